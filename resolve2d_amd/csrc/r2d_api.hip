@@ -108,7 +108,6 @@ size_t static_layout(char* base, StepDev* S, WorldDev** desc)
     take(&F.ent_cnt, (E + 1) * 4); take(&F.ent_off, (E + 1) * 4);
     take(&F.cand, (R + 1) * 16);
     take(&F.cand_flag, (R + 1) * 4); take(&F.cand_idx, (R + 1) * 4);
-    take(&F.sat_nx, (R + 1) * 4); take(&F.sat_ny, (R + 1) * 4); take(&F.sat_info, (R + 1) * 4);
     take(&F.m_ref, M * 4); take(&F.m_inc, M * 4);
     take(&F.m_nx, M * 4); take(&F.m_ny, M * 4); take(&F.m_fric, M * 4);
     take(&F.m_prev1, M * 4); take(&F.m_prev2, M * 4); take(&F.m_valid, M * 4);
@@ -118,8 +117,10 @@ size_t static_layout(char* base, StepDev* S, WorldDev** desc)
     take(&F.it_r0, I * 4); take(&F.it_r1, I * 4); take(&F.it_k0, I * 4); take(&F.it_k1, I * 4);
     take(&F.deg, (N + 1) * 4); take(&F.deg_off, (N + 1) * 4); take(&F.deg_fill, (N + 1) * 4);
     take(&F.lists, 2 * I * 4);
-    take(&F.it_color, I * 4); take(&F.it_perm, I * 4);
     take(&F.recs, I * 128);
+    take(&F.prog_rows, CHAIN_ITERS_MAX * I * 8); take(&F.prog_entries, 2 * CHAIN_ITERS_MAX * I * 4);
+    take(&F.prog_slots, CHAIN_ITERS_MAX * I * 8);
+    take(&F.plan_items, I * 16); take(&F.plan_ring, 2 * I * 16);
     take(&F.cmask, 2 * N * 8);
     take(&F.g_im, N * 4); take(&F.g_ii, N * 4); take(&F.g_cnt, N * 4);
     take(&F.cmap, N * 4); take(&F.cinv, N * 4); take(&F.w_nc, (W + 1) * 4);
@@ -285,6 +286,7 @@ struct r2d_ctx {
     void* farena = nullptr;                       // the worlds' slices (entries, candidates, manifolds, items)
     size_t farena_bytes = 0;
     uint32_t fcap_e = 0, fcap_r = 0, fcap_m = 0, fcap_i = 0;   // slice totals the arena holds
+    uint32_t fcap_k = 0;                          // ... and iterations per program
     void* fworld = nullptr;                       // per-world arrays of the fused kernel
     size_t fworld_cap = 0;
     StepDev SF{};                                 // the fused kernel's view: S with the slice arrays in farena
@@ -762,12 +764,13 @@ uint32_t grow_cap(uint32_t have, uint64_t need)
 // The fused arena: every world's slices of the entry, candidate, manifold and
 // item arrays.  With `preserve` the manifold arrays keep their contents (the
 // slices of worlds that finished before an overflow relaunch stay readable).
-int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64_t ti, bool preserve)
+int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64_t ti, uint32_t iters, bool preserve)
 {
-    if (te <= c->fcap_e && tr <= c->fcap_r && tm <= c->fcap_m && ti <= c->fcap_i && c->farena) return R2D_OK;
+    if (te <= c->fcap_e && tr <= c->fcap_r && tm <= c->fcap_m && ti <= c->fcap_i && iters <= c->fcap_k && c->farena)
+        return R2D_OK;
     if (std::max(std::max(te, tr), std::max(tm, ti)) >= 0x7fffff00ull) return R2D_E_CAPACITY;
     const uint32_t E = grow_cap(c->fcap_e, te), R = grow_cap(c->fcap_r, tr), M = grow_cap(c->fcap_m, tm),
-                   I = grow_cap(c->fcap_i, ti);
+                   I = grow_cap(c->fcap_i, ti), K = std::max(c->fcap_k, iters);
     StepDev F{};
     std::vector<std::pair<void**, size_t>> parts;
     auto add = [&](void** p, size_t bytes) { parts.push_back({p, bytes}); };
@@ -775,16 +778,17 @@ int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64
     add((void**)&F.ent_body, (size_t)E * 4); add((void**)&F.ent_bkt, (size_t)E * 4);
     add((void**)&F.ent_cnt, (size_t)E * 4);
     add((void**)&F.cand, (size_t)R * 16); add((void**)&F.cand_flag, (size_t)R * 4);
-    add((void**)&F.sat_nx, (size_t)R * 4); add((void**)&F.sat_ny, (size_t)R * 4); add((void**)&F.sat_info, (size_t)R * 4);
     add((void**)&F.m_ref, (size_t)M * 4); add((void**)&F.m_inc, (size_t)M * 4);
     add((void**)&F.m_nx, (size_t)M * 4); add((void**)&F.m_ny, (size_t)M * 4); add((void**)&F.m_fric, (size_t)M * 4);
     add((void**)&F.m_prev1, (size_t)M * 4); add((void**)&F.m_prev2, (size_t)M * 4); add((void**)&F.m_valid, (size_t)M * 4);
     add((void**)&F.m_pt, (size_t)MP_NFIELDS * 2 * M * 4);
     add((void**)&F.it_r0, (size_t)I * 4); add((void**)&F.it_r1, (size_t)I * 4);
     add((void**)&F.it_k0, (size_t)I * 4); add((void**)&F.it_k1, (size_t)I * 4);
-    add((void**)&F.it_perm, (size_t)I * 4);
     add((void**)&F.lists, 2 * (size_t)I * 4);
     add((void**)&F.recs, (size_t)I * 128);
+    add((void**)&F.prog_rows, (size_t)K * I * 8); add((void**)&F.prog_entries, 2 * (size_t)K * I * 4);
+    add((void**)&F.prog_slots, (size_t)K * I * 8);
+    add((void**)&F.plan_items, (size_t)I * 16); add((void**)&F.plan_ring, 2 * (size_t)I * 16);
     size_t bytes = 0;
     for (auto& p : parts) bytes += align256(p.second);
     void* arena = nullptr;
@@ -808,13 +812,14 @@ int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64
     }
     c->farena = arena;
     c->farena_bytes = bytes;
-    c->fcap_e = E; c->fcap_r = R; c->fcap_m = M; c->fcap_i = I;
+    c->fcap_e = E; c->fcap_r = R; c->fcap_m = M; c->fcap_i = I; c->fcap_k = K;
     O.bkt_items = F.bkt_items; O.bkt_sorted = F.bkt_sorted; O.ent_body = F.ent_body; O.ent_bkt = F.ent_bkt;
-    O.ent_cnt = F.ent_cnt; O.cand = F.cand; O.cand_flag = F.cand_flag; O.sat_nx = F.sat_nx; O.sat_ny = F.sat_ny;
-    O.sat_info = F.sat_info; O.m_ref = F.m_ref; O.m_inc = F.m_inc; O.m_nx = F.m_nx; O.m_ny = F.m_ny;
+    O.ent_cnt = F.ent_cnt; O.cand = F.cand; O.cand_flag = F.cand_flag; O.m_ref = F.m_ref; O.m_inc = F.m_inc; O.m_nx = F.m_nx; O.m_ny = F.m_ny;
     O.m_fric = F.m_fric; O.m_prev1 = F.m_prev1; O.m_prev2 = F.m_prev2; O.m_valid = F.m_valid; O.m_pt = F.m_pt;
-    O.it_r0 = F.it_r0; O.it_r1 = F.it_r1; O.it_k0 = F.it_k0; O.it_k1 = F.it_k1; O.it_perm = F.it_perm;
+    O.it_r0 = F.it_r0; O.it_r1 = F.it_r1; O.it_k0 = F.it_k0; O.it_k1 = F.it_k1;
     O.lists = F.lists; O.recs = F.recs;
+    O.prog_rows = F.prog_rows; O.prog_entries = F.prog_entries; O.prog_slots = F.prog_slots;
+    O.plan_items = F.plan_items; O.plan_ring = F.plan_ring;
     O.cap_e = E; O.cap_r = R; O.cap_m = M; O.cap_i = I;
     return R2D_OK;
 }
@@ -925,7 +930,7 @@ int fused_layout(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += cap[3];
     }
     // as much again free for worlds that outgrow their slices during the call
-    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, false))) return rc;
+    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, chain_iters(b.iters), false))) return rc;
     // workgroups take the largest worlds first (the longest steps start first)
     c->forder.resize(nw);
     for (size_t i = 0; i < nw; ++i) c->forder[i] = (uint32_t)i;
@@ -965,7 +970,7 @@ int fused_regrow(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += cap[3];
         c->hstatus[i] = WS_OK;
     }
-    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, true);
+    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, chain_iters(b.iters), true);
     if (rc) return rc;
     if ((rc = fused_upload_tables(c))) return rc;
     HIPCHK(hipMemcpyAsync(c->S.w_status, c->hstatus, nw * 4, hipMemcpyHostToDevice, c->stream));
@@ -1031,11 +1036,12 @@ StepDev fused_view(const r2d_ctx* c)
     StepDev F = c->S;
     const StepDev& O = c->SF;
     F.bkt_items = O.bkt_items; F.bkt_sorted = O.bkt_sorted; F.ent_body = O.ent_body; F.ent_bkt = O.ent_bkt;
-    F.ent_cnt = O.ent_cnt; F.cand = O.cand; F.cand_flag = O.cand_flag; F.sat_nx = O.sat_nx; F.sat_ny = O.sat_ny;
-    F.sat_info = O.sat_info; F.m_ref = O.m_ref; F.m_inc = O.m_inc; F.m_nx = O.m_nx; F.m_ny = O.m_ny;
+    F.ent_cnt = O.ent_cnt; F.cand = O.cand; F.cand_flag = O.cand_flag; F.m_ref = O.m_ref; F.m_inc = O.m_inc; F.m_nx = O.m_nx; F.m_ny = O.m_ny;
     F.m_fric = O.m_fric; F.m_prev1 = O.m_prev1; F.m_prev2 = O.m_prev2; F.m_valid = O.m_valid; F.m_pt = O.m_pt;
-    F.it_r0 = O.it_r0; F.it_r1 = O.it_r1; F.it_k0 = O.it_k0; F.it_k1 = O.it_k1; F.it_perm = O.it_perm;
+    F.it_r0 = O.it_r0; F.it_r1 = O.it_r1; F.it_k0 = O.it_k0; F.it_k1 = O.it_k1;
     F.lists = O.lists; F.recs = O.recs;
+    F.prog_rows = O.prog_rows; F.prog_entries = O.prog_entries; F.prog_slots = O.prog_slots;
+    F.plan_items = O.plan_items; F.plan_ring = O.plan_ring;
     F.cap_e = O.cap_e; F.cap_r = O.cap_r; F.cap_m = O.cap_m; F.cap_i = O.cap_i;
     F.wscr = O.wscr; F.fpool = O.fpool; F.w_done = O.w_done; F.w_cnt = O.w_cnt; F.w_man_begin = O.w_man_begin;
     F.w_man_end = O.w_man_end; F.w_order = O.w_order;
@@ -1112,7 +1118,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         maxtb = std::max(maxtb, b.descs[i].table);
     }
     if (fused) {
-        b.fused_lds = fused_lds_bytes(maxn, maxtb, fused_slots(variant), fused_threads(variant));
+        b.fused_lds = fused_lds_bytes(maxn, maxtb);
         fused = b.fused_lds <= kFusedLdsMax;
     }
     b.fused = fused;
@@ -1238,6 +1244,7 @@ int fused_launch(r2d_ctx* c, Batch& b)
     StepDev F = fused_view(c);
     F.nb = (uint32_t)b.N; F.nworlds = (uint32_t)nw; F.nbuckets = (uint32_t)b.B; F.njoints = (uint32_t)b.J;
     F.worlds = c->dworlds;
+    F.chain_iters = chain_iters(b.iters);
     if (c->profiling) {
         // The timing buffers grow rarely and by a lot: a launch that follows a
         // hipMalloc closely can stall all of its waves for several ms at once
@@ -2049,12 +2056,8 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
             if (w->slot_of(h.id1) < 0 || (h.type <= 1 && w->slot_of(h.id2) < 0)) return R2D_E_INVALID_ID;
     int variant = c->solve_variant >= 0 ? c->solve_variant : default_variant(1);
     if (!fused_available(variant)) variant = 11;
-    size_t lds = fused_lds_bytes(n, tb, fused_slots(variant), fused_threads(variant));
-    if (lds > kFusedLdsMax) {
-        variant = 11;
-        lds = fused_lds_bytes(n, tb, fused_slots(variant), fused_threads(variant));
-        if (lds > kFusedLdsMax) return R2D_E_CAPACITY;
-    }
+    const size_t lds = fused_lds_bytes(n, tb);
+    if (lds > kFusedLdsMax) return R2D_E_CAPACITY;
     if (n == 0) {   // nothing moves and no manifold exists
         w->epoch = 0;
         w->sepoch = 0;
@@ -2083,6 +2086,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     WorldDev* ddesc = nullptr;
     static_layout(base, &F, &ddesc);
     F.nb = n; F.nbuckets = tb; F.njoints = nj;
+    F.chain_iters = chain_iters(iters);
     // host values the asynchronous uploads read; the call waits for the
     // stream before they go out of scope
     WorldDev d = w->desc;

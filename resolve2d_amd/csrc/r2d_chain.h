@@ -1,0 +1,680 @@
+// The solver's chain as a program: the K iterations of a sub-step's items
+// (constraints, then manifolds) laid out ahead of time in rows of at most 64
+// lanes, which the waves then run one after another.
+//
+// The reference's solver is sequential: an item may run once every earlier
+// item on its ordering bodies has run.  That partial order is the same in
+// every sub-step of a step, so it is worked out once per step (plan_*: the
+// items ready now make the next rows, which release their successors) and
+// the sub-steps replay the rows (chain_call).  A row's lanes share no
+// ordering body and every body meets its items in the reference's order, so
+// the bits are the sequential loop's.  Nothing polls: a world whose rows all
+// fit one wave runs them in program order, LDS serving one wave's operations
+// in the order they are issued, and wider worlds put a workgroup barrier
+// between rows.
+//
+// What bounds it is the length of the dependency chain times one row: two LDS
+// reads, about 90 VALU instructions and an LDS write.  Lanes hold contact
+// points, not items: the points of a two-point manifold sit in neighbouring
+// lanes (the reference computes both from the same momenta and adds their
+// impulses up afterwards), which halves the instructions of a row, and a
+// one-point manifold (discs) costs one lane.  The 64-byte record of a row's
+// points is fetched from L2 while the two rows before it run.
+#pragma once
+
+#include "r2d_device.h"
+
+namespace r2d {
+
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+#define R2D_LDS __attribute__((address_space(3)))
+#define R2D_GLB __attribute__((address_space(1)))
+typedef R2D_LDS uint32_t* LU32;
+typedef R2D_LDS uint16_t* LU16;
+typedef R2D_LDS u2v* LU2;
+typedef R2D_LDS f2v* LF2;
+typedef R2D_LDS float* LF;
+typedef R2D_GLB f2v* GF2;
+typedef R2D_GLB uint32_t* GU32;
+typedef R2D_GLB u2v* GU2;
+typedef R2D_GLB u4v* GU4;
+typedef const R2D_GLB uint32_t* GCU32;
+typedef const R2D_GLB u2v* GCU2;
+typedef const R2D_GLB u4v* GCU4;
+
+// ------------------------------------------------------------ point records
+// 16 words.  Words 0 and 1: the two bodies and flags.
+//   contact point: 2-3 normal, 4 friction, 5 Baumgarte bias of the sub-step
+//     (-1: depth >= 0), 6-9 lever arms r1 r2, 10 / 11 effective masses
+//     (normal, tangent), 12-13 inverse masses, 14-15 inverse inertias
+//   distance joint (type 0): 2-3 direction, 4 position term, 5 / 6 power
+//     limits (min, max), 12-13 inverse masses
+//   offset distance joint (1): the same, 7-10 rotated offsets, 11 denominator,
+//     14-15 inverse inertias
+//   fixed position (2): 2-3 direction, 4 bias, 5 / 6 limits, 12 inverse mass
+//   motor (3): 2 inertia, 3 target, 4 beta, 5 / 6 limits, 7 torque
+constexpr uint32_t PR_INDEX = (1u << 26) - 1u;
+enum : uint32_t {
+    // word 0
+    PR_JOINT = 1u << 26,
+    PR_WRITE_A = 1u << 27,    // body a is an ordering body: its momentum is written
+    PR_STATIC_A = 1u << 28,   // ... though static (it gets "+= 0")
+    PR_ON = 1u << 29,         // the point exists (a manifold may have none)
+    PR_PAIR = 1u << 30,       // one of two points; the first sits in the even lane
+    PR_SECOND = 1u << 31,
+    // word 1
+    PR_WRITE_B = 1u << 26,
+    PR_STATIC_B = 1u << 27,
+    PR_WARM = 1u << 28,       // contact: warm started (no minimum impulse)
+    PR_SELF = 1u << 28,       // joint: both ends on one body
+    PR_SKIP = 1u << 29,       // joint: changes nothing this sub-step
+    PR_TYPE_SHIFT = 30        // joint type
+};
+
+__device__ __forceinline__ float asf(uint32_t x) { return __uint_as_float(x); }
+__device__ __forceinline__ uint32_t asu(float x) { return __float_as_uint(x); }
+
+// ------------------------------------------------------------------ planning
+// One successor of an item on an ordering body: the next item of the body's
+// list, or its first item in the next iteration (wrap).
+//
+// Planning state of a world in LDS, 16 bytes per item: succ (both successors,
+// 15-bit items with a wrap bit, NO_ITEM for none), state (16 bits: ordering
+// bodies still waited for, pair bit, iteration from bit 3), second (the second
+// point's index of a pair) and a ring of ready items (x: item | pair << 15 |
+// iteration << 16, y: its succ word).  Worlds that do not fit, or with more
+// items than 15 bits, keep the same in global memory (PlanGlb).
+constexpr uint32_t PLAN_MAX_ITEMS = 0x7ffe;
+constexpr uint32_t NO_ITEM16 = 0x7fffu;
+
+struct PlanEntry {
+    uint32_t item, iter, s0, s1;   // s0, s1: successor | wrap << 31, NO_ITEM for none
+    bool pair;
+};
+constexpr uint32_t NO_ITEM = 0x7fffffffu;
+constexpr uint32_t WRAP = 0x80000000u;
+
+__host__ __device__ constexpr uint32_t plan_ring(uint32_t nit, uint32_t waves) { return nit + 64u * waves; }
+// LDS words of PlanLds
+__host__ __device__ constexpr uint32_t plan_lds_words(uint32_t nit, uint32_t waves)
+{
+    return nit + 2u * ((nit + 1u) / 2u) + 2u * plan_ring(nit, waves) + 1u;
+}
+
+struct PlanLds {
+    LU32 succ, state;
+    LU16 second;
+    LU2 ring;
+    uint32_t ring_n;
+
+    __device__ __forceinline__ PlanLds(LU32 p, uint32_t nit, uint32_t waves)
+    {
+        ring_n = plan_ring(nit, waves);
+        ring = (LU2)p;                      // p is 8-byte aligned
+        succ = p + 2u * ring_n;
+        state = succ + nit;
+        second = (LU16)(state + (nit + 1u) / 2u);
+    }
+    static __device__ __forceinline__ uint32_t pack(uint32_t s0, uint32_t s1)
+    {
+        return (s0 & 0x7fffu) | ((s0 & WRAP) >> 16) | ((s1 & 0x7fffu) << 16) | (s1 & WRAP);
+    }
+    static __device__ __forceinline__ uint32_t half(uint32_t v)
+    {
+        return (v & 0x7fffu) == NO_ITEM16 ? NO_ITEM : ((v & 0x7fffu) | ((v & 0x8000u) << 16));
+    }
+    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t need, bool pair, uint32_t p1)
+    {
+        succ[j] = pack(s0, s1);
+        ((LU16)state)[j] = (uint16_t)(need | (pair ? 4u : 0u));
+        second[j] = (uint16_t)p1;
+    }
+    __device__ __forceinline__ void push_first(uint32_t at, uint32_t j, uint32_t s0, uint32_t s1, bool pair)
+    {
+        ring[at] = u2v{j | (pair ? 0x8000u : 0u), pack(s0, s1)};
+    }
+    __device__ __forceinline__ PlanEntry read(uint32_t at) const
+    {
+        const u2v v = ring[at];
+        return PlanEntry{v.x & 0x7fffu, v.x >> 16, half(v.y & 0xffffu), half(v.y >> 16), (v.x & 0x8000u) != 0u};
+    }
+    __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e)
+    {
+        ring[at] = u2v{e.item | (e.pair ? 0x8000u : 0u) | (e.iter << 16), pack(e.s0, e.s1)};
+    }
+    __device__ __forceinline__ uint32_t second_of(uint32_t j) const { return second[j]; }
+    // the item's next iteration waits for its `nb` ordering bodies
+    __device__ __forceinline__ void reset(uint32_t j, uint32_t nb)
+    {
+        __hip_atomic_fetch_add(&state[j >> 1], (nb + 8u) << (16u * (j & 1u)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    // one of item s's bodies has reached it; true when it was the last
+    __device__ __forceinline__ bool release(uint32_t s, PlanEntry& e)
+    {
+        const uint32_t sh = 16u * (s & 1u);
+        const uint32_t old = __hip_atomic_fetch_sub(&state[s >> 1], 1u << sh, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_WORKGROUP) >> sh;
+        const uint32_t n = succ[s];
+        e.item = s;
+        e.iter = (old & 0xffffu) >> 3;
+        e.pair = (old & 4u) != 0u;
+        e.s0 = half(n & 0xffffu);
+        e.s1 = half(n >> 16);
+        return (old & 3u) == 1u;
+    }
+};
+
+// the same in global memory: items (succ 0, succ 1, state, second point), ring
+// of ready items (item | pair << 31, iteration, succ 0, succ 1)
+struct PlanGlb {
+    GU4 items, ring;
+    uint32_t ring_n;
+
+    __device__ __forceinline__ PlanGlb(GU4 items_, GU4 ring_, uint32_t nit, uint32_t waves)
+        : items(items_), ring(ring_), ring_n(plan_ring(nit, waves))
+    {
+    }
+    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t need, bool pair, uint32_t p1)
+    {
+        items[j] = u4v{s0, s1, need | (pair ? 4u : 0u), p1};
+    }
+    __device__ __forceinline__ void push_first(uint32_t at, uint32_t j, uint32_t s0, uint32_t s1, bool pair)
+    {
+        ring[at] = u4v{j | (pair ? WRAP : 0u), 0u, s0, s1};
+    }
+    __device__ __forceinline__ PlanEntry read(uint32_t at) const
+    {
+        const u4v v = ring[at];
+        return PlanEntry{v.x & ~WRAP, v.y, v.z, v.w, (v.x & WRAP) != 0u};
+    }
+    __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e)
+    {
+        ring[at] = u4v{e.item | (e.pair ? WRAP : 0u), e.iter, e.s0, e.s1};
+    }
+    __device__ __forceinline__ uint32_t second_of(uint32_t j) const { return items[j].w; }
+    __device__ __forceinline__ GU32 state_of(uint32_t j) const { return (GU32)(items + j) + 2; }
+    __device__ __forceinline__ void reset(uint32_t j, uint32_t nb)
+    {
+        __hip_atomic_fetch_add(state_of(j), nb + 8u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ bool release(uint32_t s, PlanEntry& e)
+    {
+        const uint32_t old = __hip_atomic_fetch_sub(state_of(s), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        e.item = s;
+        e.iter = old >> 3;
+        e.pair = (old & 4u) != 0u;
+        e.s0 = items[s].x;
+        e.s1 = items[s].y;
+        return (old & 3u) == 1u;
+    }
+};
+
+// A world's program: rows (first entry, entries), the entries (point
+// indices: item j's first point is j, second points follow after the items),
+// and for worlds run by several waves the first row and the rows of each slot
+// (rows of one slot run side by side, one per wave).
+struct Program {
+    GU2 rows;
+    GU32 entries;
+    GU2 slots;
+};
+
+// A world's solve in LDS: what it works on (set by one thread), and the shared
+// words of planning.
+struct ChainShared {
+    uint32_t w, ibase, mbeg, nj, M, base, sub_steps, iters;
+    float dt;
+    uint32_t free_at, free_words;   // LDS from this word on is the solve's
+    uint32_t ready, pairs, live, nslots, failed, taken, entries, queued[3];
+};
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+// The arguments of an out-of-line function arrive in vector registers: what is
+// the same in every lane goes back to scalar ones.
+template <class P>
+__device__ __forceinline__ P uniform_ptr(P p)
+{
+    const uint64_t x = (uint64_t)p;
+    return (P)(((uint64_t)uniform((uint32_t)(x >> 32)) << 32) | uniform((uint32_t)x));
+}
+template <class P>
+__device__ __forceinline__ P uniform_lds(P p)
+{
+    return (P)(uintptr_t)uniform((uint32_t)(uintptr_t)p);
+}
+
+// One round of one wave: takes ready items from ring place `first` on (at most
+// `avail`, 64 lanes of points), writes their row's entries at `entry0` with
+// pairs in the lower lanes, and releases their successors.  Returns the items
+// taken; `lanes` gets the row's entries and the released items stay in e0 / e1
+// (r0 / r1: whether the lane released one).
+struct Round {
+    uint32_t taken, lanes;
+    bool left;                // this lane holds a ready item that did not fit the row
+    PlanEntry self, e0, e1;
+    bool r0, r1;
+};
+
+template <class PLAN>
+__device__ __forceinline__ Round plan_take(PLAN& P, uint32_t first, uint32_t avail, uint32_t lane)
+{
+    Round R;
+    const bool act = lane < avail;
+    uint32_t at = first + (act ? lane : 0u);
+    if (at >= P.ring_n) at -= P.ring_n;
+    R.self = P.read(at);
+    const bool pair = act && R.self.pair;
+    const uint64_t pm = __ballot(pair);
+    const uint32_t end = lane + 1u + lanes_below(pm) + (pair ? 1u : 0u);   // lanes used through this item
+    const bool take = act && end <= 64u;
+    R.taken = (uint32_t)__popcll(__ballot(take));
+    R.lanes = R.taken + (uint32_t)__popcll(__ballot(take && pair));
+    R.left = act && !take;
+    return R;
+}
+
+template <class PLAN>
+__device__ __forceinline__ void plan_run(PLAN& P, Round& R, GU32 entries, uint32_t entry0, uint32_t iters, uint32_t lane)
+{
+    const bool take = lane < R.taken;
+    const bool pair = take && R.self.pair;
+    const uint64_t pm = __ballot(pair);
+    const uint32_t below = lanes_below(pm), pairs = (uint32_t)__popcll(pm);
+    R.r0 = R.r1 = false;
+    if (take) {
+        const uint32_t j = R.self.item;
+        P.reset(j, R.self.s1 == NO_ITEM ? 1u : 2u);
+        const bool last = R.self.iter + 1u == iters;
+        if (R.self.s0 != NO_ITEM && !(last && (R.self.s0 & WRAP))) R.r0 = P.release(R.self.s0 & ~WRAP, R.e0);
+        if (R.self.s1 != NO_ITEM && !(last && (R.self.s1 & WRAP))) R.r1 = P.release(R.self.s1 & ~WRAP, R.e1);
+        const uint32_t pos = entry0 + (pair ? 2u * below : 2u * pairs + (lane - below));
+        entries[pos] = j;
+        if (pair) entries[pos + 1u] = P.second_of(j);
+    }
+}
+
+template <class PLAN>
+__device__ __forceinline__ void plan_put(PLAN& P, const Round& R, uint32_t at)
+{
+    const uint64_t m0 = __ballot(R.r0), m1 = __ballot(R.r1), m2 = __ballot(R.left);
+    const uint32_t c0 = (uint32_t)__popcll(m0), c1 = (uint32_t)__popcll(m1);
+    auto place = [&](uint32_t k) { return k >= P.ring_n ? k - P.ring_n : k; };
+    if (R.left) P.push(place(at + lanes_below(m2)), R.self);
+    const uint32_t c2 = (uint32_t)__popcll(m2);
+    if (R.r0) P.push(place(at + c2 + lanes_below(m0)), R.e0);
+    if (R.r1) P.push(place(at + c2 + c0 + lanes_below(m1)), R.e1);
+    (void)c1;
+}
+
+// The program of a world run by one wave, planned by one wave without
+// barriers; `ready` items are in the ring.  Returns the rows (0: the ordering
+// data was corrupt).
+template <class PLAN>
+__device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint32_t nit, uint32_t iters, uint32_t ready)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
+    const uint32_t total = nit * iters;
+    while (done < total && count) {
+        Round R = plan_take(P, head, count < 64u ? count : 64u, lane);
+        R.left = false;                  // stays at the head of the ring
+        if (lane == 0) G.rows[row] = u2v{entry, R.lanes};
+        plan_run(P, R, G.entries, entry, iters, lane);
+        uint32_t tail = head + count;
+        if (tail >= P.ring_n) tail -= P.ring_n;
+        plan_put(P, R, tail);
+        asm volatile("" ::: "memory");   // the next round reads what this one wrote (LDS order)
+        const uint32_t added = (uint32_t)(__popcll(__ballot(R.r0)) + __popcll(__ballot(R.r1)));
+        head += R.taken;
+        if (head >= P.ring_n) head -= P.ring_n;
+        count += added - R.taken;
+        done += R.taken;
+        entry += R.lanes;
+        row += 1u;
+    }
+    return done == total ? row : 0u;
+}
+
+// The program of a world run by `waves` waves of the workgroup, planned by
+// all of them: wave w takes the w-th 64 ready items.  Items that do not fit
+// a row go back to the end of the ring.  A barrier per slot; called by the
+// whole workgroup.  sh.taken, sh.entries, sh.queued start at 0.
+template <class PLAN>
+__device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32_t nit, uint32_t iters, uint32_t ready,
+                                               uint32_t waves, ChainShared& sh)
+{
+    const uint32_t lane = threadIdx.x & 63u, wv = uniform(threadIdx.x >> 6);
+    uint32_t head = 0, count = ready, row = 0, slot = 0;
+    const uint32_t limit = nit * iters;
+    for (; count && slot < limit; ++slot) {
+        const uint32_t want = (count + 63u) / 64u, nrows = want < waves ? want : waves;
+        const uint32_t round = slot % 3u;
+        uint32_t tail = head + count;
+        if (tail >= P.ring_n) tail -= P.ring_n;
+        if (threadIdx.x == 0) {
+            G.slots[slot] = u2v{row, nrows};
+            // every wave read it (as slot - 2's count) before the last barrier; it is added to after the next
+            sh.queued[(slot + 1u) % 3u] = 0u;
+        }
+        if (wv < nrows) {
+            const uint32_t rest = count - 64u * wv;
+            uint32_t first = head + 64u * wv;
+            if (first >= P.ring_n) first -= P.ring_n;
+            Round R = plan_take(P, first, rest < 64u ? rest : 64u, lane);
+            uint32_t e0 = 0u;
+            if (lane == 0) {
+                e0 = __hip_atomic_fetch_add(&sh.entries, R.lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(&sh.taken, R.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                G.rows[row + wv] = u2v{e0, R.lanes};
+            }
+            e0 = uniform(e0);
+            plan_run(P, R, G.entries, e0, iters, lane);
+            const uint32_t add = (uint32_t)(__popcll(__ballot(R.r0)) + __popcll(__ballot(R.r1)) + __popcll(__ballot(R.left)));
+            uint32_t at = 0u;
+            if (lane == 0)
+                at = __hip_atomic_fetch_add(&sh.queued[round], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            at = uniform(at) + tail;
+            if (at >= P.ring_n) at -= P.ring_n;
+            plan_put(P, R, at);
+        }
+        __syncthreads();
+        const uint32_t used = count < 64u * nrows ? count : 64u * nrows;
+        head += used;
+        if (head >= P.ring_n) head -= P.ring_n;
+        count = count - used + uniform(sh.queued[round]);
+        row += nrows;
+    }
+    __syncthreads();
+    return sh.taken == limit ? slot : 0u;
+}
+
+// Waves that run a world's rows: one while the items fill about as many rows
+// of 64 as a pile's chain is deep (90-150 for 4 iterations), more for larger
+// worlds, whose slots then cost a barrier each.
+constexpr uint32_t CHAIN_WAVE_ROWS = 96;
+__host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, uint32_t most)
+{
+    const uint32_t w = (uint32_t)(((uint64_t)nit * iters / 64u + CHAIN_WAVE_ROWS - 1u) / CHAIN_WAVE_ROWS);
+    return w < 1u ? 1u : (w < most ? w : most);
+}
+
+// ----------------------------------------------------------------- the chain
+// momenta of a world's bodies in LDS
+struct LdsMomenta {
+    LF2 m;
+    LF l;
+    __device__ __forceinline__ void get(uint32_t i, v2& p, float& L) const
+    {
+        const f2v v = m[i];
+        p = mk(v.x, v.y);
+        L = l[i];
+    }
+    __device__ __forceinline__ void put(uint32_t i, v2 p, float L) const
+    {
+        m[i] = f2v{p.x, p.y};
+        l[i] = L;
+    }
+};
+
+// x of the other lane of an even / odd pair
+__device__ __forceinline__ float pair_other(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, false));
+}
+
+// Constraint.solve (Constraints/*.zig) from a joint record
+template <class ST>
+__device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, const ST& st, float dt)
+{
+    const uint32_t type = q0.y >> PR_TYPE_SHIFT, a = q0.x & PR_INDEX, b = q0.y & PR_INDEX;
+    if (q0.y & PR_SKIP) return;
+    const bool self = (q0.y & PR_SELF) != 0u;
+    const float pmin = asf(q1.y), pmax = asf(q1.z);
+    v2 m1;
+    float L1;
+    st.get(a, m1, L1);
+    if (type <= 1u) {
+        v2 m2;
+        float L2;
+        st.get(b, m2, L2);
+        const v2 n = mk(asf(q0.z), asf(q0.w));
+        const float pc = asf(q1.x), im1 = asf(q3.x), im2 = asf(q3.y);
+        v2 dp;
+        if (type == 0u) {
+            // DistanceJoint.solve (DistanceJoint.zig:40-75)
+            const v2 rv = sub2(scale2(m2, im2), scale2(m1, im1));
+            float Jv = -(dot2(rv, n) + pc) / (im1 + im2);
+            const float den = 1.0f / maxn(absf(dot2(n, rv)), GRAD_DIV_LIMIT);
+            Jv = clampn(Jv, pmin * den, pmax * den);
+            dp = scale2(n, Jv);
+            m1 = sub2(m1, dp);
+            m2 = add2(self ? m1 : m2, dp);
+        } else {
+            // OffsetDistanceJoint.solve (OffsetDistanceJoint.zig:44-105)
+            const v2 rr1 = mk(asf(q1.w), asf(q2.x)), rr2 = mk(asf(q2.y), asf(q2.z));
+            const float ii1 = asf(q3.z), ii2 = asf(q3.w);
+            const float w1 = L1 * ii1, w2 = L2 * ii2;
+            const v2 v1 = add2(scale2(m1, im1), mk(-rr1.y * w1, rr1.x * w1));
+            const v2 v2v = add2(scale2(m2, im2), mk(-rr2.y * w2, rr2.x * w2));
+            const v2 dv = sub2(v2v, v1);
+            const float num = dot2(n, dv) + pc;
+            const float r1xn = cross2(rr1, n), r2xn = cross2(rr2, n);
+            float Jv = -num / asf(q2.w);
+            const float den = 1.0f / maxn(absf(dot2(n, dv)), GRAD_DIV_LIMIT);
+            Jv = clampn(Jv, pmin * den, pmax * den);
+            dp = scale2(n, Jv);
+            m1 = sub2(m1, dp);
+            L1 = L1 - Jv * r1xn;
+            m2 = add2(self ? m1 : m2, dp);
+            L2 = (self ? L1 : L2) + Jv * r2xn;
+        }
+        if (self) {
+            st.put(a, m2, type == 0u ? L1 : L2);
+        } else {
+            st.put(a, m1, L1);
+            st.put(b, m2, L2);
+        }
+    } else if (type == 2u) {
+        // FixedPositionJoint.solve (FixedPositionJoint.zig:38-72)
+        const float w = asf(q3.x);
+        const v2 n = mk(asf(q0.z), asf(q0.w));
+        const float rv = dot2(scale2(m1, w), n);
+        float Jv = -(rv - asf(q1.x)) / w;
+        const float den = 1.0f / maxn(absf(rv), ALLOWED_CONSTRAINT_VALUE);
+        Jv = clampn(Jv, pmin * den, pmax * den);
+        st.put(a, add2(m1, scale2(n, Jv)), L1);
+    } else {
+        // MotorJoint.solve (MotorJoint.zig:38-64)
+        const float I = asf(q0.z);
+        const float C = L1 / I - asf(q0.w);
+        if (absf(C) < ALLOWED_CONSTRAINT_VALUE) return;
+        const float bias = asf(q1.x) * C;
+        const float tq = asf(q1.w);
+        float Jv = tq - bias;
+        const float den = 1.0f / maxn(absf(tq / I), ALLOWED_CONSTRAINT_VALUE);
+        Jv = clampn(Jv, pmin * den, pmax * den);
+        st.put(a, m1, L1 + Jv * dt);
+    }
+}
+
+// CollisionManifold.calculateImpulses (collision.zig:135-218), one point per
+// lane.  Both points of a manifold work from the same momenta and their
+// impulses are added in point order, so the lane of the first point takes the
+// second's from its neighbour and writes the bodies.
+template <bool WARM, class ST, class ACC>
+__device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, const ST& st,
+                                              ACC acc)
+{
+    const uint32_t fa = q0.x, fb = q0.y, a = fa & PR_INDEX, b = fb & PR_INDEX;
+    v2 m1, m2;
+    float L1, L2;
+    st.get(a, m1, L1);
+    st.get(b, m2, L2);
+    const f2v old = *acc;
+    const v2 n = mk(asf(q0.z), asf(q0.w)), t = rot90cw(n);
+    const float fric = asf(q1.x), bias = asf(q1.y);
+    const v2 r1 = mk(asf(q1.z), asf(q1.w)), r2 = mk(asf(q2.x), asf(q2.y));
+    const float om1 = L1 * asf(q3.z), om2 = L2 * asf(q3.w);
+    const v2 v1 = add2(scale2(m1, asf(q3.x)), mk(-r1.y * om1, r1.x * om1));
+    const v2 v2v = add2(scale2(m2, asf(q3.y)), mk(-r2.y * om2, r2.x * om2));
+    const v2 dv = sub2(v1, v2v);
+    const float pn = (dot2(dv, n) + bias) * asf(q2.z);
+    const float pt = dot2(dv, t) * asf(q2.w);
+    const bool on = (fa & PR_ON) != 0u, sep = bias < 0.f;
+    const bool go = on && !sep && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (fb & PR_WARM) != 0u));
+    const float new_pn = maxn(0.0f, old.x + pn);
+    const float max_pt = fric * absf(new_pn);
+    const float new_pt = clampn(old.y + pt, -max_pt, max_pt);
+    const float apn = new_pn - old.x, apt = new_pt - old.y;
+    const bool clr = on && sep;
+    *acc = f2v{clr ? 0.f : (go ? new_pn : old.x), clr ? 0.f : (go ? new_pt : old.y)};
+    v2 dp = add2(scale2(n, apn), scale2(t, apt));
+    float c1 = cross2(r1, dp), c2 = cross2(r2, dp);
+    // a point that does nothing adds +0, which changes none of the sums below
+    // (0 - x and 0 + x are never -0)
+    dp.x = go ? dp.x : 0.f; dp.y = go ? dp.y : 0.f;
+    c1 = go ? c1 : 0.f; c2 = go ? c2 : 0.f;
+    float a1x = 0.f - dp.x, a1y = 0.f - dp.y, g1 = 0.f - c1;
+    float a2x = 0.f + dp.x, a2y = 0.f + dp.y, g2 = 0.f + c2;
+    if (fa & PR_PAIR) {
+        const float ox = pair_other(dp.x), oy = pair_other(dp.y), o1 = pair_other(c1), o2 = pair_other(c2);
+        a1x = a1x - ox; a1y = a1y - oy; g1 = g1 - o1;
+        a2x = a2x + ox; a2y = a2y + oy; g2 = g2 + o2;
+    }
+    if (fa & PR_STATIC_A) { a1x = 0.f; a1y = 0.f; g1 = 0.f; }
+    if (fb & PR_STATIC_B) { a2x = 0.f; a2y = 0.f; g2 = 0.f; }
+    const bool lead = !(fa & PR_SECOND);
+    if (lead && (fa & PR_WRITE_A)) st.put(a, mk(m1.x + a1x, m1.y + a1y), L1 + g1);
+    if (lead && (fb & PR_WRITE_B)) st.put(b, mk(m2.x + a2x, m2.y + a2y), L2 + g2);
+}
+
+// Runs a program: `nslots` slots, `reps` times over.  MULTI: the workgroup's
+// waves run the rows of a slot side by side, a workgroup barrier after each
+// slot (every wave of the workgroup calls it).
+//
+// A row is reached through loads that each need the one before (slot, row,
+// entry, record), all in L2: every stage runs two slots ahead of the stage
+// that uses it, so that a load has two slots' time to arrive.  Three buffers
+// a stage, the loop unrolled by three: a buffer is never copied while its
+// load is in flight.
+template <class T>
+struct InLds {
+    static constexpr bool value = false;
+};
+template <>
+struct InLds<LF2> {
+    static constexpr bool value = true;
+};
+template <>
+struct InLds<LdsMomenta> {
+    static constexpr bool value = true;
+};
+
+template <bool MULTI, bool WARM, class ST, class ACC>
+__device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, const ST& st, ACC acc,
+                                          uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+{
+    constexpr bool LDS_ONLY = InLds<ST>::value && InLds<ACC>::value;
+    rows = uniform_ptr(rows); entries = uniform_ptr(entries); slots = uniform_ptr(slots); recs = uniform_ptr(recs);
+    nslots = uniform(nslots); reps = uniform(reps); nj = uniform(nj);
+    const uint32_t lane = threadIdx.x & 63u, wave = MULTI ? uniform(threadIdx.x >> 6) : 0u;
+    const uint32_t end = nslots - 1u;
+    for (uint32_t rep = 0; rep < reps; ++rep) {
+        u2v sl[3], row[3];
+        uint32_t ent[3], point[3], cnt_e[3], cnt[3];
+        bool mine[3];
+        u4v rec[3][4];
+        // each stage loads for slot s (a slot past the end repeats the last)
+        // into buffer k
+        auto load_slot = [&](uint32_t s, int k) {
+            if constexpr (MULTI) sl[k] = slots[s < end ? s : end];
+        };
+        auto load_row = [&](uint32_t s, int k) {
+            uint32_t r = s < end ? s : end;
+            mine[k] = true;
+            if constexpr (MULTI) {
+                r = uniform(sl[k].x);
+                mine[k] = wave < uniform(sl[k].y);
+                r += mine[k] ? wave : 0u;
+            }
+            row[k] = rows[r];
+        };
+        auto load_entry = [&](int k) {
+            const uint32_t c = uniform(row[k].y);
+            ent[k] = entries[uniform(row[k].x) + (lane < c ? lane : 0u)];
+            cnt_e[k] = mine[k] ? c : 0u;
+        };
+        auto load_rec = [&](int k) {
+            const GCU4 q = recs + (size_t)ent[k] * 4u;
+            rec[k][0] = q[0]; rec[k][1] = q[1]; rec[k][2] = q[2]; rec[k][3] = q[3];
+            point[k] = ent[k];
+            cnt[k] = cnt_e[k];
+        };
+        // the first loads of every stage, as the loop's iterations -8 .. -1 would issue them
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            if (p >= 6) load_rec(p - 6);
+            if (p >= 4) load_entry((p - 4) % 3);
+            if (p >= 2) load_row((uint32_t)(p - 2), (p - 2) % 3);
+            load_slot((uint32_t)p, p % 3);
+        }
+        for (uint32_t s0 = 0; s0 < nslots; s0 += 3u) {
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                const uint32_t s = s0 + u;
+                if (s >= nslots) break;
+                load_rec((u + 2) % 3);
+                load_entry((u + 4) % 3);
+                load_row(s + 6u, u);
+                load_slot(s + 8u, (u + 8) % 3);
+                __builtin_amdgcn_sched_barrier(0);
+                if (lane < cnt[u]) {
+                    const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
+                    if (q0.x & PR_JOINT) chain_joint(q0, q1, q2, q3, st, dt);
+                    else chain_contact<WARM>(q0, q1, q2, q3, st, acc + (point[u] - nj));
+                }
+                // the next slot reads what this one wrote
+                if constexpr (MULTI) {
+                    if constexpr (LDS_ONLY) {
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                        __builtin_amdgcn_s_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                    } else {
+                        __syncthreads();
+                    }
+                } else if constexpr (LDS_ONLY) {
+                    asm volatile("" ::: "memory");   // one wave's LDS operations are served in order
+                } else {
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+                }
+            }
+        }
+    }
+}
+
+// The chain on LDS momenta as an out-of-line call: its registers are then its
+// own, whatever the step kernel holds around it.  `accg`: the accumulated
+// impulses when they do not fit LDS (acc null).
+template <bool MULTI, bool WARM>
+__device__ __attribute__((noinline)) void chain_lds(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF2 m, LF l, LF2 acc,
+                                                    uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+{
+    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform_lds(l)}, uniform_lds(acc), nslots,
+                           reps, nj, dt);
+}
+template <bool MULTI, bool WARM>
+__device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF2 m, LF l,
+                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+{
+    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform_lds(l)}, uniform_ptr(acc), nslots,
+                           reps, nj, dt);
+}
+
+}  // namespace r2d

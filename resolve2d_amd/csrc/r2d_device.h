@@ -85,8 +85,9 @@ enum : int {
 // A world's slices of the step scratch when whole steps of the world run in
 // one workgroup (k_fused): cell entries [e0, e0 + ecap] (bkt_items,
 // bkt_sorted, ent_body, ent_bkt, ent_cnt), raw candidates [r0, r0 + rcap]
-// (cand, cand_flag, sat_*), manifolds [m0, m0 + mcap), solver items
-// [i0, i0 + icap) (it_*, recs) and their lists [2 i0, 2 (i0 + icap)).
+// (cand, cand_flag), manifolds [m0, m0 + mcap), solver items [i0, i0 + icap)
+// (it_*, recs, plan_items), their lists [2 i0, 2 (i0 + icap)) and the
+// solver's program at the same multiples.
 struct WorldScratch {
     uint32_t e0, ecap, r0, rcap, m0, mcap, i0, icap;
 };
@@ -147,6 +148,14 @@ struct StepDev {
     uint4* recs;                           // [8*cap_i] solver item records (128 B each)
     uint4* rmass;                          // [cap_i] worlds beyond LDS: inverse mass and inertia of each item's
                                            // two bodies (im a, ii a, im b, ii b) for the light compact chain
+    // the solver's program (r2d_chain.h): iterations one program covers, its
+    // rows and entries, and planning state when it does not fit LDS
+    uint32_t chain_iters;
+    uint2* prog_rows;                      // [chain_iters * cap_i]
+    uint32_t* prog_entries;                // [2 * chain_iters * cap_i]
+    uint2* prog_slots;                     // [chain_iters * cap_i]
+    uint4* plan_items;                     // [cap_i]
+    uint4* plan_ring;                      // [2 * cap_i]
     // global-memory solver state (worlds too large for LDS)
     float *g_im, *g_ii;
     uint32_t* g_cnt;

@@ -39,6 +39,18 @@ int solve_variant_slots(int v);
 // worlds of at most this many bodies may take the register-slot kernel
 constexpr uint32_t SLOT_NMAX = 1024;
 
+// Iterations of a sub-step that one program covers: all of them up to 16,
+// else their largest divisor up to 16 (the program is then run that often).
+// A program's size grows with the iterations it covers.
+constexpr uint32_t CHAIN_ITERS_MAX = 16;
+inline uint32_t chain_iters(size_t iters)
+{
+    if (iters == 0) return 1u;
+    for (uint32_t k = CHAIN_ITERS_MAX; k > 1u; --k)
+        if (iters % k == 0) return k;
+    return 1u;
+}
+
 // how one batch's solve phase is split over the solve kernels
 struct SolvePlan {
     int variant = 0;
@@ -100,10 +112,7 @@ void set_solve_smem_limit();
 constexpr uint32_t FUSED_NMAX = 1024;
 bool fused_available(int variant);
 // dynamic LDS of the fused kernel for a world of n bodies and tb hash buckets
-// (slots: the variant solves with register slots, else with records;
-// threads: its workgroup size, which sizes the record chain's lane slots)
-size_t fused_lds_bytes(uint32_t n, uint32_t tb, bool slots, uint32_t threads);
-bool fused_slots(int variant);
+size_t fused_lds_bytes(uint32_t n, uint32_t tb);
 uint32_t fused_threads(int variant);
 // one workgroup per world (S.w_order), up to nsteps steps per world (S.w_done)
 // the fused kernel of a variant as compiled (registers, LDS, scratch): for error reports

@@ -27,6 +27,7 @@
 #include <algorithm>
 
 #include "r2d_device.h"
+#include "r2d_chain.h"
 #include "r2d_kernels.h"
 
 namespace r2d {
@@ -3307,49 +3308,49 @@ __device__ __forceinline__ void entry_candidates(const PairCache& P, uint32_t a,
 
 // LDS of the fused kernel for a world of n bodies and tb hash buckets
 struct FusedLds {
+    uint32_t* dcnt;    // [n] solver items per ordering body
+    uint32_t* doff;    // [n+1] -> list offsets
+    uint32_t* dfill;   // [n]
     uint32_t* coff;    // [n+1] cells per body -> entry offsets
     float *cc, *cs;    // [n] cos / sin of the angle at step start
     uint32_t* boff;    // [tb+1] bucket occupancy -> bucket offsets
     uint32_t* bfill;   // [tb]
-    uint32_t* dcnt;    // [n] solver items per ordering body
-    uint32_t* doff;    // [n+1] -> list offsets
-    uint32_t* dfill;   // [n]
-    uint32_t* solve;   // the solve path's body state
-    uint4* lanes;      // the record chain's lane slots (over the front part)
+    uint32_t* pairs;   // [5 n] pair cache, then the entries' buckets and bucket members when they fit
 };
 
-// front part of a world's fused LDS, in words
+// front part of a world's fused LDS (before the pair cache), in words
 __host__ __device__ constexpr uint32_t fused_front_words(uint32_t n, uint32_t tb) { return 6u * n + 2u * tb + 3u; }
+// the part of it that the solve still reads (dcnt, doff), 8-byte aligned
+__host__ __device__ constexpr uint32_t fused_keep_words(uint32_t n) { return (2u * n + 2u) & ~1u; }
 
-// The front part is dead during the solve's chains (the item counts per body
-// are read before them), so the record chain's lane slots (lane_words, at
-// offset 0) overlay it; the solve's part starts after the larger of the two.
-__device__ __forceinline__ FusedLds fused_carve(uint32_t* lds, uint32_t n, uint32_t tb, uint32_t lane_words)
+__device__ __forceinline__ FusedLds fused_carve(uint32_t* lds, uint32_t n, uint32_t tb)
 {
     FusedLds L;
     uint32_t* p = lds;
-    L.lanes = reinterpret_cast<uint4*>(lds);
+    L.dcnt = p; p += n;
+    L.doff = p; p += n + 1;
+    L.dfill = p; p += n;
     L.coff = p; p += n + 1;
     L.cc = (float*)p; p += n;
     L.cs = (float*)p; p += n;
     L.boff = p; p += tb + 1;
     L.bfill = p; p += tb;
-    L.dcnt = p; p += n;
-    L.doff = p; p += n + 1;
-    L.dfill = p; p += n;
-    L.solve = lds + umax(fused_front_words(n, tb), lane_words);
+    L.pairs = p;
     return L;
 }
 
-// words per body after the front part: the solve's LDS body state (register
-// slots 13, records 7), which also holds the pair cache and, when they fit,
-// the bucket arrays until the solve
-__host__ __device__ constexpr uint32_t fused_solve_words(bool slots) { return slots ? 13u : 7u; }
+// Words per body after the front part: the pair cache and room for the
+// bucket arrays.  The solve then has the whole of LDS but dcnt and doff: 15
+// words a body with 2 n buckets, 9 of them the bodies' state, and the plan
+// (4 words an item) and after it the impulses (2 a point) in what is left.
+constexpr uint32_t FUSED_TAIL_WORDS = 7;
+// Least dynamic LDS of a launch: room for the plan of a small world with many
+// joints, and no cost: the registers allow four workgroups a CU at most.
+constexpr size_t FUSED_LDS_MIN = 24 * 1024;
 
-size_t fused_lds_bytes(uint32_t n, uint32_t tb, bool slots, uint32_t threads)
+size_t fused_lds_bytes(uint32_t n, uint32_t tb)
 {
-    const size_t front = std::max<size_t>(fused_front_words(n, tb), (size_t)threads * LANE_WORDS);
-    return (front + (size_t)fused_solve_words(slots) * n) * 4u;
+    return std::max<size_t>(FUSED_LDS_MIN, (fused_front_words(n, tb) + (size_t)FUSED_TAIL_WORDS * n) * 4u);
 }
 
 // The fused kernel's narrowphase test of one candidate, as a call: out of
@@ -3437,45 +3438,584 @@ __device__ __forceinline__ void fused_overflow(const StepDev& S, uint32_t w, uin
     }
 }
 
-// The solve of a fused step: the register-slot path when the step's items
-// fit the slots, else the record path.  Inlined: a call would save and
-// restore the step's registers around it every step (scratch traffic of the
-// order of the step's own); WAVES sets the register budget of the shape.
-template <int NSLOT, int MAXT, int WAVES, bool LOCKSTEP, bool WARM>
-__device__ __forceinline__ void fused_solve(const StepDev& S, const WorldDev& D, uint32_t w, uint32_t ibase,
-                                         uint32_t nitems, uint32_t mbeg, const uint32_t* degs, float dt,
-                                         uint32_t sub_steps, uint32_t iters, uint32_t* lds, uint4* lanes,
-                                         uint32_t* s_abort)
+// ------------------------------------------------- the solve of a fused step
+// Words of LDS per body while a fused step solves: momentum (x, y, angular),
+// position and angle, then mass, inertia and flags.
+constexpr uint32_t CHAIN_BODY_WORDS = 9;
+
+// a world's bodies in LDS during its sub-steps
+struct ChainBodies {
+    LF2 m;
+    LF l, px, py, ang, mass, inertia;
+    LU32 flags;
+};
+
+// contact point record (words as in r2d_chain.h); the bodies' inverse masses
+// and inertias are 0 for static ones
+struct PointBodies {
+    uint32_t a, b, flag_a, flag_b;
+    float im1, im2, ii1, ii2;
+};
+
+// effective masses of a point (CollisionManifold.preStep, collision.zig:117-132)
+__device__ __forceinline__ void point_masses(const PointBodies& B, v2 n, v2 r1, v2 r2, float& mn, float& mt)
 {
-    if constexpr (NSLOT > 0) {
-        if (nitems <= (uint32_t)NSLOT * MAXT && !(WARM && D.warm > 0.0f)) {
-            slots_world<NSLOT, MAXT, LOCKSTEP>(S, D, w, ibase, nitems, mbeg, degs, dt, sub_steps, iters, lds,
-                                               *s_abort);
-            return;
+    const v2 t = rot90cw(n);
+    const float inv_mass = B.im1 + B.im2;
+    const float r1n = cross2(r1, n), r2n = cross2(r2, n);
+    const float kn = inv_mass + B.ii1 * (r1n * r1n) + B.ii2 * (r2n * r2n);
+    const float r1t = cross2(r1, t), r2t = cross2(r2, t);
+    const float kt = inv_mass + B.ii1 * (r1t * r1t) + B.ii2 * (r2t * r2t);
+    mn = kn > 0.0f ? 1.0f / kn : 0.0f;
+    mt = kt > 0.0f ? 1.0f / kt : 0.0f;
+}
+
+// Baumgarte bias of a sub-step of length dt (collision.zig:172), -1 for a
+// point whose depth is >= 0 (calculateImpulses resets and skips it)
+__device__ __forceinline__ float point_bias(float depth, float dt)
+{
+    return depth >= 0.f ? -1.0f : BAUMGARTE * maxn(0.0f, (-depth) - BAUMGARTE_SLOP) / dt;
+}
+
+__device__ __forceinline__ void point_store(u4v* recs, uint32_t at, const PointBodies& B, uint32_t flags, v2 n, float fric,
+                                            float bias, v2 r1, v2 r2, float mn, float mt)
+{
+    u4v* q = recs + (size_t)at * 4u;
+    q[0] = u4v{B.a | B.flag_a | flags, B.b | B.flag_b, asu(n.x), asu(n.y)};
+    q[1] = u4v{asu(fric), asu(bias), asu(r1.x), asu(r1.y)};
+    q[2] = u4v{asu(r2.x), asu(r2.y), asu(mn), asu(mt)};
+    q[3] = u4v{asu(B.im1), asu(B.im2), asu(B.ii1), asu(B.ii2)};
+}
+
+// the ordering bodies' flags and inverse masses of manifold m's bodies
+// (world slots a, b)
+__device__ __forceinline__ PointBodies point_bodies(const StepDev& S, const WorldDev& D, uint32_t base, uint32_t a, uint32_t b)
+{
+    PointBodies B;
+    B.a = a;
+    B.b = b;
+    const bool sa = (D.flags[a] & BF_STATIC) != 0, sb = (D.flags[b] & BF_STATIC) != 0;
+    const bool wa = (S.sflag[base + a] & SF_RESOURCE) != 0, wb = (S.sflag[base + b] & SF_RESOURCE) != 0;
+    const float m1 = D.mass[a], m2 = D.mass[b], i1 = D.inertia[a], i2 = D.inertia[b];
+    B.flag_a = (wa ? PR_WRITE_A : 0u) | (sa ? PR_STATIC_A : 0u);
+    B.flag_b = (wb ? PR_WRITE_B : 0u) | (sb ? PR_STATIC_B : 0u);
+    B.im1 = sa ? 0.0f : 1.0f / m1;
+    B.im2 = sb ? 0.0f : 1.0f / m2;
+    B.ii1 = sa ? 0.0f : 1.0f / i1;
+    B.ii2 = sb ? 0.0f : 1.0f / i2;
+    return B;
+}
+
+// The records of manifold m (item j of its world; a second point at p1), and
+// what preStep leaves in the manifold: friction and effective masses.
+// Returns whether updateTGSDepth is live for it: a point whose depth is not
+// within 1e-4 of its original depth, which at the step's start is the same
+// number, so NaN or so deep that 1e-4 vanishes in it.
+template <bool WARM>
+__device__ __forceinline__ bool point_build(const StepDev& S, const WorldDev& D, u4v* recs, uint32_t m, uint32_t base,
+                                            uint32_t j, uint32_t p1, float sub_dt)
+{
+    const size_t cm = S.cap_m;
+    float* P = S.m_pt;
+    const uint32_t a = S.m_ref[m] - base, b = S.m_inc[m] - base, valid = S.m_valid[m];
+    const v2 n = mk(S.m_nx[m], S.m_ny[m]);
+    v2 r1[2], r2[2];
+    float depth[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {   // in bounds whether or not the point exists
+        r1[p] = mk(P[(MP_R1X * 2 + p) * cm + m], P[(MP_R1Y * 2 + p) * cm + m]);
+        r2[p] = mk(P[(MP_R2X * 2 + p) * cm + m], P[(MP_R2Y * 2 + p) * cm + m]);
+        depth[p] = P[(MP_DEPTH * 2 + p) * cm + m];
+    }
+    const float mua = D.mu[a], mub = D.mu[b];
+    PointBodies B = point_bodies(S, D, base, a, b);
+    if (WARM && (valid & MV_WARM)) B.flag_b |= PR_WARM;
+    const float fric = sqrt_rn(mua * mub);   // preStep (collision.zig:114)
+    S.m_fric[m] = fric;
+    const bool pair = (valid & 3u) == 3u;
+    bool live = false;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const bool on = (valid & (1u << p)) != 0u;
+        if (!on && p == 1) continue;
+        float mn = 0.f, mt = 0.f;
+        if (on) {
+            point_masses(B, n, r1[p], r2[p], mn, mt);
+            P[(MP_MASS_N * 2 + p) * cm + m] = mn;
+            P[(MP_MASS_T * 2 + p) * cm + m] = mt;
+            live = live || !approx(depth[p], depth[p], 1e-4f);
+        }
+        // a manifold without points keeps one record that adds 0 to its bodies
+        const v2 z = mk(0.f, 0.f);
+        point_store(recs, p ? p1 : j, B, (on ? PR_ON : 0u) | (pair ? PR_PAIR : 0u) | (p ? PR_SECOND : 0u), n, fric,
+                    on ? point_bias(depth[p], sub_dt) : -1.0f, on ? r1[p] : z, on ? r2[p] : z, mn, mt);
+    }
+    return live;
+}
+
+// updateTGSDepth (collision.zig:73-100) for manifold m where it is live:
+// rotate lever arms by the bodies' rotation since the previous sub-step,
+// recompute depth and (preStep) the effective masses, in the step's arrays
+// and the records
+__device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u4v* recs, const ChainBodies& C, uint32_t m,
+                                          uint32_t base, uint32_t j, uint32_t p1, float sub_dt)
+{
+    const size_t cm = S.cap_m;
+    float* P = S.m_pt;
+    const uint32_t valid = S.m_valid[m];
+    bool live = false;
+    for (int p = 0; p < 2; ++p) {
+        const float od = P[(MP_ODEPTH * 2 + p) * cm + m];
+        live = live || ((valid & (1u << p)) && !approx(od, od, 1e-4f));
+    }
+    if (!live) return;
+    const uint32_t a = S.m_ref[m] - base, b = S.m_inc[m] - base;
+    const v2 n = mk(S.m_nx[m], S.m_ny[m]);
+    const float a1 = C.ang[a], a2 = C.ang[b], prev1 = S.m_prev1[m], prev2 = S.m_prev2[m];
+    const PointBodies B = point_bodies(S, D, base, a, b);
+    for (int p = 0; p < 2; ++p) {
+        if (!(valid & (1u << p))) continue;
+        const float od = P[(MP_ODEPTH * 2 + p) * cm + m];
+        if (approx(P[(MP_DEPTH * 2 + p) * cm + m], od, 1e-4f)) continue;
+        const v2 r1 = rotate2(mk(P[(MP_R1X * 2 + p) * cm + m], P[(MP_R1Y * 2 + p) * cm + m]), a1 - prev1);
+        const v2 r2 = rotate2(mk(P[(MP_R2X * 2 + p) * cm + m], P[(MP_R2Y * 2 + p) * cm + m]), a2 - prev2);
+        const v2 q1 = add2(r1, mk(C.px[a], C.py[a])), q2 = add2(r2, mk(C.px[b], C.py[b]));
+        const float depth = dot2(n, sub2(q2, q1)) + od;
+        float mn, mt;
+        point_masses(B, n, r1, r2, mn, mt);
+        P[(MP_R1X * 2 + p) * cm + m] = r1.x; P[(MP_R1Y * 2 + p) * cm + m] = r1.y;
+        P[(MP_R2X * 2 + p) * cm + m] = r2.x; P[(MP_R2Y * 2 + p) * cm + m] = r2.y;
+        P[(MP_DEPTH * 2 + p) * cm + m] = depth;
+        P[(MP_MASS_N * 2 + p) * cm + m] = mn;
+        P[(MP_MASS_T * 2 + p) * cm + m] = mt;
+        u4v* q = recs + (size_t)(p ? p1 : j) * 4u;
+        q[1] = u4v{q[1].x, asu(point_bias(depth, sub_dt)), asu(r1.x), asu(r1.y)};
+        q[2] = u4v{asu(r2.x), asu(r2.y), asu(mn), asu(mt)};
+    }
+    S.m_prev1[m] = a1;
+    S.m_prev2[m] = a2;
+}
+
+// The record of joint J for a sub-step: everything its solve reads besides
+// momenta is fixed within a sub-step (poses after the previous sub-step's
+// position integration; torque as set for this one), so the terms that
+// Constraints/*.zig derive from it are computed here, once, in their order.
+__device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const WorldDev& D, const ChainBodies& C, bool first)
+{
+    const uint32_t type = (uint32_t)J.type, a = (uint32_t)J.s1, b = type <= 1u ? (uint32_t)J.s2 : a;
+    u4v q0{PR_JOINT, type << PR_TYPE_SHIFT, 0u, 0u}, q1{}, q2{}, q3{};
+    if (J.s1 < 0 || (type <= 1u && J.s2 < 0)) {   // a removed body: refused before any solve
+        q0.y |= PR_SKIP;
+        q[0] = q0;
+        return;
+    }
+    const bool sa = (C.flags[a] & BF_STATIC) != 0, sb = (C.flags[b] & BF_STATIC) != 0;
+    q0.x |= a | PR_WRITE_A;
+    q0.y |= b | (type <= 1u ? (a == b ? PR_SELF : PR_WRITE_B) : 0u);
+    q1.y = asu(J.pmin);
+    q1.z = asu(J.pmax);
+    const float im1 = sa ? 0.0f : 1.0f / C.mass[a], im2 = sb ? 0.0f : 1.0f / C.mass[b];
+    const v2 pa = mk(C.px[a], C.py[a]), pb = mk(C.px[b], C.py[b]);
+    q3.x = asu(im1);
+    q3.y = asu(im2);
+    if (type == 0u) {
+        const v2 n = normalize2(sub2(pb, pa));
+        const float dist_err = length2(sub2(pb, pa)) - J.target;
+        q0.z = asu(n.x);
+        q0.w = asu(n.y);
+        q1.x = asu(J.beta * dist_err / maxn(J.target, 0.001f));
+    } else if (type == 1u) {
+        const float ta = C.ang[a], tb = C.ang[b];
+        const v2 rr1 = rotcs(mk(J.r1x, J.r1y), cosf_r(ta), sinf_r(ta));
+        const v2 rr2 = rotcs(mk(J.r2x, J.r2y), cosf_r(tb), sinf_r(tb));
+        const v2 a1 = add2(rr1, pa), a2 = add2(rr2, pb);
+        const v2 n = normalize2(sub2(a2, a1));
+        const float ii1 = sa ? 0.0f : 1.0f / C.inertia[a], ii2 = sb ? 0.0f : 1.0f / C.inertia[b];
+        const float dist_err = length2(sub2(a2, a1)) - J.target;
+        const float r1xn = cross2(rr1, n), r2xn = cross2(rr2, n);
+        q0.z = asu(n.x);
+        q0.w = asu(n.y);
+        q1.x = asu(J.beta * dist_err / maxn(J.target, GRAD_DIV_LIMIT));
+        q1.w = asu(rr1.x);
+        q2 = u4v{asu(rr1.y), asu(rr2.x), asu(rr2.y), asu(im1 + im2 + r1xn * r1xn * ii1 + r2xn * r2xn * ii2)};
+        q3.z = asu(ii1);
+        q3.w = asu(ii2);
+    } else if (type == 2u) {
+        const v2 delta = sub2(mk(J.tx, J.ty), pa);
+        const float dist = length2(delta);
+        if (sa || dist < ALLOWED_CONSTRAINT_VALUE) q0.y |= PR_SKIP;
+        const v2 n = scale2(delta, 1.0f / dist);
+        q0.z = asu(n.x);
+        q0.w = asu(n.y);
+        q1.x = asu(J.beta * dist);
+    } else {
+        if (sa) q0.y |= PR_SKIP;
+        q0.z = asu(C.inertia[a]);
+        q0.w = asu(J.target);
+        q1.x = asu(J.beta);
+        q1.w = asu(first ? D.tq[a] : 0.0f);
+    }
+    q[0] = q0; q[1] = q1; q[2] = q2; q[3] = q3;
+}
+
+// what a body's first pass reads of it beyond LDS
+struct BodyIn {
+    uint32_t f;
+    float mass, inertia, fx, fy, tq;
+};
+
+// Body i's part of the gap between two chains: the position integration of
+// sub-step s - 1 (lib.zig:238-249), then the forces, AABB refresh and velocity
+// integration of sub-step s (lib.zig:200-216).  In between a dynamic body's
+// force and torque are zero, so they need no memory; only the last sub-step's
+// AABB is observable.  s == sub_steps: the positions, and the state back to
+// global memory.
+template <bool WARM>
+__device__ __forceinline__ void chain_body(const WorldDev& D, const BodyArrays& A, const ChainBodies& C, int i, uint32_t s,
+                                           uint32_t sub_steps, float sub_dt, uint32_t f, float mass, float inertia, float fx,
+                                           float fy, float tq)
+{
+    const bool stat = (f & BF_STATIC) != 0;
+    const f2v m0 = C.m[i];
+    float mx = m0.x, my = m0.y, l = C.l[i], px = C.px[i], py = C.py[i], ang = C.ang[i];
+    if (s > 0 && !stat) {
+        const float qd = sub_dt / mass;
+        px = px + mx * qd;
+        py = py + my * qd;
+        ang = ang + l * sub_dt / inertia;
+        C.px[i] = px; C.py[i] = py; C.ang[i] = ang;
+    }
+    if (s == sub_steps) {
+        D.mx[i] = mx; D.my[i] = my; D.L[i] = l;
+        if (!stat) {
+            A.px[i] = px; A.py[i] = py; A.ang[i] = ang;
+            A.fx[i] = 0.0f; A.fy[i] = 0.0f; A.tq[i] = 0.0f;
+        }
+        return;
+    }
+    if (s + 1 == sub_steps) {
+        // Disc.updateAABB / Rectangle.updateAABB
+        float hw, hh;
+        if (f & BF_RECT) {
+            const float c = cosf_r(ang), sn = sinf_r(ang);
+            const float x = A.hw[i], y = A.hh[i];
+            v2 lv[4] = {mk(-x, -y), mk(-x, y), mk(x, y), mk(x, -y)};
+            hw = 0.f; hh = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v2 r = rotcs(lv[k], c, sn);
+                if (r.x > hw) hw = r.x;
+                if (r.y > hh) hh = r.y;
+            }
+        } else {
+            hw = hh = A.rad[i];
+        }
+        A.ax[i] = px; A.ay[i] = py; A.ahw[i] = hw; A.ahh[i] = hh;
+    }
+    if (stat) return;
+    for (int g = 0; g < A.ngens; ++g) {
+        const auto& G = A.gens[g];   // fields read one by one (keeps G's address space)
+        if (G.type == 0) {
+            fx += G.gx * mass;
+            fy += G.gy * mass;
+        } else if (G.slot == i) {
+            const float inv_m = 1.0f / mass;
+            const v2 v = scale2(mk(mx, my), inv_m);
+            const v2 d = sub2(mk(px, py), mk(G.ax, G.ay));
+            fx += (-G.k) * d.x - G.c * v.x;
+            fy += (-G.k) * d.y - G.c * v.y;
         }
     }
-    rec_world<true, WARM>(S, D, w, ibase, nitems, mbeg, degs, dt, sub_steps, iters, lds, lanes, *s_abort);
+    mx += fx * sub_dt;
+    my += fy * sub_dt;
+    l += tq * sub_dt;
+    if constexpr (WARM) {
+        if (A.warm > 0.0f) {
+            // warm starting: the body's share of the matched manifolds' carried impulses
+            const auto ws = warm_sum(A, i);
+            mx += ws[0];
+            my += ws[1];
+            l += ws[2];
+        }
+    }
+    C.m[i] = f2v{mx, my};
+    C.l[i] = l;
+}
+
+// The kernel's argument block and the worlds' descriptors as the out-of-line
+// parts of the solve read them: through the constant address space, so each
+// field is a scalar load where it is used instead of a scalar register held
+// (or spilled) through the whole step, and the pointers in them are known to
+// be global memory.
+typedef const __attribute__((address_space(4))) StepDev* StepArgs;
+typedef const __attribute__((address_space(4))) WorldDev* WorldArgs;
+
+// LDS of a world's solve from ChainShared::free_at on: the bodies, then the
+// plan, and where the plan was the bodies' constants and the impulses.  In
+// front of it: the items per ordering body and their offsets (n and n + 1).
+struct ChainLds {
+    ChainBodies C;
+    LU32 rest, dcnt, doff;
+    uint32_t n, rest_words, consts;
+    LF2 acc;
+    __device__ __forceinline__ ChainLds(LU32 smem, uint32_t free_at, uint32_t free_words, uint32_t n_) : n(n_)
+    {
+        dcnt = smem;
+        doff = smem + n;
+        LU32 lds = smem + free_at;
+        C.m = (LF2)lds;
+        C.l = (LF)(lds + 2u * n);
+        C.px = C.l + n; C.py = C.px + n; C.ang = C.py + n;
+        const uint32_t fixed = (6u * n + 1u) & ~1u;
+        rest = lds + fixed;
+        rest_words = free_words - fixed;
+        C.mass = (LF)rest; C.inertia = C.mass + n; C.flags = (LU32)(C.inertia + n);
+        consts = (3u * n + 1u) & ~1u;
+        acc = (LF2)(rest + consts);
+    }
+};
+
+// The plan, and meanwhile the bodies into LDS and the point records: wave 0
+// plans a world run by one wave while the other waves build; a wider world is
+// planned by all waves, then built by all.
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const uint32_t w = uniform(sh.w), ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj),
+                   M = uniform(sh.M), base = uniform(sh.base);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + w);
+    const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, kc = S.chain_iters;
+    const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n);
+    const ChainBodies& C = L.C;
+    u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
+    const uint32_t waves = chain_waves(nit, kc, (uint32_t)T / 64u);
+    const bool chain = nit > 0u && sh.iters > 0u;
+    const bool plan_in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words;
+    Program G;
+    G.rows = (GU2)(S.prog_rows + (size_t)ibase * kc);
+    G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+    G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
+    PlanLds PL(L.rest, nit, waves);
+    PlanGlb PG((GU4)(S.plan_items + ibase), (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
+    const uint32_t* lists = S.lists + 2 * (size_t)ibase;
+    // successors, and the items that wait for nothing in the first iteration
+    auto fill = [&](auto& P) {
+        for (uint32_t j = t; j < nit; j += T) {
+            const int32_t r0 = S.it_r0[ibase + j], r1 = S.it_r1[ibase + j];
+            const uint32_t k0 = S.it_k0[ibase + j], k1 = S.it_k1[ibase + j];
+            const bool pair = j >= nj && (S.m_valid[mbeg + (j - nj)] & 3u) == 3u;
+            auto next = [&](int32_t r, uint32_t k) {
+                const uint32_t x = (uint32_t)r - base, o = L.doff[x];
+                const bool wrap = k + 1u == L.dcnt[x];
+                return (lists[o + (wrap ? 0u : k + 1u)] >> 1) | (wrap ? WRAP : 0u);
+            };
+            uint32_t s0 = r0 >= 0 ? next(r0, k0) : NO_ITEM, s1 = r1 >= 0 ? next(r1, k1) : NO_ITEM;
+            const uint32_t need = (r0 >= 0 && k0 > 0u ? 1u : 0u) + (r1 >= 0 && k1 > 0u ? 1u : 0u);
+            if (s0 == NO_ITEM) { s0 = s1; s1 = NO_ITEM; }
+            if (s0 == NO_ITEM) s0 = j | WRAP;             // no ordering body: only its own iterations in turn
+            const uint32_t p1 = pair ? nit + __hip_atomic_fetch_add(&sh.pairs, 1u, __ATOMIC_RELAXED,
+                                                                    __HIP_MEMORY_SCOPE_WORKGROUP)
+                                     : 0u;
+            S.it_k0[ibase + j] = p1;                      // the ranks are not read again
+            P.init(j, s0, s1, need, pair, p1);
+            if (need == 0u)
+                P.push_first(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), j, s0,
+                             s1, pair);
+        }
+    };
+    if (plan_in_lds) fill(PL); else fill(PG);
+    __syncthreads();
+    const uint32_t ready = uniform(sh.ready);
+    auto build = [&](uint32_t t0, uint32_t stride) {
+        for (uint32_t i = t0; i < n; i += stride) {
+            C.m[i] = f2v{D.mx[i], D.my[i]};
+            C.l[i] = D.L[i];
+            C.px[i] = D.px[i]; C.py[i] = D.py[i]; C.ang[i] = D.ang[i];
+        }
+        for (uint32_t q = t0; q < M; q += stride)
+            if (point_build<WARM>(S, D, recs, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt)) sh.live = 1u;
+    };
+    uint32_t ns = 1u;
+    if (chain && waves > 1u) {
+        ns = plan_in_lds ? plan_multi(PL, G, nit, kc, ready, waves, sh) : plan_multi(PG, G, nit, kc, ready, waves, sh);
+        build(t, T);
+    } else if (t < 64u) {
+        if (chain) ns = plan_in_lds ? plan_single(PL, G, nit, kc, ready) : plan_single(PG, G, nit, kc, ready);
+    } else {
+        build(t - 64u, T - 64u);
+    }
+    if (t == 0) {
+        sh.nslots = ns;
+        sh.failed = ns == 0u;
+        if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
+    }
+    __syncthreads();
+    // accumulated impulses (normal, tangential) of the contact points, by
+    // point index less the joints: in LDS after the constants when they fit
+    const uint32_t nacc = M + uniform(sh.pairs);
+    if (L.consts + 2u * nacc <= L.rest_words) {
+        for (uint32_t q = t; q < nacc; q += T) L.acc[q] = f2v{0.f, 0.f};
+    } else {
+        GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+        for (uint32_t q = t; q < nacc; q += T) accg[q] = f2v{0.f, 0.f};
+    }
+}
+
+// the gap before sub-step s's chain (s == sub_steps: after the last one), bodies
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void chain_bodies(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const uint32_t sub_steps = uniform(sh.sub_steps);
+    const float sub_dt = sh.dt / (float)sub_steps;
+    const int n = D.nbodies;
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)n);
+    const ChainBodies& C = L.C;
+    const BodyArrays A = body_arrays(D);
+    s = uniform(s);
+    for (int i = (int)threadIdx.x; i < n; i += T) {
+        BodyIn in{0u, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (s == 0u) {
+            in = BodyIn{A.flags[i], A.mass[i], A.inertia[i], A.fx[i], A.fy[i], A.tq[i]};
+            C.mass[i] = in.mass; C.inertia[i] = in.inertia; C.flags[i] = in.f;
+        } else {
+            in.f = C.flags[i]; in.mass = C.mass[i]; in.inertia = C.inertia[i];
+        }
+        chain_body<WARM>(D, A, C, i, s, sub_steps, sub_dt, in.f, in.mass, in.inertia, in.fx, in.fy, in.tq);
+    }
+}
+
+// the gap, items: the joints' records, moved contact points, carried impulses
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M),
+                   base = uniform(sh.base), t = threadIdx.x;
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
+    u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
+    s = uniform(s);
+    for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u);
+    if (sh.live)
+        for (uint32_t q = t; q < M; q += T)
+            point_tgs(S, D, recs, L.C, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt);
+    if constexpr (WARM) {
+        if (!(D.warm > 0.0f)) return;
+        const size_t cm = S.cap_m;
+        const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+        GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+        for (uint32_t q = t; q < M; q += T) {
+            // warm starting: the carried impulse per sub-step joins the accumulators
+            const uint32_t m = mbeg + q, valid = S.m_valid[m];
+            if (!(valid & MV_WARM)) continue;
+            for (uint32_t p = 0; p < 2u; ++p) {
+                if (!(valid & (1u << p))) continue;
+                const f2v add{S.m_pt[(MP_WARM_N * 2 + p) * cm + m], S.m_pt[(MP_WARM_T * 2 + p) * cm + m]};
+                const uint32_t at = p ? S.it_k0[ibase + nj + q] - nj : q;
+                if (in_lds) L.acc[at] = L.acc[at] + add;
+                else accg[at] = accg[at] + add;
+            }
+        }
+    }
+}
+
+// the impulses -> the step's manifold arrays (what r2d_get_manifolds reports)
+template <int T>
+__device__ __attribute__((noinline)) void chain_finish(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
+    const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+    GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+    const size_t cm = S.cap_m;
+    for (uint32_t q = threadIdx.x; q < M; q += T) {
+        const uint32_t m = mbeg + q, valid = S.m_valid[m];
+        for (uint32_t p = 0; p < 2u; ++p) {
+            if (!(valid & (1u << p))) continue;
+            const uint32_t at = p ? S.it_k0[ibase + nj + q] - nj : q;
+            const f2v v = in_lds ? (f2v)L.acc[at] : (f2v)accg[at];
+            S.m_pt[(MP_ACC_PN * 2 + p) * cm + m] = v.x;
+            S.m_pt[(MP_ACC_PT * 2 + p) * cm + m] = v.y;
+        }
+    }
+}
+
+// The solve of one world's step (described by sh; sub_steps > 0): S sub-steps
+// of forces, integration, pre-step and K solver iterations (lib.zig:199-250),
+// by a workgroup of T threads.  The K iterations run as a program of rows
+// (r2d_chain.h); between the chains the bodies live in LDS.  Each part is a
+// function of its own: inlined into the step kernel they pushed it over its
+// register budget (80 spilled VGPRs, 490 spilled SGPRs, and machine code that
+// the compiler's own verifier refused).
+template <int T, bool WARM>
+__device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
+{
+    ChainShared& sh = *(ChainShared*)shl;
+    chain_prepare<T, WARM>(KS, smem, shl);
+    if (sh.failed) return;
+    const StepDev& S = *(const StepDev*)KS;
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const uint32_t sub_steps = uniform(sh.sub_steps), iters = uniform(sh.iters), nj = uniform(sh.nj);
+    const bool chain = nj + sh.M > 0u && iters > 0u, items = nj || sh.live || (WARM && D.warm > 0.0f);
+    for (uint32_t s = 0;; ++s) {
+        chain_bodies<T, WARM>(KS, smem, shl, s);
+        if (s == sub_steps) break;
+        __syncthreads();
+        if (!chain) continue;
+        if (items) {
+            chain_items<T, WARM>(KS, smem, shl, s);
+            __syncthreads();
+        }
+        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters;
+        const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
+        const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+        const GCU2 rows = (GCU2)(S.prog_rows + (size_t)ibase * kc), slots = (GCU2)(S.prog_slots + (size_t)ibase * kc);
+        const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+        const GCU4 recs = (GCU4)(S.recs + (size_t)ibase * 8);
+        GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+        const uint32_t nslots = uniform(sh.nslots), reps = iters / kc;
+        const float sub_dt = sh.dt / (float)sub_steps;
+        if (chain_waves(nj + M, kc, (uint32_t)T / 64u) > 1u) {
+            if (in_lds) chain_lds<true, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, L.acc, nslots, reps, nj, sub_dt);
+            else chain_lds_accg<true, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, accg, nslots, reps, nj, sub_dt);
+        } else if (threadIdx.x < 64u) {
+            if (in_lds) chain_lds<false, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, L.acc, nslots, reps, nj, sub_dt);
+            else chain_lds_accg<false, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, accg, nslots, reps, nj, sub_dt);
+        }
+        __syncthreads();
+    }
+    chain_finish<T>(KS, smem, shl);
 }
 
 // One workgroup per world (S.w_order), up to nsteps steps per world counted
 // in S.w_done, so a relaunch after an overflow resumes each world where it
-// stopped.  The solve takes the register-slot path when the step's items fit
-// NSLOT * MAXT slots, else the record path; both keep body state in LDS.
-template <int NSLOT, int MAXT, int WAVES, bool LOCKSTEP, bool WARM = false>
+// stopped.  lds_words: the launch's dynamic LDS.
+template <int MAXT, int WAVES, bool WARM = false>
 __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WAVES)))
-void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t nsteps)
+void k_fused(StepDev S /* first: chain_world reads it from the argument segment */, float dt, uint32_t sub_steps, uint32_t iters, uint32_t nsteps, uint32_t lds_words)
 {
     extern __shared__ __align__(16) uint32_t smem[];
     __shared__ uint32_t s_sm[16];
-    __shared__ uint32_t s_err, s_abort, s_slot;
-    __shared__ uint32_t s_lvl[3];
+    __shared__ uint32_t s_err, s_slot;
+    __shared__ ChainShared s_chain;
     const uint32_t w = S.w_order[blockIdx.x];
     const WorldDev& D = S.worlds[w];
     WorldScratch X = S.wscr[w];
     const uint32_t n = (uint32_t)D.nbodies, tb = D.table, base = D.body_base, nj = (uint32_t)D.njoints;
     const uint32_t t = threadIdx.x;
     constexpr uint32_t T = MAXT;
-    const FusedLds L = fused_carve(smem, n, tb, T * LANE_WORDS);
+    const FusedLds L = fused_carve(smem, n, tb);
     uint32_t* cnt = S.w_cnt + 8 * (size_t)w;
     uint64_t* ts = S.w_tstamp ? S.w_tstamp + (size_t)w * (S.tcap + 1) : nullptr;
     uint32_t step = S.w_done[w];
@@ -3495,9 +4035,8 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
         // ---- broadphase: per body (k_prep)
         if (t == 0) s_err = 0u;
         __syncthreads();
-        // stale AABBs and flags in LDS for the pair filters below (the solve's
-        // words are free until the solve)
-        const PairCache P = pair_cache(L.solve, n);
+        // stale AABBs and flags in LDS for the pair filters below
+        const PairCache P = pair_cache(L.pairs, n);
         for (uint32_t i = t; i < n; i += T) {
             const Prep o = prep_body(D, i);
             P.ax[i] = D.ax[i]; P.ay[i] = D.ay[i]; P.ahw[i] = D.ahw[i]; P.ahh[i] = D.ahh[i];
@@ -3520,10 +4059,10 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
         uint32_t* ent_body = S.ent_body + X.e0;
         uint32_t* ecnt = S.ent_cnt + X.e0;      // raw candidates per entry -> offsets
         // the entries' buckets and the bucket members are read in serial
-        // loops: in LDS after the pair cache when they fit the solve's words
-        // (3 E <= 8 n; E is about 1.5 n for bodies up to a cell wide)
-        const bool e_lds = 3 * (size_t)E <= (size_t)(fused_solve_words(NSLOT > 0) - PAIR_CACHE_WORDS) * n;
-        uint32_t* e_free = L.solve + PAIR_CACHE_WORDS * n;
+        // loops: in LDS after the pair cache when they fit (E is about 1.5 n
+        // for bodies up to a cell wide)
+        const bool e_lds = 3 * (size_t)E <= (size_t)(lds_words - fused_front_words(n, tb) - PAIR_CACHE_WORDS * n);
+        uint32_t* e_free = L.pairs + PAIR_CACHE_WORDS * n;
         uint32_t* ent_bkt = e_lds ? e_free : S.ent_bkt + X.e0;
         uint32_t* items = e_lds ? e_free + E : S.bkt_items + X.e0;
         uint32_t* sorted = e_lds ? e_free + 2 * E : S.bkt_sorted + X.e0;
@@ -3658,7 +4197,6 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
             }
             S.it_r0[X.i0 + j] = r0;
             S.it_r1[X.i0 + j] = r1;
-            S.it_perm[X.i0 + j] = j;
             if (r0 >= 0) atomicAdd(&L.dcnt[r0 - (int32_t)base], 1u);
             if (r1 >= 0) atomicAdd(&L.dcnt[r1 - (int32_t)base], 1u);
         }
@@ -3667,14 +4205,14 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
         __syncthreads();
         group_scan(L.doff, n, s_sm);
         // per-body item lists (k_list_fill), ranks in item order (k_list_rank).
-        // When the lists fit the front part of LDS (its cell, trig and bucket
-        // arrays are dead after the contacts), they are filled there in any
+        // When the lists fit LDS behind the items per body (the cell, trig,
+        // bucket and pair arrays are dead after the contacts), they are filled there in any
         // order and each entry then finds its rank by counting the smaller
         // entries of its body's list (independent LDS reads) and goes to that
         // place of the global lists; else they are filled in global memory and
         // sorted per body.
         uint32_t* const ul = L.coff;
-        const bool lds_lists = L.doff[n] <= 3u * n + 2u * tb + 2u;
+        const bool lds_lists = L.doff[n] <= lds_words - (3u * n + 1u);
         uint32_t* const fill = lds_lists ? ul : lists;
         for (uint32_t j = t; j < nit; j += T) {
             const int32_t r0 = S.it_r0[X.i0 + j], r1 = S.it_r1[X.i0 + j];
@@ -3718,12 +4256,6 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
             }
         }
         __syncthreads();
-        // execution positions by dependency level when a lane holds more than
-        // one item (with a lane per item the order of positions is moot); its
-        // work arrays in the solve's part of LDS, free until the solve
-        if (nit > T)
-            level_order(S.it_r0 + X.i0, S.it_r1 + X.i0, S.it_k0 + X.i0, S.it_k1 + X.i0, S.it_perm + X.i0, lists, L.doff,
-                        base, 0u, nit, L.solve, fused_solve_words(NSLOT > 0) * n, s_lvl);
         if (WARM && D.warm > 0.0f) {
             // warm starting: match last step's manifolds, then each body's carried impulse
             for (uint32_t q = t; q < M; q += T) warm_match(S, D, X.m0 + q, base, sub_steps);
@@ -3733,12 +4265,20 @@ void k_fused(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t n
         }
         mark(FP_SCHED);
         // ---- solve
-        fused_solve<NSLOT, MAXT, WAVES, LOCKSTEP, WARM>(S, D, w, X.i0, nit, X.m0, L.dcnt, dt, sub_steps, iters, L.solve,
-                                                  L.lanes,
-                                                  &s_abort);
+        // (all of LDS but the items per body and their offsets is dead by now)
+        if (sub_steps > 0u) {
+            if (t == 0) {
+                const uint32_t keep = fused_keep_words(n);
+                s_chain = ChainShared{w, X.i0, X.m0, nj, M, base, sub_steps, iters, dt, keep, lds_words - keep,
+                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}};
+            }
+            __syncthreads();
+            chain_world<MAXT, WARM>((StepArgs)__builtin_amdgcn_kernarg_segment_ptr(), (LU32)smem,
+                                    (R2D_LDS ChainShared*)&s_chain);
+        }
         __syncthreads();
         mark(FP_SOLVE);
-        if (s_abort) break;                     // the solve stalled: status set
+        if (sub_steps > 0u && s_chain.failed) break;   // status set
         if (WARM && D.warm > 0.0f) {
             // warm starting: this step's manifolds become the next step's tables
             for (uint32_t x = t; x < n; x += T) D.wcnt[x] = 0u;
@@ -3791,7 +4331,7 @@ size_t solve_lds_bytes(int nbodies) { return (size_t)nbodies * 7u * 4u; }
 
 typedef void (*SlotFn)(StepDev, float, uint32_t, uint32_t, uint32_t);
 typedef void (*RecFn)(StepDev, float, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
-typedef void (*FusedFn)(StepDev, float, uint32_t, uint32_t, uint32_t);
+typedef void (*FusedFn)(StepDev, float, uint32_t, uint32_t, uint32_t, uint32_t);
 struct SolveVariant {
     SlotFn slot_fn;      // register-slot kernel (nullptr: none)
     unsigned slot_threads;
@@ -3808,45 +4348,40 @@ struct SolveVariant {
 // 4,096-body world)
 static const SolveVariant kSolveVariants[SOLVE_TABLE] = {
     {nullptr, 0, 0, k_solve<1024>, 1024, nullptr},
-    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<256, 2>, 256, k_fused<4, 256, 3, false>},
-    {k_solve_slots<2, 512, 3>, 512, 2, k_solve<256, 2>, 256, k_fused<2, 512, 3, false>},
-    {k_solve_slots<3, 256, 3>, 256, 3, k_solve<256, 2>, 256, k_fused<3, 256, 3, false>},
-    {k_solve_slots<4, 256, 2>, 256, 4, k_solve<256, 2>, 256, k_fused<4, 256, 2, false>},
-    {k_solve_slots<8, 128, 2>, 128, 8, k_solve<256, 2>, 256, k_fused<8, 128, 2, false>},
+    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<256, 2>, 256, k_fused<256, 3>},
+    {k_solve_slots<2, 512, 3>, 512, 2, k_solve<256, 2>, 256, k_fused<512, 3>},
+    {k_solve_slots<3, 256, 3>, 256, 3, k_solve<256, 2>, 256, k_fused<256, 3>},
+    {k_solve_slots<4, 256, 2>, 256, 4, k_solve<256, 2>, 256, k_fused<256, 2>},
+    {k_solve_slots<8, 128, 2>, 128, 8, k_solve<256, 2>, 256, k_fused<128, 2>},
     {nullptr, 0, 0, k_solve<256, 2>, 256, nullptr},
-    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<128, 2>, 128, k_fused<4, 256, 3, false>},
+    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<128, 2>, 128, k_fused<256, 3>},
     // the lockstep slot walk takes the phase kernels only: its fused kernel
     // hung once in a test with no cause found, so it is not built
     {k_solve_slots<3, 256, 3, true>, 256, 3, k_solve<256, 2>, 256, nullptr},
     // records only (as variant 6), fused with 3 or 4 waves per SIMD: fewer
     // registers than the slots, so more worlds resident per CU
-    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<0, 256, 3, false>},
-    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<0, 256, 4, false>},
+    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<256, 3>},
+    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<256, 4>},
     // records only, 192-thread workgroups: with the records' smaller LDS
     // state, four worlds of 500 bodies are resident per CU
-    {nullptr, 0, 0, k_solve<192, 3>, 192, k_fused<0, 192, 3, false>},
+    {nullptr, 0, 0, k_solve<192, 3>, 192, k_fused<192, 3>},
     // records only, 128-thread workgroups at 2 waves per SIMD: the same four
     // worlds per CU with the full register file (no spills)
-    {nullptr, 0, 0, k_solve<128, 2>, 128, k_fused<0, 128, 2, false>},
+    {nullptr, 0, 0, k_solve<128, 2>, 128, k_fused<128, 2>},
     // records only, 512-thread workgroups at 2 waves per SIMD (the full
     // register file): for a few worlds, each alone on a CU, whose chains are
     // latency-bound; up to 512 items no lane ever changes record
-    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<0, 512, 2, false>},
+    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<512, 2>},
     // WIDE_VARIANT: 768 lanes at 3 waves per SIMD (the register budget of
     // variant 11), up to 768 items without a pickup.  A lane that holds two
     // items serialises them, which can triple a chain (the 20-row pyramid's
     // 520-590 items: 148 links per sub-step with a lane per item, 403-437
     // with 512 lanes), so the widest shape that does not spill wins
-    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<0, 768, 3, false>, 768},
+    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<768, 3>, 768},
     // WARM_VARIANT: batches with a warm-started world (the shape of variant
     // 11 with the warm-start passes compiled in; the kernels above carry none)
-    {nullptr, 0, 0, k_solve<192, 3, true>, 192, k_fused<0, 192, 3, false, true>},
+    {nullptr, 0, 0, k_solve<192, 3, true>, 192, k_fused<192, 3, true>},
 };
-
-bool fused_slots(int v)
-{
-    return v >= 0 && v < SOLVE_TABLE && kSolveVariants[v].slot_fn != nullptr;
-}
 
 uint32_t fused_threads(int v)
 {
@@ -3875,7 +4410,8 @@ void launch_fused(const StepDev& S, int v, uint32_t nworlds, float dt, uint32_t 
 {
     const SolveVariant& sv = kSolveVariants[v];
     const unsigned threads = fused_threads(v);
-    hipLaunchKernelGGL(sv.fused_fn, dim3(nworlds), dim3(threads), lds, st, S, dt, sub_steps, iters, nsteps);
+    hipLaunchKernelGGL(sv.fused_fn, dim3(nworlds), dim3(threads), lds, st, S, dt, sub_steps, iters, nsteps,
+                       (uint32_t)(lds / 4u));
 }
 
 unsigned solve_variant_threads(int v) { return kSolveVariants[v < SOLVE_TABLE && v >= 0 ? v : 0].threads; }
