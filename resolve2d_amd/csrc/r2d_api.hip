@@ -120,7 +120,7 @@ size_t static_layout(char* base, StepDev* S, WorldDev** desc)
     take(&F.recs, I * 128);
     take(&F.prog_rows, CHAIN_ITERS_MAX * I * 8); take(&F.prog_entries, 2 * CHAIN_ITERS_MAX * I * 4);
     take(&F.prog_slots, CHAIN_ITERS_MAX * I * 8);
-    take(&F.plan_items, I * 16); take(&F.plan_ring, 2 * I * 16);
+    take(&F.plan_items, 2 * I * 16); take(&F.plan_ring, 2 * I * 16);
     take(&F.cmask, 2 * N * 8);
     take(&F.g_im, N * 4); take(&F.g_ii, N * 4); take(&F.g_cnt, N * 4);
     take(&F.cmap, N * 4); take(&F.cinv, N * 4); take(&F.w_nc, (W + 1) * 4);
@@ -788,7 +788,7 @@ int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64
     add((void**)&F.recs, (size_t)I * 128);
     add((void**)&F.prog_rows, (size_t)K * I * 8); add((void**)&F.prog_entries, 2 * (size_t)K * I * 4);
     add((void**)&F.prog_slots, (size_t)K * I * 8);
-    add((void**)&F.plan_items, (size_t)I * 16); add((void**)&F.plan_ring, 2 * (size_t)I * 16);
+    add((void**)&F.plan_items, 2 * (size_t)I * 16); add((void**)&F.plan_ring, 2 * (size_t)I * 16);
     size_t bytes = 0;
     for (auto& p : parts) bytes += align256(p.second);
     void* arena = nullptr;

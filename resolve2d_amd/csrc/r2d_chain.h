@@ -47,8 +47,8 @@ typedef const R2D_GLB u4v* GCU4;
 // ------------------------------------------------------------ point records
 // 16 words.  Words 0 and 1: the two bodies and flags.
 //   contact point: 2-3 normal, 4 friction, 5 Baumgarte bias of the sub-step
-//     (-1: depth >= 0), 6-9 lever arms r1 r2, 10 / 11 effective masses
-//     (normal, tangent), 12-13 inverse masses, 14-15 inverse inertias
+//     (-1: depth >= 0, or no point), 6-9 lever arms r1 r2, 10 / 11 effective
+//     masses (normal, tangent), 12-13 inverse masses, 14-15 inverse inertias
 //   distance joint (type 0): 2-3 direction, 4 position term, 5 / 6 power
 //     limits (min, max), 12-13 inverse masses
 //   offset distance joint (1): the same, 7-10 rotated offsets, 11 denominator,
@@ -57,51 +57,53 @@ typedef const R2D_GLB u4v* GCU4;
 //   motor (3): 2 inertia, 3 target, 4 beta, 5 / 6 limits, 7 torque
 constexpr uint32_t PR_INDEX = (1u << 26) - 1u;
 enum : uint32_t {
-    // word 0
-    PR_JOINT = 1u << 26,
-    PR_WRITE_A = 1u << 27,    // body a is an ordering body: its momentum is written
-    PR_STATIC_A = 1u << 28,   // ... though static (it gets "+= 0")
-    PR_ON = 1u << 29,         // the point exists (a manifold may have none)
-    PR_PAIR = 1u << 30,       // one of two points; the first sits in the even lane
-    PR_SECOND = 1u << 31,
-    // word 1
-    PR_WRITE_B = 1u << 26,
-    PR_STATIC_B = 1u << 27,
-    PR_WARM = 1u << 28,       // contact: warm started (no minimum impulse)
-    PR_SELF = 1u << 28,       // joint: both ends on one body
-    PR_SKIP = 1u << 29,       // joint: changes nothing this sub-step
-    PR_TYPE_SHIFT = 30        // joint type
+    PR_WRITE = 1u << 31,      // word 0 / 1, contacts: body a / b is an ordering body (its momentum is written)
+                              // and this is the manifold's first point
+    PR_STATIC = 1u << 30,     // word 0 / 1, contacts: the body is static (an ordering one gets "+= 0")
+    PR_JOINT = 1u << 26,      // word 0
+    PR_SELF = 1u << 27,       // word 0, joints: both ends on one body
+    PR_SKIP = 1u << 28,       // word 0, joints: changes nothing this sub-step
+    PR_WARM = 1u << 26,       // word 1, contacts: warm started (no minimum impulse)
+    PR_TYPE_SHIFT = 28        // word 1, joints: type
 };
 
 __device__ __forceinline__ float asf(uint32_t x) { return __uint_as_float(x); }
 __device__ __forceinline__ uint32_t asu(float x) { return __float_as_uint(x); }
 
 // ------------------------------------------------------------------ planning
-// One successor of an item on an ordering body: the next item of the body's
-// list, or its first item in the next iteration (wrap).
+// An item waits for its ordering bodies (one or two) to reach it; run, it
+// releases the next item of each body's list, or the list's first item for
+// the next iteration.  One round of a wave (plan_take, plan_run, plan_put)
+// turns up to 64 lanes of ready items into a row.  A round is bound by its
+// instructions and two LDS round trips: the entry of a ready item carries
+// what the round that runs it needs, and the state word needs no decoding --
+// (ordering bodies waited for) << 16 | iterations left, so a release
+// subtracts 1 << 16 and made its item ready when 1 body and at least one
+// iteration were left, and running an item adds its bodies and takes an
+// iteration off.  An item with one ordering body releases the spare item (the
+// last place), which never becomes ready.
 //
-// Planning state of a world in LDS, 16 bytes per item: succ (both successors,
-// 15-bit items with a wrap bit, NO_ITEM for none), state (16 bits: ordering
-// bodies still waited for, pair bit, iteration from bit 3), second (the second
-// point's index of a pair) and a ring of ready items (x: item | pair << 15 |
-// iteration << 16, y: its succ word).  Worlds that do not fit, or with more
-// items than 15 bits, keep the same in global memory (PlanGlb).
+// Planning state in LDS, 4.5 words an item: succ (both successors, 15 bits
+// each; bit 31: one ordering body), state, second (second point of a pair,
+// counted from 1) and a ring of ready items (x: item | second << 16, y: succ).
+// Worlds that do not fit, or with more items than 15 bits, keep the same in
+// global memory (PlanGlb).
 constexpr uint32_t PLAN_MAX_ITEMS = 0x7ffe;
-constexpr uint32_t NO_ITEM16 = 0x7fffu;
+constexpr uint32_t STATE_BODY = 1u << 16;
 
 struct PlanEntry {
-    uint32_t item, iter, s0, s1;   // s0, s1: successor | wrap << 31, NO_ITEM for none
-    bool pair;
+    uint32_t item, second, s0, s1;   // s1: SINGLE in the top bit when there is one ordering body
 };
-constexpr uint32_t NO_ITEM = 0x7fffffffu;
-constexpr uint32_t WRAP = 0x80000000u;
+constexpr uint32_t SINGLE = 0x80000000u;
 
 __host__ __device__ constexpr uint32_t plan_ring(uint32_t nit, uint32_t waves) { return nit + 64u * waves; }
 // LDS words of PlanLds
 __host__ __device__ constexpr uint32_t plan_lds_words(uint32_t nit, uint32_t waves)
 {
-    return nit + 2u * ((nit + 1u) / 2u) + 2u * plan_ring(nit, waves) + 1u;
+    return 2u * plan_ring(nit, waves) + 2u * (nit + 1u) + (nit + 2u) / 2u;
 }
+// a state that made its item ready when a release found it
+__device__ __forceinline__ bool state_ready(uint32_t old) { return old - (STATE_BODY + 1u) < STATE_BODY - 1u; }
 
 struct PlanLds {
     LU32 succ, state;
@@ -114,61 +116,45 @@ struct PlanLds {
         ring_n = plan_ring(nit, waves);
         ring = (LU2)p;                      // p is 8-byte aligned
         succ = p + 2u * ring_n;
-        state = succ + nit;
-        second = (LU16)(state + (nit + 1u) / 2u);
+        state = succ + nit + 1u;
+        second = (LU16)(state + nit + 1u);
     }
     static __device__ __forceinline__ uint32_t pack(uint32_t s0, uint32_t s1)
     {
-        return (s0 & 0x7fffu) | ((s0 & WRAP) >> 16) | ((s1 & 0x7fffu) << 16) | (s1 & WRAP);
+        return s0 | ((s1 & 0x7fffu) << 16) | (s1 & SINGLE);
     }
-    static __device__ __forceinline__ uint32_t half(uint32_t v)
+    static __device__ __forceinline__ PlanEntry unpack(uint32_t x, uint32_t y)
     {
-        return (v & 0x7fffu) == NO_ITEM16 ? NO_ITEM : ((v & 0x7fffu) | ((v & 0x8000u) << 16));
+        return PlanEntry{x & 0xffffu, x >> 16, y & 0x7fffu, ((y >> 16) & 0x7fffu) | (y & SINGLE)};
     }
-    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t need, bool pair, uint32_t p1)
+    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t st, uint32_t sec)
     {
         succ[j] = pack(s0, s1);
-        ((LU16)state)[j] = (uint16_t)(need | (pair ? 4u : 0u));
-        second[j] = (uint16_t)p1;
-    }
-    __device__ __forceinline__ void push_first(uint32_t at, uint32_t j, uint32_t s0, uint32_t s1, bool pair)
-    {
-        ring[at] = u2v{j | (pair ? 0x8000u : 0u), pack(s0, s1)};
+        state[j] = st;
+        second[j] = (uint16_t)sec;
     }
     __device__ __forceinline__ PlanEntry read(uint32_t at) const
     {
         const u2v v = ring[at];
-        return PlanEntry{v.x & 0x7fffu, v.x >> 16, half(v.y & 0xffffu), half(v.y >> 16), (v.x & 0x8000u) != 0u};
+        return unpack(v.x, v.y);
     }
     __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e)
     {
-        ring[at] = u2v{e.item | (e.pair ? 0x8000u : 0u) | (e.iter << 16), pack(e.s0, e.s1)};
+        ring[at] = u2v{e.item | (e.second << 16), pack(e.s0, e.s1)};
     }
-    __device__ __forceinline__ uint32_t second_of(uint32_t j) const { return second[j]; }
-    // the item's next iteration waits for its `nb` ordering bodies
-    __device__ __forceinline__ void reset(uint32_t j, uint32_t nb)
+    __device__ __forceinline__ void rearm(uint32_t j, uint32_t by)
     {
-        __hip_atomic_fetch_add(&state[j >> 1], (nb + 8u) << (16u * (j & 1u)), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(&state[j], by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    // one of item s's bodies has reached it; true when it was the last
-    __device__ __forceinline__ bool release(uint32_t s, PlanEntry& e)
+    __device__ __forceinline__ uint32_t release(uint32_t s)
     {
-        const uint32_t sh = 16u * (s & 1u);
-        const uint32_t old = __hip_atomic_fetch_sub(&state[s >> 1], 1u << sh, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_WORKGROUP) >> sh;
-        const uint32_t n = succ[s];
-        e.item = s;
-        e.iter = (old & 0xffffu) >> 3;
-        e.pair = (old & 4u) != 0u;
-        e.s0 = half(n & 0xffffu);
-        e.s1 = half(n >> 16);
-        return (old & 3u) == 1u;
+        return __hip_atomic_fetch_sub(&state[s], STATE_BODY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
+    __device__ __forceinline__ PlanEntry entry(uint32_t s) const { return unpack(s | ((uint32_t)second[s] << 16), succ[s]); }
 };
 
-// the same in global memory: items (succ 0, succ 1, state, second point), ring
-// of ready items (item | pair << 31, iteration, succ 0, succ 1)
+// the same in global memory: items (succ 0, succ 1, state, second), ring of
+// ready items (item, second, succ 0, succ 1)
 struct PlanGlb {
     GU4 items, ring;
     uint32_t ring_n;
@@ -177,45 +163,38 @@ struct PlanGlb {
         : items(items_), ring(ring_), ring_n(plan_ring(nit, waves))
     {
     }
-    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t need, bool pair, uint32_t p1)
+    __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t st, uint32_t sec)
     {
-        items[j] = u4v{s0, s1, need | (pair ? 4u : 0u), p1};
-    }
-    __device__ __forceinline__ void push_first(uint32_t at, uint32_t j, uint32_t s0, uint32_t s1, bool pair)
-    {
-        ring[at] = u4v{j | (pair ? WRAP : 0u), 0u, s0, s1};
+        items[j] = u4v{s0, s1, st, sec};
     }
     __device__ __forceinline__ PlanEntry read(uint32_t at) const
     {
         const u4v v = ring[at];
-        return PlanEntry{v.x & ~WRAP, v.y, v.z, v.w, (v.x & WRAP) != 0u};
+        return PlanEntry{v.x, v.y, v.z, v.w};
     }
-    __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e)
-    {
-        ring[at] = u4v{e.item | (e.pair ? WRAP : 0u), e.iter, e.s0, e.s1};
-    }
-    __device__ __forceinline__ uint32_t second_of(uint32_t j) const { return items[j].w; }
+    __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e) { ring[at] = u4v{e.item, e.second, e.s0, e.s1}; }
     __device__ __forceinline__ GU32 state_of(uint32_t j) const { return (GU32)(items + j) + 2; }
-    __device__ __forceinline__ void reset(uint32_t j, uint32_t nb)
+    __device__ __forceinline__ void rearm(uint32_t j, uint32_t by)
     {
-        __hip_atomic_fetch_add(state_of(j), nb + 8u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(state_of(j), by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    __device__ __forceinline__ bool release(uint32_t s, PlanEntry& e)
+    __device__ __forceinline__ uint32_t release(uint32_t s)
     {
-        const uint32_t old = __hip_atomic_fetch_sub(state_of(s), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        e.item = s;
-        e.iter = old >> 3;
-        e.pair = (old & 4u) != 0u;
-        e.s0 = items[s].x;
-        e.s1 = items[s].y;
-        return (old & 3u) == 1u;
+        return __hip_atomic_fetch_sub(state_of(s), STATE_BODY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ PlanEntry entry(uint32_t s) const
+    {
+        const GU32 p = (GU32)(items + s);
+        return PlanEntry{s, p[3], p[0], p[1]};
     }
 };
 
-// A world's program: rows (first entry, entries), the entries (point
-// indices: item j's first point is j, second points follow after the items),
+// A world's program: rows (first entry; entries | pairs << 8 | ROW_JOINTS when
+// one is a joint), the entries (point indices: item j's first point is j,
+// second points follow after the items; pairs first),
 // and for worlds run by several waves the first row and the rows of each slot
 // (rows of one slot run side by side, one per wave).
+constexpr uint32_t ROW_JOINTS = 1u << 16;
 struct Program {
     GU2 rows;
     GU32 entries;
@@ -228,7 +207,7 @@ struct ChainShared {
     uint32_t w, ibase, mbeg, nj, M, base, sub_steps, iters;
     float dt;
     uint32_t free_at, free_words;   // LDS from this word on is the solve's
-    uint32_t ready, pairs, live, nslots, failed, taken, entries, queued[3];
+    uint32_t ready, pairs, live, fix, nslots, failed, taken, entries, queued[3];
 };
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
@@ -251,52 +230,54 @@ __device__ __forceinline__ P uniform_lds(P p)
 }
 
 // One round of one wave: takes ready items from ring place `first` on (at most
-// `avail`, 64 lanes of points), writes their row's entries at `entry0` with
-// pairs in the lower lanes, and releases their successors.  Returns the items
-// taken; `lanes` gets the row's entries and the released items stay in e0 / e1
-// (r0 / r1: whether the lane released one).
+// `avail`, 64 lanes of points; plan_take), then writes their row's entries at
+// `entry0` with pairs in the lower lanes and releases their successors
+// (plan_run: the released items are in e0 / e1, r0 / r1 whether the lane
+// released one).
 struct Round {
-    uint32_t taken, lanes;
-    bool left;                // this lane holds a ready item that did not fit the row
+    uint32_t taken, lanes, word;   // items, points, second word of the row
+    bool take, left;               // this lane's item is in the row / did not fit it
+    uint32_t below, pairs;         // pairs in lower lanes / in the row
     PlanEntry self, e0, e1;
     bool r0, r1;
 };
 
 template <class PLAN>
-__device__ __forceinline__ Round plan_take(PLAN& P, uint32_t first, uint32_t avail, uint32_t lane)
+__device__ __forceinline__ Round plan_take(PLAN& P, uint32_t first, uint32_t avail, uint32_t lane, uint32_t nj)
 {
     Round R;
     const bool act = lane < avail;
     uint32_t at = first + (act ? lane : 0u);
-    if (at >= P.ring_n) at -= P.ring_n;
+    at = at < at - P.ring_n ? at : at - P.ring_n;   // at - ring_n wraps round to a large number below the ring's end
     R.self = P.read(at);
-    const bool pair = act && R.self.pair;
-    const uint64_t pm = __ballot(pair);
-    const uint32_t end = lane + 1u + lanes_below(pm) + (pair ? 1u : 0u);   // lanes used through this item
-    const bool take = act && end <= 64u;
-    R.taken = (uint32_t)__popcll(__ballot(take));
-    R.lanes = R.taken + (uint32_t)__popcll(__ballot(take && pair));
-    R.left = act && !take;
+    const bool pair = act && R.self.second != 0u;
+    R.below = lanes_below(__ballot(pair));
+    R.take = act && lane + 1u + R.below + (pair ? 1u : 0u) <= 64u;   // lanes used through this item
+    const uint64_t tm = __ballot(R.take);
+    R.taken = (uint32_t)__popcll(tm);
+    R.pairs = (uint32_t)__popcll(tm & __ballot(pair));
+    R.lanes = R.taken + R.pairs;
+    R.word = R.lanes | (R.pairs << 8) | (__ballot(R.take && R.self.item < nj) ? ROW_JOINTS : 0u);
+    R.left = act && !R.take;
     return R;
 }
 
 template <class PLAN>
-__device__ __forceinline__ void plan_run(PLAN& P, Round& R, GU32 entries, uint32_t entry0, uint32_t iters, uint32_t lane)
+__device__ __forceinline__ void plan_run(PLAN& P, Round& R, GU32 entries, uint32_t entry0, uint32_t nit, uint32_t lane)
 {
-    const bool take = lane < R.taken;
-    const bool pair = take && R.self.pair;
-    const uint64_t pm = __ballot(pair);
-    const uint32_t below = lanes_below(pm), pairs = (uint32_t)__popcll(pm);
     R.r0 = R.r1 = false;
-    if (take) {
-        const uint32_t j = R.self.item;
-        P.reset(j, R.self.s1 == NO_ITEM ? 1u : 2u);
-        const bool last = R.self.iter + 1u == iters;
-        if (R.self.s0 != NO_ITEM && !(last && (R.self.s0 & WRAP))) R.r0 = P.release(R.self.s0 & ~WRAP, R.e0);
-        if (R.self.s1 != NO_ITEM && !(last && (R.self.s1 & WRAP))) R.r1 = P.release(R.self.s1 & ~WRAP, R.e1);
-        const uint32_t pos = entry0 + (pair ? 2u * below : 2u * pairs + (lane - below));
+    if (R.take) {
+        const uint32_t j = R.self.item, s0 = R.self.s0, s1 = R.self.s1 & ~SINGLE;
+        P.rearm(j, (R.self.s1 & SINGLE ? STATE_BODY : 2u * STATE_BODY) - 1u);
+        const uint32_t o0 = P.release(s0), o1 = P.release(s1);
+        R.e0 = P.entry(s0);
+        R.e1 = P.entry(s1);
+        const bool pair = R.self.second != 0u;
+        const uint32_t pos = entry0 + (pair ? 2u * R.below : 2u * R.pairs + (lane - R.below));
         entries[pos] = j;
-        if (pair) entries[pos + 1u] = P.second_of(j);
+        if (pair) entries[pos + 1u] = nit + R.self.second - 1u;
+        R.r0 = state_ready(o0);
+        R.r1 = state_ready(o1);
     }
 }
 
@@ -304,29 +285,28 @@ template <class PLAN>
 __device__ __forceinline__ void plan_put(PLAN& P, const Round& R, uint32_t at)
 {
     const uint64_t m0 = __ballot(R.r0), m1 = __ballot(R.r1), m2 = __ballot(R.left);
-    const uint32_t c0 = (uint32_t)__popcll(m0), c1 = (uint32_t)__popcll(m1);
-    auto place = [&](uint32_t k) { return k >= P.ring_n ? k - P.ring_n : k; };
+    const uint32_t c0 = (uint32_t)__popcll(m0), c2 = (uint32_t)__popcll(m2);
+    auto place = [&](uint32_t k) { return k < k - P.ring_n ? k : k - P.ring_n; };
     if (R.left) P.push(place(at + lanes_below(m2)), R.self);
-    const uint32_t c2 = (uint32_t)__popcll(m2);
     if (R.r0) P.push(place(at + c2 + lanes_below(m0)), R.e0);
     if (R.r1) P.push(place(at + c2 + c0 + lanes_below(m1)), R.e1);
-    (void)c1;
 }
 
 // The program of a world run by one wave, planned by one wave without
 // barriers; `ready` items are in the ring.  Returns the rows (0: the ordering
 // data was corrupt).
 template <class PLAN>
-__device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint32_t nit, uint32_t iters, uint32_t ready)
+__device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint32_t nit, uint32_t nj, uint32_t iters,
+                                                uint32_t ready)
 {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
     const uint32_t total = nit * iters;
     while (done < total && count) {
-        Round R = plan_take(P, head, count < 64u ? count : 64u, lane);
+        Round R = plan_take(P, head, count < 64u ? count : 64u, lane, nj);
         R.left = false;                  // stays at the head of the ring
-        if (lane == 0) G.rows[row] = u2v{entry, R.lanes};
-        plan_run(P, R, G.entries, entry, iters, lane);
+        if (lane == 0) G.rows[row] = u2v{entry, R.word};
+        plan_run(P, R, G.entries, entry, nit, lane);
         uint32_t tail = head + count;
         if (tail >= P.ring_n) tail -= P.ring_n;
         plan_put(P, R, tail);
@@ -347,8 +327,8 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
 // a row go back to the end of the ring.  A barrier per slot; called by the
 // whole workgroup.  sh.taken, sh.entries, sh.queued start at 0.
 template <class PLAN>
-__device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32_t nit, uint32_t iters, uint32_t ready,
-                                               uint32_t waves, ChainShared& sh)
+__device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32_t nit, uint32_t nj, uint32_t iters,
+                                               uint32_t ready, uint32_t waves, ChainShared& sh)
 {
     const uint32_t lane = threadIdx.x & 63u, wv = uniform(threadIdx.x >> 6);
     uint32_t head = 0, count = ready, row = 0, slot = 0;
@@ -367,15 +347,15 @@ __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32
             const uint32_t rest = count - 64u * wv;
             uint32_t first = head + 64u * wv;
             if (first >= P.ring_n) first -= P.ring_n;
-            Round R = plan_take(P, first, rest < 64u ? rest : 64u, lane);
+            Round R = plan_take(P, first, rest < 64u ? rest : 64u, lane, nj);
             uint32_t e0 = 0u;
             if (lane == 0) {
                 e0 = __hip_atomic_fetch_add(&sh.entries, R.lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_fetch_add(&sh.taken, R.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                G.rows[row + wv] = u2v{e0, R.lanes};
+                G.rows[row + wv] = u2v{e0, R.word};
             }
             e0 = uniform(e0);
-            plan_run(P, R, G.entries, e0, iters, lane);
+            plan_run(P, R, G.entries, e0, nit, lane);
             const uint32_t add = (uint32_t)(__popcll(__ballot(R.r0)) + __popcll(__ballot(R.r1)) + __popcll(__ballot(R.left)));
             uint32_t at = 0u;
             if (lane == 0)
@@ -406,21 +386,16 @@ __host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, ui
 }
 
 // ----------------------------------------------------------------- the chain
-// momenta of a world's bodies in LDS
+// momenta (x, y, angular) of a world's bodies in LDS, 16 bytes a body; the
+// place after the last body takes the writes that are not to be kept
+typedef float f3v __attribute__((ext_vector_type(3)));
+typedef R2D_LDS f3v* LF3;
 struct LdsMomenta {
-    LF2 m;
-    LF l;
-    __device__ __forceinline__ void get(uint32_t i, v2& p, float& L) const
-    {
-        const f2v v = m[i];
-        p = mk(v.x, v.y);
-        L = l[i];
-    }
-    __device__ __forceinline__ void put(uint32_t i, v2 p, float L) const
-    {
-        m[i] = f2v{p.x, p.y};
-        l[i] = L;
-    }
+    LF3 m;
+    uint32_t none;
+    __device__ __forceinline__ f3v get(uint32_t i) const { return m[i]; }
+    __device__ __forceinline__ void put(uint32_t i, f3v v) const { m[i] = v; }
+    __device__ __forceinline__ void put_if(bool keep, uint32_t i, f3v v) const { m[keep ? i : none] = v; }
 };
 
 // x of the other lane of an even / odd pair
@@ -433,17 +408,17 @@ __device__ __forceinline__ float pair_other(float x)
 template <class ST>
 __device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, const ST& st, float dt)
 {
-    const uint32_t type = q0.y >> PR_TYPE_SHIFT, a = q0.x & PR_INDEX, b = q0.y & PR_INDEX;
-    if (q0.y & PR_SKIP) return;
-    const bool self = (q0.y & PR_SELF) != 0u;
+    const uint32_t type = (q0.y >> PR_TYPE_SHIFT) & 3u, a = q0.x & PR_INDEX, b = q0.y & PR_INDEX;
+    if (q0.x & PR_SKIP) return;
+    const bool self = (q0.x & PR_SELF) != 0u;
     const float pmin = asf(q1.y), pmax = asf(q1.z);
-    v2 m1;
-    float L1;
-    st.get(a, m1, L1);
+    const f3v s1 = st.get(a);
+    v2 m1 = mk(s1.x, s1.y);
+    float L1 = s1.z;
     if (type <= 1u) {
-        v2 m2;
-        float L2;
-        st.get(b, m2, L2);
+        const f3v s2 = st.get(b);
+        v2 m2 = mk(s2.x, s2.y);
+        float L2 = s2.z;
         const v2 n = mk(asf(q0.z), asf(q0.w));
         const float pc = asf(q1.x), im1 = asf(q3.x), im2 = asf(q3.y);
         v2 dp;
@@ -475,12 +450,9 @@ __device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const 
             m2 = add2(self ? m1 : m2, dp);
             L2 = (self ? L1 : L2) + Jv * r2xn;
         }
-        if (self) {
-            st.put(a, m2, type == 0u ? L1 : L2);
-        } else {
-            st.put(a, m1, L1);
-            st.put(b, m2, L2);
-        }
+        // the second end last: with both ends on one body it is the sum of both
+        if (!self) st.put(a, f3v{m1.x, m1.y, L1});
+        st.put(b, f3v{m2.x, m2.y, type == 0u && self ? L1 : L2});
     } else if (type == 2u) {
         // FixedPositionJoint.solve (FixedPositionJoint.zig:38-72)
         const float w = asf(q3.x);
@@ -489,7 +461,8 @@ __device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const 
         float Jv = -(rv - asf(q1.x)) / w;
         const float den = 1.0f / maxn(absf(rv), ALLOWED_CONSTRAINT_VALUE);
         Jv = clampn(Jv, pmin * den, pmax * den);
-        st.put(a, add2(m1, scale2(n, Jv)), L1);
+        m1 = add2(m1, scale2(n, Jv));
+        st.put(a, f3v{m1.x, m1.y, L1});
     } else {
         // MotorJoint.solve (MotorJoint.zig:38-64)
         const float I = asf(q0.z);
@@ -500,59 +473,63 @@ __device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const 
         float Jv = tq - bias;
         const float den = 1.0f / maxn(absf(tq / I), ALLOWED_CONSTRAINT_VALUE);
         Jv = clampn(Jv, pmin * den, pmax * den);
-        st.put(a, m1, L1 + Jv * dt);
+        st.put(a, f3v{m1.x, m1.y, L1 + Jv * dt});
     }
 }
 
 // CollisionManifold.calculateImpulses (collision.zig:135-218), one point per
 // lane.  Both points of a manifold work from the same momenta and their
 // impulses are added in point order, so the lane of the first point takes the
-// second's from its neighbour and writes the bodies.
+// second's from its neighbour and writes the bodies.  `paired` lanes, from
+// lane 0 on, hold pairs.  A separated point's impulses are zero already (its
+// depth is the step's, or was reset with it), so it need only change nothing.
+// fix: some static body is an ordering body.
+//
+// A row is bound by its instructions (one wave issues about one every five
+// cycles: 115 vector and 35 scalar ones took 1,090 cycles), so nothing here
+// branches but on what the whole row shares: a write that is not to be kept
+// goes to a spare place instead of being masked.  s1, s2, old: the bodies'
+// momenta and the point's impulses, read ahead.
 template <bool WARM, class ST, class ACC>
 __device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, const ST& st,
-                                              ACC acc)
+                                              f3v s1, f3v s2, f2v old, ACC acc, uint32_t lane, uint32_t paired, bool fix)
 {
-    const uint32_t fa = q0.x, fb = q0.y, a = fa & PR_INDEX, b = fb & PR_INDEX;
-    v2 m1, m2;
-    float L1, L2;
-    st.get(a, m1, L1);
-    st.get(b, m2, L2);
-    const f2v old = *acc;
+    const uint32_t a = q0.x & PR_INDEX, b = q0.y & PR_INDEX;
     const v2 n = mk(asf(q0.z), asf(q0.w)), t = rot90cw(n);
     const float fric = asf(q1.x), bias = asf(q1.y);
     const v2 r1 = mk(asf(q1.z), asf(q1.w)), r2 = mk(asf(q2.x), asf(q2.y));
-    const float om1 = L1 * asf(q3.z), om2 = L2 * asf(q3.w);
-    const v2 v1 = add2(scale2(m1, asf(q3.x)), mk(-r1.y * om1, r1.x * om1));
-    const v2 v2v = add2(scale2(m2, asf(q3.y)), mk(-r2.y * om2, r2.x * om2));
+    const float om1 = s1.z * asf(q3.z), om2 = s2.z * asf(q3.w);
+    const v2 v1 = add2(scale2(mk(s1.x, s1.y), asf(q3.x)), mk(-r1.y * om1, r1.x * om1));
+    const v2 v2v = add2(scale2(mk(s2.x, s2.y), asf(q3.y)), mk(-r2.y * om2, r2.x * om2));
     const v2 dv = sub2(v1, v2v);
     const float pn = (dot2(dv, n) + bias) * asf(q2.z);
     const float pt = dot2(dv, t) * asf(q2.w);
-    const bool on = (fa & PR_ON) != 0u, sep = bias < 0.f;
-    const bool go = on && !sep && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (fb & PR_WARM) != 0u));
+    const bool go = !(bias < 0.f) && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (q0.y & PR_WARM) != 0u));
     const float new_pn = maxn(0.0f, old.x + pn);
     const float max_pt = fric * absf(new_pn);
     const float new_pt = clampn(old.y + pt, -max_pt, max_pt);
     const float apn = new_pn - old.x, apt = new_pt - old.y;
-    const bool clr = on && sep;
-    *acc = f2v{clr ? 0.f : (go ? new_pn : old.x), clr ? 0.f : (go ? new_pt : old.y)};
+    *acc = f2v{go ? new_pn : old.x, go ? new_pt : old.y};
     v2 dp = add2(scale2(n, apn), scale2(t, apt));
     float c1 = cross2(r1, dp), c2 = cross2(r2, dp);
     // a point that does nothing adds +0, which changes none of the sums below
     // (0 - x and 0 + x are never -0)
     dp.x = go ? dp.x : 0.f; dp.y = go ? dp.y : 0.f;
     c1 = go ? c1 : 0.f; c2 = go ? c2 : 0.f;
-    float a1x = 0.f - dp.x, a1y = 0.f - dp.y, g1 = 0.f - c1;
-    float a2x = 0.f + dp.x, a2y = 0.f + dp.y, g2 = 0.f + c2;
-    if (fa & PR_PAIR) {
-        const float ox = pair_other(dp.x), oy = pair_other(dp.y), o1 = pair_other(c1), o2 = pair_other(c2);
-        a1x = a1x - ox; a1y = a1y - oy; g1 = g1 - o1;
-        a2x = a2x + ox; a2y = a2y + oy; g2 = g2 + o2;
+    f3v d1{0.f - dp.x, 0.f - dp.y, 0.f - c1}, d2{0.f + dp.x, 0.f + dp.y, 0.f + c2};
+    if (paired) {
+        if (lane < paired) {
+            const float ox = pair_other(dp.x), oy = pair_other(dp.y), o1 = pair_other(c1), o2 = pair_other(c2);
+            d1 = f3v{d1.x - ox, d1.y - oy, d1.z - o1};
+            d2 = f3v{d2.x + ox, d2.y + oy, d2.z + o2};
+        }
     }
-    if (fa & PR_STATIC_A) { a1x = 0.f; a1y = 0.f; g1 = 0.f; }
-    if (fb & PR_STATIC_B) { a2x = 0.f; a2y = 0.f; g2 = 0.f; }
-    const bool lead = !(fa & PR_SECOND);
-    if (lead && (fa & PR_WRITE_A)) st.put(a, mk(m1.x + a1x, m1.y + a1y), L1 + g1);
-    if (lead && (fb & PR_WRITE_B)) st.put(b, mk(m2.x + a2x, m2.y + a2y), L2 + g2);
+    if (fix) {
+        if (q0.x & PR_STATIC) d1 = f3v{0.f, 0.f, 0.f};
+        if (q0.y & PR_STATIC) d2 = f3v{0.f, 0.f, 0.f};
+    }
+    st.put_if((int32_t)q0.x < 0, a, f3v{s1.x + d1.x, s1.y + d1.y, s1.z + d1.z});
+    st.put_if((int32_t)q0.y < 0, b, f3v{s2.x + d2.x, s2.y + d2.y, s2.z + d2.z});
 }
 
 // Runs a program: `nslots` slots, `reps` times over.  MULTI: the workgroup's
@@ -579,7 +556,7 @@ struct InLds<LdsMomenta> {
 
 template <bool MULTI, bool WARM, class ST, class ACC>
 __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, const ST& st, ACC acc,
-                                          uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+                                          uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
 {
     constexpr bool LDS_ONLY = InLds<ST>::value && InLds<ACC>::value;
     rows = uniform_ptr(rows); entries = uniform_ptr(entries); slots = uniform_ptr(slots); recs = uniform_ptr(recs);
@@ -608,7 +585,7 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
         };
         auto load_entry = [&](int k) {
             const uint32_t c = uniform(row[k].y);
-            ent[k] = entries[uniform(row[k].x) + (lane < c ? lane : 0u)];
+            ent[k] = entries[uniform(row[k].x) + (lane < (c & 0xffu) ? lane : 0u)];
             cnt_e[k] = mine[k] ? c : 0u;
         };
         auto load_rec = [&](int k) {
@@ -630,16 +607,28 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
             for (int u = 0; u < 3; ++u) {
                 const uint32_t s = s0 + u;
                 if (s >= nslots) break;
+                // this row's LDS reads first: the fetches below are issued
+                // while they are under way (lanes without an entry and joints
+                // read something harmless)
+                const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
+                const uint32_t rc = cnt[u], pt = point[u];
+                const uint32_t ai = (uint32_t)max((int32_t)(pt - nj), 0);
+                const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
+                const f2v old = acc[ai];
+                __builtin_amdgcn_sched_barrier(0);
                 load_rec((u + 2) % 3);
                 load_entry((u + 4) % 3);
                 load_row(s + 6u, u);
                 load_slot(s + 8u, (u + 8) % 3);
                 __builtin_amdgcn_sched_barrier(0);
-                if (lane < cnt[u]) {
-                    const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
-                    if (q0.x & PR_JOINT) chain_joint(q0, q1, q2, q3, st, dt);
-                    else chain_contact<WARM>(q0, q1, q2, q3, st, acc + (point[u] - nj));
+                bool act = lane < (rc & 0xffu);
+                if (rc & ROW_JOINTS) {
+                    const bool joint = (q0.x & PR_JOINT) != 0u;
+                    if (act && joint) chain_joint(q0, q1, q2, q3, st, dt);
+                    act = act && !joint;
                 }
+                if (act)
+                    chain_contact<WARM>(q0, q1, q2, q3, st, s1, s2, old, acc + ai, lane, (rc >> 7) & 0x1feu, fix);
                 // the next slot reads what this one wrote
                 if constexpr (MULTI) {
                     if constexpr (LDS_ONLY) {
@@ -663,18 +652,18 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
 // own, whatever the step kernel holds around it.  `accg`: the accumulated
 // impulses when they do not fit LDS (acc null).
 template <bool MULTI, bool WARM>
-__device__ __attribute__((noinline)) void chain_lds(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF2 m, LF l, LF2 acc,
-                                                    uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+__device__ __attribute__((noinline)) void chain_lds(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
+                                                    LF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
 {
-    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform_lds(l)}, uniform_lds(acc), nslots,
-                           reps, nj, dt);
+    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_lds(acc), nslots,
+                           reps, nj, uniform(fix) != 0u, dt);
 }
 template <bool MULTI, bool WARM>
-__device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF2 m, LF l,
-                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, float dt)
+__device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
+                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
 {
-    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform_lds(l)}, uniform_ptr(acc), nslots,
-                           reps, nj, dt);
+    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), nslots,
+                           reps, nj, uniform(fix) != 0u, dt);
 }
 
 }  // namespace r2d

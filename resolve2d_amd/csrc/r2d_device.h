@@ -154,7 +154,7 @@ struct StepDev {
     uint2* prog_rows;                      // [chain_iters * cap_i]
     uint32_t* prog_entries;                // [2 * chain_iters * cap_i]
     uint2* prog_slots;                     // [chain_iters * cap_i]
-    uint4* plan_items;                     // [cap_i]
+    uint4* plan_items;                     // [2 * cap_i]
     uint4* plan_ring;                      // [2 * cap_i]
     // global-memory solver state (worlds too large for LDS)
     float *g_im, *g_ii;

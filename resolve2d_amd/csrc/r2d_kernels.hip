@@ -3320,8 +3320,8 @@ struct FusedLds {
 
 // front part of a world's fused LDS (before the pair cache), in words
 __host__ __device__ constexpr uint32_t fused_front_words(uint32_t n, uint32_t tb) { return 6u * n + 2u * tb + 3u; }
-// the part of it that the solve still reads (dcnt, doff), 8-byte aligned
-__host__ __device__ constexpr uint32_t fused_keep_words(uint32_t n) { return (2u * n + 2u) & ~1u; }
+// the part of it that the solve still reads (dcnt, doff), 16-byte aligned
+__host__ __device__ constexpr uint32_t fused_keep_words(uint32_t n) { return (2u * n + 4u) & ~3u; }
 
 __device__ __forceinline__ FusedLds fused_carve(uint32_t* lds, uint32_t n, uint32_t tb)
 {
@@ -3340,10 +3340,11 @@ __device__ __forceinline__ FusedLds fused_carve(uint32_t* lds, uint32_t n, uint3
 }
 
 // Words per body after the front part: the pair cache and room for the
-// bucket arrays.  The solve then has the whole of LDS but dcnt and doff: 15
-// words a body with 2 n buckets, 9 of them the bodies' state, and the plan
-// (4 words an item) and after it the impulses (2 a point) in what is left.
-constexpr uint32_t FUSED_TAIL_WORDS = 7;
+// bucket arrays.  The solve then has the whole of LDS but dcnt and doff: 16
+// words a body with 2 n buckets, 7 of them momenta and poses, and in the rest
+// the plan (4 words an item), then 3 words a body and the impulses (2 a
+// point).  A world of 500 bodies takes 36 KB: four to a CU.
+constexpr uint32_t FUSED_TAIL_WORDS = 8;
 // Least dynamic LDS of a launch: room for the plan of a small world with many
 // joints, and no cost: the registers allow four workgroups a CU at most.
 constexpr size_t FUSED_LDS_MIN = 24 * 1024;
@@ -3439,14 +3440,11 @@ __device__ __forceinline__ void fused_overflow(const StepDev& S, uint32_t w, uin
 }
 
 // ------------------------------------------------- the solve of a fused step
-// Words of LDS per body while a fused step solves: momentum (x, y, angular),
-// position and angle, then mass, inertia and flags.
-constexpr uint32_t CHAIN_BODY_WORDS = 9;
-
-// a world's bodies in LDS during its sub-steps
+// a world's bodies in LDS during its sub-steps: momenta (16 bytes a body and a
+// spare one), position and angle, then mass, inertia and flags
 struct ChainBodies {
-    LF2 m;
-    LF l, px, py, ang, mass, inertia;
+    LF3 m;
+    LF px, py, ang, mass, inertia;
     LU32 flags;
 };
 
@@ -3477,11 +3475,12 @@ __device__ __forceinline__ float point_bias(float depth, float dt)
     return depth >= 0.f ? -1.0f : BAUMGARTE * maxn(0.0f, (-depth) - BAUMGARTE_SLOP) / dt;
 }
 
-__device__ __forceinline__ void point_store(u4v* recs, uint32_t at, const PointBodies& B, uint32_t flags, v2 n, float fric,
+__device__ __forceinline__ void point_store(u4v* recs, uint32_t at, const PointBodies& B, bool second, v2 n, float fric,
                                             float bias, v2 r1, v2 r2, float mn, float mt)
 {
     u4v* q = recs + (size_t)at * 4u;
-    q[0] = u4v{B.a | B.flag_a | flags, B.b | B.flag_b, asu(n.x), asu(n.y)};
+    const uint32_t drop = second ? ~(uint32_t)PR_WRITE : ~0u;   // the first point writes the bodies
+    q[0] = u4v{B.a | (B.flag_a & drop), B.b | (B.flag_b & drop), asu(n.x), asu(n.y)};
     q[1] = u4v{asu(fric), asu(bias), asu(r1.x), asu(r1.y)};
     q[2] = u4v{asu(r2.x), asu(r2.y), asu(mn), asu(mt)};
     q[3] = u4v{asu(B.im1), asu(B.im2), asu(B.ii1), asu(B.ii2)};
@@ -3497,8 +3496,8 @@ __device__ __forceinline__ PointBodies point_bodies(const StepDev& S, const Worl
     const bool sa = (D.flags[a] & BF_STATIC) != 0, sb = (D.flags[b] & BF_STATIC) != 0;
     const bool wa = (S.sflag[base + a] & SF_RESOURCE) != 0, wb = (S.sflag[base + b] & SF_RESOURCE) != 0;
     const float m1 = D.mass[a], m2 = D.mass[b], i1 = D.inertia[a], i2 = D.inertia[b];
-    B.flag_a = (wa ? PR_WRITE_A : 0u) | (sa ? PR_STATIC_A : 0u);
-    B.flag_b = (wb ? PR_WRITE_B : 0u) | (sb ? PR_STATIC_B : 0u);
+    B.flag_a = (wa ? PR_WRITE : 0u) | (sa ? PR_STATIC : 0u);
+    B.flag_b = (wb ? PR_WRITE : 0u) | (sb ? PR_STATIC : 0u);
     B.im1 = sa ? 0.0f : 1.0f / m1;
     B.im2 = sb ? 0.0f : 1.0f / m2;
     B.ii1 = sa ? 0.0f : 1.0f / i1;
@@ -3510,9 +3509,10 @@ __device__ __forceinline__ PointBodies point_bodies(const StepDev& S, const Worl
 // what preStep leaves in the manifold: friction and effective masses.
 // Returns whether updateTGSDepth is live for it: a point whose depth is not
 // within 1e-4 of its original depth, which at the step's start is the same
-// number, so NaN or so deep that 1e-4 vanishes in it.
+// number, so NaN or so deep that 1e-4 vanishes in it (1), and whether one of
+// its bodies is static and an ordering body (2).
 template <bool WARM>
-__device__ __forceinline__ bool point_build(const StepDev& S, const WorldDev& D, u4v* recs, uint32_t m, uint32_t base,
+__device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev& D, u4v* recs, uint32_t m, uint32_t base,
                                             uint32_t j, uint32_t p1, float sub_dt)
 {
     const size_t cm = S.cap_m;
@@ -3532,7 +3532,6 @@ __device__ __forceinline__ bool point_build(const StepDev& S, const WorldDev& D,
     if (WARM && (valid & MV_WARM)) B.flag_b |= PR_WARM;
     const float fric = sqrt_rn(mua * mub);   // preStep (collision.zig:114)
     S.m_fric[m] = fric;
-    const bool pair = (valid & 3u) == 3u;
     bool live = false;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -3547,18 +3546,21 @@ __device__ __forceinline__ bool point_build(const StepDev& S, const WorldDev& D,
         }
         // a manifold without points keeps one record that adds 0 to its bodies
         const v2 z = mk(0.f, 0.f);
-        point_store(recs, p ? p1 : j, B, (on ? PR_ON : 0u) | (pair ? PR_PAIR : 0u) | (p ? PR_SECOND : 0u), n, fric,
-                    on ? point_bias(depth[p], sub_dt) : -1.0f, on ? r1[p] : z, on ? r2[p] : z, mn, mt);
+        point_store(recs, p ? p1 : j, B, p != 0, n, fric, on ? point_bias(depth[p], sub_dt) : -1.0f, on ? r1[p] : z,
+                    on ? r2[p] : z, mn, mt);
     }
-    return live;
+    const uint32_t both = PR_WRITE | PR_STATIC;
+    return (live ? 1u : 0u) | ((B.flag_a & both) == both || (B.flag_b & both) == both ? 2u : 0u);
 }
 
 // updateTGSDepth (collision.zig:73-100) for manifold m where it is live:
 // rotate lever arms by the bodies' rotation since the previous sub-step,
 // recompute depth and (preStep) the effective masses, in the step's arrays
-// and the records
+// and the records; reset(p): point p is separated now, its impulses are reset
+// (calculateImpulses does so in the sub-step's first iteration)
+template <class RESET>
 __device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u4v* recs, const ChainBodies& C, uint32_t m,
-                                          uint32_t base, uint32_t j, uint32_t p1, float sub_dt)
+                                          uint32_t base, uint32_t j, uint32_t p1, float sub_dt, RESET reset)
 {
     const size_t cm = S.cap_m;
     float* P = S.m_pt;
@@ -3588,6 +3590,7 @@ __device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u
         P[(MP_DEPTH * 2 + p) * cm + m] = depth;
         P[(MP_MASS_N * 2 + p) * cm + m] = mn;
         P[(MP_MASS_T * 2 + p) * cm + m] = mt;
+        if (depth >= 0.f) reset(p);
         u4v* q = recs + (size_t)(p ? p1 : j) * 4u;
         q[1] = u4v{q[1].x, asu(point_bias(depth, sub_dt)), asu(r1.x), asu(r1.y)};
         q[2] = u4v{asu(r2.x), asu(r2.y), asu(mn), asu(mt)};
@@ -3605,13 +3608,13 @@ __device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const World
     const uint32_t type = (uint32_t)J.type, a = (uint32_t)J.s1, b = type <= 1u ? (uint32_t)J.s2 : a;
     u4v q0{PR_JOINT, type << PR_TYPE_SHIFT, 0u, 0u}, q1{}, q2{}, q3{};
     if (J.s1 < 0 || (type <= 1u && J.s2 < 0)) {   // a removed body: refused before any solve
-        q0.y |= PR_SKIP;
+        q0.x |= PR_SKIP;
         q[0] = q0;
         return;
     }
     const bool sa = (C.flags[a] & BF_STATIC) != 0, sb = (C.flags[b] & BF_STATIC) != 0;
-    q0.x |= a | PR_WRITE_A;
-    q0.y |= b | (type <= 1u ? (a == b ? PR_SELF : PR_WRITE_B) : 0u);
+    q0.x |= a | (type <= 1u && a == b ? PR_SELF : 0u);
+    q0.y |= b;
     q1.y = asu(J.pmin);
     q1.z = asu(J.pmax);
     const float im1 = sa ? 0.0f : 1.0f / C.mass[a], im2 = sb ? 0.0f : 1.0f / C.mass[b];
@@ -3643,13 +3646,13 @@ __device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const World
     } else if (type == 2u) {
         const v2 delta = sub2(mk(J.tx, J.ty), pa);
         const float dist = length2(delta);
-        if (sa || dist < ALLOWED_CONSTRAINT_VALUE) q0.y |= PR_SKIP;
+        if (sa || dist < ALLOWED_CONSTRAINT_VALUE) q0.x |= PR_SKIP;
         const v2 n = scale2(delta, 1.0f / dist);
         q0.z = asu(n.x);
         q0.w = asu(n.y);
         q1.x = asu(J.beta * dist);
     } else {
-        if (sa) q0.y |= PR_SKIP;
+        if (sa) q0.x |= PR_SKIP;
         q0.z = asu(C.inertia[a]);
         q0.w = asu(J.target);
         q1.x = asu(J.beta);
@@ -3676,8 +3679,8 @@ __device__ __forceinline__ void chain_body(const WorldDev& D, const BodyArrays& 
                                            float fy, float tq)
 {
     const bool stat = (f & BF_STATIC) != 0;
-    const f2v m0 = C.m[i];
-    float mx = m0.x, my = m0.y, l = C.l[i], px = C.px[i], py = C.py[i], ang = C.ang[i];
+    const f3v m0 = C.m[i];
+    float mx = m0.x, my = m0.y, l = m0.z, px = C.px[i], py = C.py[i], ang = C.ang[i];
     if (s > 0 && !stat) {
         const float qd = sub_dt / mass;
         px = px + mx * qd;
@@ -3738,8 +3741,7 @@ __device__ __forceinline__ void chain_body(const WorldDev& D, const BodyArrays& 
             l += ws[2];
         }
     }
-    C.m[i] = f2v{mx, my};
-    C.l[i] = l;
+    C.m[i] = f3v{mx, my, l};
 }
 
 // The kernel's argument block and the worlds' descriptors as the out-of-line
@@ -3763,10 +3765,9 @@ struct ChainLds {
         dcnt = smem;
         doff = smem + n;
         LU32 lds = smem + free_at;
-        C.m = (LF2)lds;
-        C.l = (LF)(lds + 2u * n);
-        C.px = C.l + n; C.py = C.px + n; C.ang = C.py + n;
-        const uint32_t fixed = (6u * n + 1u) & ~1u;
+        C.m = (LF3)lds;
+        C.px = (LF)(lds + 4u * (n + 1u)); C.py = C.px + n; C.ang = C.py + n;
+        const uint32_t fixed = (4u * (n + 1u) + 3u * n + 1u) & ~1u;
         rest = lds + fixed;
         rest_words = free_words - fixed;
         C.mass = (LF)rest; C.inertia = C.mass + n; C.flags = (LU32)(C.inertia + n);
@@ -3799,7 +3800,7 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * kc);
     G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
     PlanLds PL(L.rest, nit, waves);
-    PlanGlb PG((GU4)(S.plan_items + ibase), (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
+    PlanGlb PG((GU4)(S.plan_items + 2 * (size_t)ibase), (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
     const uint32_t* lists = S.lists + 2 * (size_t)ibase;
     // successors, and the items that wait for nothing in the first iteration
     auto fill = [&](auto& P) {
@@ -3808,42 +3809,46 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
             const uint32_t k0 = S.it_k0[ibase + j], k1 = S.it_k1[ibase + j];
             const bool pair = j >= nj && (S.m_valid[mbeg + (j - nj)] & 3u) == 3u;
             auto next = [&](int32_t r, uint32_t k) {
-                const uint32_t x = (uint32_t)r - base, o = L.doff[x];
-                const bool wrap = k + 1u == L.dcnt[x];
-                return (lists[o + (wrap ? 0u : k + 1u)] >> 1) | (wrap ? WRAP : 0u);
+                const uint32_t x = (uint32_t)r - base;
+                return lists[L.doff[x] + (k + 1u == L.dcnt[x] ? 0u : k + 1u)] >> 1;
             };
-            uint32_t s0 = r0 >= 0 ? next(r0, k0) : NO_ITEM, s1 = r1 >= 0 ? next(r1, k1) : NO_ITEM;
+            // one ordering body (or none: the item then only follows itself)
+            const bool two = r0 >= 0 && r1 >= 0;
+            const uint32_t s0 = r0 >= 0 ? next(r0, k0) : r1 >= 0 ? next(r1, k1) : j;
+            const uint32_t s1 = two ? next(r1, k1) : nit | SINGLE;
             const uint32_t need = (r0 >= 0 && k0 > 0u ? 1u : 0u) + (r1 >= 0 && k1 > 0u ? 1u : 0u);
-            if (s0 == NO_ITEM) { s0 = s1; s1 = NO_ITEM; }
-            if (s0 == NO_ITEM) s0 = j | WRAP;             // no ordering body: only its own iterations in turn
-            const uint32_t p1 = pair ? nit + __hip_atomic_fetch_add(&sh.pairs, 1u, __ATOMIC_RELAXED,
+            const uint32_t sec = pair ? 1u + __hip_atomic_fetch_add(&sh.pairs, 1u, __ATOMIC_RELAXED,
                                                                     __HIP_MEMORY_SCOPE_WORKGROUP)
-                                     : 0u;
-            S.it_k0[ibase + j] = p1;                      // the ranks are not read again
-            P.init(j, s0, s1, need, pair, p1);
+                                      : 0u;
+            S.it_k0[ibase + j] = nit + sec - 1u;          // the second point's index; the ranks are not read again
+            P.init(j, s0, s1, need * STATE_BODY + kc, sec);
             if (need == 0u)
-                P.push_first(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), j, s0,
-                             s1, pair);
+                P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
+                       PlanEntry{j, sec, s0, s1});
         }
+        if (t == 0u) P.init(nit, nit, nit | SINGLE, 0u, 0u);   // the spare item: no iterations, never ready
     };
     if (plan_in_lds) fill(PL); else fill(PG);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
     auto build = [&](uint32_t t0, uint32_t stride) {
         for (uint32_t i = t0; i < n; i += stride) {
-            C.m[i] = f2v{D.mx[i], D.my[i]};
-            C.l[i] = D.L[i];
+            C.m[i] = f3v{D.mx[i], D.my[i], D.L[i]};
             C.px[i] = D.px[i]; C.py[i] = D.py[i]; C.ang[i] = D.ang[i];
         }
-        for (uint32_t q = t0; q < M; q += stride)
-            if (point_build<WARM>(S, D, recs, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt)) sh.live = 1u;
+        for (uint32_t q = t0; q < M; q += stride) {
+            const uint32_t f = point_build<WARM>(S, D, recs, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt);
+            if (f & 1u) sh.live = 1u;
+            if (f & 2u) sh.fix = 1u;
+        }
     };
     uint32_t ns = 1u;
     if (chain && waves > 1u) {
-        ns = plan_in_lds ? plan_multi(PL, G, nit, kc, ready, waves, sh) : plan_multi(PG, G, nit, kc, ready, waves, sh);
+        ns = plan_in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh)
+                         : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
         build(t, T);
     } else if (t < 64u) {
-        if (chain) ns = plan_in_lds ? plan_single(PL, G, nit, kc, ready) : plan_single(PG, G, nit, kc, ready);
+        if (chain) ns = plan_in_lds ? plan_single(PL, G, nit, nj, kc, ready) : plan_single(PG, G, nit, nj, kc, ready);
     } else {
         build(t - 64u, T - 64u);
     }
@@ -3904,14 +3909,20 @@ __device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     s = uniform(s);
     for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u);
+    const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+    GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
     if (sh.live)
-        for (uint32_t q = t; q < M; q += T)
-            point_tgs(S, D, recs, L.C, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt);
+        for (uint32_t q = t; q < M; q += T) {
+            const uint32_t p1 = S.it_k0[ibase + nj + q];
+            point_tgs(S, D, recs, L.C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
+                const uint32_t at = p ? p1 - nj : q;
+                if (in_lds) L.acc[at] = f2v{0.f, 0.f};
+                else accg[at] = f2v{0.f, 0.f};
+            });
+        }
     if constexpr (WARM) {
         if (!(D.warm > 0.0f)) return;
         const size_t cm = S.cap_m;
-        const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
-        GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         for (uint32_t q = t; q < M; q += T) {
             // warm starting: the carried impulse per sub-step joins the accumulators
             const uint32_t m = mbeg + q, valid = S.m_valid[m];
@@ -3986,12 +3997,13 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const uint32_t nslots = uniform(sh.nslots), reps = iters / kc;
         const float sub_dt = sh.dt / (float)sub_steps;
+        const bool fix = uniform(sh.fix) != 0u;
         if (chain_waves(nj + M, kc, (uint32_t)T / 64u) > 1u) {
-            if (in_lds) chain_lds<true, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, L.acc, nslots, reps, nj, sub_dt);
-            else chain_lds_accg<true, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, accg, nslots, reps, nj, sub_dt);
+            if (in_lds) chain_lds<true, WARM>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, fix, sub_dt);
+            else chain_lds_accg<true, WARM>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, fix, sub_dt);
         } else if (threadIdx.x < 64u) {
-            if (in_lds) chain_lds<false, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, L.acc, nslots, reps, nj, sub_dt);
-            else chain_lds_accg<false, WARM>(rows, entries, slots, recs, L.C.m, L.C.l, accg, nslots, reps, nj, sub_dt);
+            if (in_lds) chain_lds<false, WARM>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, fix, sub_dt);
+            else chain_lds_accg<false, WARM>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, fix, sub_dt);
         }
         __syncthreads();
     }
@@ -4270,7 +4282,7 @@ void k_fused(StepDev S /* first: chain_world reads it from the argument segment 
             if (t == 0) {
                 const uint32_t keep = fused_keep_words(n);
                 s_chain = ChainShared{w, X.i0, X.m0, nj, M, base, sub_steps, iters, dt, keep, lds_words - keep,
-                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}};
+                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}};
             }
             __syncthreads();
             chain_world<MAXT, WARM>((StepArgs)__builtin_amdgcn_kernarg_segment_ptr(), (LU32)smem,
