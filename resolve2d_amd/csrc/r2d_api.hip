@@ -122,8 +122,6 @@ size_t static_layout(char* base, StepDev* S, WorldDev** desc)
     take(&F.prog_slots, CHAIN_ITERS_MAX * I * 8);
     take(&F.plan_items, 2 * I * 16); take(&F.plan_ring, 2 * I * 16);
     take(&F.cmask, 2 * N * 8);
-    take(&F.g_im, N * 4); take(&F.g_ii, N * 4); take(&F.g_cnt, N * 4);
-    take(&F.cmap, N * 4); take(&F.cinv, N * 4); take(&F.w_nc, (W + 1) * 4);
     take(&F.counters, 64 * 4);
     take(&F.partials, 1024 * 4);
     take(&F.wscr, W * sizeof(WorldScratch));
@@ -242,8 +240,6 @@ struct r2d_world {
 struct r2d_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    hipStream_t aux[2] = {nullptr, nullptr};      // side streams of the solve phase
-    hipEvent_t fork = nullptr, join[2] = {nullptr, nullptr};
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;   // brackets of the last launched batch
     hipEvent_t ev_kend = nullptr;                      // end of the last fused kernel
     r2d_server* server = nullptr;
@@ -253,7 +249,7 @@ struct r2d_ctx {
     size_t arena_bytes = 0;
     StepDev S{};
     uint32_t cap_n = 0, cap_b = 0, cap_w = 0, cap_j = 0;
-    uint32_t cap_e = 0, cap_r = 0, cap_m = 0, cap_i = 0;
+    uint32_t cap_e = 0, cap_r = 0, cap_m = 0, cap_i = 0, cap_k = 0;
     WorldDev* dworlds = nullptr;
     size_t dworlds_cap = 0;
     uint32_t* hcounters = nullptr;     // pinned
@@ -321,7 +317,7 @@ struct r2d_ctx {
     std::unordered_map<void*, size_t> pool_class;  // every block handed out -> its class
     size_t pool_cached = 0;                        // bytes in the free lists
 
-    Streams streams() const { return Streams{stream, {aux[0], aux[1]}, fork, {join[0], join[1]}, trace}; }
+    Streams streams() const { return Streams{stream, trace}; }
 };
 
 namespace {
@@ -619,9 +615,9 @@ WorldDev make_desc(r2d_world* w)
 
 // carve the step scratch for the current capacities
 int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, uint32_t e, uint32_t r, uint32_t m,
-                   uint32_t it)
+                   uint32_t it, uint32_t k)
 {
-    if (n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w && j <= c->cap_j && e <= c->cap_e && r <= c->cap_r &&
+    if (k <= c->cap_k && n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w && j <= c->cap_j && e <= c->cap_e && r <= c->cap_r &&
         m <= c->cap_m && it <= c->cap_i && c->arena)
         return R2D_OK;
     auto grow = [](uint32_t have, uint32_t need) {
@@ -629,6 +625,7 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
         uint64_t v = (uint64_t)need + need / 2 + 256;
         return (uint32_t)std::min<uint64_t>(v, 0xffffff00ull);
     };
+    c->cap_k = std::max(c->cap_k, k);
     c->cap_n = grow(c->cap_n, n); c->cap_b = grow(c->cap_b, b); c->cap_w = grow(c->cap_w, wn);
     c->cap_j = grow(c->cap_j, j); c->cap_e = grow(c->cap_e, e); c->cap_r = grow(c->cap_r, r);
     c->cap_m = grow(c->cap_m, m); c->cap_i = grow(c->cap_i, std::max(it, c->cap_m + c->cap_j));
@@ -661,12 +658,13 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.deg, (N + 1) * 4); add((void**)&S.deg_off, (N + 1) * 4); add((void**)&S.deg_fill, (N + 1) * 4);
     add((void**)&S.lists, 2 * I * 4);
     add((void**)&S.it_color, I * 4);
-    add((void**)&S.it_perm, I * 4);
     add((void**)&S.recs, I * 128);
-    add((void**)&S.rmass, I * 16);
+    const size_t K = c->cap_k;
+    add((void**)&S.prog_rows, K * I * 8); add((void**)&S.prog_entries, 2 * K * I * 4); add((void**)&S.prog_slots, K * I * 8);
+    add((void**)&S.plan_items, 2 * I * 16); add((void**)&S.plan_ring, 2 * I * 16);
     add((void**)&S.cmask, 2 * N * 8);
-    add((void**)&S.g_im, N * 4); add((void**)&S.g_ii, N * 4); add((void**)&S.g_cnt, N * 4);
-    add((void**)&S.cmap, N * 4); add((void**)&S.cinv, N * 4); add((void**)&S.w_nc, (W + 1) * 4);
+    add((void**)&S.g_cnt, N * 4); add((void**)&S.cmap, N * 4); add((void**)&S.g_mom, (N + W) * 16);
+    add((void**)&S.w_chain, (W + 1) * sizeof(WorldChain));
     add((void**)&S.counters, 64 * 4);
     add((void**)&S.partials, 1024 * 4);
     for (auto& p : parts) off += align256(p.second);
@@ -1126,7 +1124,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     if (fused) {
         // the step scratch holds the per-body and per-world arrays; the
         // worlds' slices live in the fused arena
-        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1)))
+        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1, 1)))
             return rc;
         return fused_layout(c, b);
     }
@@ -1134,7 +1132,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     uint32_t est_r = std::max<uint32_t>(c->cap_r, (uint32_t)(8 * b.N + 1024));
     uint32_t est_m = std::max<uint32_t>(c->cap_m, (uint32_t)(4 * b.N + 1024));
     return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m,
-                          (uint32_t)b.J + est_m);
+                          (uint32_t)b.J + est_m, chain_iters(b.iters));
 }
 
 // sum the phase times of the timed steps recorded so far
@@ -1171,6 +1169,7 @@ int batch_launch(r2d_ctx* c, Batch& b)
     StepDev S = c->S;
     S.nb = (uint32_t)b.N; S.nworlds = (uint32_t)nw; S.nbuckets = (uint32_t)b.B; S.njoints = (uint32_t)b.J;
     S.worlds = c->dworlds;
+    S.chain_iters = chain_iters(b.iters);
     const Streams ss = c->streams();
     const uint32_t sub = (uint32_t)b.sub, iters = (uint32_t)b.iters;
     auto eager_phase = [&](int ph) { launch_phase(S, ss, ph, b.dt, sub, iters, b.plan); };
@@ -1424,7 +1423,7 @@ int batch_wait(r2d_ctx* c, Batch& b)
             if (c->hcounters[C_OVERFLOW] & 4u) m = c->hcounters[C_MANIFOLDS] * 2;
             if (c->hcounters[C_OVERFLOW] & 8u) it = c->hcounters[C_ITEMS] * 2;
             int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e + 1, r + 1,
-                                    m + 1, it + 1);
+                                    m + 1, it + 1, chain_iters(b.iters));
             if (rc) return rc;
         }
         if (b.done >= b.steps) break;
@@ -1717,9 +1716,6 @@ R2D_EXPORT int r2d_ctx_create(int device, r2d_ctx** out)
     if (hipDeviceGetAttribute(&c->num_cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         c->num_cus = 0;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return R2D_E_DEVICE; }
-    for (int i = 0; i < 2; ++i) HIPCHK(hipStreamCreateWithFlags(&c->aux[i], hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
-    for (int i = 0; i < 2; ++i) HIPCHK(hipEventCreateWithFlags(&c->join[i], hipEventDisableTiming));
     HIPCHK(hipEventCreate(&c->ev_begin));
     HIPCHK(hipEventCreate(&c->ev_end));
     HIPCHK(hipEventCreate(&c->ev_kend));
@@ -1754,8 +1750,6 @@ R2D_EXPORT int r2d_ctx_destroy(r2d_ctx* c)
     if (c->hcounters) (void)hipHostFree(c->hcounters);
     if (c->hstatus) (void)hipHostFree(c->hstatus);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
-    (void)hipEventDestroy(c->fork);
-    for (int i = 0; i < 2; ++i) (void)hipEventDestroy(c->join[i]);
     (void)hipEventDestroy(c->ev_begin);
     (void)hipEventDestroy(c->ev_end);
     (void)hipEventDestroy(c->ev_kend);
@@ -1770,7 +1764,6 @@ R2D_EXPORT int r2d_ctx_destroy(r2d_ctx* c)
     if (c->hfsum) (void)hipHostFree(c->hfsum);
     if (c->ingest) (void)hipFree(c->ingest);
     pool_destroy(c);
-    for (int i = 0; i < 2; ++i) (void)hipStreamDestroy(c->aux[i]);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return R2D_OK;

@@ -390,12 +390,22 @@ __host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, ui
 // place after the last body takes the writes that are not to be kept
 typedef float f3v __attribute__((ext_vector_type(3)));
 typedef R2D_LDS f3v* LF3;
+typedef R2D_GLB f3v* GF3;
 struct LdsMomenta {
     LF3 m;
     uint32_t none;
     __device__ __forceinline__ f3v get(uint32_t i) const { return m[i]; }
     __device__ __forceinline__ void put(uint32_t i, f3v v) const { m[i] = v; }
     __device__ __forceinline__ void put_if(bool keep, uint32_t i, f3v v) const { m[keep ? i : none] = v; }
+};
+
+// the same in global memory
+struct GlbMomenta {
+    GF3 m;
+    uint32_t none;
+    __device__ __forceinline__ f3v get(uint32_t i) const { return m[i]; }
+    __device__ __forceinline__ void put(uint32_t i, f3v v) const { m[i] = v; }
+    __device__ __forceinline__ void put_if(bool keep, uint32_t i, f3v v) const { if (keep) m[i] = v; }
 };
 
 // x of the other lane of an even / odd pair
@@ -663,6 +673,15 @@ __device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entrie
                                                          GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
 {
     chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), nslots,
+                           reps, nj, uniform(fix) != 0u, dt);
+}
+
+// momenta and impulses in global memory
+template <bool MULTI, bool WARM>
+__device__ __attribute__((noinline)) void chain_glb(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, GF3 m, uint32_t none,
+                                                    GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
+{
+    chain_run<MULTI, WARM>(rows, entries, slots, recs, GlbMomenta{uniform_ptr(m), uniform(none)}, uniform_ptr(acc), nslots,
                            reps, nj, uniform(fix) != 0u, dt);
 }
 

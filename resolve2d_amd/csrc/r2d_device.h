@@ -102,6 +102,15 @@ enum : int32_t {
 };
 
 // per-step scratch, sized by capacities chosen on the host
+constexpr uint32_t UNTOUCHED = 0xffffffffu;
+// a world's chain in the separate launches
+struct WorldChain {
+    uint32_t bodies;    // places: bodies its items touch
+    uint32_t pairs;     // manifolds of two points
+    uint32_t flags;     // 1: updateTGSDepth is live; 2: some static body is an ordering body
+    uint32_t slots;     // of its program
+};
+
 struct StepDev {
     uint32_t nb;             // batch bodies N
     uint32_t nworlds;        // W
@@ -143,11 +152,8 @@ struct StepDev {
     uint32_t *deg, *deg_off, *deg_fill;    // [N+1]
     uint32_t* lists;                       // [2*cap_i]
     uint32_t* it_color;                    // [cap_i] colour (0 in reference order)
-    uint32_t* it_perm;                     // [cap_i] world-local items in execution order
     uint64_t* cmask;                       // [2*N] colours used per body (coloured schedule)
-    uint4* recs;                           // [8*cap_i] solver item records (128 B each)
-    uint4* rmass;                          // [cap_i] worlds beyond LDS: inverse mass and inertia of each item's
-                                           // two bodies (im a, ii a, im b, ii b) for the light compact chain
+    uint4* recs;                           // [8*cap_i] contact point and joint records (two of 64 B an item)
     // the solver's program (r2d_chain.h): iterations one program covers, its
     // rows and entries, and planning state when it does not fit LDS
     uint32_t chain_iters;
@@ -156,12 +162,11 @@ struct StepDev {
     uint2* prog_slots;                     // [chain_iters * cap_i]
     uint4* plan_items;                     // [2 * cap_i]
     uint4* plan_ring;                      // [2 * cap_i]
-    // global-memory solver state (worlds too large for LDS)
-    float *g_im, *g_ii;
-    uint32_t* g_cnt;
-    uint32_t* cmap;          // [N] worlds beyond LDS: compact chain index of each body (or ~0)
-    uint32_t* cinv;          // [N] compact index -> world slot, at the world's body base
-    uint32_t* w_nc;          // [W] bodies in the compact chain
+    // the solve in separate launches
+    uint32_t* g_cnt;         // [N] colouring: items of a body that have their colour
+    uint32_t* cmap;          // [N] each body's place in its world's chain (UNTOUCHED: no item touches it)
+    uint4* g_mom;            // [N + W] momenta by place, each world's from its body base + its index on
+    WorldChain* w_chain;     // [W+1]
     uint32_t* counters;
     uint32_t* partials;                    // scan scratch
     // whole steps of each world in one workgroup (k_fused)

@@ -16,9 +16,6 @@ namespace r2d {
 enum { KT_BROAD_BEGIN = 0, KT_NARROW_BEGIN, KT_SCHED_BEGIN, KT_SOLVE_BEGIN, KT_END, KT_N };
 
 
-// bytes of LDS the solve kernel needs for a world of n bodies
-size_t solve_lds_bytes(int nbodies);
-
 // the four phases of one step, enqueued in this order on one stream
 enum { PH_BROAD = 0, PH_NARROW, PH_SCHED, PH_SOLVE, PH_N };
 
@@ -33,11 +30,6 @@ constexpr size_t WIDE_MAX_WORLDS = 64;
 // the variant every batch with a warm-started world takes (not tunable)
 constexpr int WARM_VARIANT = SOLVE_VARIANTS;
 constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 1;
-unsigned solve_variant_threads(int v);
-int solve_variant_slots(int v);
-
-// worlds of at most this many bodies may take the register-slot kernel
-constexpr uint32_t SLOT_NMAX = 1024;
 
 // Iterations of a sub-step that one program covers: all of them up to 16,
 // else their largest divisor up to 16 (the program is then run that often).
@@ -51,23 +43,21 @@ inline uint32_t chain_iters(size_t iters)
     return 1u;
 }
 
-// how one batch's solve phase is split over the solve kernels
+// The separate launches' chain: batches of at most this many worlds (one per
+// CU) take wide workgroups and all of LDS.
+constexpr size_t CHAIN_WIDE_WORLDS = 256;
+constexpr size_t CHAIN_LDS = 159 * 1024, CHAIN_LDS_MIN = 16 * 1024, CHAIN_LDS_BODY = 40;
+
+// how one batch's solve phase is launched
 struct SolvePlan {
-    int variant = 0;
-    uint32_t slot_cap = 0;    // items a world may have to take the slot kernel (0: no slot kernel)
-    uint32_t slot_nmax = 0;   // bodies a world may have to take the slot kernel
-    uint32_t lds_nmax = 0;    // bodies a world may have to keep its body state in LDS
-    uint32_t slot_maxn = 0;   // largest world each launch may take: sizes its LDS
-    uint32_t lds_maxn = 0;
-    uint32_t any_slot = 0, any_lds = 0, any_big = 0;
+    uint32_t lds = 0;          // dynamic LDS of a world's workgroup
+    uint32_t lds_nmax = 0;     // bodies a world may have to keep its momenta in LDS
+    uint32_t wide = 0;         // wide workgroups
     uint32_t any_colored = 0;  // some world uses the coloured schedule
     uint32_t any_warm = 0;     // some world is warm started
-    uint32_t n_big = 0;        // worlds beyond LDS
-    uint32_t n_lds = 0;        // worlds of the record kernel with LDS body state
-    uint32_t rec_wide = 0;     // they take the 512-lane record kernel (few worlds, each alone on a CU)
 };
-// lds_limit: largest world (bodies) that keeps its body state in LDS (0: as
-// many as LDS holds); larger worlds use the global-memory record kernel
+// lds_limit: largest world (bodies) that keeps its momenta in LDS (0: as many
+// as LDS holds)
 SolvePlan plan_solve(int variant, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
                      bool any_warm, bool allow_wide = true);
 
@@ -89,12 +79,9 @@ struct KernelTrace {
     ~KernelTrace();
 };
 
-// the context's main stream plus two side streams for the solve kernels
+// the context's stream
 struct Streams {
     hipStream_t main;
-    hipStream_t aux[2];
-    hipEvent_t fork;
-    hipEvent_t join[2];
     KernelTrace* trace;
 };
 

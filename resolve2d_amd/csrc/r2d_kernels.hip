@@ -820,6 +820,34 @@ __global__ void k_joint_mark(StepDev S)
     }
 }
 
+// A rank among the active lanes of a wave that are `on`, added to the counter
+// of each one's world: one atomic per world and wave.
+__device__ __forceinline__ uint32_t world_rank(const StepDev& S, bool on, uint32_t w, uint32_t WorldChain::* counter)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t rank = 0;
+    for (uint64_t todo = __ballot(on); todo;) {
+        const uint32_t lead = (uint32_t)__builtin_ctzll(todo);
+        const uint64_t same = __ballot(on && w == (uint32_t)__shfl((int)w, (int)lead)) & todo;
+        uint32_t at = 0;
+        if (lane == lead) at = atomicAdd(&(S.w_chain[w].*counter), (uint32_t)__popcll(same));
+        at = (uint32_t)__shfl((int)at, (int)lead);
+        if ((same >> lane) & 1u) rank = at + lanes_below(same);
+        todo &= ~same;
+    }
+    return rank;
+}
+
+// batch body x of world w takes part in the step's items: its place in the
+// world's chain (any numbering gives the same results)
+__device__ __forceinline__ void chain_touch(const StepDev& S, bool on, uint32_t w, uint32_t x)
+{
+    bool mine = false;
+    if (on && S.cmap[x] == UNTOUCHED) mine = atomicCAS(&S.cmap[x], UNTOUCHED, UNTOUCHED - 1u) == UNTOUCHED;
+    const uint32_t c = world_rank(S, mine, w, &WorldChain::bodies);
+    if (mine) S.cmap[x] = c;
+}
+
 __global__ void k_items_joints(StepDev S)
 {
     if (S.counters[C_OVERFLOW]) return;
@@ -841,6 +869,8 @@ __global__ void k_items_joints(StepDev S)
         S.it_r1[item] = r1;
         if (r0 >= 0) atomicAdd(&S.deg[r0], 1u);
         if (r1 >= 0) atomicAdd(&S.deg[r1], 1u);
+        chain_touch(S, r0 >= 0, lo, (uint32_t)r0);
+        chain_touch(S, r1 >= 0, lo, (uint32_t)r1);
     }
 }
 
@@ -858,6 +888,19 @@ __global__ void k_items_mans(StepDev S)
         S.it_r1[item] = r1;
         if (r0 >= 0) atomicAdd(&S.deg[r0], 1u);
         if (r1 >= 0) atomicAdd(&S.deg[r1], 1u);
+        chain_touch(S, true, w, ref);
+        chain_touch(S, true, w, inc);
+    }
+}
+
+// what the step's items are counted into, at zero
+__global__ void k_items_clear(StepDev S)
+{
+    for (uint32_t x = grid_tid(); x <= S.nb; x += grid_stride()) {
+        S.deg[x] = 0u;
+        S.deg_fill[x] = 0u;
+        if (x < S.nb) S.cmap[x] = UNTOUCHED;
+        if (x <= S.nworlds) S.w_chain[x] = WorldChain{};
     }
 }
 
@@ -881,142 +924,32 @@ __device__ __forceinline__ void st_rel(uint32_t* p, uint32_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// polls of one item before its world is stopped as stalled: ~2 s of waiting
-// with the poll's sleep; a wave can wait behind other worlds' waves on its
-// SIMD for a tenth of that and still be making progress
-constexpr uint32_t SPIN_LIMIT = 1u << 26;
 // the colouring polls global memory (~1 us a poll): its own, smaller limit
 constexpr uint32_t COLOR_SPIN_LIMIT = 1u << 22;
 
 // Coloured schedule (a world with r2d_set_schedule(w, 1)): greedy colouring
 // of the world's items in item order -- an item takes the smallest colour
 // unused by earlier items sharing one of its ordering bodies; past 127
-// colours an item takes 128 + its index, a colour of its own -- then the
-// execution order (colour, item).  One workgroup per world.  The colouring
-// runs as a dataflow over per-body counters in item order (an item waits
-// until every earlier item on its bodies has taken its colour), the pattern
-// of the solver; the order is a stable block-wide counting sort.  Worlds in
-// the reference order get colour 0 and the identity order.
-// Reference order: the execution positions of a world's items (it_perm) by
-// level -- an item's level is 1 + the larger level of its predecessors, the
-// items just before it in its ordering bodies' lists.  Items of one level
-// share no ordering body, so their order among themselves is free.  The solve's lanes
-// take positions t, t + T, ... of each pass in turn; with positions in item
-// order a lane's next item often waits behind a long chain while items at
-// later positions could run, and the lane holds them back.  Any order that
-// lists every item after its predecessors keeps the dataflow free of
-// deadlock (the earliest unfinished item in (pass, position) order is always
-// its lane's current item, and its predecessors have run), and the counters
-// still give each body its items in the reference order, so the results are
-// the same bits; only which lane runs what, and when, changes.  Work arrays
-// in LDS (lds_words): levels, packed predecessors, level counts, 3 nit + 2
-// words; a world with more items keeps the item order.  Levels are found by
-// sweeps in which each thread walks a contiguous chunk of items in item
-// order (a predecessor in the same chunk is seen in the same sweep), until a
-// sweep changes nothing.  The world's item arrays start at its first item
-// (r0s .. perm); a body r's item list is lists[off[r - base] ..], whose
-// entries are (item + sub) * 2 + side.  Not inlined: it runs once per step,
-// and kept out of the caller it leaves the caller's register allocation as
-// it is (the fused step kernel is at its register budget).
-__device__ __attribute__((noinline)) void level_order(const int32_t* r0s, const int32_t* r1s, const uint32_t* k0s,
-                                                      const uint32_t* k1s, uint32_t* perm, const uint32_t* lists,
-                                                      const uint32_t* off, uint32_t base, uint32_t sub, uint32_t nit,
-                                                      uint32_t* lds, uint32_t lds_words, uint32_t* flags)
+// colours an item takes 128 + its index, a colour of its own.  One workgroup
+// per world.  The colouring runs as a dataflow over per-body counters in item
+// order: an item waits until every earlier item on its bodies has taken its
+// colour.  Worlds in the reference order take no part.
+__global__ __launch_bounds__(256) void k_color(StepDev S)
 {
-    const uint32_t T = blockDim.x, t = threadIdx.x;
-    if (nit < 2u || nit >= 0xffffu || 3u * nit + 2u > lds_words) {
-        for (uint32_t p = t; p < nit; p += T) perm[p] = p;
-        return;
-    }
-    uint32_t* lev = lds;
-    uint32_t* pred = lds + nit;
-    uint32_t* hist = lds + 2u * nit;
-    for (uint32_t p = t; p < nit; p += T) {
-        const int32_t r0 = r0s[p], r1 = r1s[p];
-        uint32_t q0 = 0xffffu, q1 = 0xffffu;
-        if (r0 >= 0 && k0s[p] > 0u) q0 = (lists[off[(uint32_t)r0 - base] + k0s[p] - 1u] >> 1) - sub;
-        if (r1 >= 0 && k1s[p] > 0u) q1 = (lists[off[(uint32_t)r1 - base] + k1s[p] - 1u] >> 1) - sub;
-        pred[p] = q0 | (q1 << 16);
-        lev[p] = 1u;
-    }
-    if (t == 0) { flags[0] = 0u; flags[1] = 0u; flags[2] = 0u; }
-    __syncthreads();
-    const uint32_t chunk = (nit + T - 1) / T;
-    const uint32_t lo = umin(t * chunk, nit), hi = umin(lo + chunk, nit);
-    // sweep p reports a change in flags[p % 3] and clears the flag of sweep
-    // p + 1, which every thread read before the previous barrier
-    for (uint32_t sweep = 0;; ++sweep) {
-        bool changed = false;
-        for (uint32_t p = lo; p < hi; ++p) {
-            const uint32_t pw = pred[p];
-            const uint32_t q0 = pw & 0xffffu, q1 = pw >> 16;
-            uint32_t l = 1u;
-            if (q0 != 0xffffu)
-                l = umax(l, 1u + __hip_atomic_load(&lev[q0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-            if (q1 != 0xffffu)
-                l = umax(l, 1u + __hip_atomic_load(&lev[q1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-            if (l != __hip_atomic_load(&lev[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
-                __hip_atomic_store(&lev[p], l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                changed = true;
-            }
-        }
-        if (changed) flags[sweep % 3u] = 1u;
-        if (t == 0) flags[(sweep + 1u) % 3u] = 0u;
-        __syncthreads();
-        if (!flags[sweep % 3u]) break;
-    }
-    // counting sort by level: counts, exclusive offsets, then each item takes
-    // the next free position of its level
-    if (t == 0) flags[0] = 0u;
-    __syncthreads();
-    for (uint32_t p = lo; p < hi; ++p) atomicMax(&flags[0], lev[p]);
-    __syncthreads();
-    const uint32_t top = flags[0];
-    for (uint32_t l = t; l <= top + 1u; l += T) hist[l] = 0u;
-    __syncthreads();
-    for (uint32_t p = t; p < nit; p += T) atomicAdd(&hist[lev[p]], 1u);
-    __syncthreads();
-    if (t < 64u) {
-        const uint32_t len = top + 1u, c = (len + 63u) / 64u;
-        const uint32_t a = umin(t * c, len), b = umin(a + c, len);
-        uint32_t sum = 0u;
-        for (uint32_t l = a; l < b; ++l) sum += hist[l];
-        uint32_t run = wave_incl_scan(sum) - sum;
-        for (uint32_t l = a; l < b; ++l) {
-            const uint32_t x = hist[l];
-            hist[l] = run;
-            run += x;
-        }
-    }
-    __syncthreads();
-    for (uint32_t p = t; p < nit; p += T) perm[atomicAdd(&hist[lev[p]], 1u)] = p;
-    __syncthreads();
-}
-
-__global__ __launch_bounds__(256) void k_color(StepDev S, uint32_t lds_words)
-{
-    extern __shared__ __align__(16) uint32_t dyn[];
-    __shared__ uint32_t s_scan[256];
-    __shared__ uint32_t s_maxc, s_abort, s_base;
-    __shared__ uint32_t s_flags[3];
+    __shared__ uint32_t s_abort;
     if (S.counters[C_OVERFLOW]) return;
     const uint32_t w = blockIdx.x;
     const WorldDev& D = S.worlds[w];
     const uint32_t i0 = S.w_item_base[w], nit = S.w_item_base[w + 1] - i0;
     const uint32_t T = blockDim.x, t = threadIdx.x;
-    if (D.sched == 0) {
-        for (uint32_t p = t; p < nit; p += T) S.it_color[i0 + p] = 0u;
-        level_order(S.it_r0 + i0, S.it_r1 + i0, S.it_k0 + i0, S.it_k1 + i0, S.it_perm + i0, S.lists, S.deg_off, 0u,
-                    i0, nit, dyn, lds_words, s_flags);
-        return;
-    }
+    if (D.sched == 0) return;
     const uint32_t base = D.body_base;
     for (int b = t; b < D.nbodies; b += T) {
         S.cmask[2 * (base + b)] = 0ull;
         S.cmask[2 * (base + b) + 1] = 0ull;
         S.g_cnt[base + b] = 0u;
     }
-    if (t == 0) { s_maxc = 0u; s_abort = 0u; s_base = 0u; }
+    if (t == 0) s_abort = 0u;
     __syncthreads();
     uint32_t spins = 0;
     for (uint32_t p = t; p < nit;) {
@@ -1042,7 +975,6 @@ __global__ __launch_bounds__(256) void k_color(StepDev S, uint32_t lds_words)
             }
             if (r0 >= 0) st_rel(&S.g_cnt[r0], S.it_k0[it] + 1u);
             if (r1 >= 0) st_rel(&S.g_cnt[r1], S.it_k1[it] + 1u);
-            atomicMax(&s_maxc, umin(c, 128u));
             p += T;
             spins = 0;
         } else {
@@ -1054,31 +986,6 @@ __global__ __launch_bounds__(256) void k_color(StepDev S, uint32_t lds_words)
             }
             __builtin_amdgcn_s_sleep(1);
         }
-    }
-    __syncthreads();
-    if (s_abort) return;
-    // execution order: stable counting sort by min(colour, 128); each thread
-    // owns a contiguous chunk of items, bins are placed one after another
-    const uint32_t chunk = (nit + T - 1) / T;
-    const uint32_t lo = umin(t * chunk, nit), hi = umin(lo + chunk, nit);
-    const uint32_t maxc = s_maxc;
-    for (uint32_t bin = 0; bin <= maxc; ++bin) {
-        uint32_t cnt = 0;
-        for (uint32_t p = lo; p < hi; ++p) cnt += umin(S.it_color[i0 + p], 128u) == bin;
-        s_scan[t] = cnt;
-        __syncthreads();
-        for (uint32_t d = 1; d < T; d <<= 1) {
-            uint32_t v = t >= d ? s_scan[t - d] : 0u;
-            __syncthreads();
-            s_scan[t] += v;
-            __syncthreads();
-        }
-        uint32_t off = s_base + s_scan[t] - cnt;
-        for (uint32_t p = lo; p < hi; ++p)
-            if (umin(S.it_color[i0 + p], 128u) == bin) S.it_perm[i0 + off++] = p;
-        __syncthreads();
-        if (t == T - 1) s_base += s_scan[T - 1];
-        __syncthreads();
     }
 }
 
@@ -1112,561 +1019,6 @@ __global__ void k_list_rank(StepDev S)
 }
 
 // ---------------------------------------------------------------- solver
-template <bool LDS>
-struct SolverState {
-    float *mx, *my, *L, *im, *ii;
-    uint32_t *cnt, *deg;
-};
-
-
-
-// ------------------------------------------------------- solver item records
-// Each solver item of a step gets one 128-byte record at its execution
-// position, built in parallel at the first sub-step: the ordering bodies and
-// ranks, and for a manifold its normal, friction, both points' lever arms,
-// depths, effective masses (identical every sub-step unless updateTGSDepth
-// moves the point) and accumulated impulses.  A worker holds a record before
-// the item's dependencies are met (item_chain reads its next record while it
-// still waits on the current one; item_chain_lanes copies it into the lane's
-// LDS slot), so a link of a dependency chain touches only LDS body state.
-enum : uint32_t {
-    RF_JOINT = 1u, RF_P0 = 2u, RF_P1 = 4u, RF_W1 = 8u, RF_W2 = 16u, RF_S1 = 32u, RF_S2 = 64u,
-    RF_TGS = 128u,           // a point's depth is not its original depth: updateTGSDepth is live
-    RF_WARM = 256u           // warm started: each sub-step adds MP_WARM_N / MP_WARM_T to the impulses
-};
-constexpr uint32_t NONE = 0xffffffffu;
-
-// words: 0 flags, 1 body a (manifold ref / joint r0), 2 body b (inc / r1),
-// 3 index (manifold in the step arrays / world-local joint), 4-5 ranks at the
-// ordering bodies, 6 the ordering bodies' item counts, 7 the compact chain
-// indices (worlds beyond LDS); then the six rows a chain link reads: 8-10
-// normal + friction, 11-17 point 0 (r1x r1y r2x r2y depth mass_n mass_t),
-// 18-24 point 1, 25-26 the points' Baumgarte biases, 28-31 impulses (pn0 pt0
-// pn1 pt1)
-struct Rec {
-    uint32_t flags, a, b, idx, rk0, rk1;
-    float nx, ny, fric;
-    float p[2][7];
-    float acc[4];
-    uint32_t degs;       // items at r0 | items at r1 << 16; DEGS_WIDE when either needs more than 16 bits
-    float bias[2];       // Baumgarte bias of the sub-step per point, -1 when depth >= 0
-    uint32_t cpair;      // worlds beyond LDS: compact chain indices of (a, b) / the joint's (s1, s2)
-};
-constexpr uint32_t DEGS_WIDE = 0xffffffffu;
-
-constexpr uint32_t REC_LINK = 2;    // first of the six rows a chain link reads
-constexpr uint32_t REC_ACC = 7;     // the impulses' row
-
-__device__ __forceinline__ void rec_load(Rec& r, const uint4* q)
-{
-    const uint4 v0 = q[0], v1 = q[1], v2 = q[2], v3 = q[3], v4 = q[4], v5 = q[5], v6 = q[6], v7 = q[7];
-    r.flags = v0.x; r.a = v0.y; r.b = v0.z; r.idx = v0.w;
-    r.rk0 = v1.x; r.rk1 = v1.y; r.degs = v1.z; r.cpair = v1.w;
-    r.nx = __uint_as_float(v2.x); r.ny = __uint_as_float(v2.y); r.fric = __uint_as_float(v2.z);
-    r.p[0][0] = __uint_as_float(v2.w);
-    r.p[0][1] = __uint_as_float(v3.x); r.p[0][2] = __uint_as_float(v3.y); r.p[0][3] = __uint_as_float(v3.z);
-    r.p[0][4] = __uint_as_float(v3.w);
-    r.p[0][5] = __uint_as_float(v4.x); r.p[0][6] = __uint_as_float(v4.y); r.p[1][0] = __uint_as_float(v4.z);
-    r.p[1][1] = __uint_as_float(v4.w);
-    r.p[1][2] = __uint_as_float(v5.x); r.p[1][3] = __uint_as_float(v5.y); r.p[1][4] = __uint_as_float(v5.z);
-    r.p[1][5] = __uint_as_float(v5.w);
-    r.p[1][6] = __uint_as_float(v6.x); r.bias[0] = __uint_as_float(v6.y); r.bias[1] = __uint_as_float(v6.z);
-    r.acc[0] = __uint_as_float(v7.x); r.acc[1] = __uint_as_float(v7.y);
-    r.acc[2] = __uint_as_float(v7.z); r.acc[3] = __uint_as_float(v7.w);
-}
-
-// a record read by the compact chain: its bodies as compact indices
-__device__ __forceinline__ void rec_to_compact(Rec& r)
-{
-    const uint32_t c0 = r.cpair & 0xffffu, c1 = r.cpair >> 16;
-    r.a = c0;
-    if (r.flags & RF_JOINT) r.b = (r.b == NONE) ? NONE : c1;
-    else r.b = c1;
-}
-
-__device__ __forceinline__ void rec_store(const Rec& r, uint4* q)
-{
-    q[0] = make_uint4(r.flags, r.a, r.b, r.idx);
-    q[1] = make_uint4(r.rk0, r.rk1, r.degs, r.cpair);
-    q[2] = make_uint4(__float_as_uint(r.nx), __float_as_uint(r.ny), __float_as_uint(r.fric),
-                      __float_as_uint(r.p[0][0]));
-    q[3] = make_uint4(__float_as_uint(r.p[0][1]), __float_as_uint(r.p[0][2]), __float_as_uint(r.p[0][3]),
-                      __float_as_uint(r.p[0][4]));
-    q[4] = make_uint4(__float_as_uint(r.p[0][5]), __float_as_uint(r.p[0][6]), __float_as_uint(r.p[1][0]),
-                      __float_as_uint(r.p[1][1]));
-    q[5] = make_uint4(__float_as_uint(r.p[1][2]), __float_as_uint(r.p[1][3]), __float_as_uint(r.p[1][4]),
-                      __float_as_uint(r.p[1][5]));
-    q[6] = make_uint4(__float_as_uint(r.p[1][6]), __float_as_uint(r.bias[0]), __float_as_uint(r.bias[1]), 0u);
-    q[7] = make_uint4(__float_as_uint(r.acc[0]), __float_as_uint(r.acc[1]), __float_as_uint(r.acc[2]),
-                      __float_as_uint(r.acc[3]));
-}
-
-__device__ __forceinline__ int32_t rec_r0(const Rec& r)
-{
-    if (r.flags & RF_JOINT) return r.a == NONE ? -1 : (int32_t)r.a;
-    return (r.flags & RF_W1) ? (int32_t)r.a : -1;
-}
-__device__ __forceinline__ int32_t rec_r1(const Rec& r)
-{
-    if (r.flags & RF_JOINT) return r.b == NONE ? -1 : (int32_t)r.b;
-    return (r.flags & RF_W2) ? (int32_t)r.b : -1;
-}
-
-// the ordering bodies' item counts, packed when both fit 16 bits
-template <class ST>
-__device__ __forceinline__ uint32_t rec_degs(const Rec& r, const ST& st)
-{
-    int32_t q0 = rec_r0(r), q1 = rec_r1(r);
-    uint32_t d0 = q0 >= 0 ? st.deg[q0] : 0u, d1 = q1 >= 0 ? st.deg[q1] : 0u;
-    return (d0 > 0xffffu || d1 > 0xffffu) ? DEGS_WIDE : (d0 | (d1 << 16));
-}
-
-// Baumgarte bias of each point for a sub-step of length dt (collision.zig:172),
-// -1 for a point whose depth is >= 0 (calculateImpulses resets and skips it)
-__device__ __forceinline__ void rec_biases(Rec& r, float dt)
-{
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        float depth = r.p[p][4];
-        r.bias[p] = depth >= 0.f ? -1.0f : BAUMGARTE * maxn(0.0f, (-depth) - BAUMGARTE_SLOP) / dt;
-    }
-}
-
-// CollisionManifold.preStep effective masses (collision.zig:117-132) for one point
-template <class ST>
-__device__ __forceinline__ void rec_masses(Rec& r, const ST& st, int p)
-{
-    float im1 = st.im[r.a], im2 = st.im[r.b], ii1 = st.ii[r.a], ii2 = st.ii[r.b];
-    float inv_mass = im1 + im2;
-    v2 n = mk(r.nx, r.ny), t = rot90cw(n);
-    v2 r1 = mk(r.p[p][0], r.p[p][1]), r2 = mk(r.p[p][2], r.p[p][3]);
-    float r1n = cross2(r1, n), r2n = cross2(r2, n);
-    float kn = inv_mass + ii1 * (r1n * r1n) + ii2 * (r2n * r2n);
-    float r1t = cross2(r1, t), r2t = cross2(r2, t);
-    float kt = inv_mass + ii1 * (r1t * r1t) + ii2 * (r2t * r2t);
-    r.p[p][5] = kn > 0.0f ? 1.0f / kn : 0.0f;
-    r.p[p][6] = kt > 0.0f ? 1.0f / kt : 0.0f;
-}
-
-// record of the item at execution position `pos` (first sub-step)
-template <bool WARM = false, class ST>
-__device__ __forceinline__ void rec_build(Rec& r, const StepDev& S, const WorldDev& D, const ST& st, uint32_t pos,
-                                          uint32_t ibase, uint32_t nj, uint32_t mbeg, uint32_t base)
-{
-    const size_t cm = S.cap_m;
-    const float* P = S.m_pt;
-    uint32_t j = S.it_perm[ibase + pos];
-    uint32_t item = ibase + j;
-    r.rk0 = S.it_k0[item];
-    r.rk1 = S.it_k1[item];
-    r.nx = r.ny = r.fric = 0.0f;
-    r.degs = 0u;
-    r.bias[0] = r.bias[1] = -1.0f;
-    r.cpair = 0u;
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int f = 0; f < 7; ++f) r.p[p][f] = 0.0f;
-#pragma unroll
-    for (int f = 0; f < 4; ++f) r.acc[f] = 0.0f;
-    if (j < nj) {
-        int32_t r0 = S.it_r0[item], r1 = S.it_r1[item];
-        r.flags = RF_JOINT;
-        r.a = r0 >= 0 ? (uint32_t)(r0 - (int32_t)base) : NONE;
-        r.b = r1 >= 0 ? (uint32_t)(r1 - (int32_t)base) : NONE;
-        r.idx = j;
-        return;
-    }
-    uint32_t m = mbeg + (j - nj);
-    r.idx = m;
-    r.a = S.m_ref[m] - base;
-    r.b = S.m_inc[m] - base;
-    r.flags = 0u;
-    if (S.sflag[base + r.a] & SF_RESOURCE) r.flags |= RF_W1;
-    if (S.sflag[base + r.b] & SF_RESOURCE) r.flags |= RF_W2;
-    if (D.flags[r.a] & BF_STATIC) r.flags |= RF_S1;
-    if (D.flags[r.b] & BF_STATIC) r.flags |= RF_S2;
-    r.nx = S.m_nx[m];
-    r.ny = S.m_ny[m];
-    r.fric = sqrt_rn(D.mu[r.a] * D.mu[r.b]);   // preStep (collision.zig:114)
-    uint32_t valid = S.m_valid[m];
-    if constexpr (WARM)
-        if (valid & MV_WARM) r.flags |= RF_WARM;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        if (!(valid & (1u << p))) continue;
-        r.flags |= (RF_P0 << p);
-        r.p[p][0] = P[(MP_R1X * 2 + p) * cm + m];
-        r.p[p][1] = P[(MP_R1Y * 2 + p) * cm + m];
-        r.p[p][2] = P[(MP_R2X * 2 + p) * cm + m];
-        r.p[p][3] = P[(MP_R2Y * 2 + p) * cm + m];
-        r.p[p][4] = P[(MP_DEPTH * 2 + p) * cm + m];
-        if (!approx(r.p[p][4], P[(MP_ODEPTH * 2 + p) * cm + m], 1e-4f)) r.flags |= RF_TGS;
-        rec_masses(r, st, p);
-    }
-}
-
-// updateTGSDepth (collision.zig:73-100) for a record whose points may move:
-// rotate lever arms by the bodies' rotation since the previous sub-step,
-// recompute depth and (preStep) the effective masses
-// DV: WorldDev or PassArrays (the body arrays it reads: ang, px, py)
-template <class ST, class DV>
-__device__ __forceinline__ void rec_tgs(Rec& r, const StepDev& S, const DV& D, const ST& st, bool = false)
-{
-    const uint32_t m = r.idx;
-    const size_t cm = S.cap_m;
-    const float* P = S.m_pt;
-    // everything the update may read, loaded before any of it is tested (one
-    // round trip instead of three dependent ones; the indices are valid
-    // whether or not a point is present or moved)
-    const float a1 = D.ang[r.a], a2 = D.ang[r.b];
-    const float prev1 = S.m_prev1[m], prev2 = S.m_prev2[m];
-    const float ods[2] = {P[(MP_ODEPTH * 2 + 0) * cm + m], P[(MP_ODEPTH * 2 + 1) * cm + m]};
-    const v2 pa = mk(D.px[r.a], D.py[r.a]), pb = mk(D.px[r.b], D.py[r.b]);
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        if (!(r.flags & (RF_P0 << p))) continue;
-        const float od = ods[p];
-        if (approx(r.p[p][4], od, 1e-4f)) continue;
-        v2 rr1 = rotate2(mk(r.p[p][0], r.p[p][1]), a1 - prev1);
-        v2 rr2 = rotate2(mk(r.p[p][2], r.p[p][3]), a2 - prev2);
-        v2 q1 = add2(rr1, pa);
-        v2 q2 = add2(rr2, pb);
-        float dd = dot2(mk(r.nx, r.ny), sub2(q2, q1));
-        r.p[p][4] = dd + od;
-        r.p[p][0] = rr1.x; r.p[p][1] = rr1.y; r.p[p][2] = rr2.x; r.p[p][3] = rr2.y;
-        rec_masses(r, st, p);
-    }
-    S.m_prev1[m] = a1;
-    S.m_prev2[m] = a2;
-}
-
-// What a joint link reads besides the bodies' momentum and inverse masses:
-// parameters and the pose of its bodies, constant within a sub-step.
-struct JointIn {
-    uint32_t type;
-    bool stat1;                       // body 1 is static (fixed / motor joints skip)
-    float pmax, pmin, beta, target;
-    float r1x, r1y, r2x, r2y, tx, ty;
-    v2 pa, pb;                        // positions
-    float ca, sa, cb, sb;             // cos / sin of the angles (offset joints)
-    float I1, tq1;                    // inertia and torque of body 1 (motor joints)
-};
-
-// Constraint.solve (Constraints/*.zig) with momentum / inverse masses at st
-// indices a and b
-template <class ST>
-__device__ __forceinline__ void joint_apply(const JointIn& j, const ST& st, uint32_t a, uint32_t b, float dt)
-{
-    const float pmax = j.pmax, pmin = j.pmin, beta = j.beta, target = j.target;
-    if (j.type == 0) {
-        // DistanceJoint.solve (DistanceJoint.zig:40-75)
-        float w1 = st.im[a], w2 = st.im[b];
-        v2 v1 = scale2(mk(st.mx[a], st.my[a]), w1);
-        v2 v2v = scale2(mk(st.mx[b], st.my[b]), w2);
-        v2 rv = sub2(v2v, v1);
-        v2 pa = j.pa, pb = j.pb;
-        v2 n = normalize2(sub2(pb, pa));
-        float dist_err = length2(sub2(pb, pa)) - target;
-        float pc = beta * dist_err / maxn(target, 0.001f);
-        float Jv = -(dot2(rv, n) + pc) / (w1 + w2);
-        float ndv = dot2(n, rv);
-        float den = 1.0f / maxn(absf(ndv), GRAD_DIV_LIMIT);
-        Jv = clampn(Jv, pmin * den, pmax * den);
-        v2 dp = scale2(n, Jv);
-        st.mx[a] -= dp.x; st.my[a] -= dp.y;
-        st.mx[b] += dp.x; st.my[b] += dp.y;
-    } else if (j.type == 1) {
-        // OffsetDistanceJoint.solve (OffsetDistanceJoint.zig:44-105)
-        v2 r1 = mk(j.r1x, j.r1y), r2 = mk(j.r2x, j.r2y);
-        v2 rr1 = rotcs(r1, j.ca, j.sa), rr2 = rotcs(r2, j.cb, j.sb);
-        v2 a1 = add2(rr1, j.pa);
-        v2 a2 = add2(rr2, j.pb);
-        v2 n = normalize2(sub2(a2, a1));
-        float im1 = st.im[a], im2 = st.im[b], ii1 = st.ii[a], ii2 = st.ii[b];
-        v2 vl1 = scale2(mk(st.mx[a], st.my[a]), im1);
-        float w1 = st.L[a] * ii1;
-        v2 vl2 = scale2(mk(st.mx[b], st.my[b]), im2);
-        float w2 = st.L[b] * ii2;
-        v2 v1 = add2(vl1, mk(-rr1.y * w1, rr1.x * w1));
-        v2 v2v = add2(vl2, mk(-rr2.y * w2, rr2.x * w2));
-        v2 dv = sub2(v2v, v1);
-        float dist_err = length2(sub2(a2, a1)) - target;
-        float pc = beta * dist_err / maxn(target, GRAD_DIV_LIMIT);
-        float num = dot2(n, dv) + pc;
-        float r1xn = cross2(rr1, n), r2xn = cross2(rr2, n);
-        float den = im1 + im2 + r1xn * r1xn * ii1 + r2xn * r2xn * ii2;
-        float Jv = -num / den;
-        float ndv = dot2(n, dv);
-        float den2 = 1.0f / maxn(absf(ndv), GRAD_DIV_LIMIT);
-        Jv = clampn(Jv, pmin * den2, pmax * den2);
-        v2 dp = scale2(n, Jv);
-        st.mx[a] -= dp.x; st.my[a] -= dp.y;
-        st.L[a] -= Jv * r1xn;
-        st.mx[b] += dp.x; st.my[b] += dp.y;
-        st.L[b] += Jv * r2xn;
-    } else if (j.type == 2) {
-        // FixedPositionJoint.solve (FixedPositionJoint.zig:38-72)
-        if (j.stat1) return;
-        float w = st.im[a];
-        v2 v = scale2(mk(st.mx[a], st.my[a]), w);
-        v2 delta = sub2(mk(j.tx, j.ty), j.pa);
-        float dist = length2(delta);
-        if (dist < ALLOWED_CONSTRAINT_VALUE) return;
-        v2 n = scale2(delta, 1.0f / dist);
-        float bias = beta * dist;
-        float rv = dot2(v, n);
-        float Jv = -(rv - bias) / w;
-        float den = 1.0f / maxn(absf(rv), ALLOWED_CONSTRAINT_VALUE);
-        Jv = clampn(Jv, pmin * den, pmax * den);
-        v2 dp = scale2(n, Jv);
-        st.mx[a] += dp.x; st.my[a] += dp.y;
-    } else {
-        // MotorJoint.solve (MotorJoint.zig:38-64)
-        if (j.stat1) return;
-        float I = j.I1;
-        float omega = st.L[a] / I;
-        float C = omega - target;
-        if (absf(C) < ALLOWED_CONSTRAINT_VALUE) return;
-        float bias = beta * C;
-        float tq = j.tq1;
-        float Jv = tq - bias;
-        float rel = tq / I;
-        float den = 1.0f / maxn(absf(rel), ALLOWED_CONSTRAINT_VALUE);
-        Jv = clampn(Jv, pmin * den, pmax * den);
-        st.L[a] += Jv * dt;
-    }
-}
-
-// Joint records keep what the link reads in the fields a contact uses for its
-// points: p[0] = pmax pmin beta r1x r1y r2x r2y, p[1][0..2] = target tx ty,
-// p[1][3..6] = positions of the two bodies, (nx, ny, fric, acc[0]) = cos / sin
-// of both angles, acc[1] / acc[2] = inertia / torque of body 1; the type in
-// flags bits 24-30 and RF_S1 when body 1 is static.
-__device__ __forceinline__ void rec_joint_params(Rec& r, const Joint& J, const WorldDev& D)
-{
-    r.flags |= (uint32_t)J.type << 24;
-    if (D.flags[J.s1] & BF_STATIC) r.flags |= RF_S1;
-    r.p[0][0] = J.pmax; r.p[0][1] = J.pmin; r.p[0][2] = J.beta;
-    r.p[0][3] = J.r1x; r.p[0][4] = J.r1y; r.p[0][5] = J.r2x; r.p[0][6] = J.r2y;
-    r.p[1][0] = J.target; r.p[1][1] = J.tx; r.p[1][2] = J.ty;
-}
-
-// the sub-step's pose of a joint record's bodies (after the previous
-// sub-step's position integration; torque as set for this sub-step);
-// DV: WorldDev or PassArrays
-template <class DV>
-__device__ __forceinline__ void rec_joint_pose(Rec& r, const Joint& J, const DV& D)
-{
-    const int32_t a = J.s1, b = J.s2;
-    r.p[1][3] = D.px[a]; r.p[1][4] = D.py[a];
-    r.acc[1] = D.inertia[a];
-    r.acc[2] = D.tq[a];
-    if (J.type == 1) {
-        float angle_a = D.ang[a], angle_b = D.ang[b];
-        r.nx = cosf_r(angle_a); r.ny = sinf_r(angle_a);
-        r.fric = cosf_r(angle_b); r.acc[0] = sinf_r(angle_b);
-    }
-    if (J.type <= 1) { r.p[1][5] = D.px[b]; r.p[1][6] = D.py[b]; }
-}
-
-template <class ST>
-__device__ __forceinline__ void rec_solve_joint(const Rec& r, const ST& st, uint32_t ua, uint32_t ub, float dt)
-{
-    JointIn j;
-    j.type = (r.flags >> 24) & 0x7fu;
-    j.stat1 = (r.flags & RF_S1) != 0;
-    j.pmax = r.p[0][0]; j.pmin = r.p[0][1]; j.beta = r.p[0][2];
-    j.r1x = r.p[0][3]; j.r1y = r.p[0][4]; j.r2x = r.p[0][5]; j.r2y = r.p[0][6];
-    j.target = r.p[1][0]; j.tx = r.p[1][1]; j.ty = r.p[1][2];
-    j.pa = mk(r.p[1][3], r.p[1][4]); j.pb = mk(r.p[1][5], r.p[1][6]);
-    j.ca = r.nx; j.sa = r.ny; j.cb = r.fric; j.sb = r.acc[0];
-    j.I1 = r.acc[1]; j.tq1 = r.acc[2];
-    joint_apply(j, st, ua, ub, dt);
-}
-
-// one body's solver state as read by a chain link
-struct BodyState {
-    float mx, my, L, im, ii;
-};
-
-__device__ __forceinline__ float lds_relaxed(const float* p)
-{
-    return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_WORKGROUP));
-}
-
-// a body's state read without ordering: only for LDS, where one workgroup's
-// operations are served in order (see the dataflow loops)
-template <class ST>
-__device__ __forceinline__ BodyState body_state(const ST& st, uint32_t i)
-{
-    return BodyState{lds_relaxed(&st.mx[i]), lds_relaxed(&st.my[i]), lds_relaxed(&st.L[i]), lds_relaxed(&st.im[i]),
-                     lds_relaxed(&st.ii[i])};
-}
-
-// The light compact chain's state (worlds beyond LDS whose touched bodies
-// exceed the full compact state but whose momentum and counters fit LDS):
-// momentum and counter of each touched body in LDS under its compact index;
-// a link's inverse masses and inertias come with its item (a sixth row of the
-// lane slot, from S.rmass), and the pair proxies answer st.im[i] / st.ii[i]
-// for the item's two bodies (the first body's index, else the second's); an
-// item count per body (only items whose counts need more than 16 bits read
-// it) is looked up in global memory.
-struct PairValue {
-    uint32_t a;
-    float va, vb;
-    __device__ __forceinline__ float operator[](uint32_t i) const { return i == a ? va : vb; }
-};
-struct DegLookup {
-    const uint32_t* deg;
-    const uint32_t* cinv;
-    uint32_t base;
-    __device__ __forceinline__ uint32_t operator[](uint32_t c) const { return deg[base + cinv[base + c]]; }
-};
-struct LiteState {
-    float *mx, *my, *L;
-    uint32_t* cnt;
-    PairValue im, ii;
-    DegLookup deg;
-    const uint4* rmass;      // the world's item masses, by execution position
-};
-template <class ST>
-struct IsLite {
-    static constexpr bool value = false;
-};
-template <>
-struct IsLite<LiteState> {
-    static constexpr bool value = true;
-};
-
-__device__ __forceinline__ BodyState body_state(const LiteState& st, uint32_t i)
-{
-    return BodyState{lds_relaxed(&st.mx[i]), lds_relaxed(&st.my[i]), lds_relaxed(&st.L[i]), st.im[i], st.ii[i]};
-}
-
-// the same with ordinary loads (after the item's counters were acquired)
-template <class ST>
-__device__ __forceinline__ BodyState body_state_ordered(const ST& st, uint32_t i)
-{
-    return BodyState{st.mx[i], st.my[i], st.L[i], st.im[i], st.ii[i]};
-}
-
-// CollisionManifold.calculateImpulses (collision.zig:135-218) on a slot or a
-// record, with both bodies' state already read (the link's only reads of
-// them) and the Baumgarte bias of the sub-step precomputed
-// ((0.02 max(0, -depth - 0.005)) / dt, collision.zig:172; -1 marks depth >= 0)
-template <bool WARM = false, class Item, class ST>
-__device__ __forceinline__ void contact_impulses(Item& z, uint32_t l1, uint32_t l2, const BodyState& b1,
-                                                 const BodyState& b2, const ST& st)
-{
-    v2 vl1 = scale2(mk(b1.mx, b1.my), b1.im);
-    float om1 = b1.L * b1.ii;
-    v2 vl2 = scale2(mk(b2.mx, b2.my), b2.im);
-    float om2 = b2.L * b2.ii;
-    v2 n = mk(z.nx, z.ny);
-    v2 t = rot90cw(n);
-    v2 app1 = mk(0.f, 0.f), app2 = mk(0.f, 0.f);
-    float rot1 = 0.f, rot2 = 0.f;
-    // straight-line code with selects: a point that is absent, separated
-    // (bias < 0: its impulses reset) or below the minimum impulse changes
-    // nothing else, exactly as skipping it would.  A warm-started manifold
-    // has no minimum: its accumulated impulse may shrink (clamped at 0), so a
-    // carried impulse that is too large can be taken back.
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        // the second point only when a lane running this link has one (a
-        // wave whose links are all one-point manifolds skips its half of the
-        // instructions; for an absent point the selects below change nothing)
-        if (p == 1 && __ballot((z.flags & RF_P1) != 0u) == 0ull) break;
-        const bool on = (z.flags & (RF_P0 << p)) != 0u;
-        const bool sep = z.bias[p] < 0.f;
-        v2 r1 = mk(z.p[p][0], z.p[p][1]), r2 = mk(z.p[p][2], z.p[p][3]);
-        v2 v1 = add2(vl1, mk(-r1.y * om1, r1.x * om1));
-        v2 v2v = add2(vl2, mk(-r2.y * om2, r2.x * om2));
-        v2 dv = sub2(v1, v2v);
-        float num = dot2(dv, n) + z.bias[p];
-        float pn = num * z.p[p][5];
-        const bool go = on && !sep && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (z.flags & RF_WARM) != 0u));
-        num = dot2(dv, t);
-        float pt = num * z.p[p][6];
-        float acc_pn = z.acc[2 * p], acc_pt = z.acc[2 * p + 1];
-        float new_pn = maxn(0.0f, acc_pn + pn);
-        float applied_pn = new_pn - acc_pn;
-        float max_pt = z.fric * absf(new_pn);
-        float new_pt = clampn(acc_pt + pt, -max_pt, max_pt);
-        float applied_pt = new_pt - acc_pt;
-        const bool clr = on && sep;
-        z.acc[2 * p] = clr ? 0.f : (go ? new_pn : acc_pn);
-        z.acc[2 * p + 1] = clr ? 0.f : (go ? new_pt : acc_pt);
-        v2 dp = add2(scale2(n, applied_pn), scale2(t, applied_pt));
-        const bool g1 = go && !(z.flags & RF_S1), g2 = go && !(z.flags & RF_S2);
-        const float a1x = app1.x - dp.x, a1y = app1.y - dp.y, q1 = rot1 - cross2(r1, dp);
-        const float a2x = app2.x + dp.x, a2y = app2.y + dp.y, q2 = rot2 + cross2(r2, dp);
-        app1.x = g1 ? a1x : app1.x; app1.y = g1 ? a1y : app1.y; rot1 = g1 ? q1 : rot1;
-        app2.x = g2 ? a2x : app2.x; app2.y = g2 ? a2y : app2.y; rot2 = g2 ? q2 : rot2;
-    }
-    if (z.flags & RF_W1) { st.mx[l1] = b1.mx + app1.x; st.my[l1] = b1.my + app1.y; st.L[l1] = b1.L + rot1; }
-    if (z.flags & RF_W2) { st.mx[l2] = b2.mx + app2.x; st.my[l2] = b2.my + app2.y; st.L[l2] = b2.L + rot2; }
-}
-
-// record -> the step's manifold arrays (what r2d_get_manifolds reports)
-__device__ __forceinline__ void rec_writeback(const Rec& r, const StepDev& S)
-{
-    if (r.flags & RF_JOINT) return;
-    const size_t cm = S.cap_m;
-    float* P = S.m_pt;
-    const uint32_t m = r.idx;
-    S.m_fric[m] = r.fric;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        if (!(r.flags & (RF_P0 << p))) continue;
-        P[(MP_ACC_PN * 2 + p) * cm + m] = r.acc[2 * p];
-        P[(MP_ACC_PT * 2 + p) * cm + m] = r.acc[2 * p + 1];
-        P[(MP_MASS_N * 2 + p) * cm + m] = r.p[p][5];
-        P[(MP_MASS_T * 2 + p) * cm + m] = r.p[p][6];
-        P[(MP_R1X * 2 + p) * cm + m] = r.p[p][0];
-        P[(MP_R1Y * 2 + p) * cm + m] = r.p[p][1];
-        P[(MP_R2X * 2 + p) * cm + m] = r.p[p][2];
-        P[(MP_R2Y * 2 + p) * cm + m] = r.p[p][3];
-        P[(MP_DEPTH * 2 + p) * cm + m] = r.p[p][4];
-    }
-}
-
-// LDS of the register-slot kernel: 13 words of body state per body
-__host__ __device__ inline size_t slot_lds_bytes(int nbodies) { return (size_t)nbodies * 13u * 4u; }
-
-// Which solve kernel steps a world: 0 the register-slot kernel (at most
-// slot_nmax bodies and slot_cap items), 1 the record kernel with LDS body
-// state (at most lds_nmax bodies), 2 the record kernel with body state in
-// global memory.  Every kernel evaluates the same rule, so each world is
-// stepped by exactly one of them.
-__device__ __forceinline__ int solve_route(uint32_t n, uint32_t nitems, uint32_t slot_cap, uint32_t slot_nmax,
-                                           uint32_t lds_nmax, bool warm)
-{
-    if (slot_cap && !warm && n <= slot_nmax && nitems <= slot_cap) return 0;
-    if (n <= lds_nmax) return 1;
-    return 2;
-}
-
-// ---------------------------------------------- solve building blocks
-// Per-body and per-item parts of Solver.process's sub-step loop
-// (lib.zig:199-250), shared by the one-workgroup-per-world kernels and by the
-// grid-wide kernels used for worlds whose body state does not fit LDS.
-
-// inverse mass / inertia (static: 0) and item count of body i (degs: the
-// world's item counts per body)
-template <class ST>
-__device__ __forceinline__ void body_setup(const WorldDev& D, const ST& st, int i, bool copy_state,
-                                           const uint32_t* degs)
-{
-    bool stat = (D.flags[i] & BF_STATIC) != 0;
-    if (copy_state) { st.mx[i] = D.mx[i]; st.my[i] = D.my[i]; st.L[i] = D.L[i]; }
-    st.im[i] = stat ? 0.0f : 1.0f / D.mass[i];
-    st.ii[i] = stat ? 0.0f : 1.0f / D.inertia[i];
-    st.deg[i] = degs[i];
-}
-
 // The body arrays that the per-body passes of a sub-step read and write,
 // copied out of the world's descriptor once per pass and typed by address
 // space: global for the body arrays (their loads and stores then wait on the
@@ -1698,146 +1050,7 @@ __device__ __forceinline__ BodyArrays body_arrays(const WorldDev& D)
 
 // body i's warm impulse per sub-step (momentum x, y, angular: the first
 // three floats of its float4)
-__device__ __forceinline__ const float* warm_sum(const WorldDev& D, int i)
-{
-    return reinterpret_cast<const float*>(&D.wsum[i]);
-}
 __device__ __forceinline__ GlbCF warm_sum(const BodyArrays& D, int i) { return D.wsum + 4 * i; }
-
-// what body_forces reads of body i, loaded before any of it is used (one
-// round trip; every index is valid whatever the flags)
-struct ForceIn {
-    uint32_t f;
-    float fx, fy, mass, px, py, tq, ang, hw, hh, rad;
-};
-template <class DV>
-__device__ __forceinline__ ForceIn force_in(const DV& D, int i)
-{
-    return ForceIn{D.flags[i], D.fx[i], D.fy[i], D.mass[i], D.px[i], D.py[i], D.tq[i], D.ang[i], D.hw[i], D.hh[i],
-                   D.rad[i]};
-}
-
-// forces (lib.zig:200-205), AABB refresh + velocity integration
-// (lib.zig:207-216) for body i from its loaded inputs; clears its solver
-// counter.  DV: WorldDev or BodyArrays.
-template <bool WARM = false, class ST, class DV>
-__device__ __forceinline__ void body_forces_in(const DV& D, const ST& st, int i, const ForceIn& in, bool last,
-                                               float sub_dt)
-{
-    const uint32_t f = in.f;
-    const float fx0 = in.fx, fy0 = in.fy, mass = in.mass, px = in.px, py = in.py, tq = in.tq;
-    const float ang = in.ang, bhw = in.hw, bhh = in.hh, rad = in.rad;
-    const bool stat = (f & BF_STATIC) != 0;
-    float fx = fx0, fy = fy0;
-    if (!stat) {
-        for (int g = 0; g < D.ngens; ++g) {
-            const auto& G = D.gens[g];   // fields read one by one (keeps G's address space)
-            if (G.type == 0) {
-                fx += G.gx * mass;
-                fy += G.gy * mass;
-            } else if (G.slot == i) {
-                float inv_m = 1.0f / mass;
-                v2 v = scale2(mk(st.mx[i], st.my[i]), inv_m);
-                v2 d = sub2(mk(px, py), mk(G.ax, G.ay));
-                fx += (-G.k) * d.x - G.c * v.x;
-                fy += (-G.k) * d.y - G.c * v.y;
-            }
-        }
-    }
-    if (last) {
-        // Disc.updateAABB / Rectangle.updateAABB; only the last refresh is observable
-        float hw, hh;
-        if (f & BF_RECT) {
-            float c = cosf_r(ang), sn = sinf_r(ang);
-            float x = bhw, y = bhh;
-            v2 lv[4] = {mk(-x, -y), mk(-x, y), mk(x, y), mk(x, -y)};
-            hw = 0.f; hh = 0.f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                v2 r = rotcs(lv[k], c, sn);
-                if (r.x > hw) hw = r.x;
-                if (r.y > hh) hh = r.y;
-            }
-        } else {
-            hw = rad; hh = rad;
-        }
-        D.ax[i] = px; D.ay[i] = py; D.ahw[i] = hw; D.ahh[i] = hh;
-    }
-    if (!stat) {
-        st.mx[i] += fx * sub_dt;
-        st.my[i] += fy * sub_dt;
-        st.L[i] += tq * sub_dt;
-        if constexpr (WARM) {
-            if (D.warm > 0.0f) {
-                // warm starting: the body's share of the matched manifolds' carried impulses
-                const auto ws = warm_sum(D, i);
-                st.mx[i] += ws[0];
-                st.my[i] += ws[1];
-                st.L[i] += ws[2];
-            }
-        }
-    }
-    D.fx[i] = fx; D.fy[i] = fy;
-    st.cnt[i] = 0u;
-}
-
-template <bool WARM = false, class ST, class DV>
-__device__ __forceinline__ void body_forces(const DV& D, const ST& st, int i, bool last, float sub_dt)
-{
-    body_forces_in<WARM>(D, st, i, force_in(D, i), last, sub_dt);
-}
-
-// what body_positions reads of body i, loaded before any of it is used
-struct PosIn {
-    uint32_t f;
-    float mass, inertia, px, py, ang;
-};
-template <class DV>
-__device__ __forceinline__ PosIn pos_in(const DV& D, int i)
-{
-    return PosIn{D.flags[i], D.mass[i], D.inertia[i], D.px[i], D.py[i], D.ang[i]};
-}
-
-// position integration (lib.zig:238-249) for body i from its loaded inputs;
-// DV: WorldDev or BodyArrays
-template <class ST, class DV>
-__device__ __forceinline__ void body_positions_in(const DV& D, const ST& st, int i, const PosIn& in, float sub_dt)
-{
-    const uint32_t f = in.f;
-    const float mass = in.mass, inertia = in.inertia, px = in.px, py = in.py, ang = in.ang;
-    if (f & BF_STATIC) return;
-    float qd = sub_dt / mass;
-    D.px[i] = px + st.mx[i] * qd;
-    D.py[i] = py + st.my[i] * qd;
-    D.ang[i] = ang + st.L[i] * sub_dt / inertia;
-    D.fx[i] = 0.0f; D.fy[i] = 0.0f;
-    D.tq[i] = 0.0f;
-}
-
-template <class ST, class DV>
-__device__ __forceinline__ void body_positions(const DV& D, const ST& st, int i, float sub_dt)
-{
-    body_positions_in(D, st, i, pos_in(D, i), sub_dt);
-}
-
-// A per-body pass over [0, n) in rounds of K bodies per thread: each round
-// loads the inputs of all its bodies before it applies the update to any, so
-// their loads are in flight together (bodies are independent in these
-// passes, so the order changes no result).
-template <int K, class In, class Load, class Apply>
-__device__ __forceinline__ void body_pass(int n, Load load, Apply apply)
-{
-    const int T = blockDim.x;
-    for (int i0 = threadIdx.x; i0 < n; i0 += K * T) {
-        In in[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-            if (i0 + k * T < n) in[k] = load(i0 + k * T);
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-            if (i0 + k * T < n) apply(i0 + k * T, in[k]);
-    }
-}
 
 // ------------------------------------------------------------ warm starting
 // Opt-in, not in the reference (its roadmap item "persist manifolds across
@@ -1954,566 +1167,6 @@ __device__ __forceinline__ void warm_save(const StepDev& S, const WorldDev& D, u
     e[2] = make_uint4(__float_as_uint(P[(MP_ACC_PT * 2 + 1) * cm + m]), 0u, 0u, 0u);
 }
 
-// the record of execution position pos (first sub-step's preStep)
-template <bool WARM = false, class ST>
-__device__ __forceinline__ void item_build(const StepDev& S, const WorldDev& D, const ST& st, uint4* recs, uint32_t pos,
-                                           uint32_t ibase, uint32_t mbeg, float sub_dt)
-{
-    Rec r;
-    rec_build<WARM>(r, S, D, st, pos, ibase, (uint32_t)D.njoints, mbeg, D.body_base);
-    r.degs = rec_degs(r, st);
-    if (r.flags & RF_JOINT) {
-        const Joint& J = D.joints[r.idx];
-        rec_joint_params(r, J, D);
-        rec_joint_pose(r, J, D);
-    } else {
-        rec_biases(r, sub_dt);
-    }
-    rec_store(r, recs + (size_t)pos * 8);
-}
-
-// The body arrays that the per-sub-step item pass reads, copied out of the
-// world's descriptor once per pass: through a reference to the descriptor
-// (global memory) the compiler reloads each pointer for every item, since it
-// cannot tell that the pass's own stores leave the descriptor unchanged.
-struct PassArrays {
-    const float *px, *py, *ang, *inertia, *tq;
-    const Joint* joints;
-};
-__device__ __forceinline__ PassArrays pass_arrays(const WorldDev& D)
-{
-    return PassArrays{D.px, D.py, D.ang, D.inertia, D.tq, D.joints};
-}
-
-// updateTGSDepth (collision.zig:73-100): live only for records flagged at
-// build time; every manifold's previous angles end as the last sub-step's.
-// DV: WorldDev or PassArrays.
-// h: the record's header row (recs[pos * 8])
-template <bool WARM = false, class ST, class DV>
-__device__ __forceinline__ void item_tgs_h(const StepDev& S, const DV& D, const ST& st, uint4* recs, uint32_t pos,
-                                           uint4 h, bool last, float sub_dt)
-{
-    uint4* q = recs + (size_t)pos * 8;
-    if (h.x & RF_JOINT) {
-        Rec r;
-        rec_load(r, q);
-        rec_joint_pose(r, D.joints[h.w], D);
-        rec_store(r, q);
-        return;
-    }
-    if (WARM && (h.x & RF_WARM)) {
-        // warm starting: the carried impulse per sub-step joins the accumulators
-        const size_t cm = S.cap_m;
-        const float* P = S.m_pt;
-        uint4 a = q[REC_ACC];
-        if (h.x & RF_P0) {
-            a.x = __float_as_uint(__uint_as_float(a.x) + P[(MP_WARM_N * 2 + 0) * cm + h.w]);
-            a.y = __float_as_uint(__uint_as_float(a.y) + P[(MP_WARM_T * 2 + 0) * cm + h.w]);
-        }
-        if (h.x & RF_P1) {
-            a.z = __float_as_uint(__uint_as_float(a.z) + P[(MP_WARM_N * 2 + 1) * cm + h.w]);
-            a.w = __float_as_uint(__uint_as_float(a.w) + P[(MP_WARM_T * 2 + 1) * cm + h.w]);
-        }
-        q[REC_ACC] = a;
-    }
-    if (h.x & RF_TGS) {
-        Rec r;
-        rec_load(r, q);
-        rec_tgs(r, S, D, st);
-        rec_biases(r, sub_dt);
-        rec_store(r, q);
-    } else if (last) {
-        S.m_prev1[h.w] = D.ang[h.y];
-        S.m_prev2[h.w] = D.ang[h.z];
-    }
-}
-
-template <bool WARM = false, class ST, class DV>
-__device__ __forceinline__ void item_tgs(const StepDev& S, const DV& D, const ST& st, uint4* recs, uint32_t pos,
-                                         bool last, float sub_dt)
-{
-    item_tgs_h<WARM>(S, D, st, recs, pos, recs[(size_t)pos * 8], last, sub_dt);
-}
-
-// K iterations of one sub-step's (constraints, manifolds) for the world of
-// this workgroup, as an ordered dataflow
-template <bool LDS, bool COMPACT, bool WARM = false, class ST>
-__device__ __forceinline__ void item_chain(const StepDev& S, const WorldDev& D, const ST& st, uint4* recs,
-                                           uint32_t nitems, uint32_t iters, float sub_dt, uint32_t w,
-                                           uint32_t& s_abort)
-{
-    // K iterations of (constraints, manifolds) as one ordered dataflow.  With
-    // LDS body state a link's counters and its bodies' state are read
-    // together (LDS serves one workgroup's operations in order, so state read
-    // after a counter that shows the item ready is what its predecessor
-    // released; values read for an item that is not ready are discarded);
-    // with body state in global memory the state is read after an acquire.
-    {
-        const uint32_t p_begin = threadIdx.x, p_step = blockDim.x;
-        uint32_t pcur = p_begin, kcur = (p_begin < nitems) ? 0u : iters;
-        Rec cur, nxt;
-        uint32_t cur_pos = 0, cur_k = 0, nxt_pos = 0, nxt_k = 0;
-        bool have = false, has_nxt = false;
-        if (kcur < iters) {
-            rec_load(nxt, recs + (size_t)pcur * 8);
-            if (COMPACT) rec_to_compact(nxt);
-            nxt_pos = pcur; nxt_k = kcur; has_nxt = true;
-            pcur += p_step;
-            if (pcur >= nitems) { pcur = p_begin; ++kcur; }
-        }
-        int32_t r0 = -1, r1 = -1;
-        uint32_t t0 = 0, t1 = 0;
-        uint32_t spins = 0;
-        while (true) {
-            if (!have) {
-                if (!has_nxt) break;
-                cur = nxt;
-                cur_pos = nxt_pos;
-                cur_k = nxt_k;
-                has_nxt = false;
-                have = true;
-                // prefetch the following position; the same position in the
-                // next iteration reads impulses this record is about to write,
-                // so that case is forwarded from registers instead
-                if (kcur < iters) {
-                    if (pcur != cur_pos) {
-                        rec_load(nxt, recs + (size_t)pcur * 8);
-                        if (COMPACT) rec_to_compact(nxt);
-                    }
-                    nxt_pos = pcur; nxt_k = kcur; has_nxt = true;
-                    pcur += p_step;
-                    if (pcur >= nitems) { pcur = p_begin; ++kcur; }
-                }
-                r0 = rec_r0(cur);
-                r1 = rec_r1(cur);
-                if (cur.degs != DEGS_WIDE) {
-                    t0 = cur_k * (cur.degs & 0xffffu) + cur.rk0;
-                    t1 = cur_k * (cur.degs >> 16) + cur.rk1;
-                } else {
-                    if (r0 >= 0) t0 = cur_k * st.deg[r0] + cur.rk0;
-                    if (r1 >= 0) t1 = cur_k * st.deg[r1] + cur.rk1;
-                }
-            }
-            const bool contact = !(cur.flags & RF_JOINT);
-            BodyState b1{}, b2{};
-            bool ready;
-            if (LDS) {
-                uint32_t c0 = r0 >= 0 ? __hip_atomic_load(&st.cnt[r0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                      : t0;
-                uint32_t c1 = r1 >= 0 ? __hip_atomic_load(&st.cnt[r1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                      : t1;
-                __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                if (contact) {
-                    b1 = body_state(st, cur.a);
-                    b2 = body_state(st, cur.b);
-                }
-                ready = c0 == t0 && c1 == t1;
-            } else {
-                ready = true;
-                if (r0 >= 0) ready = ld_acq(&st.cnt[r0]) == t0;
-                if (ready && r1 >= 0) ready = ld_acq(&st.cnt[r1]) == t1;
-                if (ready && contact) {
-                    b1 = body_state_ordered(st, cur.a);
-                    b2 = body_state_ordered(st, cur.b);
-                }
-            }
-            if (ready) {
-                // a wave with a ready link issues ahead of the waves that poll
-                __builtin_amdgcn_s_setprio(2);
-                if (!contact) {
-                    const uint32_t ua = COMPACT ? (cur.cpair & 0xffffu) : cur.a;
-                    const uint32_t ub = COMPACT ? (cur.cpair >> 16) : (cur.b == NONE ? cur.a : cur.b);
-                    rec_solve_joint(cur, st, ua, ub, sub_dt);
-                } else {
-                    contact_impulses<WARM>(cur, cur.a, cur.b, b1, b2, st);
-                    recs[(size_t)cur_pos * 8 + REC_ACC] = make_uint4(__float_as_uint(cur.acc[0]),
-                                                                     __float_as_uint(cur.acc[1]),
-                                                                     __float_as_uint(cur.acc[2]),
-                                                                     __float_as_uint(cur.acc[3]));
-                }
-                if (LDS) {
-                    // the state writes above reach LDS before the counters (in order)
-                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                    if (r0 >= 0) __hip_atomic_store(&st.cnt[r0], t0 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (r1 >= 0) __hip_atomic_store(&st.cnt[r1], t1 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                } else {
-                    if (r0 >= 0) st_rel(&st.cnt[r0], t0 + 1u);
-                    if (r1 >= 0) st_rel(&st.cnt[r1], t1 + 1u);
-                }
-                __builtin_amdgcn_s_setprio(0);
-                if (has_nxt && nxt_pos == cur_pos) nxt = cur;
-                have = false;
-                spins = 0;
-            } else {
-                // every item's predecessors precede it, so some item is always
-                // ready; a stall this long means corrupt ordering data: stop
-                if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
-                if (++spins > SPIN_LIMIT) {
-                    __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    S.w_status[w] = 5;
-                    break;
-                }
-            }
-            // a wave with no lane ready yields its SIMD
-            if (__ballot(ready) == 0ull) __builtin_amdgcn_s_sleep(1);
-        }
-    }
-}
-
-// Keeps the compiler from moving LDS accesses across this point, without a
-// wait: one workgroup's LDS operations are served in the order they are
-// issued, so program order is all the dataflow needs.
-__device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
-
-// A lane's slot: the five rows of its current record that a chain link reads
-// besides the header and the impulses (rows REC_LINK.., copied as they are):
-// (nx ny fric p00) (p01 p02 p03 p04) (p05 p06 p10 p11) (p12 p13 p14 p15)
-// (p16 bias0 bias1 -).
-constexpr uint32_t LANE_ROWS = REC_ACC - REC_LINK;
-constexpr uint32_t LANE_WORDS = LANE_ROWS * 4;
-static_assert(REC_LINK == 2 && REC_ACC == 7 && LANE_ROWS == 5, "lane_load reads rows REC_LINK..REC_ACC-1 in this order");
-// the record kernel takes the lane slots up to this workgroup size (larger
-// ones keep the chain's records in registers)
-constexpr uint32_t LANES_MAXT = 512;
-// the record kernel's workgroup when a batch holds few worlds with LDS body state
-constexpr int REC_WIDE_THREADS = 512;
-__host__ __device__ constexpr size_t rec_lane_bytes(uint32_t threads)
-{
-    return threads <= LANES_MAXT ? (size_t)threads * LANE_WORDS * 4u : 0u;
-}
-
-// a contact's impulses back to its record
-__device__ __forceinline__ void rec_put_acc(uint4* recs, uint32_t pos, const float* acc)
-{
-    recs[(size_t)pos * 8 + REC_ACC] = make_uint4(__float_as_uint(acc[0]), __float_as_uint(acc[1]),
-                                                 __float_as_uint(acc[2]), __float_as_uint(acc[3]));
-}
-
-// a lane's slot rows are blockDim.x apart (row r of lane t at lanes[r * T + t]):
-// a wave's 16-byte row reads and writes then cover consecutive LDS words,
-// free of bank conflicts (rows contiguous per lane, 80 bytes apart, were not)
-__device__ __forceinline__ void lane_load(Rec& r, const uint4* q, uint32_t stride)
-{
-    const uint4 a = q[0], b = q[stride], c = q[2 * stride], d = q[3 * stride], e = q[4 * stride];
-    r.nx = __uint_as_float(a.x); r.ny = __uint_as_float(a.y); r.fric = __uint_as_float(a.z);
-    r.p[0][0] = __uint_as_float(a.w);
-    r.p[0][1] = __uint_as_float(b.x); r.p[0][2] = __uint_as_float(b.y); r.p[0][3] = __uint_as_float(b.z);
-    r.p[0][4] = __uint_as_float(b.w);
-    r.p[0][5] = __uint_as_float(c.x); r.p[0][6] = __uint_as_float(c.y); r.p[1][0] = __uint_as_float(c.z);
-    r.p[1][1] = __uint_as_float(c.w);
-    r.p[1][2] = __uint_as_float(d.x); r.p[1][3] = __uint_as_float(d.y); r.p[1][4] = __uint_as_float(d.z);
-    r.p[1][5] = __uint_as_float(d.w);
-    r.p[1][6] = __uint_as_float(e.x); r.bias[0] = __uint_as_float(e.y); r.bias[1] = __uint_as_float(e.z);
-}
-
-// The same ordered dataflow as item_chain (body state in LDS), with a
-// lane's current record kept in its LDS slot (lanes: blockDim.x slots of
-// LANE_WORDS, 16-byte aligned) instead of registers: the loop carries only
-// the header (flags, bodies, ranks, targets) and the impulses, so an
-// iteration moves no record between registers, and a poll reads just the two
-// counters.  The slot and the bodies' state are read in one batch once the
-// item is ready.  A link issues no global memory operation: a contact's
-// impulses go back to its record when the lane moves to another position
-// and when the chain ends (a wave's memory counter is waited on as a whole,
-// so a store per link would make every later wait of the wave wait for it);
-// a lane whose next position is its current one (one item per iteration)
-// keeps slot and impulses.  COMPACT: body state under the compact chain
-// indices of worlds beyond LDS (record row 1 .w), as in rec_to_compact.
-// GLOBAL: body state and counters in global memory (worlds whose touched
-// bodies do not fit LDS): counters are polled with acquire loads and
-// released with release stores, and the state is read after the acquire.
-// HYBRID (with GLOBAL): the state stays in global memory but the counters
-// are in LDS (lcnt) under the compact chain indices, so a poll is an LDS
-// read; acquire / release at workgroup scope order the state around them.
-template <bool COMPACT = false, bool GLOBAL = false, bool WARM = false, bool HYBRID = false, class ST>
-__device__ __forceinline__ void item_chain_lanes(int32_t* w_status, const ST& st, uint4* recs, uint4* lanes,
-                                                 uint32_t nitems, uint32_t iters, float sub_dt, uint32_t w,
-                                                 uint32_t& s_abort, uint32_t* lcnt = nullptr)
-{
-    static_assert(!HYBRID || (GLOBAL && !COMPACT), "the LDS counters go with global-memory state");
-    constexpr bool LITE = IsLite<ST>::value;
-    static_assert(!LITE || (COMPACT && !GLOBAL), "the light state is a compact LDS state");
-    const uint32_t p_begin = threadIdx.x, p_step = blockDim.x;
-    uint4* slot = lanes + threadIdx.x;          // row r at slot[r * p_step]
-    uint32_t pos = p_begin, k = (p_begin < nitems) ? 0u : iters;
-    uint32_t held = NONE;                    // position whose record the slot holds
-    uint32_t flags = 0, a = 0, b = 0, rk0 = 0, rk1 = 0, degs = 0;
-    int32_t r0 = -1, r1 = -1;
-    uint32_t t0 = 0, t1 = 0, n0 = 0, n1 = 0;  // the counters' targets and released values
-    uint32_t* const cbase = HYBRID ? lcnt : st.cnt;
-    uint32_t *p0 = cbase, *p1 = cbase;       // the counters polled (body 0's when none)
-    uint32_t cpair = 0;                      // HYBRID: the compact indices of a and b
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};     // the held record's impulses
-    bool have = false;
-    uint32_t spins = 0;
-    while (true) {
-        if (!have) {
-            if (k >= iters) break;
-            if (pos != held) {
-                if (held != NONE && !(flags & RF_JOINT)) rec_put_acc(recs, held, acc);
-                const uint4* q = recs + (size_t)pos * 8;
-                const uint4 h0 = q[0], h1 = q[1], ac = q[REC_ACC];
-                // every row's load is issued before any is written to the
-                // slot (one round trip for the record): without the barrier
-                // the scheduler may put each row's load after the previous
-                // row's LDS write, one round trip per row
-                const uint4 w0 = q[REC_LINK], w1 = q[REC_LINK + 1], w2 = q[REC_LINK + 2], w3 = q[REC_LINK + 3],
-                            w4 = q[REC_LINK + 4];
-                __builtin_amdgcn_sched_barrier(0);
-                slot[0] = w0;
-                slot[p_step] = w1;
-                slot[2 * p_step] = w2;
-                slot[3 * p_step] = w3;
-                slot[4 * p_step] = w4;
-                if constexpr (LITE) slot[LANE_ROWS * p_step] = st.rmass[pos];
-                flags = h0.x; a = h0.y; b = h0.z; rk0 = h1.x; rk1 = h1.y; degs = h1.z;
-                if (HYBRID) cpair = h1.w;
-                if (COMPACT) {
-                    const uint32_t c0 = h1.w & 0xffffu, c1 = h1.w >> 16;
-                    a = c0;
-                    b = ((flags & RF_JOINT) && b == NONE) ? NONE : c1;
-                }
-                acc[0] = __uint_as_float(ac.x); acc[1] = __uint_as_float(ac.y);
-                acc[2] = __uint_as_float(ac.z); acc[3] = __uint_as_float(ac.w);
-                held = pos;
-            }
-            if (flags & RF_JOINT) {
-                r0 = a == NONE ? -1 : (int32_t)a;
-                r1 = b == NONE ? -1 : (int32_t)b;
-            } else {
-                r0 = (flags & RF_W1) ? (int32_t)a : -1;
-                r1 = (flags & RF_W2) ? (int32_t)b : -1;
-            }
-            if (degs != DEGS_WIDE) {
-                t0 = k * (degs & 0xffffu) + rk0;
-                t1 = k * (degs >> 16) + rk1;
-            } else {
-                t0 = r0 >= 0 ? k * st.deg[r0] + rk0 : 0u;
-                t1 = r1 >= 0 ? k * st.deg[r1] + rk1 : 0u;
-            }
-            n0 = t0 + 1u;
-            n1 = t1 + 1u;
-            if (HYBRID) {
-                p0 = cbase + (r0 >= 0 ? (cpair & 0xffffu) : 0u);
-                p1 = cbase + (r1 >= 0 ? (cpair >> 16) : 0u);
-            } else {
-                p0 = cbase + (r0 >= 0 ? r0 : 0);
-                p1 = cbase + (r1 >= 0 ? r1 : 0);
-            }
-            have = true;
-        }
-        // a poll reads the two counters only (a lane without an ordering
-        // body reads body 0's and ignores it); the bodies' state is read once
-        // the item is ready, in the same batch as the slot (LDS serves one
-        // workgroup's operations in order, so it is what the predecessors
-        // released)
-        const bool contact = !(flags & RF_JOINT);
-        bool ready;
-        if (HYBRID) {
-            ready = r0 < 0 || __hip_atomic_load(p0, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == t0;
-            if (ready && r1 >= 0) ready = __hip_atomic_load(p1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == t1;
-        } else if (GLOBAL) {
-            ready = r0 < 0 || ld_acq(p0) == t0;
-            if (ready && r1 >= 0) ready = ld_acq(p1) == t1;
-        } else {
-            const uint32_t c0 = __hip_atomic_load(p0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            const uint32_t c1 = __hip_atomic_load(p1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            ready = (r0 < 0 || c0 == t0) && (r1 < 0 || c1 == t1);
-        }
-        if (ready) {
-            // a wave with a ready link issues ahead of the waves that poll
-            __builtin_amdgcn_s_setprio(2);
-            lds_order();
-            Rec cur;
-            cur.flags = flags; cur.a = a; cur.b = b;
-            lane_load(cur, slot, p_step);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) cur.acc[f] = acc[f];
-            // the light state's masses of this item's bodies, from its slot
-            ST sl = st;
-            if constexpr (LITE) {
-                const uint4 m = slot[LANE_ROWS * p_step];
-                sl.im = PairValue{a, __uint_as_float(m.x), __uint_as_float(m.z)};
-                sl.ii = PairValue{a, __uint_as_float(m.y), __uint_as_float(m.w)};
-            }
-            const BodyState b1 = GLOBAL ? body_state_ordered(sl, contact ? a : 0u) : body_state(sl, contact ? a : 0u);
-            const BodyState b2 = GLOBAL ? body_state_ordered(sl, contact ? b : 0u) : body_state(sl, contact ? b : 0u);
-            if (!contact) {
-                rec_solve_joint(cur, sl, a, b == NONE ? a : b, sub_dt);
-            } else {
-                contact_impulses<WARM>(cur, a, b, b1, b2, sl);
-#pragma unroll
-                for (int f = 0; f < 4; ++f) acc[f] = cur.acc[f];
-            }
-            // the state writes above reach LDS before the counters (in order)
-            lds_order();
-            if (HYBRID) {
-                if (r0 >= 0) __hip_atomic_store(p0, n0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (r1 >= 0) __hip_atomic_store(p1, n1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            } else if (GLOBAL) {
-                if (r0 >= 0) st_rel(p0, n0);
-                if (r1 >= 0) st_rel(p1, n1);
-            } else {
-                if (r0 >= 0) __hip_atomic_store(p0, n0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (r1 >= 0) __hip_atomic_store(p1, n1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            __builtin_amdgcn_s_setprio(0);
-            pos += p_step;
-            if (pos >= nitems) { pos = p_begin; ++k; }
-            have = false;
-            spins = 0;
-        } else {
-            // every item's predecessors precede it, so some item is always
-            // ready; a stall this long means corrupt ordering data: stop
-            ++spins;
-            if ((spins & 255u) == 0u) {
-                if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
-                if (spins > SPIN_LIMIT) {
-                    __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    w_status[w] = 5;
-                    break;
-                }
-            }
-        }
-        // no sleep between polls: a sleeping wave notices a released
-        // counter later, and the ready waves of other worlds on the SIMD
-        // issue ahead of it anyway
-    }
-    if (held != NONE && !(flags & RF_JOINT)) rec_put_acc(recs, held, acc);
-}
-
-// The LDS-state chain of a sub-step as an out-of-line call.  Its register
-// allocation is then its own: inlined, any change of register pressure
-// elsewhere in the step kernel reshaped the loop (at worst a record pickup
-// became one global round trip per row instead of one for all rows).  It
-// takes pointers typed by address space (LDS: the body state laid out as in
-// rec_world, the lane slots and the abort flag; global: the records and the
-// world status) and values only, so the callee keeps LDS and global
-// instructions and no argument block is copied.
-typedef __attribute__((address_space(3))) uint32_t* LdsU32;
-typedef __attribute__((address_space(3))) uint4* LdsU4;
-typedef __attribute__((address_space(1))) int32_t* GlbI32;
-typedef __attribute__((address_space(1))) uint4* GlbU4;
-template <bool WARM>
-__device__ __attribute__((noinline)) void chain_lds_call(GlbI32 w_status, LdsU32 lds, uint32_t n, GlbU4 recs,
-                                                        LdsU4 lanes, uint32_t nitems, uint32_t iters, float sub_dt,
-                                                        uint32_t w, LdsU32 s_abort)
-{
-    SolverState<true> st;
-    st.mx = (float*)(uint32_t*)lds;
-    st.my = st.mx + n;
-    st.L = st.my + n;
-    st.im = st.L + n;
-    st.ii = st.im + n;
-    st.cnt = (uint32_t*)(st.ii + n);
-    st.deg = st.cnt + n;
-    item_chain_lanes<false, false, WARM>((int32_t*)w_status, st, (uint4*)recs, (uint4*)lanes, nitems, iters, sub_dt, w,
-                                         *(uint32_t*)s_abort);
-}
-
-// the records' impulses, effective masses, lever arms and depths -> the
-// step's manifold arrays (what r2d_get_manifolds reports)
-__device__ __forceinline__ void item_writeback(const StepDev& S, uint4* recs, uint32_t pos)
-{
-    Rec r;
-    rec_load(r, recs + (size_t)pos * 8);
-    rec_writeback(r, S);
-}
-
-// One workgroup steps one world: S sub-steps of forces, integration,
-// pre-step and K solver iterations (lib.zig:199-250).  Solver items run as a
-// dataflow: an item may run once every earlier item (in the schedule's order)
-// that touches one of its ordering bodies has run, which gives the same bits
-// as the sequential loop.  Workers own execution positions tid, tid+blockDim,
-// ... and take them in (iteration, position) order, the order the ranks use,
-// so the earliest unfinished item always has a worker.  Body state lives in
-// LDS (lds: solve_lds_bytes(n) bytes); records at the world's item range
-// [ibase, ibase + nitems) of S.recs; degs: the world's item counts per body.
-// LANES: the chain keeps each lane's current record in its slot of `lanes`
-// (LDS, blockDim.x * LANE_WORDS words, 16-byte aligned, disjoint from lds).
-template <bool LANES, bool WARM = false>
-__device__ __forceinline__ void rec_world(const StepDev& S, const WorldDev& D, uint32_t w, uint32_t ibase,
-                                          uint32_t nitems, uint32_t mbeg, const uint32_t* degs, float dt,
-                                          uint32_t sub_steps, uint32_t iters, uint32_t* lds, uint4* lanes,
-                                          uint32_t& s_abort)
-{
-    if (threadIdx.x == 0) s_abort = 0u;
-    const int n = D.nbodies;
-    const float sub_dt = dt / (float)sub_steps;
-    uint4* recs = S.recs + (size_t)ibase * 8;
-
-    SolverState<true> st;
-    st.mx = (float*)lds;
-    st.my = st.mx + n;
-    st.L = st.my + n;
-    st.im = st.L + n;
-    st.ii = st.im + n;
-    st.cnt = (uint32_t*)(st.ii + n);
-    st.deg = st.cnt + n;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) body_setup(D, st, i, true, degs);
-    __syncthreads();
-    for (uint32_t pos = threadIdx.x; pos < nitems; pos += blockDim.x)
-        item_build<WARM>(S, D, st, recs, pos, ibase, mbeg, sub_dt);
-    for (uint32_t s = 0; s < sub_steps; ++s) {
-        const bool last = s + 1 == sub_steps;
-        const BodyArrays bf = body_arrays(D);
-        body_pass<3, ForceIn>(
-            n, [&](int i) { return force_in(bf, i); },
-            [&](int i, const ForceIn& in) { body_forces_in<WARM>(bf, st, i, in, last, sub_dt); });
-        __syncthreads();
-        {
-            // the next record's header is loaded while this one is updated
-            const PassArrays pa = pass_arrays(D);
-            uint32_t pos = threadIdx.x;
-            uint4 hn = pos < nitems ? recs[(size_t)pos * 8] : make_uint4(0u, 0u, 0u, 0u);
-            for (; pos < nitems; pos += blockDim.x) {
-                const uint4 h = hn;
-                if (pos + blockDim.x < nitems) hn = recs[(size_t)(pos + blockDim.x) * 8];
-                item_tgs_h<WARM>(S, pa, st, recs, pos, h, last, sub_dt);
-            }
-        }
-        __syncthreads();
-        if constexpr (LANES)
-            chain_lds_call<WARM>((GlbI32)S.w_status, (LdsU32)lds, (uint32_t)n, (GlbU4)recs, (LdsU4)lanes, nitems, iters,
-                                 sub_dt, w, (LdsU32)&s_abort);
-        else item_chain<true, false, WARM>(S, D, st, recs, nitems, iters, sub_dt, w, s_abort);
-        __syncthreads();
-        const BodyArrays bp = body_arrays(D);
-        body_pass<3, PosIn>(
-            n, [&](int i) { return pos_in(bp, i); },
-            [&](int i, const PosIn& in) { body_positions_in(bp, st, i, in, sub_dt); });
-        __syncthreads();
-    }
-    for (uint32_t pos = threadIdx.x; pos < nitems; pos += blockDim.x) item_writeback(S, recs, pos);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        D.mx[i] = st.mx[i]; D.my[i] = st.my[i]; D.L[i] = st.L[i];
-    }
-}
-
-// the record kernel: the worlds solve_route gives it, one workgroup each
-template <int MAXT, int WAVES = 1, bool WARM = false>
-__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WAVES)))
-void k_solve(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t slot_cap, uint32_t slot_nmax,
-             uint32_t lds_nmax)
-{
-    extern __shared__ __align__(16) uint32_t smem[];
-    __shared__ uint32_t s_abort;
-    if (S.counters[C_OVERFLOW]) return;
-    const uint32_t w = S.w_order[blockIdx.x];
-    if (S.w_status[w] != 0) return;
-    const uint32_t ibase = S.w_item_base[w];
-    const uint32_t nitems = S.w_item_base[w + 1] - ibase;
-    const WorldDev& D = S.worlds[w];
-    if (solve_route((uint32_t)D.nbodies, nitems, slot_cap, slot_nmax, lds_nmax, D.warm > 0.0f) != 1) return;
-    // LDS: the chain's lane slots (workgroups of at most LANES_MAXT threads),
-    // then the body state
-    constexpr bool LANES = MAXT <= LANES_MAXT;
-    uint4* lanes = LANES ? reinterpret_cast<uint4*>(smem) : nullptr;
-    uint32_t* body = smem + (LANES ? MAXT * LANE_WORDS : 0u);
-    rec_world<LANES, WARM>(S, D, w, ibase, nitems, S.w_man_begin[w], S.deg + D.body_base, dt, sub_steps, iters, body,
-                     lanes, s_abort);
-}
-
 // ---------------------------------- warm starting in the phase kernels
 // grid-wide over the step's manifolds / bodies; worlds without warm starting
 // (and stopped worlds) are skipped
@@ -2564,673 +1217,6 @@ __global__ void k_warm_save(StepDev S)
         if (D.warm > 0.0f && S.w_status[w] == 0)
             warm_save(S, D, m, S.w_man_begin[w], S.w_man_begin[w + 1], D.body_base);
     }
-}
-
-// ------------------------------------- worlds beyond LDS: split sub-steps
-// For a world whose body state does not fit LDS (more than lds_nmax bodies)
-// the per-body and per-item parts run as grid-wide kernels over all such
-// worlds' bodies, and only the dependency chains run one workgroup per world;
-// body state, counters and records stay in global memory between launches.
-__device__ __forceinline__ bool big_world(const WorldDev& D, uint32_t lds_nmax)
-{
-    return (uint32_t)D.nbodies > lds_nmax;
-}
-
-__device__ __forceinline__ SolverState<false> global_state(const StepDev& S, const WorldDev& D)
-{
-    SolverState<false> st;
-    st.mx = D.mx; st.my = D.my; st.L = D.L;
-    st.im = S.g_im + D.body_base; st.ii = S.g_ii + D.body_base;
-    st.cnt = S.g_cnt + D.body_base; st.deg = S.deg + D.body_base;
-    return st;
-}
-
-// phase 0: body setup; 1: forces + velocities (sub-step s); 2: positions
-__global__ void k_big_bodies(StepDev S, uint32_t lds_nmax, int phase, uint32_t s, uint32_t sub_steps, float sub_dt)
-{
-    if (S.counters[C_OVERFLOW]) return;
-    for (uint32_t x = grid_tid(); x < S.nb; x += grid_stride()) {
-        const uint32_t w = S.bworld[x];
-        if (S.w_status[w] != 0) continue;
-        const WorldDev& D = S.worlds[w];
-        if (!big_world(D, lds_nmax)) continue;
-        const SolverState<false> st = global_state(S, D);
-        const int i = (int)(x - D.body_base);
-        if (phase == 0) body_setup(D, st, i, false, S.deg + D.body_base);
-        else if (phase == 1) body_forces<true>(D, st, i, s + 1 == sub_steps, sub_dt);
-        else body_positions(D, st, i, sub_dt);
-    }
-}
-
-// the per-item parts, gridDim.y workgroups per world: phase 0 builds the
-// records, 1 is updateTGSDepth (sub-step s), 2 writes back
-constexpr unsigned BIG_THREADS = 256;
-constexpr unsigned BIG_SPLIT = 32;
-__global__ __launch_bounds__(BIG_THREADS) void k_big_item_pass(StepDev S, uint32_t lds_nmax, int phase, uint32_t s,
-                                                            uint32_t sub_steps, float sub_dt)
-{
-    if (S.counters[C_OVERFLOW]) return;
-    const uint32_t w = blockIdx.x;
-    if (S.w_status[w] != 0) return;
-    const WorldDev& D = S.worlds[w];
-    if (!big_world(D, lds_nmax)) return;
-    const SolverState<false> st = global_state(S, D);
-    const uint32_t ibase = S.w_item_base[w], nitems = S.w_item_base[w + 1] - ibase, mbeg = S.w_man_begin[w];
-    uint4* recs = S.recs + (size_t)ibase * 8;
-    for (uint32_t pos = blockIdx.y * blockDim.x + threadIdx.x; pos < nitems; pos += gridDim.y * blockDim.x) {
-        if (phase == 0) item_build<true>(S, D, st, recs, pos, ibase, mbeg, sub_dt);
-        else if (phase == 1) item_tgs<true>(S, D, st, recs, pos, s + 1 == sub_steps, sub_dt);
-        else item_writeback(S, recs, pos);
-    }
-}
-
-// after the records: the compact chain indices, one workgroup per world
-__global__ __launch_bounds__(BIG_THREADS) void k_big_items(StepDev S, uint32_t lds_nmax)
-{
-    __shared__ uint32_t s_scan[BIG_THREADS];
-    __shared__ uint32_t s_total;
-    if (S.counters[C_OVERFLOW]) return;
-    const uint32_t w = blockIdx.x;
-    if (S.w_status[w] != 0) return;
-    const WorldDev& D = S.worlds[w];
-    if (!big_world(D, lds_nmax)) return;
-    const uint32_t ibase = S.w_item_base[w], nitems = S.w_item_base[w + 1] - ibase;
-    const uint32_t base = D.body_base, T = blockDim.x, t = threadIdx.x;
-    const int n = D.nbodies;
-    uint4* recs = S.recs + (size_t)ibase * 8;
-    // compact chain indices: the bodies the items touch, numbered in slot order
-    const uint32_t UNUSED = 0xffffffffu;
-    for (int i = t; i < n; i += T) S.cmap[base + i] = UNUSED;
-    __syncthreads();
-    for (uint32_t pos = t; pos < nitems; pos += T) {
-        const uint4 h = recs[(size_t)pos * 8];
-        if (h.x & RF_JOINT) {
-            const Joint& J = D.joints[h.w];
-            S.cmap[base + J.s1] = 0u;
-            if (J.s2 >= 0) S.cmap[base + J.s2] = 0u;
-        } else {
-            S.cmap[base + h.y] = 0u;
-            S.cmap[base + h.z] = 0u;
-        }
-    }
-    __syncthreads();
-    // each wave numbers a contiguous range of slots, 64 at a time (coalesced
-    // loads, ranks from the wave's ballot): count, the waves' offsets, assign
-    constexpr uint32_t NW = BIG_THREADS / 64;
-    const uint32_t lane = t & 63u, wv = t >> 6;
-    const uint32_t span = (((uint32_t)n + NW - 1) / NW + 63u) & ~63u;
-    const uint32_t lo = umin(wv * span, (uint32_t)n), hi = umin(lo + span, (uint32_t)n);
-    const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t cnt = 0;
-    for (uint32_t i0 = lo; i0 < hi; i0 += 64u) {
-        const uint32_t i = i0 + lane;
-        cnt += (uint32_t)__popcll(__ballot(i < hi && S.cmap[base + i] == 0u));
-    }
-    if (lane == 0) s_scan[wv] = cnt;
-    __syncthreads();
-    uint32_t c = 0, total = 0;
-    for (uint32_t k = 0; k < NW; ++k) {
-        c += k < wv ? s_scan[k] : 0u;
-        total += s_scan[k];
-    }
-    for (uint32_t i0 = lo; i0 < hi; i0 += 64u) {
-        const uint32_t i = i0 + lane;
-        const bool hit = i < hi && S.cmap[base + i] == 0u;
-        const uint64_t bal = __ballot(hit);
-        if (hit) {
-            const uint32_t ci = c + (uint32_t)__popcll(bal & below);
-            S.cmap[base + i] = ci;
-            S.cinv[base + ci] = i;
-        }
-        c += (uint32_t)__popcll(bal);
-    }
-    if (t == 0) s_total = total;
-    __syncthreads();
-    const uint32_t nc = s_total;
-    if (t == 0) S.w_nc[w] = nc;
-    if (nc >= 0xffffu) return;   // the compact chain is not used (LDS holds far fewer)
-    for (uint32_t pos = t; pos < nitems; pos += T) {
-        uint4* q = recs + (size_t)pos * 8;
-        const uint4 h = q[0];
-        uint32_t c0, c1, s0, s1;
-        if (h.x & RF_JOINT) {
-            const Joint& J = D.joints[h.w];
-            c0 = S.cmap[base + J.s1];
-            c1 = J.s2 >= 0 ? S.cmap[base + J.s2] : 0xffffu;
-            s0 = (uint32_t)J.s1;
-            s1 = J.s2 >= 0 ? (uint32_t)J.s2 : s0;
-        } else {
-            c0 = S.cmap[base + h.y];
-            c1 = S.cmap[base + h.z];
-            s0 = h.y;
-            s1 = h.z;
-        }
-        q[1].w = c0 | (c1 << 16);
-        // the light compact chain's masses of the item's bodies
-        S.rmass[ibase + pos] = make_uint4(__float_as_uint(S.g_im[base + s0]), __float_as_uint(S.g_ii[base + s0]),
-                                          __float_as_uint(S.g_im[base + s1]), __float_as_uint(S.g_ii[base + s1]));
-    }
-}
-
-// LDS bytes of the compact chain per body (momentum, inverse masses, counter, item count)
-constexpr size_t COMPACT_BYTES = 7 * 4;
-constexpr size_t LITE_BYTES = 4 * 4;   // the light compact state: momentum and counter
-// the light compact chain runs in the 256-lane compact launch, with lane
-// slots of six rows; both chain launches decide with this one size, so
-// exactly one of them takes each world
-constexpr uint32_t LITE_LANES = 256;
-constexpr size_t LITE_SLOT_BYTES = (size_t)LITE_LANES * (LANE_ROWS + 1) * 16u;
-constexpr size_t COMPACT_LDS = 160 * 1024 - 1024;
-// lanes of the global-memory chain's workgroup
-constexpr int BIG_GLOBAL_THREADS = 1024;
-
-// one sub-step's K iterations; one workgroup per world.  When the bodies the
-// items touch fit LDS, their state is gathered there under compact indices,
-// the chain runs on LDS, and the state is scattered back; otherwise the
-// chain runs on global memory.  PART 0 takes only the worlds of the first
-// kind, 1 only those of the second (launched with more lanes: a lane owns
-// fewer positions, so fewer of its items wait behind one whose operands are
-// not ready, and the chain's loads and polls, all to L2, overlap more).
-template <int MAXT, bool WARM = false, int PART = 0>
-__global__ __launch_bounds__(MAXT) void k_big_chain(StepDev S, uint32_t lds_nmax, uint32_t iters, float sub_dt)
-{
-    extern __shared__ __align__(16) uint32_t smem[];
-    __shared__ uint32_t s_abort;
-    if (S.counters[C_OVERFLOW]) return;
-    const uint32_t w = S.w_order[blockIdx.x];
-    if (S.w_status[w] != 0) return;
-    const WorldDev& D = S.worlds[w];
-    if (!big_world(D, lds_nmax)) return;
-    if (threadIdx.x == 0) s_abort = 0u;
-    __syncthreads();
-    const uint32_t ibase = S.w_item_base[w], nitems = S.w_item_base[w + 1] - ibase;
-    const uint32_t base = D.body_base;
-    uint4* recs = S.recs + (size_t)ibase * 8;
-    const uint32_t nc = S.w_nc[w];
-    const bool compact = (size_t)nc * COMPACT_BYTES <= COMPACT_LDS;
-    // the light compact state (momentum and counters, 16 B per touched body,
-    // beside lane slots of six rows) for the worlds the full one does not fit
-    const bool lite = !compact && nc < 0xffffu && (size_t)nc * LITE_BYTES + LITE_SLOT_BYTES <= COMPACT_LDS;
-    static_assert(PART != 0 || MAXT == LITE_LANES, "the light chain's slots are sized for the compact launch");
-    if ((compact || lite) != (PART == 0)) return;   // uniform: the other launch takes this world
-    // the lane-slot chain when the slots fit beside the compact state
-    constexpr size_t LANE_BYTES = (size_t)MAXT * LANE_WORDS * 4u;
-    const bool lanes = (size_t)nc * COMPACT_BYTES + LANE_BYTES <= COMPACT_LDS;
-    if constexpr (PART == 0) {
-        if (lite) {
-            LiteState st;
-            st.mx = (float*)(smem + LITE_SLOT_BYTES / 4);
-            st.my = st.mx + nc;
-            st.L = st.my + nc;
-            st.cnt = (uint32_t*)(st.L + nc);
-            st.im = PairValue{0u, 0.f, 0.f};
-            st.ii = PairValue{0u, 0.f, 0.f};
-            st.deg = DegLookup{S.deg, S.cinv, base};
-            st.rmass = S.rmass + ibase;
-            for (uint32_t c = threadIdx.x; c < nc; c += blockDim.x) {
-                const uint32_t i = S.cinv[base + c];
-                st.mx[c] = D.mx[i]; st.my[c] = D.my[i]; st.L[c] = D.L[i];
-                st.cnt[c] = 0u;
-            }
-            __syncthreads();
-            item_chain_lanes<true, false, WARM>(S.w_status, st, recs, reinterpret_cast<uint4*>(smem), nitems, iters, sub_dt, w,
-                                                s_abort);
-            __syncthreads();
-            for (uint32_t c = threadIdx.x; c < nc; c += blockDim.x) {
-                const uint32_t i = S.cinv[base + c];
-                D.mx[i] = st.mx[c]; D.my[i] = st.my[c]; D.L[i] = st.L[c];
-            }
-            return;
-        }
-        SolverState<true> st;
-        st.mx = (float*)(smem + (lanes ? MAXT * LANE_WORDS : 0u));
-        st.my = st.mx + nc;
-        st.L = st.my + nc;
-        st.im = st.L + nc;
-        st.ii = st.im + nc;
-        st.cnt = (uint32_t*)(st.ii + nc);
-        st.deg = st.cnt + nc;
-        for (uint32_t c = threadIdx.x; c < nc; c += blockDim.x) {
-            const uint32_t i = S.cinv[base + c];
-            st.mx[c] = D.mx[i]; st.my[c] = D.my[i]; st.L[c] = D.L[i];
-            st.im[c] = S.g_im[base + i]; st.ii[c] = S.g_ii[base + i];
-            st.cnt[c] = 0u;
-            st.deg[c] = S.deg[base + i];
-        }
-        __syncthreads();
-        if (lanes)
-            item_chain_lanes<true, false, WARM>(S.w_status, st, recs, reinterpret_cast<uint4*>(smem), nitems, iters, sub_dt, w,
-                                                s_abort);
-        else item_chain<true, true, WARM>(S, D, st, recs, nitems, iters, sub_dt, w, s_abort);
-        __syncthreads();
-        for (uint32_t c = threadIdx.x; c < nc; c += blockDim.x) {
-            const uint32_t i = S.cinv[base + c];
-            D.mx[i] = st.mx[c]; D.my[i] = st.my[c]; D.L[i] = st.L[c];
-        }
-    } else {
-        (void)lanes;
-        // body state in global memory; the lane slots take the start of LDS,
-        // then the counters under the compact indices when they fit (the
-        // compact indices exist below 65,535 touched bodies), else the
-        // counters stay in global memory too
-        const SolverState<false> st = global_state(S, D);
-        uint4* slots = reinterpret_cast<uint4*>(smem);
-        if (nc < 0xffffu && (size_t)nc * 4u + LANE_BYTES <= COMPACT_LDS) {
-            uint32_t* lcnt = smem + (size_t)MAXT * LANE_WORDS;
-            for (uint32_t c = threadIdx.x; c < nc; c += blockDim.x) lcnt[c] = 0u;
-            __syncthreads();
-            item_chain_lanes<false, true, WARM, true>(S.w_status, st, recs, slots, nitems, iters, sub_dt, w, s_abort, lcnt);
-        } else {
-            item_chain_lanes<false, true, WARM>(S.w_status, st, recs, slots, nitems, iters, sub_dt, w, s_abort);
-        }
-    }
-}
-
-// ------------------------------------------------------ register-slot solver
-// For worlds with at most NSLOT * MAXT solver items (and < 65,535 bodies) each
-// thread keeps all of its items -- execution positions tid, tid + MAXT, ... --
-// in registers for the whole step, and the body state a chain link reads
-// (momentum, inverse masses, pose, cos / sin of the angle, inertia, torque)
-// sits in LDS, so the dependency-chain loop issues no global memory operation:
-// a wave's vector-memory wait is wave-wide, and any load inside the loop would
-// put HBM latency on every chain link.
-struct Slot {
-    uint32_t flags;          // RF_* bits | joint type << 24 | SLOT_USED; 0 = unused
-    uint32_t pair;           // manifold: ref | inc << 16; joint: r0 | r1 << 16 (0xffff = none)
-    uint32_t ranks;          // rank at r0 | rank at r1 << 16
-    uint32_t idx;            // manifold index / joint body slots (s1 | s2 << 16)
-    float nx, ny, fric;
-    float p[2][7];           // manifold: r1x r1y r2x r2y depth mass_n mass_t per point
-                             // joint: pmax pmin beta r1x r1y r2x r2y | target tx ty
-    float acc[4];            // pn0 pt0 pn1 pt1
-    uint32_t degs;           // items at r0 | items at r1 << 16 (ordering bodies)
-    float bias[2];           // per point: Baumgarte bias of this sub-step, -1 when depth >= 0
-};
-constexpr uint32_t SLOT_USED = 0x80000000u;
-
-struct SlotState {
-    float *mx, *my, *L, *im, *ii;
-    uint32_t *cnt, *deg;
-    float *px, *py, *c, *s, *I, *tq;
-};
-
-__device__ __forceinline__ void slot_from_rec(Slot& z, const Rec& r)
-{
-    z.flags = r.flags | SLOT_USED;
-    z.pair = (r.a & 0xffffu) | (r.b << 16);
-    z.ranks = (r.rk0 & 0xffffu) | (r.rk1 << 16);
-    z.idx = r.idx;
-    z.nx = r.nx; z.ny = r.ny; z.fric = r.fric;
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int f = 0; f < 7; ++f) z.p[p][f] = r.p[p][f];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) z.acc[f] = r.acc[f];
-}
-
-__device__ __forceinline__ void rec_from_slot(Rec& r, const Slot& z)
-{
-    r.flags = z.flags & ~SLOT_USED;
-    uint32_t a = z.pair & 0xffffu, b = z.pair >> 16;
-    r.a = (a == 0xffffu) ? NONE : a;
-    r.b = (b == 0xffffu) ? NONE : b;
-    r.rk0 = z.ranks & 0xffffu; r.rk1 = z.ranks >> 16;
-    r.idx = z.idx;
-    r.nx = z.nx; r.ny = z.ny; r.fric = z.fric;
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int f = 0; f < 7; ++f) r.p[p][f] = z.p[p][f];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) r.acc[f] = z.acc[f];
-}
-
-// joint slot: parameters from the world's joint record
-__device__ __forceinline__ void slot_joint(Slot& z, const Joint& J, const WorldDev& D)
-{
-    z.flags |= (uint32_t)J.type << 24;
-    if (D.flags[J.s1] & BF_STATIC) z.flags |= RF_S1;
-    z.idx = ((uint32_t)J.s1 & 0xffffu) | ((uint32_t)(J.s2 < 0 ? 0xffff : J.s2) << 16);
-    z.p[0][0] = J.pmax; z.p[0][1] = J.pmin; z.p[0][2] = J.beta;
-    z.p[0][3] = J.r1x; z.p[0][4] = J.r1y; z.p[0][5] = J.r2x; z.p[0][6] = J.r2y;
-    z.p[1][0] = J.target; z.p[1][1] = J.tx; z.p[1][2] = J.ty;
-}
-
-// Constraint.solve for a joint slot: pose, cos / sin, inertia and torque from LDS
-__device__ __forceinline__ void slot_solve_joint(const Slot& z, const SlotState& st, float dt)
-{
-    const uint32_t a = z.idx & 0xffffu, b = z.idx >> 16;
-    JointIn j;
-    j.type = (z.flags >> 24) & 0x7fu;
-    j.stat1 = (z.flags & RF_S1) != 0;
-    j.pmax = z.p[0][0]; j.pmin = z.p[0][1]; j.beta = z.p[0][2];
-    j.r1x = z.p[0][3]; j.r1y = z.p[0][4]; j.r2x = z.p[0][5]; j.r2y = z.p[0][6];
-    j.target = z.p[1][0]; j.tx = z.p[1][1]; j.ty = z.p[1][2];
-    j.pa = mk(st.px[a], st.py[a]);
-    j.ca = st.c[a]; j.sa = st.s[a];
-    j.I1 = st.I[a]; j.tq1 = st.tq[a];
-    if (j.type <= 1) {
-        j.pb = mk(st.px[b], st.py[b]);
-        j.cb = st.c[b]; j.sb = st.s[b];
-    } else {
-        j.pb = mk(0.f, 0.f);
-        j.cb = j.sb = 0.f;
-    }
-    joint_apply(j, st, a, b, dt);
-}
-
-// ordering bodies of a slot (-1: none) and the Baumgarte biases of a sub-step
-__device__ __forceinline__ void slot_ordering(const Slot& z, int32_t& r0, int32_t& r1)
-{
-    uint32_t a = z.pair & 0xffffu, b = z.pair >> 16;
-    if (z.flags & RF_JOINT) {
-        r0 = a == 0xffffu ? -1 : (int32_t)a;
-        r1 = b == 0xffffu ? -1 : (int32_t)b;
-    } else {
-        r0 = (z.flags & RF_W1) ? (int32_t)a : -1;
-        r1 = (z.flags & RF_W2) ? (int32_t)b : -1;
-    }
-}
-
-__device__ __forceinline__ void slot_biases(Slot& z, float dt)
-{
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        float depth = z.p[p][4];
-        z.bias[p] = depth >= 0.f ? -1.0f : BAUMGARTE * maxn(0.0f, (-depth) - BAUMGARTE_SLOP) / dt;
-    }
-}
-
-// LOCKSTEP: a wave takes its lanes' slot z together, z = 0, 1, ... in turn
-// (each slot's registers addressed directly, no per-lane selection of the
-// current slot), instead of every lane walking its own slots independently.
-// Both orders are deadlock-free: a wave works on positions in increasing
-// (iteration, slot, lane) order, the order of the dependencies.
-// One world's step on the register-slot path, one workgroup of MAXT threads
-// (nitems <= NSLOT * MAXT; lds: slot_lds_bytes(n) bytes; degs: the world's
-// item counts per body).
-template <int NSLOT, int MAXT, bool LOCKSTEP>
-__device__ __forceinline__ void slots_world(const StepDev& S, const WorldDev& D, uint32_t w, uint32_t ibase,
-                                            uint32_t nitems, uint32_t mbeg, const uint32_t* degs, float dt,
-                                            uint32_t sub_steps, uint32_t iters, uint32_t* lds, uint32_t& s_abort)
-{
-    const int n = D.nbodies;
-    if (threadIdx.x == 0) s_abort = 0u;
-    const uint32_t base = D.body_base;
-    const uint32_t nj = D.njoints;
-    const float fsub = (float)sub_steps;
-    const float sub_dt = dt / fsub;
-
-    SlotState st;
-    st.mx = (float*)lds;
-    st.my = st.mx + n;
-    st.L = st.my + n;
-    st.im = st.L + n;
-    st.ii = st.im + n;
-    st.cnt = (uint32_t*)(st.ii + n);
-    st.deg = st.cnt + n;
-    st.px = (float*)(st.deg + n);
-    st.py = st.px + n;
-    st.c = st.py + n;
-    st.s = st.c + n;
-    st.I = st.s + n;
-    st.tq = st.I + n;
-    for (int i = threadIdx.x; i < n; i += MAXT) {
-        bool stat = (D.flags[i] & BF_STATIC) != 0;
-        st.mx[i] = D.mx[i]; st.my[i] = D.my[i]; st.L[i] = D.L[i];
-        st.im[i] = stat ? 0.0f : 1.0f / D.mass[i];
-        st.ii[i] = stat ? 0.0f : 1.0f / D.inertia[i];
-        st.deg[i] = degs[i];
-        st.I[i] = D.inertia[i];
-    }
-    __syncthreads();
-    Slot sl[NSLOT];
-    uint32_t nslot = 0;
-#pragma unroll
-    for (int z = 0; z < NSLOT; ++z) {
-        sl[z].flags = 0u;
-        uint32_t pos = threadIdx.x + (uint32_t)z * MAXT;
-        if (pos < nitems) {
-            Rec r;
-            rec_build(r, S, D, st, pos, ibase, nj, mbeg, base);
-            slot_from_rec(sl[z], r);
-            if (r.flags & RF_JOINT) slot_joint(sl[z], D.joints[r.idx], D);
-            int32_t q0, q1;
-            slot_ordering(sl[z], q0, q1);
-            sl[z].degs = (q0 >= 0 ? st.deg[q0] : 0u) | ((q1 >= 0 ? st.deg[q1] : 0u) << 16);
-            nslot = (uint32_t)z + 1u;
-        }
-    }
-
-    for (uint32_t s = 0; s < sub_steps; ++s) {
-        // forces (lib.zig:200-205), AABB refresh + velocity integration (lib.zig:207-216)
-        for (int i = threadIdx.x; i < n; i += MAXT) {
-            uint32_t f = D.flags[i];
-            bool stat = (f & BF_STATIC) != 0;
-            float fx = D.fx[i], fy = D.fy[i];
-            float px = D.px[i], py = D.py[i], a = D.ang[i];
-            for (int g = 0; g < D.ngens; ++g) {
-                const Gen& G = D.gens[g];
-                if (stat) continue;
-                if (G.type == 0) {
-                    fx += G.gx * D.mass[i];
-                    fy += G.gy * D.mass[i];
-                } else if (G.slot == i) {
-                    float inv_m = 1.0f / D.mass[i];
-                    v2 v = scale2(mk(st.mx[i], st.my[i]), inv_m);
-                    v2 d = sub2(mk(px, py), mk(G.ax, G.ay));
-                    fx += (-G.k) * d.x - G.c * v.x;
-                    fy += (-G.k) * d.y - G.c * v.y;
-                }
-            }
-            // cos / sin of the angle: offset joints read them in the solve
-            float c = 0.0f, sn = 0.0f;
-            if (nj || (s + 1 == sub_steps && (f & BF_RECT))) { c = cosf_r(a); sn = sinf_r(a); }
-            if (s + 1 == sub_steps) {
-                float hw, hh;
-                if (f & BF_RECT) {
-                    float x = D.hw[i], y = D.hh[i];
-                    v2 lv[4] = {mk(-x, -y), mk(-x, y), mk(x, y), mk(x, -y)};
-                    hw = 0.f; hh = 0.f;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        v2 r = rotcs(lv[k], c, sn);
-                        if (r.x > hw) hw = r.x;
-                        if (r.y > hh) hh = r.y;
-                    }
-                } else {
-                    hw = D.rad[i]; hh = D.rad[i];
-                }
-                D.ax[i] = px; D.ay[i] = py; D.ahw[i] = hw; D.ahh[i] = hh;
-            }
-            if (!stat) {
-                st.mx[i] += fx * sub_dt;
-                st.my[i] += fy * sub_dt;
-                st.L[i] += D.tq[i] * sub_dt;
-            }
-            D.fx[i] = fx; D.fy[i] = fy;
-            st.px[i] = px; st.py[i] = py; st.c[i] = c; st.s[i] = sn;
-            st.tq[i] = D.tq[i];
-            st.cnt[i] = 0u;
-        }
-        __syncthreads();
-        // updateTGSDepth (collision.zig:73-100)
-#pragma unroll
-        for (int z = 0; z < NSLOT; ++z) {
-            uint32_t fl = sl[z].flags;
-            if (!fl || (fl & RF_JOINT)) continue;
-            if (fl & RF_TGS) {
-                Rec r;
-                rec_from_slot(r, sl[z]);
-                rec_tgs(r, S, D, st, true);
-                slot_from_rec(sl[z], r);
-            } else if (s + 1 == sub_steps) {
-                S.m_prev1[sl[z].idx] = D.ang[sl[z].pair & 0xffffu];
-                S.m_prev2[sl[z].idx] = D.ang[sl[z].pair >> 16];
-            }
-            slot_biases(sl[z], sub_dt);
-        }
-        if constexpr (LOCKSTEP) {
-            // lockstep over slots: see the kernel's comment; reads as in the
-            // independent walk below
-            for (uint32_t k = 0; k < iters; ++k) {
-#pragma unroll
-                for (int z = 0; z < NSLOT; ++z) {
-                    Slot& it = sl[z];
-                    bool done = !it.flags;
-                    int32_t r0 = -1, r1 = -1;
-                    slot_ordering(it, r0, r1);
-                    const uint32_t t0 = k * (it.degs & 0xffffu) + (it.ranks & 0xffffu);
-                    const uint32_t t1 = k * (it.degs >> 16) + (it.ranks >> 16);
-                    const bool contact = !(it.flags & RF_JOINT);
-                    uint32_t spins = 0;
-                    while (!done) {
-                        uint32_t c0 = r0 >= 0 ? __hip_atomic_load(&st.cnt[r0], __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_WORKGROUP)
-                                              : t0;
-                        uint32_t c1 = r1 >= 0 ? __hip_atomic_load(&st.cnt[r1], __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_WORKGROUP)
-                                              : t1;
-                        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                        BodyState b1{}, b2{};
-                        if (contact) {
-                            b1 = body_state(st, it.pair & 0xffffu);
-                            b2 = body_state(st, it.pair >> 16);
-                        }
-                        const bool ready = c0 == t0 && c1 == t1;
-                        if (ready) {
-                            if (!contact) slot_solve_joint(it, st, sub_dt);
-                            else contact_impulses(it, it.pair & 0xffffu, it.pair >> 16, b1, b2, st);
-                            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                            if (r0 >= 0)
-                                __hip_atomic_store(&st.cnt[r0], t0 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            if (r1 >= 0)
-                                __hip_atomic_store(&st.cnt[r1], t1 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                            done = true;
-                        } else {
-                            if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
-                                done = true;
-                            } else if (++spins > SPIN_LIMIT) {
-                                __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                                S.w_status[w] = 5;
-                                done = true;
-                            }
-                        }
-                        if (__ballot(ready) == 0ull) __builtin_amdgcn_s_sleep(1);
-                    }
-                }
-            }
-        } else
-        // K iterations as an ordered dataflow over register-resident items.  A
-        // link's counters and its bodies' state are read together: LDS serves
-        // one workgroup's operations in order, so state read after a counter
-        // that shows the item ready is the state its predecessor released
-        // (values read for an item that is not ready are discarded)
-        {
-            uint32_t k = nslot ? 0u : iters, cz = 0, spins = 0;
-            bool have = false;
-            Slot cur;
-            int32_t r0 = -1, r1 = -1;
-            uint32_t t0 = 0, t1 = 0;
-            while (k < iters) {
-                if (!have) {
-#pragma unroll
-                    for (int z = 0; z < NSLOT; ++z)
-                        if ((uint32_t)z == cz) cur = sl[z];
-                    have = true;
-                    slot_ordering(cur, r0, r1);
-                    t0 = k * (cur.degs & 0xffffu) + (cur.ranks & 0xffffu);
-                    t1 = k * (cur.degs >> 16) + (cur.ranks >> 16);
-                }
-                uint32_t c0 = r0 >= 0 ? __hip_atomic_load(&st.cnt[r0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                      : t0;
-                uint32_t c1 = r1 >= 0 ? __hip_atomic_load(&st.cnt[r1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                      : t1;
-                __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                const bool contact = !(cur.flags & RF_JOINT);
-                BodyState b1{}, b2{};
-                if (contact) {
-                    b1 = body_state(st, cur.pair & 0xffffu);
-                    b2 = body_state(st, cur.pair >> 16);
-                }
-                const bool ready = c0 == t0 && c1 == t1;
-                if (ready) {
-                    // a wave with a ready link issues ahead of the waves that poll
-                    __builtin_amdgcn_s_setprio(2);
-                    if (!contact) {
-                        slot_solve_joint(cur, st, sub_dt);
-                    } else {
-                        contact_impulses(cur, cur.pair & 0xffffu, cur.pair >> 16, b1, b2, st);
-#pragma unroll
-                        for (int z = 0; z < NSLOT; ++z)
-                            if ((uint32_t)z == cz)
-#pragma unroll
-                                for (int f = 0; f < 4; ++f) sl[z].acc[f] = cur.acc[f];
-                    }
-                    // the state writes above reach LDS before the counters (in order)
-                    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                    if (r0 >= 0) __hip_atomic_store(&st.cnt[r0], t0 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (r1 >= 0) __hip_atomic_store(&st.cnt[r1], t1 + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    __builtin_amdgcn_s_setprio(0);
-                    have = false;
-                    spins = 0;
-                    if (++cz == nslot) { cz = 0; ++k; }
-                } else {
-                    // every item's predecessors precede it, so some item is always
-                    // ready; a stall this long means corrupt ordering data: stop
-                    if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
-                    if (++spins > SPIN_LIMIT) {
-                        __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        S.w_status[w] = 5;
-                        break;
-                    }
-                }
-                // a wave with no lane ready yields its SIMD
-                if (__ballot(ready) == 0ull) __builtin_amdgcn_s_sleep(1);
-            }
-        }
-        __syncthreads();
-        // position integration (lib.zig:238-249)
-        for (int i = threadIdx.x; i < n; i += MAXT) {
-            if (D.flags[i] & BF_STATIC) continue;
-            float qd = sub_dt / D.mass[i];
-            D.px[i] += st.mx[i] * qd;
-            D.py[i] += st.my[i] * qd;
-            D.ang[i] += st.L[i] * sub_dt / D.inertia[i];
-            D.fx[i] = 0.0f; D.fy[i] = 0.0f;
-            D.tq[i] = 0.0f;
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int z = 0; z < NSLOT; ++z) {
-        if (!sl[z].flags || (sl[z].flags & RF_JOINT)) continue;
-        Rec r;
-        rec_from_slot(r, sl[z]);
-        rec_writeback(r, S);
-    }
-    for (int i = threadIdx.x; i < n; i += MAXT) {
-        D.mx[i] = st.mx[i]; D.my[i] = st.my[i]; D.L[i] = st.L[i];
-    }
-}
-
-// the register-slot kernel: the worlds solve_route gives it, one workgroup each
-template <int NSLOT, int MAXT, int WAVES, bool LOCKSTEP = false>
-__global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WAVES)))
-void k_solve_slots(StepDev S, float dt, uint32_t sub_steps, uint32_t iters, uint32_t slot_nmax)
-{
-    extern __shared__ __align__(16) uint32_t smem[];
-    __shared__ uint32_t s_abort;
-    if (S.counters[C_OVERFLOW]) return;
-    const uint32_t w = S.w_order[blockIdx.x];
-    if (S.w_status[w] != 0) return;
-    const uint32_t ibase = S.w_item_base[w];
-    const uint32_t nitems = S.w_item_base[w + 1] - ibase;
-    const WorldDev& D = S.worlds[w];
-    if (solve_route((uint32_t)D.nbodies, nitems, (uint32_t)NSLOT * MAXT, slot_nmax, 0u, D.warm > 0.0f) != 0) return;
-    slots_world<NSLOT, MAXT, LOCKSTEP>(S, D, w, ibase, nitems, S.w_man_begin[w], S.deg + D.body_base, dt, sub_steps,
-                                       iters, smem, s_abort);
 }
 
 // ------------------------------------------------------ fused world steps
@@ -3440,12 +1426,16 @@ __device__ __forceinline__ void fused_overflow(const StepDev& S, uint32_t w, uin
 }
 
 // ------------------------------------------------- the solve of a fused step
+// what the gap between two chains reads of a world's bodies, in LDS or global
+template <class F, class U>
+struct BodyPoses {
+    F px, py, ang, mass, inertia;
+    U flags;
+};
 // a world's bodies in LDS during its sub-steps: momenta (16 bytes a body and a
 // spare one), position and angle, then mass, inertia and flags
-struct ChainBodies {
+struct ChainBodies : BodyPoses<LF, LU32> {
     LF3 m;
-    LF px, py, ang, mass, inertia;
-    LU32 flags;
 };
 
 // contact point record (words as in r2d_chain.h); the bodies' inverse masses
@@ -3510,10 +1500,11 @@ __device__ __forceinline__ PointBodies point_bodies(const StepDev& S, const Worl
 // Returns whether updateTGSDepth is live for it: a point whose depth is not
 // within 1e-4 of its original depth, which at the step's start is the same
 // number, so NaN or so deep that 1e-4 vanishes in it (1), and whether one of
-// its bodies is static and an ordering body (2).
-template <bool WARM>
+// its bodies is static and an ordering body (2).  place(slot): where the
+// chain keeps a body's momentum.
+template <bool WARM, class PLACE>
 __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev& D, u4v* recs, uint32_t m, uint32_t base,
-                                            uint32_t j, uint32_t p1, float sub_dt)
+                                            uint32_t j, uint32_t p1, float sub_dt, PLACE place)
 {
     const size_t cm = S.cap_m;
     float* P = S.m_pt;
@@ -3529,6 +1520,8 @@ __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev
     }
     const float mua = D.mu[a], mub = D.mu[b];
     PointBodies B = point_bodies(S, D, base, a, b);
+    B.a = place(a);
+    B.b = place(b);
     if (WARM && (valid & MV_WARM)) B.flag_b |= PR_WARM;
     const float fric = sqrt_rn(mua * mub);   // preStep (collision.zig:114)
     S.m_fric[m] = fric;
@@ -3558,8 +1551,8 @@ __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev
 // recompute depth and (preStep) the effective masses, in the step's arrays
 // and the records; reset(p): point p is separated now, its impulses are reset
 // (calculateImpulses does so in the sub-step's first iteration)
-template <class RESET>
-__device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u4v* recs, const ChainBodies& C, uint32_t m,
+template <class POSES, class RESET>
+__device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u4v* recs, const POSES& C, uint32_t m,
                                           uint32_t base, uint32_t j, uint32_t p1, float sub_dt, RESET reset)
 {
     const size_t cm = S.cap_m;
@@ -3603,7 +1596,9 @@ __device__ __forceinline__ void point_tgs(const StepDev& S, const WorldDev& D, u
 // momenta is fixed within a sub-step (poses after the previous sub-step's
 // position integration; torque as set for this one), so the terms that
 // Constraints/*.zig derive from it are computed here, once, in their order.
-__device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const WorldDev& D, const ChainBodies& C, bool first)
+template <class POSES, class PLACE>
+__device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const WorldDev& D, const POSES& C, bool first,
+                                             PLACE place)
 {
     const uint32_t type = (uint32_t)J.type, a = (uint32_t)J.s1, b = type <= 1u ? (uint32_t)J.s2 : a;
     u4v q0{PR_JOINT, type << PR_TYPE_SHIFT, 0u, 0u}, q1{}, q2{}, q3{};
@@ -3613,8 +1608,8 @@ __device__ __forceinline__ void joint_record(u4v* q, const Joint& J, const World
         return;
     }
     const bool sa = (C.flags[a] & BF_STATIC) != 0, sb = (C.flags[b] & BF_STATIC) != 0;
-    q0.x |= a | (type <= 1u && a == b ? PR_SELF : 0u);
-    q0.y |= b;
+    q0.x |= place(a) | (type <= 1u && a == b ? PR_SELF : 0u);
+    q0.y |= place(b);
     q1.y = asu(J.pmin);
     q1.z = asu(J.pmax);
     const float im1 = sa ? 0.0f : 1.0f / C.mass[a], im2 = sb ? 0.0f : 1.0f / C.mass[b];
@@ -3668,39 +1663,41 @@ struct BodyIn {
 };
 
 // Body i's part of the gap between two chains: the position integration of
-// sub-step s - 1 (lib.zig:238-249), then the forces, AABB refresh and velocity
-// integration of sub-step s (lib.zig:200-216).  In between a dynamic body's
-// force and torque are zero, so they need no memory; only the last sub-step's
-// AABB is observable.  s == sub_steps: the positions, and the state back to
-// global memory.
-template <bool WARM>
-__device__ __forceinline__ void chain_body(const WorldDev& D, const BodyArrays& A, const ChainBodies& C, int i, uint32_t s,
-                                           uint32_t sub_steps, float sub_dt, uint32_t f, float mass, float inertia, float fx,
-                                           float fy, float tq)
+// sub-step s - 1 (lib.zig:238-249; body_move), then the forces, AABB refresh
+// and velocity integration of sub-step s (lib.zig:200-216; body_push).  In
+// between a dynamic body's force and torque are zero, so they need no memory;
+// only the last sub-step's AABB is observable.  After the last chain: the
+// positions, and the state back to global memory (body_done).
+struct BodyState {
+    f3v m;
+    float px, py, ang;
+};
+__device__ __forceinline__ void body_move(BodyState& b, float mass, float inertia, float sub_dt)
 {
-    const bool stat = (f & BF_STATIC) != 0;
-    const f3v m0 = C.m[i];
-    float mx = m0.x, my = m0.y, l = m0.z, px = C.px[i], py = C.py[i], ang = C.ang[i];
-    if (s > 0 && !stat) {
-        const float qd = sub_dt / mass;
-        px = px + mx * qd;
-        py = py + my * qd;
-        ang = ang + l * sub_dt / inertia;
-        C.px[i] = px; C.py[i] = py; C.ang[i] = ang;
+    const float qd = sub_dt / mass;
+    b.px = b.px + b.m.x * qd;
+    b.py = b.py + b.m.y * qd;
+    b.ang = b.ang + b.m.z * sub_dt / inertia;
+}
+
+__device__ __forceinline__ void body_done(const WorldDev& D, const BodyArrays& A, int i, bool stat, const BodyState& b)
+{
+    D.mx[i] = b.m.x; D.my[i] = b.m.y; D.L[i] = b.m.z;
+    if (!stat) {
+        A.px[i] = b.px; A.py[i] = b.py; A.ang[i] = b.ang;
+        A.fx[i] = 0.0f; A.fy[i] = 0.0f; A.tq[i] = 0.0f;
     }
-    if (s == sub_steps) {
-        D.mx[i] = mx; D.my[i] = my; D.L[i] = l;
-        if (!stat) {
-            A.px[i] = px; A.py[i] = py; A.ang[i] = ang;
-            A.fx[i] = 0.0f; A.fy[i] = 0.0f; A.tq[i] = 0.0f;
-        }
-        return;
-    }
-    if (s + 1 == sub_steps) {
+}
+
+template <bool WARM>
+__device__ __forceinline__ f3v body_push(const BodyArrays& A, int i, bool last, const BodyState& b, BodyIn in, float sub_dt)
+{
+    const bool stat = (in.f & BF_STATIC) != 0;
+    if (last) {
         // Disc.updateAABB / Rectangle.updateAABB
         float hw, hh;
-        if (f & BF_RECT) {
-            const float c = cosf_r(ang), sn = sinf_r(ang);
+        if (in.f & BF_RECT) {
+            const float c = cosf_r(b.ang), sn = sinf_r(b.ang);
             const float x = A.hw[i], y = A.hh[i];
             v2 lv[4] = {mk(-x, -y), mk(-x, y), mk(x, y), mk(x, -y)};
             hw = 0.f; hh = 0.f;
@@ -3713,35 +1710,36 @@ __device__ __forceinline__ void chain_body(const WorldDev& D, const BodyArrays& 
         } else {
             hw = hh = A.rad[i];
         }
-        A.ax[i] = px; A.ay[i] = py; A.ahw[i] = hw; A.ahh[i] = hh;
+        A.ax[i] = b.px; A.ay[i] = b.py; A.ahw[i] = hw; A.ahh[i] = hh;
     }
-    if (stat) return;
+    if (stat) return b.m;
     for (int g = 0; g < A.ngens; ++g) {
         const auto& G = A.gens[g];   // fields read one by one (keeps G's address space)
         if (G.type == 0) {
-            fx += G.gx * mass;
-            fy += G.gy * mass;
+            in.fx += G.gx * in.mass;
+            in.fy += G.gy * in.mass;
         } else if (G.slot == i) {
-            const float inv_m = 1.0f / mass;
-            const v2 v = scale2(mk(mx, my), inv_m);
-            const v2 d = sub2(mk(px, py), mk(G.ax, G.ay));
-            fx += (-G.k) * d.x - G.c * v.x;
-            fy += (-G.k) * d.y - G.c * v.y;
+            const float inv_m = 1.0f / in.mass;
+            const v2 v = scale2(mk(b.m.x, b.m.y), inv_m);
+            const v2 d = sub2(mk(b.px, b.py), mk(G.ax, G.ay));
+            in.fx += (-G.k) * d.x - G.c * v.x;
+            in.fy += (-G.k) * d.y - G.c * v.y;
         }
     }
-    mx += fx * sub_dt;
-    my += fy * sub_dt;
-    l += tq * sub_dt;
+    f3v m = b.m;
+    m.x += in.fx * sub_dt;
+    m.y += in.fy * sub_dt;
+    m.z += in.tq * sub_dt;
     if constexpr (WARM) {
         if (A.warm > 0.0f) {
             // warm starting: the body's share of the matched manifolds' carried impulses
-            const auto ws = warm_sum(A, i);
-            mx += ws[0];
-            my += ws[1];
-            l += ws[2];
+            const GlbCF ws = warm_sum(A, i);
+            m.x += ws[0];
+            m.y += ws[1];
+            m.z += ws[2];
         }
     }
-    C.m[i] = f3v{mx, my, l};
+    return m;
 }
 
 // The kernel's argument block and the worlds' descriptors as the out-of-line
@@ -3837,7 +1835,8 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
             C.px[i] = D.px[i]; C.py[i] = D.py[i]; C.ang[i] = D.ang[i];
         }
         for (uint32_t q = t0; q < M; q += stride) {
-            const uint32_t f = point_build<WARM>(S, D, recs, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt);
+            const uint32_t f = point_build<WARM>(S, D, recs, mbeg + q, base, nj + q, S.it_k0[ibase + nj + q], sub_dt,
+                                                 [](uint32_t x) { return x; });
             if (f & 1u) sh.live = 1u;
             if (f & 2u) sh.fix = 1u;
         }
@@ -3891,7 +1890,14 @@ __device__ __attribute__((noinline)) void chain_bodies(StepArgs KS, LU32 smem, R
         } else {
             in.f = C.flags[i]; in.mass = C.mass[i]; in.inertia = C.inertia[i];
         }
-        chain_body<WARM>(D, A, C, i, s, sub_steps, sub_dt, in.f, in.mass, in.inertia, in.fx, in.fy, in.tq);
+        const bool stat = (in.f & BF_STATIC) != 0;
+        BodyState b{C.m[i], C.px[i], C.py[i], C.ang[i]};
+        if (s > 0u && !stat) {
+            body_move(b, in.mass, in.inertia, sub_dt);
+            C.px[i] = b.px; C.py[i] = b.py; C.ang[i] = b.ang;
+        }
+        if (s == sub_steps) body_done(D, A, i, stat, b);
+        else C.m[i] = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
     }
 }
 
@@ -3908,7 +1914,7 @@ __device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     s = uniform(s);
-    for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u);
+    for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u, [](uint32_t x) { return x; });
     const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
     GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
     if (sh.live)
@@ -3978,16 +1984,17 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
     const StepDev& S = *(const StepDev*)KS;
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
     const uint32_t sub_steps = uniform(sh.sub_steps), iters = uniform(sh.iters), nj = uniform(sh.nj);
-    const bool chain = nj + sh.M > 0u && iters > 0u, items = nj || sh.live || (WARM && D.warm > 0.0f);
+    const bool any = nj + sh.M > 0u, items = nj || sh.live || (WARM && D.warm > 0.0f);
     for (uint32_t s = 0;; ++s) {
         chain_bodies<T, WARM>(KS, smem, shl, s);
         if (s == sub_steps) break;
         __syncthreads();
-        if (!chain) continue;
+        if (!any) continue;
         if (items) {
             chain_items<T, WARM>(KS, smem, shl, s);
             __syncthreads();
         }
+        if (iters == 0u) continue;
         const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters;
         const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
         const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
@@ -4008,6 +2015,258 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         __syncthreads();
     }
     chain_finish<T>(KS, smem, shl);
+}
+
+// ------------------------------------------- the solve in separate launches
+// For the worlds whose step is not one kernel: grid-wide kernels over all
+// worlds' bodies and items around a workgroup per world that plans, then (once
+// per sub-step) runs its program.  The momenta of the bodies that take part in
+// items live under chain places (cmap) in g_mom between the launches, 16 bytes
+// each, so that a chain takes them into LDS with plain wide copies; poses stay
+// in the world's arrays.
+typedef BodyPoses<GlbCF, GlbCU> GlobalPoses;
+__device__ __forceinline__ GlobalPoses global_poses(const WorldDev& D)
+{
+    GlobalPoses P;
+    P.px = (GlbCF)D.px; P.py = (GlbCF)D.py; P.ang = (GlbCF)D.ang; P.mass = (GlbCF)D.mass; P.inertia = (GlbCF)D.inertia;
+    P.flags = (GlbCU)D.flags;
+    return P;
+}
+// a world's momenta: one place more than its bodies
+__device__ __forceinline__ GF3 world_momenta(const StepDev& S, const WorldDev& D, uint32_t w)
+{
+    return (GF3)(S.g_mom + D.body_base + w);
+}
+
+// the planning state of item j of a world, and where its second point is
+__device__ __forceinline__ void plan_item(const StepDev& S, uint32_t ibase, uint32_t j, uint32_t nit, uint32_t second)
+{
+    const uint32_t it = ibase + j;
+    const int32_t r0 = S.it_r0[it], r1 = S.it_r1[it];
+    auto next = [&](int32_t r, uint32_t k, uint32_t& need) {
+        const uint32_t o = S.deg_off[r], c = S.deg_off[r + 1] - o;
+        need += k > 0u ? 1u : 0u;
+        return (S.lists[o + (k + 1u == c ? 0u : k + 1u)] >> 1) - ibase;
+    };
+    uint32_t need = 0u, s0 = j, s1 = nit | SINGLE;   // no ordering body: the item only follows itself
+    if (r0 >= 0) s0 = next(r0, S.it_k0[it], need);
+    if (r1 >= 0) {
+        const uint32_t q = next(r1, S.it_k1[it], need);
+        if (r0 >= 0) s1 = q; else s0 = q;
+    }
+    S.it_k0[it] = nit + second - 1u;                 // the ranks are not read again
+    S.plan_items[2 * (size_t)ibase + j] = make_uint4(s0, s1, need * STATE_BODY + S.chain_iters, second);
+}
+
+// per item: planning state, and the records of a manifold's points
+template <bool WARM>
+__global__ __launch_bounds__(256) void k_chain_build(StepDev S, float sub_dt)
+{
+    if (S.counters[C_OVERFLOW]) return;
+    for (uint32_t q = grid_tid(); q < S.njoints; q += grid_stride()) {
+        uint32_t lo = 0, hi = S.nworlds;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (S.worlds[mid].joint_base <= q) lo = mid; else hi = mid;
+        }
+        const uint32_t ibase = S.w_item_base[lo];
+        plan_item(S, ibase, q - S.worlds[lo].joint_base, S.w_item_base[lo + 1] - ibase, 0u);
+    }
+    const uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
+    for (uint32_t m = grid_tid(); m < M; m += grid_stride()) {
+        const uint32_t w = S.bworld[S.m_ref[m]];
+        const WorldDev& D = S.worlds[w];
+        const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, base = D.body_base;
+        const uint32_t j = (uint32_t)D.njoints + (m - S.w_man_begin[w]);
+        const bool pair = (S.m_valid[m] & 3u) == 3u;
+        const uint32_t rank = world_rank(S, pair, w, &WorldChain::pairs), second = pair ? 1u + rank : 0u;
+        plan_item(S, ibase, j, nit, second);
+        const uint32_t f = point_build<WARM>(S, D, reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8), m, base, j,
+                                             nit + second - 1u, sub_dt, [&](uint32_t x) { return S.cmap[base + x]; });
+        if (f) atomicOr(&S.w_chain[w].flags, f);
+    }
+}
+
+// the program of each world, one workgroup each
+template <int T>
+__global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
+{
+    extern __shared__ __align__(16) uint32_t smem[];
+    __shared__ ChainShared sh;
+    if (S.counters[C_OVERFLOW]) return;
+    const uint32_t w = S.w_order[blockIdx.x];
+    const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, nj = (uint32_t)S.worlds[w].njoints;
+    if (S.w_status[w] != 0 || nit == 0u) return;
+    const uint32_t t = threadIdx.x, kc = S.chain_iters, waves = chain_waves(nit, kc, (uint32_t)T / 64u);
+    const bool in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= lds_words;
+    if (t == 0) {
+        sh.ready = sh.taken = sh.entries = 0u;
+        sh.queued[0] = sh.queued[1] = sh.queued[2] = 0u;
+    }
+    __syncthreads();
+    Program G;
+    G.rows = (GU2)(S.prog_rows + (size_t)ibase * kc);
+    G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+    G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
+    const GU4 items = (GU4)(S.plan_items + 2 * (size_t)ibase);
+    PlanLds PL((LU32)smem, nit, waves);
+    PlanGlb PG(items, (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
+    auto start = [&](auto& P, bool init) {
+        for (uint32_t j = t; j < nit; j += T) {
+            const u4v v = items[j];
+            if (init) P.init(j, v.x, v.y, v.z, v.w);
+            if (v.z < STATE_BODY)
+                P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
+                       PlanEntry{j, v.w, v.x, v.y});
+        }
+        if (t == 0u) P.init(nit, nit, nit | SINGLE, 0u, 0u);   // the spare item: no iterations, never ready
+    };
+    if (in_lds) start(PL, true); else start(PG, false);
+    __syncthreads();
+    const uint32_t ready = uniform(sh.ready);
+    uint32_t ns = 0u;
+    if (waves > 1u)
+        ns = in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh) : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
+    else if (t < 64u)
+        ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready) : plan_single(PG, G, nit, nj, kc, ready);
+    if (t == 0) {
+        S.w_chain[w].slots = ns;
+        if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
+    }
+}
+
+// The gap before sub-step s's chain (s == sub_steps: after the last one):
+// bodies, and after the last one the impulses into the step's manifold arrays
+// (what r2d_get_manifolds reports)
+template <bool WARM>
+__global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uint32_t sub_steps, float sub_dt)
+{
+    if (S.counters[C_OVERFLOW]) return;
+    for (uint32_t x = grid_tid(); x < S.nb; x += grid_stride()) {
+        const uint32_t w = S.bworld[x];
+        if (S.w_status[w] != 0) continue;
+        const WorldDev& D = S.worlds[w];
+        const BodyArrays A = body_arrays(D);
+        const int i = (int)(x - D.body_base);
+        const uint32_t c = S.cmap[x];
+        const bool touched = c != UNTOUCHED;
+        const GF3 mom = world_momenta(S, D, w) + (touched ? c : 0u);
+        BodyIn in{A.flags[i], A.mass[i], A.inertia[i], 0.f, 0.f, 0.f};
+        BodyState b;
+        if (s > 0u && touched) b.m = *mom; else b.m = f3v{D.mx[i], D.my[i], D.L[i]};
+        b.px = A.px[i]; b.py = A.py[i]; b.ang = A.ang[i];
+        const bool stat = (in.f & BF_STATIC) != 0;
+        if (s == 0u) { in.fx = A.fx[i]; in.fy = A.fy[i]; in.tq = A.tq[i]; }
+        else if (!stat) {
+            body_move(b, in.mass, in.inertia, sub_dt);
+            if (s < sub_steps) { A.px[i] = b.px; A.py[i] = b.py; A.ang[i] = b.ang; }
+        }
+        if (s == sub_steps) { body_done(D, A, i, stat, b); continue; }
+        const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
+        if (touched) *mom = m;
+        else { D.mx[i] = m.x; D.my[i] = m.y; D.L[i] = m.z; }
+    }
+    if (s != sub_steps) return;
+    const size_t cm = S.cap_m;
+    const uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
+    for (uint32_t m = grid_tid(); m < M; m += grid_stride()) {
+        const uint32_t w = S.bworld[S.m_ref[m]];
+        if (S.w_status[w] != 0) continue;
+        const uint32_t ibase = S.w_item_base[w], q = m - S.w_man_begin[w], nj = (uint32_t)S.worlds[w].njoints;
+        const GF2 acc = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+        const uint32_t valid = S.m_valid[m];
+        for (uint32_t p = 0; p < 2u; ++p) {
+            if (!(valid & (1u << p))) continue;
+            const f2v v = acc[p ? S.it_k0[ibase + nj + q] - nj : q];
+            S.m_pt[(MP_ACC_PN * 2 + p) * cm + m] = v.x;
+            S.m_pt[(MP_ACC_PT * 2 + p) * cm + m] = v.y;
+        }
+    }
+}
+
+// Sub-step s's joint records, moved contact points and carried impulses, and
+// its K iterations, one workgroup per world.  Momenta in LDS for worlds of at
+// most lds_nmax bodies whose places fit it, and beside them the impulses when
+// they fit too; otherwise they stay in global memory.
+template <int T, bool WARM>
+__global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t iters, float sub_dt, uint32_t lds_words,
+                                                 uint32_t lds_nmax)
+{
+    extern __shared__ __align__(16) uint32_t smem[];
+    if (S.counters[C_OVERFLOW]) return;
+    const uint32_t w = S.w_order[blockIdx.x];
+    const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase;
+    if (S.w_status[w] != 0 || nit == 0u) return;
+    const WorldDev& D = S.worlds[w];
+    const WorldChain W = S.w_chain[w];
+    const uint32_t t = threadIdx.x, nj = (uint32_t)D.njoints, M = nit - nj, mbeg = S.w_man_begin[w], base = D.body_base;
+    const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + 1u);
+    const bool m_lds = (uint32_t)D.nbodies <= lds_nmax && mwords <= lds_words;
+    const bool a_lds = m_lds && mwords + 2u * nacc <= lds_words;
+    const LF3 m = (LF3)(LU32)smem;
+    const LF2 acc = (LF2)((LU32)smem + mwords);
+    const GF3 mom = world_momenta(S, D, w);
+    const GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+    u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
+    if (m_lds)
+        for (uint32_t c = t; c < nc; c += T) m[c] = mom[c];
+    if (s == 0u)
+        for (uint32_t q = t; q < nacc; q += T) {
+            if (a_lds) acc[q] = f2v{0.f, 0.f}; else accg[q] = f2v{0.f, 0.f};
+        }
+    else if (a_lds)
+        for (uint32_t q = t; q < nacc; q += T) acc[q] = accg[q];
+    const GlobalPoses C = global_poses(D);
+    for (uint32_t j = t; j < nj; j += T)
+        joint_record(recs + (size_t)j * 4u, D.joints[j], D, C, s == 0u, [&](uint32_t x) { return S.cmap[base + x]; });
+    __syncthreads();
+    if (W.flags & 1u) {
+        for (uint32_t q = t; q < M; q += T) {
+            const uint32_t p1 = S.it_k0[ibase + nj + q];
+            point_tgs(S, D, recs, C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
+                const uint32_t at = p ? p1 - nj : q;
+                if (a_lds) acc[at] = f2v{0.f, 0.f}; else accg[at] = f2v{0.f, 0.f};
+            });
+        }
+    }
+    if constexpr (WARM) {
+        if (D.warm > 0.0f) {
+            const size_t cm = S.cap_m;
+            for (uint32_t q = t; q < M; q += T) {
+                // warm starting: the carried impulse per sub-step joins the accumulators
+                const uint32_t mi = mbeg + q, valid = S.m_valid[mi];
+                if (!(valid & MV_WARM)) continue;
+                for (uint32_t p = 0; p < 2u; ++p) {
+                    if (!(valid & (1u << p))) continue;
+                    const f2v add{S.m_pt[(MP_WARM_N * 2 + p) * cm + mi], S.m_pt[(MP_WARM_T * 2 + p) * cm + mi]};
+                    const uint32_t at = p ? S.it_k0[ibase + nj + q] - nj : q;
+                    if (a_lds) acc[at] = acc[at] + add; else accg[at] = accg[at] + add;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (iters > 0u) {
+        const uint32_t kc = S.chain_iters, reps = iters / kc, ns = W.slots;
+        const GCU2 rows = (GCU2)(S.prog_rows + (size_t)ibase * kc), slots = (GCU2)(S.prog_slots + (size_t)ibase * kc);
+        const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+        const GCU4 rec = (GCU4)(S.recs + (size_t)ibase * 8);
+        const bool fix = (W.flags & 2u) != 0u;
+        if (chain_waves(nit, kc, (uint32_t)T / 64u) > 1u) {
+            if (a_lds) chain_lds<true, WARM>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<true, WARM>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, fix, sub_dt);
+            else chain_glb<true, WARM>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, fix, sub_dt);
+        } else if (t < 64u) {
+            if (a_lds) chain_lds<false, WARM>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<false, WARM>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, fix, sub_dt);
+            else chain_glb<false, WARM>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, fix, sub_dt);
+        }
+        __syncthreads();
+    }
+    if (m_lds)
+        for (uint32_t c = t; c < nc; c += T) mom[c] = m[c];
+    if (a_lds)
+        for (uint32_t q = t; q < nacc; q += T) accg[q] = acc[q];
 }
 
 // One workgroup per world (S.w_order), up to nsteps steps per world counted
@@ -4339,67 +2598,38 @@ static inline unsigned blocks_for(uint64_t n, unsigned bs, unsigned cap = 4096)
     return (unsigned)b;
 }
 
-size_t solve_lds_bytes(int nbodies) { return (size_t)nbodies * 7u * 4u; }
-
-typedef void (*SlotFn)(StepDev, float, uint32_t, uint32_t, uint32_t);
-typedef void (*RecFn)(StepDev, float, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
 typedef void (*FusedFn)(StepDev, float, uint32_t, uint32_t, uint32_t, uint32_t);
 struct SolveVariant {
-    SlotFn slot_fn;      // register-slot kernel (nullptr: none)
-    unsigned slot_threads;
-    int slots;
-    RecFn rec_fn;        // record kernel (LDS body state) for the worlds the slot kernel leaves
-    unsigned threads;
-    FusedFn fused_fn;    // whole steps per workgroup with the slot kernel's shape (nullptr: none)
-    unsigned fused_t;    // the fused kernel's workgroup size when it is neither slot_threads nor threads
+    unsigned threads;    // workgroup of the separate launches' chain (CHAIN_THREADS or CHAIN_NARROW)
+    FusedFn fused_fn;    // whole steps per workgroup (nullptr: none)
+    unsigned fused_t;    // its workgroup size
 };
-// solve variants: the register-slot kernel's slots x workgroup size, and the
-// record kernel's workgroup size for worlds with more items than slots
-// (fewer waves per world keep a dependency chain's wave from sharing its
-// SIMD with the world's other waves: 256 threads beat 1,024 by about 3x on a
-// 4,096-body world)
+constexpr unsigned CHAIN_THREADS = 512, CHAIN_NARROW = 256;
+// Solve variants: shapes of the kernels that run worlds' programs.  The fused
+// kernels differ in threads and in waves per SIMD (registers); 0, 6 and 8
+// have none and take the separate launches.
 static const SolveVariant kSolveVariants[SOLVE_TABLE] = {
-    {nullptr, 0, 0, k_solve<1024>, 1024, nullptr},
-    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<256, 2>, 256, k_fused<256, 3>},
-    {k_solve_slots<2, 512, 3>, 512, 2, k_solve<256, 2>, 256, k_fused<512, 3>},
-    {k_solve_slots<3, 256, 3>, 256, 3, k_solve<256, 2>, 256, k_fused<256, 3>},
-    {k_solve_slots<4, 256, 2>, 256, 4, k_solve<256, 2>, 256, k_fused<256, 2>},
-    {k_solve_slots<8, 128, 2>, 128, 8, k_solve<256, 2>, 256, k_fused<128, 2>},
-    {nullptr, 0, 0, k_solve<256, 2>, 256, nullptr},
-    {k_solve_slots<4, 256, 3>, 256, 4, k_solve<128, 2>, 128, k_fused<256, 3>},
-    // the lockstep slot walk takes the phase kernels only: its fused kernel
-    // hung once in a test with no cause found, so it is not built
-    {k_solve_slots<3, 256, 3, true>, 256, 3, k_solve<256, 2>, 256, nullptr},
-    // records only (as variant 6), fused with 3 or 4 waves per SIMD: fewer
-    // registers than the slots, so more worlds resident per CU
-    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<256, 3>},
-    {nullptr, 0, 0, k_solve<256, 2>, 256, k_fused<256, 4>},
-    // records only, 192-thread workgroups: with the records' smaller LDS
-    // state, four worlds of 500 bodies are resident per CU
-    {nullptr, 0, 0, k_solve<192, 3>, 192, k_fused<192, 3>},
-    // records only, 128-thread workgroups at 2 waves per SIMD: the same four
-    // worlds per CU with the full register file (no spills)
-    {nullptr, 0, 0, k_solve<128, 2>, 128, k_fused<128, 2>},
-    // records only, 512-thread workgroups at 2 waves per SIMD (the full
-    // register file): for a few worlds, each alone on a CU, whose chains are
-    // latency-bound; up to 512 items no lane ever changes record
-    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<512, 2>},
-    // WIDE_VARIANT: 768 lanes at 3 waves per SIMD (the register budget of
-    // variant 11), up to 768 items without a pickup.  A lane that holds two
-    // items serialises them, which can triple a chain (the 20-row pyramid's
-    // 520-590 items: 148 links per sub-step with a lane per item, 403-437
-    // with 512 lanes), so the widest shape that does not spill wins
-    {nullptr, 0, 0, k_solve<REC_WIDE_THREADS, 1>, REC_WIDE_THREADS, k_fused<768, 3>, 768},
-    // WARM_VARIANT: batches with a warm-started world (the shape of variant
-    // 11 with the warm-start passes compiled in; the kernels above carry none)
-    {nullptr, 0, 0, k_solve<192, 3, true>, 192, k_fused<192, 3, true>},
+    {CHAIN_THREADS, nullptr, 0},
+    {CHAIN_NARROW, k_fused<256, 3>, 256},
+    {CHAIN_NARROW, k_fused<512, 3>, 512},
+    {CHAIN_NARROW, k_fused<256, 3>, 256},
+    {CHAIN_NARROW, k_fused<256, 2>, 256},
+    {CHAIN_NARROW, k_fused<128, 2>, 128},
+    {CHAIN_NARROW, nullptr, 0},
+    {CHAIN_NARROW, k_fused<256, 3>, 256},
+    {CHAIN_NARROW, nullptr, 0},
+    {CHAIN_NARROW, k_fused<256, 3>, 256},
+    {CHAIN_NARROW, k_fused<256, 4>, 256},
+    {CHAIN_NARROW, k_fused<192, 3>, 192},
+    {CHAIN_NARROW, k_fused<128, 2>, 128},
+    {CHAIN_THREADS, k_fused<512, 2>, 512},
+    {CHAIN_THREADS, k_fused<768, 3>, 768},      // WIDE_VARIANT
+    {CHAIN_NARROW, k_fused<192, 3, true>, 192}, // WARM_VARIANT (the kernels above carry no warm-start passes)
 };
 
 uint32_t fused_threads(int v)
 {
-    const SolveVariant& sv = kSolveVariants[v];
-    if (sv.fused_t) return sv.fused_t;
-    return sv.slot_fn ? (uint32_t)sv.slot_threads : (uint32_t)sv.threads;
+    return kSolveVariants[v].fused_t;
 }
 
 // a fused kernel runs only at the workgroup size it was compiled for (its
@@ -4425,9 +2655,6 @@ void launch_fused(const StepDev& S, int v, uint32_t nworlds, float dt, uint32_t 
     hipLaunchKernelGGL(sv.fused_fn, dim3(nworlds), dim3(threads), lds, st, S, dt, sub_steps, iters, nsteps,
                        (uint32_t)(lds / 4u));
 }
-
-unsigned solve_variant_threads(int v) { return kSolveVariants[v < SOLVE_TABLE && v >= 0 ? v : 0].threads; }
-int solve_variant_slots(int v) { return kSolveVariants[v < SOLVE_TABLE && v >= 0 ? v : 0].slots; }
 
 void KernelTrace::mark(const char* name, hipStream_t st)
 {
@@ -4494,27 +2721,16 @@ SolvePlan plan_solve(int variant, const uint32_t* nbodies, size_t nw, uint32_t l
     SolvePlan p;
     p.any_colored = any_colored ? 1u : 0u;
     p.any_warm = any_warm ? 1u : 0u;
-    p.variant = (variant >= 0 && variant < SOLVE_TABLE) ? variant : 0;
-    const SolveVariant& v = kSolveVariants[p.variant];
-    p.slot_cap = v.slot_fn ? (uint32_t)v.slots * v.slot_threads : 0u;
-    p.slot_nmax = v.slot_fn ? SLOT_NMAX : 0u;
-    p.lds_nmax = (uint32_t)((160u * 1024u - 1024u - rec_lane_bytes(v.threads)) / solve_lds_bytes(1));
-    if (lds_limit) p.lds_nmax = std::min(p.lds_nmax, lds_limit);
-    for (size_t i = 0; i < nw; ++i) {
-        uint32_t n = nbodies[i];
-        if (p.slot_cap && n <= p.slot_nmax) { p.any_slot = 1; p.slot_maxn = std::max(p.slot_maxn, n); }
-        if (n <= p.lds_nmax) { p.any_lds = 1; p.lds_maxn = std::max(p.lds_maxn, n); p.n_lds += 1; }
-        else { p.any_big = 1; p.n_big += 1; }
-    }
-    // A few worlds, each alone on a CU, are latency-bound on their chains:
-    // more lanes hold fewer positions each and wait less (4,096-body world:
-    // 0.71 -> 0.58 ms per step with 512 lanes).  Many worlds share CUs and
-    // are issue-bound: the variant's shape.  The wide kernel's lane slots
-    // leave LDS for fewer bodies.
-    const uint32_t wide_nmax = (uint32_t)((160u * 1024u - 1024u - rec_lane_bytes(REC_WIDE_THREADS)) /
-                                          solve_lds_bytes(1));
-    p.rec_wide = (allow_wide && p.any_lds && !any_warm && p.n_lds <= 64u && p.lds_maxn <= wide_nmax &&
-                  kSolveVariants[p.variant].threads < REC_WIDE_THREADS) ? 1u : 0u;
+    p.lds_nmax = lds_limit ? lds_limit : 0xffffffffu;
+    p.wide = nw <= CHAIN_WIDE_WORLDS && allow_wide ? 1u : 0u;
+    if (variant >= 0 && variant < SOLVE_TABLE && kSolveVariants[variant].threads == CHAIN_THREADS) p.wide = 1u;
+    // LDS: worlds that are alone on their CU take all of it; of larger batches
+    // each world takes what its momenta (16 bytes a touched body), impulses (8
+    // a point) and plan (18 an item) commonly need, so that CUs hold several
+    uint32_t maxn = 0;
+    for (size_t i = 0; i < nw; ++i) maxn = std::max(maxn, nbodies[i]);
+    const size_t want = std::max<size_t>(CHAIN_LDS_MIN, (size_t)maxn * CHAIN_LDS_BODY);
+    p.lds = (uint32_t)(nw <= CHAIN_WIDE_WORLDS ? CHAIN_LDS : std::min<size_t>(CHAIN_LDS, want));
     return p;
 }
 
@@ -4571,10 +2787,8 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
         tmark(ss, "k_world_ranges", st);
         hipLaunchKernelGGL(k_joint_mark, dim3(blocks_for(S.njoints, BS)), dim3(BS), 0, st, S);
         tmark(ss, "k_joint_mark", st);
-        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(S.nb + 1, BS)), dim3(BS), 0, st, S.deg, S.nb + 1);
-        tmark(ss, "k_zero_u32", st);
-        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(S.nb + 1, BS)), dim3(BS), 0, st, S.deg_fill, S.nb + 1);
-        tmark(ss, "k_zero_u32", st);
+        hipLaunchKernelGGL(k_items_clear, dim3(blocks_for(S.nb + 1, BS)), dim3(BS), 0, st, S);
+        tmark(ss, "k_items_clear", st);
         hipLaunchKernelGGL(k_items_joints, dim3(blocks_for(S.njoints, BS)), dim3(BS), 0, st, S);
         tmark(ss, "k_items_joints", st);
         hipLaunchKernelGGL(k_items_mans, dim3(GRID), dim3(BS), 0, st, S);
@@ -4585,13 +2799,10 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
         tmark(ss, "k_list_fill", st);
         hipLaunchKernelGGL(k_list_rank<false>, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
         tmark(ss, "k_list_rank<false>", st);
-        {
-            // the level order's work arrays: 96 KB for batches of up to 256
-            // worlds (items per world up to ~8,000), 32 KB for larger ones
-            const size_t lds = S.nworlds <= 256u ? 96u * 1024u : 32u * 1024u;
-            hipLaunchKernelGGL(k_color, dim3(S.nworlds), dim3(256), lds, st, S, (uint32_t)(lds / 4u));
+        if (sp.any_colored) {
+            hipLaunchKernelGGL(k_color, dim3(S.nworlds), dim3(256), 0, st, S);
+            tmark(ss, "k_color", st);
         }
-        tmark(ss, "k_color", st);
         hipLaunchKernelGGL(k_world_order, dim3(1), dim3(1024), 0, st, S);
         tmark(ss, "k_world_order", st);
         if (sp.any_colored) {
@@ -4606,77 +2817,28 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
         }
         break;
     default: {
-        // the three solve kernels take disjoint sets of worlds (solve_route);
-        // the record kernels run on side streams beside the slot kernel
-        const SolveVariant& v = kSolveVariants[sp.variant];
-        const bool run_slot = v.slot_fn && sp.any_slot, run_lds = sp.any_lds != 0, run_big = sp.any_big != 0;
-        if (run_lds || run_big) {
-            (void)hipEventRecord(ss.fork, st);
-            if (run_big) (void)hipStreamWaitEvent(ss.aux[1], ss.fork, 0);
-            if (run_lds) (void)hipStreamWaitEvent(ss.aux[0], ss.fork, 0);
-        }
-        if (run_big) {
-            // worlds beyond LDS: grid-wide body and item phases around a
-            // one-workgroup-per-world chain kernel, all on the second side stream
-            const hipStream_t sb = ss.aux[1];
-            const float sub_dt = dt / (float)sub_steps;
-            const unsigned gb = blocks_for(S.nb, BS);
-            // the per-item passes: up to BIG_SPLIT workgroups per world beyond
-            // LDS, fewer when there are many of them or many other worlds
-            // (every world gets the same count and the others exit at once)
-            const uint32_t split = std::max<uint32_t>(
-                1u, std::min<uint32_t>({BIG_SPLIT, 256u / std::max<uint32_t>(sp.n_big, 1u),
-                                        8192u / std::max<uint32_t>(S.nworlds, 1u)}));
-            const dim3 gi(S.nworlds, split);
-            hipLaunchKernelGGL(k_big_bodies, dim3(gb), dim3(BS), 0, sb, S, sp.lds_nmax, 0, 0u, sub_steps, sub_dt);
-            hipLaunchKernelGGL(k_big_item_pass, gi, dim3(BIG_THREADS), 0, sb, S, sp.lds_nmax, 0, 0u, sub_steps, sub_dt);
-            hipLaunchKernelGGL(k_big_items, dim3(S.nworlds), dim3(BIG_THREADS), 0, sb, S, sp.lds_nmax);
-            for (uint32_t s = 0; s < sub_steps; ++s) {
-                hipLaunchKernelGGL(k_big_bodies, dim3(gb), dim3(BS), 0, sb, S, sp.lds_nmax, 1, s, sub_steps, sub_dt);
-                hipLaunchKernelGGL(k_big_item_pass, gi, dim3(BIG_THREADS), 0, sb, S, sp.lds_nmax, 1, s, sub_steps,
-                                   sub_dt);
-                // worlds whose touched bodies fit LDS, then those that do not
-                // the second launch's LDS: its lane slots, then the counters
-                constexpr size_t GLOBAL_LDS = COMPACT_LDS;
-                if (sp.any_warm) {
-                    hipLaunchKernelGGL((k_big_chain<256, true, 0>), dim3(S.nworlds), dim3(256), COMPACT_LDS, sb, S,
-                                       sp.lds_nmax, iters, sub_dt);
-                    hipLaunchKernelGGL((k_big_chain<BIG_GLOBAL_THREADS, true, 1>), dim3(S.nworlds),
-                                       dim3(BIG_GLOBAL_THREADS), GLOBAL_LDS, sb, S, sp.lds_nmax, iters, sub_dt);
-                } else {
-                    hipLaunchKernelGGL((k_big_chain<256, false, 0>), dim3(S.nworlds), dim3(256), COMPACT_LDS, sb, S,
-                                       sp.lds_nmax, iters, sub_dt);
-                    hipLaunchKernelGGL((k_big_chain<BIG_GLOBAL_THREADS, false, 1>), dim3(S.nworlds),
-                                       dim3(BIG_GLOBAL_THREADS), GLOBAL_LDS, sb, S, sp.lds_nmax, iters, sub_dt);
-                }
-                hipLaunchKernelGGL(k_big_bodies, dim3(gb), dim3(BS), 0, sb, S, sp.lds_nmax, 2, s, sub_steps, sub_dt);
+        const float sub_dt = dt / (float)sub_steps;
+        auto pick = [&](auto warm, auto cold) { return sp.any_warm ? warm : cold; };
+        const unsigned T = sp.wide ? CHAIN_THREADS : CHAIN_NARROW;
+        const uint32_t words = sp.lds / 4u;
+        if (sub_steps > 0) {   // without sub-steps nothing of a world changes
+            hipLaunchKernelGGL(pick(k_chain_build<true>, k_chain_build<false>), dim3(GRID), dim3(BS), 0, st, S, sub_dt);
+            tmark(ss, "k_chain_build", st);
+            if (iters > 0) {
+                hipLaunchKernelGGL(sp.wide ? k_chain_plan<CHAIN_THREADS> : k_chain_plan<CHAIN_NARROW>, dim3(S.nworlds), dim3(T),
+                                   sp.lds, st, S, words);
+                tmark(ss, "k_chain_plan", st);
             }
-            hipLaunchKernelGGL(k_big_item_pass, gi, dim3(BIG_THREADS), 0, sb, S, sp.lds_nmax, 2, 0u, sub_steps, sub_dt);
-            tmark(ss, "k_big (global state)", sb);
         }
-        if (run_lds && sp.rec_wide) {
-            hipLaunchKernelGGL((k_solve<REC_WIDE_THREADS, 1>), dim3(S.nworlds), dim3(REC_WIDE_THREADS),
-                               solve_lds_bytes((int)sp.lds_maxn) + rec_lane_bytes(REC_WIDE_THREADS), ss.aux[0], S, dt,
-                               sub_steps, iters, sp.slot_cap, sp.slot_nmax, sp.lds_nmax);
-            tmark(ss, "k_solve (record, wide)", ss.aux[0]);
-        } else if (run_lds) {
-            hipLaunchKernelGGL(v.rec_fn, dim3(S.nworlds), dim3(v.threads),
-                               solve_lds_bytes((int)sp.lds_maxn) + rec_lane_bytes(v.threads),
-                               ss.aux[0], S, dt, sub_steps, iters, sp.slot_cap, sp.slot_nmax, sp.lds_nmax);
-            tmark(ss, "k_solve (record)", ss.aux[0]);
-        }
-        if (run_slot) {
-            hipLaunchKernelGGL(v.slot_fn, dim3(S.nworlds), dim3(v.slot_threads), slot_lds_bytes((int)sp.slot_maxn),
-                               st, S, dt, sub_steps, iters, sp.slot_nmax);
-            tmark(ss, "k_solve_slots", st);
-        }
-        if (run_lds) {
-            (void)hipEventRecord(ss.join[0], ss.aux[0]);
-            (void)hipStreamWaitEvent(st, ss.join[0], 0);
-        }
-        if (run_big) {
-            (void)hipEventRecord(ss.join[1], ss.aux[1]);
-            (void)hipStreamWaitEvent(st, ss.join[1], 0);
+        for (uint32_t s = 0; sub_steps > 0; ++s) {
+            hipLaunchKernelGGL(pick(k_chain_bodies<true>, k_chain_bodies<false>), dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S, s,
+                               sub_steps, sub_dt);
+            tmark(ss, "k_chain_bodies", st);
+            if (s == sub_steps) break;
+            auto run = sp.wide ? pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>)
+                               : pick(k_chain_run<CHAIN_NARROW, true>, k_chain_run<CHAIN_NARROW, false>);
+            hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax);
+            tmark(ss, "k_chain_run", st);
         }
         if (sp.any_warm) {
             hipLaunchKernelGGL(k_warm_clear, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
@@ -4693,26 +2855,16 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
 
 void set_solve_smem_limit()
 {
-    (void)hipFuncSetAttribute((const void*)k_color, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_big_chain<256, false, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_solve<REC_WIDE_THREADS, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_big_chain<256, true, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_big_chain<BIG_GLOBAL_THREADS, false, 1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)k_big_chain<BIG_GLOBAL_THREADS, true, 1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    auto allow = [](const void* f) { (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); };
+    allow((const void*)k_chain_plan<CHAIN_THREADS>);
+    allow((const void*)k_chain_plan<CHAIN_NARROW>);
+    allow((const void*)k_chain_run<CHAIN_THREADS, false>);
+    allow((const void*)k_chain_run<CHAIN_THREADS, true>);
+    allow((const void*)k_chain_run<CHAIN_NARROW, false>);
+    allow((const void*)k_chain_run<CHAIN_NARROW, true>);
     for (int v = 0; v < SOLVE_TABLE; ++v) {
-        if (kSolveVariants[v].slot_fn)
-            (void)hipFuncSetAttribute((const void*)kSolveVariants[v].slot_fn,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)kSolveVariants[v].rec_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
         if (kSolveVariants[v].fused_fn) {
-            (void)hipFuncSetAttribute((const void*)kSolveVariants[v].fused_fn,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            allow((const void*)kSolveVariants[v].fused_fn);
             hipFuncAttributes fa{};
             g_fused_width_ok[v] = hipFuncGetAttributes(&fa, (const void*)kSolveVariants[v].fused_fn) == hipSuccess &&
                                   fa.maxThreadsPerBlock == (int)fused_threads(v);
