@@ -661,6 +661,7 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.recs, I * 128);
     const size_t K = c->cap_k;
     add((void**)&S.prog_rows, K * I * 8); add((void**)&S.prog_entries, 2 * K * I * 4); add((void**)&S.prog_slots, K * I * 8);
+    add((void**)&S.prog_recs, 2 * K * I * 64 + W * 512);
     add((void**)&S.plan_items, 2 * I * 16); add((void**)&S.plan_ring, 2 * I * 16);
     add((void**)&S.cmask, 2 * N * 8);
     add((void**)&S.g_cnt, N * 4); add((void**)&S.cmap, N * 4); add((void**)&S.g_mom, (N + W) * 16);

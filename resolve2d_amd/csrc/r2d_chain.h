@@ -201,6 +201,23 @@ struct Program {
     GU2 slots;
 };
 
+// Records in program order: entry e's four words of 16 bytes, in blocks of
+// four entries, so that a row's lanes read whole 64-byte pieces.  Gathered by
+// point, each of a row's four loads touches 64 cache lines, which the CU's
+// one address unit takes about 256 cycles a row for: nothing to one wave (a
+// row takes 890), but the bound of four or eight waves' slots (4,096-body
+// pile: 106 -> 88 us a sub-step).  Joints' records, which change every
+// sub-step, stay one a joint: after the entries, in the same blocks.
+__device__ __forceinline__ size_t entry_at(uint32_t e) { return (size_t)(e >> 2) * 16u + (e & 3u); }
+constexpr uint32_t ENTRY_WORD = 4;   // from one word of an entry to the next
+__device__ __forceinline__ void entry_copy(GU4 to, uint32_t e, GCU4 recs, uint32_t point)
+{
+    const GCU4 q = recs + (size_t)point * 4u;
+    const u4v a = q[0], b = q[1], c = q[2], d = q[3];
+    const GU4 p = to + entry_at(e);
+    p[0] = a; p[ENTRY_WORD] = b; p[2 * ENTRY_WORD] = c; p[3 * ENTRY_WORD] = d;
+}
+
 // A world's solve in LDS: what it works on (set by one thread), and the shared
 // words of planning.
 struct ChainShared {
@@ -294,10 +311,10 @@ __device__ __forceinline__ void plan_put(PLAN& P, const Round& R, uint32_t at)
 
 // The program of a world run by one wave, planned by one wave without
 // barriers; `ready` items are in the ring.  Returns the rows (0: the ordering
-// data was corrupt).
+// data was corrupt) and the entries.
 template <class PLAN>
 __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint32_t nit, uint32_t nj, uint32_t iters,
-                                                uint32_t ready)
+                                                uint32_t ready, uint32_t& entries)
 {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
@@ -319,6 +336,7 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
         entry += R.lanes;
         row += 1u;
     }
+    entries = entry;
     return done == total ? row : 0u;
 }
 
@@ -375,13 +393,17 @@ __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32
     return sh.taken == limit ? slot : 0u;
 }
 
-// Waves that run a world's rows: one while the items fill about as many rows
-// of 64 as a pile's chain is deep (90-150 for 4 iterations), more for larger
-// worlds, whose slots then cost a barrier each.
-constexpr uint32_t CHAIN_WAVE_ROWS = 96;
-__host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, uint32_t most)
+// Waves that run a world's rows: one for each `rows` rows of 64 its items fill
+// (a pile's chain is 90-150 slots deep for 4 iterations).  In the one-kernel
+// step a slot of several waves costs about two rows of one, so they pay from
+// 96 rows on (97 worlds x 8 steps: 3.40 ms, with 48 4.45 ms).  In the separate
+// launches, records in program order, wider is better down to a wave for 32
+// rows (solve of a 4,096-body pile, 96 / 48 / 24 rows: 529 / 499 / 498 us;
+// coloured 417 / 311 / 308).
+constexpr uint32_t FUSED_WAVE_ROWS = 96, CHAIN_WAVE_ROWS = 32;
+__host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, uint32_t most, uint32_t rows)
 {
-    const uint32_t w = (uint32_t)(((uint64_t)nit * iters / 64u + CHAIN_WAVE_ROWS - 1u) / CHAIN_WAVE_ROWS);
+    const uint32_t w = (uint32_t)(((uint64_t)nit * iters / 64u + rows - 1u) / rows);
     return w < 1u ? 1u : (w < most ? w : most);
 }
 
@@ -544,7 +566,8 @@ __device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, cons
 
 // Runs a program: `nslots` slots, `reps` times over.  MULTI: the workgroup's
 // waves run the rows of a slot side by side, a workgroup barrier after each
-// slot (every wave of the workgroup calls it).
+// slot (every wave of the workgroup calls it).  DIRECT: recs are in program
+// order (entry_at), joint j's the entry jbase + j; otherwise by point.
 //
 // A row is reached through loads that each need the one before (slot, row,
 // entry, record), all in L2: every stage runs two slots ahead of the stage
@@ -564,18 +587,18 @@ struct InLds<LdsMomenta> {
     static constexpr bool value = true;
 };
 
-template <bool MULTI, bool WARM, class ST, class ACC>
+template <bool MULTI, bool WARM, bool DIRECT, class ST, class ACC>
 __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, const ST& st, ACC acc,
-                                          uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
+                                          uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
 {
     constexpr bool LDS_ONLY = InLds<ST>::value && InLds<ACC>::value;
     rows = uniform_ptr(rows); entries = uniform_ptr(entries); slots = uniform_ptr(slots); recs = uniform_ptr(recs);
-    nslots = uniform(nslots); reps = uniform(reps); nj = uniform(nj);
+    nslots = uniform(nslots); reps = uniform(reps); nj = uniform(nj); jbase = uniform(jbase);
     const uint32_t lane = threadIdx.x & 63u, wave = MULTI ? uniform(threadIdx.x >> 6) : 0u;
     const uint32_t end = nslots - 1u;
     for (uint32_t rep = 0; rep < reps; ++rep) {
         u2v sl[3], row[3];
-        uint32_t ent[3], point[3], cnt_e[3], cnt[3];
+        uint32_t ent[3], at[3], point[3], cnt_e[3], cnt[3];
         bool mine[3];
         u4v rec[3][4];
         // each stage loads for slot s (a slot past the end repeats the last)
@@ -595,13 +618,19 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
         };
         auto load_entry = [&](int k) {
             const uint32_t c = uniform(row[k].y);
-            ent[k] = entries[uniform(row[k].x) + (lane < (c & 0xffu) ? lane : 0u)];
+            const uint32_t e = uniform(row[k].x) + (lane < (c & 0xffu) ? lane : 0u);
+            ent[k] = entries[e];
+            at[k] = e;
             cnt_e[k] = mine[k] ? c : 0u;
         };
         auto load_rec = [&](int k) {
-            const GCU4 q = recs + (size_t)ent[k] * 4u;
-            rec[k][0] = q[0]; rec[k][1] = q[1]; rec[k][2] = q[2]; rec[k][3] = q[3];
+            const GCU4 q = recs + (DIRECT ? entry_at(ent[k] < nj ? jbase + ent[k] : at[k]) : (size_t)ent[k] * 4u);
+            constexpr uint32_t W = DIRECT ? ENTRY_WORD : 1u;
+            rec[k][0] = q[0]; rec[k][1] = q[W]; rec[k][2] = q[2 * W]; rec[k][3] = q[3 * W];
+            // a register of its own: shared with ent it would be moved, and so
+            // waited for, in the slot that loads the next entry
             point[k] = ent[k];
+            asm("" : "+v"(point[k]));
             cnt[k] = cnt_e[k];
         };
         // the first loads of every stage, as the loop's iterations -8 .. -1 would issue them
@@ -611,78 +640,84 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
             if (p >= 4) load_entry((p - 4) % 3);
             if (p >= 2) load_row((uint32_t)(p - 2), (p - 2) % 3);
             load_slot((uint32_t)p, p % 3);
+            __builtin_amdgcn_sched_barrier(0);   // in the loop's order: its waits count from either
         }
-        for (uint32_t s0 = 0; s0 < nslots; s0 += 3u) {
-#pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const uint32_t s = s0 + u;
-                if (s >= nslots) break;
-                // this row's LDS reads first: the fetches below are issued
-                // while they are under way (lanes without an entry and joints
-                // read something harmless)
-                const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
-                const uint32_t rc = cnt[u], pt = point[u];
-                const uint32_t ai = (uint32_t)max((int32_t)(pt - nj), 0);
-                const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
-                const f2v old = acc[ai];
-                __builtin_amdgcn_sched_barrier(0);
-                load_rec((u + 2) % 3);
-                load_entry((u + 4) % 3);
-                load_row(s + 6u, u);
-                load_slot(s + 8u, (u + 8) % 3);
-                __builtin_amdgcn_sched_barrier(0);
-                bool act = lane < (rc & 0xffu);
-                if (rc & ROW_JOINTS) {
-                    const bool joint = (q0.x & PR_JOINT) != 0u;
-                    if (act && joint) chain_joint(q0, q1, q2, q3, st, dt);
-                    act = act && !joint;
-                }
-                if (act)
-                    chain_contact<WARM>(q0, q1, q2, q3, st, s1, s2, old, acc + ai, lane, (rc >> 7) & 0x1feu, fix);
-                // the next slot reads what this one wrote
-                if constexpr (MULTI) {
-                    if constexpr (LDS_ONLY) {
-                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-                        __builtin_amdgcn_s_barrier();
-                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-                    } else {
-                        __syncthreads();
-                    }
-                } else if constexpr (LDS_ONLY) {
-                    asm volatile("" ::: "memory");   // one wave's LDS operations are served in order
-                } else {
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-                }
+        auto run_slot = [&](uint32_t s, int u) __attribute__((always_inline)) {
+            // this row's LDS reads first: the fetches below are issued while
+            // they are under way (lanes without an entry and joints read
+            // something harmless)
+            const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
+            const uint32_t rc = cnt[u], pt = point[u];
+            const uint32_t ai = (uint32_t)max((int32_t)(pt - nj), 0);
+            const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
+            const f2v old = acc[ai];
+            __builtin_amdgcn_sched_barrier(0);
+            load_rec((u + 2) % 3);
+            load_entry((u + 4) % 3);
+            load_row(s + 6u, u);
+            load_slot(s + 8u, (u + 8) % 3);
+            __builtin_amdgcn_sched_barrier(0);
+            bool act = lane < (rc & 0xffu);
+            if (rc & ROW_JOINTS) {
+                const bool joint = (q0.x & PR_JOINT) != 0u;
+                if (act && joint) chain_joint(q0, q1, q2, q3, st, dt);
+                act = act && !joint;
             }
+            if (act) chain_contact<WARM>(q0, q1, q2, q3, st, s1, s2, old, acc + ai, lane, (rc >> 7) & 0x1feu, fix);
+            // the next slot reads what this one wrote
+            if constexpr (MULTI) {
+                if constexpr (LDS_ONLY) {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                } else {
+                    __syncthreads();
+                }
+            } else if constexpr (LDS_ONLY) {
+                asm volatile("" ::: "memory");   // one wave's LDS operations are served in order
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+            }
+        };
+        // whole rounds of the three buffers, then what is left: a way out of
+        // the middle of the loop would make its waits those of the shortest
+        // path round it (a row's fetches waited for one slot after their issue)
+        uint32_t s = 0;
+        for (; s + 3u <= nslots; s += 3u) {
+            run_slot(s, 0);
+            run_slot(s + 1u, 1);
+            run_slot(s + 2u, 2);
         }
+        if (s < nslots) run_slot(s, 0);
+        if (s + 1u < nslots) run_slot(s + 1u, 1);
     }
 }
 
 // The chain on LDS momenta as an out-of-line call: its registers are then its
 // own, whatever the step kernel holds around it.  `accg`: the accumulated
 // impulses when they do not fit LDS (acc null).
-template <bool MULTI, bool WARM>
+template <bool MULTI, bool WARM, bool DIRECT>
 __device__ __attribute__((noinline)) void chain_lds(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
-                                                    LF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
+                                                    LF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
 {
-    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_lds(acc), nslots,
-                           reps, nj, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_lds(acc), nslots,
+                           reps, nj, jbase, uniform(fix) != 0u, dt);
 }
-template <bool MULTI, bool WARM>
+template <bool MULTI, bool WARM, bool DIRECT>
 __device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
-                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
+                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
 {
-    chain_run<MULTI, WARM>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), nslots,
-                           reps, nj, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), nslots,
+                           reps, nj, jbase, uniform(fix) != 0u, dt);
 }
 
 // momenta and impulses in global memory
-template <bool MULTI, bool WARM>
+template <bool MULTI, bool WARM, bool DIRECT>
 __device__ __attribute__((noinline)) void chain_glb(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, GF3 m, uint32_t none,
-                                                    GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, bool fix, float dt)
+                                                    GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
 {
-    chain_run<MULTI, WARM>(rows, entries, slots, recs, GlbMomenta{uniform_ptr(m), uniform(none)}, uniform_ptr(acc), nslots,
-                           reps, nj, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, GlbMomenta{uniform_ptr(m), uniform(none)}, uniform_ptr(acc), nslots,
+                           reps, nj, jbase, uniform(fix) != 0u, dt);
 }
 
 }  // namespace r2d

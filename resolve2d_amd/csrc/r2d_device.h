@@ -109,6 +109,7 @@ struct WorldChain {
     uint32_t pairs;     // manifolds of two points
     uint32_t flags;     // 1: updateTGSDepth is live; 2: some static body is an ordering body
     uint32_t slots;     // of its program
+    uint32_t entries;   // of its program
 };
 
 struct StepDev {
@@ -160,6 +161,7 @@ struct StepDev {
     uint2* prog_rows;                      // [chain_iters * cap_i]
     uint32_t* prog_entries;                // [2 * chain_iters * cap_i]
     uint2* prog_slots;                     // [chain_iters * cap_i]
+    uint4* prog_recs;                      // [8 * chain_iters * cap_i + 32 W] separate launches: records in program order
     uint4* plan_items;                     // [2 * cap_i]
     uint4* plan_ring;                      // [2 * cap_i]
     // the solve in separate launches

@@ -1790,7 +1790,7 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n);
     const ChainBodies& C = L.C;
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
-    const uint32_t waves = chain_waves(nit, kc, (uint32_t)T / 64u);
+    const uint32_t waves = chain_waves(nit, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS);
     const bool chain = nit > 0u && sh.iters > 0u;
     const bool plan_in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words;
     Program G;
@@ -1847,7 +1847,9 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
                          : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
         build(t, T);
     } else if (t < 64u) {
-        if (chain) ns = plan_in_lds ? plan_single(PL, G, nit, nj, kc, ready) : plan_single(PG, G, nit, nj, kc, ready);
+        uint32_t entries;
+        if (chain)
+            ns = plan_in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
     } else {
         build(t - 64u, T - 64u);
     }
@@ -2005,12 +2007,12 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         const uint32_t nslots = uniform(sh.nslots), reps = iters / kc;
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = uniform(sh.fix) != 0u;
-        if (chain_waves(nj + M, kc, (uint32_t)T / 64u) > 1u) {
-            if (in_lds) chain_lds<true, WARM>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, fix, sub_dt);
-            else chain_lds_accg<true, WARM>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, fix, sub_dt);
+        if (chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u) {
+            if (in_lds) chain_lds<true, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, 0u, fix, sub_dt);
+            else chain_lds_accg<true, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, 0u, fix, sub_dt);
         } else if (threadIdx.x < 64u) {
-            if (in_lds) chain_lds<false, WARM>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, fix, sub_dt);
-            else chain_lds_accg<false, WARM>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, fix, sub_dt);
+            if (in_lds) chain_lds<false, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, 0u, fix, sub_dt);
+            else chain_lds_accg<false, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, 0u, fix, sub_dt);
         }
         __syncthreads();
     }
@@ -2036,6 +2038,13 @@ __device__ __forceinline__ GlobalPoses global_poses(const WorldDev& D)
 __device__ __forceinline__ GF3 world_momenta(const StepDev& S, const WorldDev& D, uint32_t w)
 {
     return (GF3)(S.g_mom + D.body_base + w);
+}
+
+// a world's records in program order: entries, then joints, in blocks of four, each last one
+// perhaps not full (up to 3 + 3 places beyond 2 kc an item)
+__device__ __forceinline__ GU4 world_records(const StepDev& S, uint32_t w, uint32_t ibase)
+{
+    return (GU4)(S.prog_recs + (size_t)ibase * 8u * S.chain_iters + (size_t)w * 32u);
 }
 
 // the planning state of item j of a world, and where its second point is
@@ -2097,7 +2106,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     const uint32_t w = S.w_order[blockIdx.x];
     const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, nj = (uint32_t)S.worlds[w].njoints;
     if (S.w_status[w] != 0 || nit == 0u) return;
-    const uint32_t t = threadIdx.x, kc = S.chain_iters, waves = chain_waves(nit, kc, (uint32_t)T / 64u);
+    const uint32_t t = threadIdx.x, kc = S.chain_iters, waves = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
     const bool in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= lds_words;
     if (t == 0) {
         sh.ready = sh.taken = sh.entries = 0u;
@@ -2124,20 +2133,22 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     if (in_lds) start(PL, true); else start(PG, false);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
-    uint32_t ns = 0u;
+    uint32_t ns = 0u, entries = 0u;
     if (waves > 1u)
         ns = in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh) : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
     else if (t < 64u)
-        ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready) : plan_single(PG, G, nit, nj, kc, ready);
+        ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
     if (t == 0) {
         S.w_chain[w].slots = ns;
+        S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
 }
 
 // The gap before sub-step s's chain (s == sub_steps: after the last one):
-// bodies, and after the last one the impulses into the step's manifold arrays
-// (what r2d_get_manifolds reports)
+// bodies; before the first one the points' records into program order, after
+// the last one the impulses into the step's manifold arrays (what
+// r2d_get_manifolds reports)
 template <bool WARM>
 __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uint32_t sub_steps, float sub_dt)
 {
@@ -2165,6 +2176,21 @@ __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uin
         const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
         if (touched) *mom = m;
         else { D.mx[i] = m.x; D.my[i] = m.y; D.L[i] = m.z; }
+    }
+    if (s == 0u) {
+        // each world's entries over gridDim / worlds workgroups
+        const uint32_t parts = gridDim.x > S.nworlds ? gridDim.x / S.nworlds : 1u, kc = S.chain_iters;
+        for (uint32_t b = blockIdx.x; b < parts * S.nworlds; b += gridDim.x) {
+            const uint32_t w = b % S.nworlds, ibase = S.w_item_base[w], nj = (uint32_t)S.worlds[w].njoints;
+            if (S.w_status[w] != 0 || S.w_item_base[w + 1] == ibase) continue;
+            const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+            const GU4 to = world_records(S, w, ibase);
+            const uint32_t n = S.w_chain[w].entries;
+            for (uint32_t e = (b / S.nworlds) * blockDim.x + threadIdx.x; e < n; e += parts * blockDim.x) {
+                const uint32_t p = entries[e];
+                if (p >= nj) entry_copy(to, e, (GCU4)(S.recs + (size_t)ibase * 8), p);
+            }
+        }
     }
     if (s != sub_steps) return;
     const size_t cm = S.cap_m;
@@ -2216,9 +2242,17 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         }
     else if (a_lds)
         for (uint32_t q = t; q < nacc; q += T) acc[q] = accg[q];
+    const uint32_t kc = S.chain_iters;
+    const GU4 prog = world_records(S, w, ibase);
+    const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+    const uint32_t jbase = (W.entries + 3u) & ~3u;   // 2 kc nit places hold the entries and a record a joint
     const GlobalPoses C = global_poses(D);
-    for (uint32_t j = t; j < nj; j += T)
-        joint_record(recs + (size_t)j * 4u, D.joints[j], D, C, s == 0u, [&](uint32_t x) { return S.cmap[base + x]; });
+    for (uint32_t j = t; j < nj && iters > 0u; j += T) {
+        u4v q[4];
+        joint_record(q, D.joints[j], D, C, s == 0u, [&](uint32_t x) { return S.cmap[base + x]; });
+        const GU4 to = prog + entry_at(jbase + j);
+        for (int p = 0; p < 4; ++p) to[p * ENTRY_WORD] = q[p];
+    }
     __syncthreads();
     if (W.flags & 1u) {
         for (uint32_t q = t; q < M; q += T) {
@@ -2227,6 +2261,11 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
                 const uint32_t at = p ? p1 - nj : q;
                 if (a_lds) acc[at] = f2v{0.f, 0.f}; else accg[at] = f2v{0.f, 0.f};
             });
+        }
+        __syncthreads();
+        for (uint32_t e = t; e < W.entries && iters > 0u; e += T) {
+            const uint32_t p = entries[e];
+            if (p >= nj) entry_copy(prog, e, (GCU4)(S.recs + (size_t)ibase * 8), p);
         }
     }
     if constexpr (WARM) {
@@ -2247,19 +2286,18 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     }
     __syncthreads();
     if (iters > 0u) {
-        const uint32_t kc = S.chain_iters, reps = iters / kc, ns = W.slots;
+        const uint32_t reps = iters / kc, ns = W.slots;
         const GCU2 rows = (GCU2)(S.prog_rows + (size_t)ibase * kc), slots = (GCU2)(S.prog_slots + (size_t)ibase * kc);
-        const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
-        const GCU4 rec = (GCU4)(S.recs + (size_t)ibase * 8);
+        const GCU4 rec = (GCU4)prog;
         const bool fix = (W.flags & 2u) != 0u;
-        if (chain_waves(nit, kc, (uint32_t)T / 64u) > 1u) {
-            if (a_lds) chain_lds<true, WARM>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<true, WARM>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, fix, sub_dt);
-            else chain_glb<true, WARM>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, fix, sub_dt);
+        if (chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
+            if (a_lds) chain_lds<true, WARM, true>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, jbase, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<true, WARM, true>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
+            else chain_glb<true, WARM, true>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
         } else if (t < 64u) {
-            if (a_lds) chain_lds<false, WARM>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<false, WARM>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, fix, sub_dt);
-            else chain_glb<false, WARM>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, fix, sub_dt);
+            if (a_lds) chain_lds<false, WARM, true>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, jbase, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<false, WARM, true>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
+            else chain_glb<false, WARM, true>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
         }
         __syncthreads();
     }
@@ -2831,8 +2869,9 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             }
         }
         for (uint32_t s = 0; sub_steps > 0; ++s) {
-            hipLaunchKernelGGL(pick(k_chain_bodies<true>, k_chain_bodies<false>), dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S, s,
-                               sub_steps, sub_dt);
+            // (the first one also copies records, about four a body)
+            hipLaunchKernelGGL(pick(k_chain_bodies<true>, k_chain_bodies<false>), dim3(blocks_for(s ? S.nb : 4ull * S.nb, BS)),
+                               dim3(BS), 0, st, S, s, sub_steps, sub_dt);
             tmark(ss, "k_chain_bodies", st);
             if (s == sub_steps) break;
             auto run = sp.wide ? pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>)
