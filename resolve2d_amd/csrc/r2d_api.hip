@@ -87,7 +87,7 @@ constexpr uint32_t ST_I = ST_M + ST_J;
 // Returns the bytes used; a null base only measures.
 size_t static_layout(char* base, StepDev* S, WorldDev** desc)
 {
-    const size_t N = ST_N, B = ST_B, E = ST_E, R = ST_R, M = ST_M, I = ST_I, W = 1;
+    const size_t N = ST_N, B = ST_B, E = ST_E, R = ST_R, M = ST_M, I = ST_I + 1, W = 1;
     size_t o = 0;
     auto take = [&](auto** p, size_t bytes) {
         using T = std::remove_reference_t<decltype(*p)>;
@@ -660,7 +660,7 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.it_color, I * 4);
     add((void**)&S.recs, I * 128);
     const size_t K = c->cap_k;
-    add((void**)&S.prog_rows, K * I * 8); add((void**)&S.prog_entries, 2 * K * I * 4); add((void**)&S.prog_slots, K * I * 8);
+    add((void**)&S.prog_rows, K * I * 8); add((void**)&S.prog_entries, (2 * K * I + 8 * W) * 4); add((void**)&S.prog_slots, K * I * 8);
     add((void**)&S.prog_recs, 2 * K * I * 64 + W * 512);
     add((void**)&S.plan_items, 2 * I * 16); add((void**)&S.plan_ring, 2 * I * 16);
     add((void**)&S.cmask, 2 * N * 8);
@@ -890,7 +890,7 @@ void fused_used(const r2d_ctx* c, uint64_t end[4])
         end[0] = std::max<uint64_t>(end[0], (uint64_t)x.e0 + x.ecap + 1);
         end[1] = std::max<uint64_t>(end[1], (uint64_t)x.r0 + x.rcap + 1);
         end[2] = std::max<uint64_t>(end[2], (uint64_t)x.m0 + x.mcap);
-        end[3] = std::max<uint64_t>(end[3], (uint64_t)x.i0 + x.icap);
+        end[3] = std::max<uint64_t>(end[3], (uint64_t)x.i0 + x.icap + 1);
     }
 }
 
@@ -926,7 +926,7 @@ int fused_layout(r2d_ctx* c, Batch& b)
         fused_caps(b.worlds[i], cap);
         c->fscr[i] = WorldScratch{(uint32_t)te, cap[0], (uint32_t)tr, cap[1], (uint32_t)tm, cap[2], (uint32_t)ti,
                                   cap[3]};
-        te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += cap[3];
+        te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
     }
     // as much again free for worlds that outgrow their slices during the call
     if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, chain_iters(b.iters), false))) return rc;
@@ -966,7 +966,7 @@ int fused_regrow(r2d_ctx* c, Batch& b)
         for (int k = 0; k < 4; ++k) w->fz[k] = cap[k];
         c->fscr[i] = WorldScratch{(uint32_t)te, cap[0], (uint32_t)tr, cap[1], (uint32_t)tm, cap[2], (uint32_t)ti,
                                   cap[3]};
-        te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += cap[3];
+        te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
         c->hstatus[i] = WS_OK;
     }
     int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, chain_iters(b.iters), true);
@@ -2088,7 +2088,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     const WorldScratch x{0u, ST_E, 0u, ST_R, 0u, ST_M, 0u, ST_I};
     // free ends at the capacities: a world that outgrows a slice stops
     // before its step (WS_OVERFLOW) instead of taking more
-    const uint32_t pool[8] = {ST_E + 1, ST_R + 1, ST_M, ST_I, ST_E + 1, ST_R + 1, ST_M, ST_I};
+    const uint32_t pool[8] = {ST_E + 1, ST_R + 1, ST_M, ST_I + 1, ST_E + 1, ST_R + 1, ST_M, ST_I + 1};
     const uint32_t order = 0u;
     HIPCHK(hipMemcpyAsync(ddesc, &d, sizeof d, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(F.wscr, &x, sizeof x, hipMemcpyHostToDevice, st));

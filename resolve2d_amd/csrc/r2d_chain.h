@@ -67,6 +67,9 @@ enum : uint32_t {
     PR_TYPE_SHIFT = 28        // word 1, joints: type
 };
 
+// the record of a lane without a point: bias -1, no body to write
+__device__ __forceinline__ u4v idle_word(int word) { return word == 1 ? u4v{0u, 0xbf800000u, 0u, 0u} : u4v{0u, 0u, 0u, 0u}; }
+
 __device__ __forceinline__ float asf(uint32_t x) { return __uint_as_float(x); }
 __device__ __forceinline__ uint32_t asu(float x) { return __float_as_uint(x); }
 
@@ -189,8 +192,8 @@ struct PlanGlb {
     }
 };
 
-// A world's program: rows (first entry; entries | pairs << 8 | ROW_JOINTS when
-// one is a joint), the entries (point indices: item j's first point is j,
+// A world's program: rows (first entry; entries | lanes of pairs << 8 |
+// ROW_JOINTS when one is a joint), the entries (point indices: item j's first point is j,
 // second points follow after the items; pairs first),
 // and for worlds run by several waves the first row and the rows of each slot
 // (rows of one slot run side by side, one per wave).
@@ -274,7 +277,7 @@ __device__ __forceinline__ Round plan_take(PLAN& P, uint32_t first, uint32_t ava
     R.taken = (uint32_t)__popcll(tm);
     R.pairs = (uint32_t)__popcll(tm & __ballot(pair));
     R.lanes = R.taken + R.pairs;
-    R.word = R.lanes | (R.pairs << 8) | (__ballot(R.take && R.self.item < nj) ? ROW_JOINTS : 0u);
+    R.word = R.lanes | (R.pairs << 9) | (__ballot(R.take && R.self.item < nj) ? ROW_JOINTS : 0u);
     R.left = act && !R.take;
     return R;
 }
@@ -515,20 +518,29 @@ __device__ __forceinline__ void chain_joint(const u4v& q0, const u4v& q1, const 
 // second's from its neighbour and writes the bodies.  `paired` lanes, from
 // lane 0 on, hold pairs.  A separated point's impulses are zero already (its
 // depth is the step's, or was reset with it), so it need only change nothing.
-// fix: some static body is an ordering body.
 //
-// A row is bound by its instructions (one wave issues about one every five
-// cycles: 115 vector and 35 scalar ones took 1,090 cycles), so nothing here
-// branches but on what the whole row shares: a write that is not to be kept
-// goes to a spare place instead of being masked.  s1, s2, old: the bodies'
-// momenta and the point's impulses, read ahead.
+// A row is bound by its instructions (a wave issues about one every five
+// cycles), so nothing here branches but on what the whole row shares: a write
+// that is not to be kept goes to a spare place, a lane without a point has a
+// point that does nothing (bias -1, no body to write, a spare impulse).
+// fl_a, fl_b: words 0 and 1 for their flags; s1, s2, old: the bodies' momenta
+// and the point's impulses, read ahead.
+//
+// The reference sums an impulse up from +0 and adds the sum to the bodies; it
+// does so too where a point does nothing, and to a static body that is an
+// ordering body it adds +0.  `fix` does that to the letter.  Without it the
+// impulses are added to each other and then to the momenta, with zeros where
+// a point does nothing: the same bits as long as no momentum is -0 (which no
+// item makes of others), all normals and arms are finite and no ordering body
+// is static, which is what the caller asks for.
 template <bool WARM, class ST, class ACC>
-__device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, const ST& st,
-                                              f3v s1, f3v s2, f2v old, ACC acc, uint32_t lane, uint32_t paired, bool fix)
+__device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, const u4v& q2, const u4v& q3, uint32_t fl_a,
+                                              uint32_t fl_b, float bias, const ST& st, f3v s1, f3v s2, f2v old, ACC acc,
+                                              uint32_t lane, uint32_t paired, bool fix)
 {
     const uint32_t a = q0.x & PR_INDEX, b = q0.y & PR_INDEX;
     const v2 n = mk(asf(q0.z), asf(q0.w)), t = rot90cw(n);
-    const float fric = asf(q1.x), bias = asf(q1.y);
+    const float fric = asf(q1.x);
     const v2 r1 = mk(asf(q1.z), asf(q1.w)), r2 = mk(asf(q2.x), asf(q2.y));
     const float om1 = s1.z * asf(q3.z), om2 = s2.z * asf(q3.w);
     const v2 v1 = add2(scale2(mk(s1.x, s1.y), asf(q3.x)), mk(-r1.y * om1, r1.x * om1));
@@ -536,44 +548,71 @@ __device__ __forceinline__ void chain_contact(const u4v& q0, const u4v& q1, cons
     const v2 dv = sub2(v1, v2v);
     const float pn = (dot2(dv, n) + bias) * asf(q2.z);
     const float pt = dot2(dv, t) * asf(q2.w);
-    const bool go = !(bias < 0.f) && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (q0.y & PR_WARM) != 0u));
+    const bool go = !(bias < 0.f) && (!(pn < MIN_MANIFOLD_IMPULSE) || (WARM && (fl_b & PR_WARM) != 0u));
     const float new_pn = maxn(0.0f, old.x + pn);
     const float max_pt = fric * absf(new_pn);
-    const float new_pt = clampn(old.y + pt, -max_pt, max_pt);
-    const float apn = new_pn - old.x, apt = new_pt - old.y;
+    // clampn(old.y + pt, -max_pt, max_pt): a NaN of one side leaves the other
+    // (fminf, and a comparison that NaN passes), -0 wins over +0 below
+    const float up_pt = __builtin_fminf(old.y + pt, max_pt);
+    const float new_pt = !(up_pt <= -max_pt) ? up_pt : -max_pt;
+    float apn = new_pn - old.x, apt = new_pt - old.y;
     *acc = f2v{go ? new_pn : old.x, go ? new_pt : old.y};
-    v2 dp = add2(scale2(n, apn), scale2(t, apt));
-    float c1 = cross2(r1, dp), c2 = cross2(r2, dp);
-    // a point that does nothing adds +0, which changes none of the sums below
-    // (0 - x and 0 + x are never -0)
-    dp.x = go ? dp.x : 0.f; dp.y = go ? dp.y : 0.f;
-    c1 = go ? c1 : 0.f; c2 = go ? c2 : 0.f;
-    f3v d1{0.f - dp.x, 0.f - dp.y, 0.f - c1}, d2{0.f + dp.x, 0.f + dp.y, 0.f + c2};
-    if (paired) {
+    f3v m1, m2;
+    if (__builtin_expect(!fix, 1)) {
+        apn = go ? apn : 0.f;
+        apt = go ? apt : 0.f;
+        v2 dp = add2(scale2(n, apn), scale2(t, apt));
+        float c1 = cross2(r1, dp), c2 = cross2(r2, dp);
+        if (lane < paired) {
+            dp.x = dp.x + pair_other(dp.x);
+            dp.y = dp.y + pair_other(dp.y);
+            c1 = c1 + pair_other(c1);
+            c2 = c2 + pair_other(c2);
+        }
+        m1 = f3v{s1.x - dp.x, s1.y - dp.y, s1.z - c1};
+        m2 = f3v{s2.x + dp.x, s2.y + dp.y, s2.z + c2};
+    } else {
+        v2 dp = add2(scale2(n, apn), scale2(t, apt));
+        float c1 = cross2(r1, dp), c2 = cross2(r2, dp);
+        dp.x = go ? dp.x : 0.f; dp.y = go ? dp.y : 0.f;
+        c1 = go ? c1 : 0.f; c2 = go ? c2 : 0.f;
+        f3v d1{0.f - dp.x, 0.f - dp.y, 0.f - c1}, d2{0.f + dp.x, 0.f + dp.y, 0.f + c2};
         if (lane < paired) {
             const float ox = pair_other(dp.x), oy = pair_other(dp.y), o1 = pair_other(c1), o2 = pair_other(c2);
             d1 = f3v{d1.x - ox, d1.y - oy, d1.z - o1};
             d2 = f3v{d2.x + ox, d2.y + oy, d2.z + o2};
         }
+        if (fl_a & PR_STATIC) d1 = f3v{0.f, 0.f, 0.f};
+        if (fl_b & PR_STATIC) d2 = f3v{0.f, 0.f, 0.f};
+        m1 = f3v{s1.x + d1.x, s1.y + d1.y, s1.z + d1.z};
+        m2 = f3v{s2.x + d2.x, s2.y + d2.y, s2.z + d2.z};
     }
-    if (fix) {
-        if (q0.x & PR_STATIC) d1 = f3v{0.f, 0.f, 0.f};
-        if (q0.y & PR_STATIC) d2 = f3v{0.f, 0.f, 0.f};
-    }
-    st.put_if((int32_t)q0.x < 0, a, f3v{s1.x + d1.x, s1.y + d1.y, s1.z + d1.z});
-    st.put_if((int32_t)q0.y < 0, b, f3v{s2.x + d2.x, s2.y + d2.y, s2.z + d2.z});
+    st.put_if((int32_t)fl_a < 0, a, m1);
+    st.put_if((int32_t)fl_b < 0, b, m2);
 }
 
-// Runs a program: `nslots` slots, `reps` times over.  MULTI: the workgroup's
-// waves run the rows of a slot side by side, a workgroup barrier after each
-// slot (every wave of the workgroup calls it).  DIRECT: recs are in program
-// order (entry_at), joint j's the entry jbase + j; otherwise by point.
+// what the chain reads in global memory, and its sizes: points are those of
+// index nj + nacc, the one that does nothing, and below; `idle` is its place
+// among the entries; DIRECT programs have joint j's record at entry jbase + j
+struct ChainProgram {
+    GCU2 rows;
+    GCU32 entries;
+    GCU2 slots;
+    GCU4 recs;
+    uint32_t nslots, reps, nj, nacc, idle, jbase;
+};
+
+// Runs a program `reps` times over.  MULTI: the workgroup's waves run the rows
+// of a slot side by side, a workgroup barrier after each slot (every wave of
+// the workgroup calls it).  DIRECT: recs are in program order (entry_at),
+// otherwise by point.
 //
-// A row is reached through loads that each need the one before (slot, row,
-// entry, record), all in L2: every stage runs two slots ahead of the stage
-// that uses it, so that a load has two slots' time to arrive.  Three buffers
-// a stage, the loop unrolled by three: a buffer is never copied while its
-// load is in flight.
+// A row is reached through loads that each need the one before (row, entry,
+// record), all in L2.  The rows of 63 slots are read at once, one a lane, a
+// batch ahead; entries and records run two slots ahead of the stage that uses
+// them, so that a load has two slots' time to arrive.  Three buffers a stage,
+// the loop unrolled by three: a buffer is never copied while its load is in
+// flight.
 template <class T>
 struct InLds {
     static constexpr bool value = false;
@@ -588,82 +627,95 @@ struct InLds<LdsMomenta> {
 };
 
 template <bool MULTI, bool WARM, bool DIRECT, class ST, class ACC>
-__device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, const ST& st, ACC acc,
-                                          uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
+__device__ __forceinline__ void chain_run(ChainProgram G, const ST& st, ACC acc, bool fix, float dt)
 {
     constexpr bool LDS_ONLY = InLds<ST>::value && InLds<ACC>::value;
-    rows = uniform_ptr(rows); entries = uniform_ptr(entries); slots = uniform_ptr(slots); recs = uniform_ptr(recs);
-    nslots = uniform(nslots); reps = uniform(reps); nj = uniform(nj); jbase = uniform(jbase);
+    constexpr uint32_t BATCH = 63, AHEAD = 4;   // slots a batch; slots the entry stage runs ahead
+    const GCU2 rows = uniform_ptr(G.rows), slots = uniform_ptr(G.slots);
+    const GCU32 entries = uniform_ptr(G.entries);
+    const GCU4 recs = uniform_ptr(G.recs);
+    const uint32_t nslots = uniform(G.nslots), reps = uniform(G.reps), nj = uniform(G.nj), nacc = uniform(G.nacc),
+                   idle = uniform(G.idle), jbase = uniform(G.jbase);
     const uint32_t lane = threadIdx.x & 63u, wave = MULTI ? uniform(threadIdx.x >> 6) : 0u;
     const uint32_t end = nslots - 1u;
     for (uint32_t rep = 0; rep < reps; ++rep) {
-        u2v sl[3], row[3];
         uint32_t ent[3], at[3], point[3], cnt_e[3], cnt[3];
-        bool mine[3];
         u4v rec[3][4];
-        // each stage loads for slot s (a slot past the end repeats the last)
-        // into buffer k
-        auto load_slot = [&](uint32_t s, int k) {
-            if constexpr (MULTI) sl[k] = slots[s < end ? s : end];
+        // the rows of slots `first` + lane (past the end: the last again),
+        // and in worlds of several waves, before them, the slots
+        auto batch_slots = [&](uint32_t first) -> u2v {
+            const uint32_t s = first + lane;
+            if constexpr (MULTI) return slots[s < end ? s : end];
+            return u2v{s < end ? s : end, 1u};
         };
-        auto load_row = [&](uint32_t s, int k) {
-            uint32_t r = s < end ? s : end;
-            mine[k] = true;
-            if constexpr (MULTI) {
-                r = uniform(sl[k].x);
-                mine[k] = wave < uniform(sl[k].y);
-                r += mine[k] ? wave : 0u;
-            }
-            row[k] = rows[r];
+        auto batch_rows = [&](u2v sl) -> u2v {
+            const bool mine = wave < sl.y;
+            u2v r = rows[sl.x + (mine ? wave : 0u)];
+            if constexpr (MULTI) r.y = mine ? r.y : 0u;
+            return r;
         };
-        auto load_entry = [&](int k) {
-            const uint32_t c = uniform(row[k].y);
-            const uint32_t e = uniform(row[k].x) + (lane < (c & 0xffu) ? lane : 0u);
-            ent[k] = entries[e];
+        // each stage loads into buffer k; lanes without a point take the idle one
+        auto load_entry = [&](u2v batch, uint32_t i, int k) {
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)batch.x, (int)i);
+            const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)batch.y, (int)i);
+            const uint32_t e = lane < (c & 0xffu) ? first + lane : idle;
+            ent[k] = *(const R2D_GLB uint32_t*)((const R2D_GLB char*)entries + (size_t)(uint32_t)(e * 4u));
             at[k] = e;
-            cnt_e[k] = mine[k] ? c : 0u;
+            cnt_e[k] = c;
         };
         auto load_rec = [&](int k) {
-            const GCU4 q = recs + (DIRECT ? entry_at(ent[k] < nj ? jbase + ent[k] : at[k]) : (size_t)ent[k] * 4u);
-            constexpr uint32_t W = DIRECT ? ENTRY_WORD : 1u;
-            rec[k][0] = q[0]; rec[k][1] = q[W]; rec[k][2] = q[2 * W]; rec[k][3] = q[3 * W];
+            if constexpr (DIRECT) {
+                const GCU4 q = recs + entry_at(ent[k] < nj ? jbase + ent[k] : at[k]);
+                rec[k][0] = q[0]; rec[k][1] = q[ENTRY_WORD]; rec[k][2] = q[2 * ENTRY_WORD]; rec[k][3] = q[3 * ENTRY_WORD];
+            } else {
+                const GCU4 q = (GCU4)((const R2D_GLB char*)recs + (size_t)(uint32_t)(ent[k] * 64u));
+                rec[k][0] = q[0]; rec[k][1] = q[1]; rec[k][2] = q[2]; rec[k][3] = q[3];
+            }
             // a register of its own: shared with ent it would be moved, and so
             // waited for, in the slot that loads the next entry
             point[k] = ent[k];
             asm("" : "+v"(point[k]));
             cnt[k] = cnt_e[k];
         };
-        // the first loads of every stage, as the loop's iterations -8 .. -1 would issue them
-#pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            if (p >= 6) load_rec(p - 6);
-            if (p >= 4) load_entry((p - 4) % 3);
-            if (p >= 2) load_row((uint32_t)(p - 2), (p - 2) % 3);
-            load_slot((uint32_t)p, p % 3);
-            __builtin_amdgcn_sched_barrier(0);   // in the loop's order: its waits count from either
-        }
-        auto run_slot = [&](uint32_t s, int u) __attribute__((always_inline)) {
+        // the first loads of every stage, as the loop's iterations -4 .. -1
+        // would issue them, in its order: its waits count from either
+        u2v batch = batch_rows(batch_slots(0u));
+        u2v sl = batch_slots(AHEAD + BATCH);
+        u2v next = batch_rows(batch_slots(AHEAD));
+        load_entry(batch, 0u, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_entry(batch, 1u, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load_rec(0);
+        load_entry(batch, 2u, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        load_rec(1);
+        load_entry(batch, 3u, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        auto run_slot = [&](uint32_t i, int u) __attribute__((always_inline)) {
             // this row's LDS reads first: the fetches below are issued while
-            // they are under way (lanes without an entry and joints read
-            // something harmless)
+            // they are under way (joints read something harmless)
             const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
-            const uint32_t rc = cnt[u], pt = point[u];
-            const uint32_t ai = (uint32_t)max((int32_t)(pt - nj), 0);
+            const uint32_t rc = cnt[u], left = point[u] - nj;
+            const uint32_t ai = left < nacc ? left : nacc;   // joints, and lanes without a point: the spare one
             const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
             const f2v old = acc[ai];
             __builtin_amdgcn_sched_barrier(0);
             load_rec((u + 2) % 3);
-            load_entry((u + 4) % 3);
-            load_row(s + 6u, u);
-            load_slot(s + 8u, (u + 8) % 3);
+            load_entry(batch, i, (u + 4) % 3);
             __builtin_amdgcn_sched_barrier(0);
-            bool act = lane < (rc & 0xffu);
+            uint32_t fl_a = q0.x, fl_b = q0.y;
+            float bias = asf(q1.y);
             if (rc & ROW_JOINTS) {
+                asm volatile("");   // one branch for the row: not folded into the lanes' test
                 const bool joint = (q0.x & PR_JOINT) != 0u;
-                if (act && joint) chain_joint(q0, q1, q2, q3, st, dt);
-                act = act && !joint;
+                if (joint) chain_joint(q0, q1, q2, q3, st, dt);
+                // as a point it does nothing
+                fl_a = joint ? 0u : fl_a;
+                fl_b = joint ? 0u : fl_b;
+                bias = joint ? -1.0f : bias;
             }
-            if (act) chain_contact<WARM>(q0, q1, q2, q3, st, s1, s2, old, acc + ai, lane, (rc >> 7) & 0x1feu, fix);
+            chain_contact<WARM>(q0, q1, q2, q3, fl_a, fl_b, bias, st, s1, s2, old, acc + ai, lane, (rc >> 8) & 0xffu, fix);
             // the next slot reads what this one wrote
             if constexpr (MULTI) {
                 if constexpr (LDS_ONLY) {
@@ -679,17 +731,27 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
             }
         };
-        // whole rounds of the three buffers, then what is left: a way out of
-        // the middle of the loop would make its waits those of the shortest
-        // path round it (a row's fetches waited for one slot after their issue)
-        uint32_t s = 0;
-        for (; s + 3u <= nslots; s += 3u) {
-            run_slot(s, 0);
-            run_slot(s + 1u, 1);
-            run_slot(s + 2u, 2);
+        // whole rounds of the three buffers, a batch of them at a time, then
+        // what is left: a way out of the middle of the loop would make its
+        // waits those of the shortest path round it (a row's fetches waited
+        // for one slot after their issue)
+        uint32_t rounds = nslots / 3u, s = 0;
+        while (rounds) {
+            batch = next;
+            next = batch_rows(sl);
+            sl = batch_slots(s + AHEAD + 2u * BATCH);
+            const uint32_t now = rounds < BATCH / 3u ? rounds : BATCH / 3u;
+            for (uint32_t i = 0; i < 3u * now; i += 3u) {
+                run_slot(i, 0);
+                run_slot(i + 1u, 1);
+                run_slot(i + 2u, 2);
+            }
+            rounds -= now;
+            s += 3u * now;
         }
-        if (s < nslots) run_slot(s, 0);
-        if (s + 1u < nslots) run_slot(s + 1u, 1);
+        // (what these fetch is past the end and not used)
+        if (s < nslots) run_slot(0u, 0);
+        if (s + 1u < nslots) run_slot(1u, 1);
     }
 }
 
@@ -697,27 +759,20 @@ __device__ __forceinline__ void chain_run(GCU2 rows, GCU32 entries, GCU2 slots, 
 // own, whatever the step kernel holds around it.  `accg`: the accumulated
 // impulses when they do not fit LDS (acc null).
 template <bool MULTI, bool WARM, bool DIRECT>
-__device__ __attribute__((noinline)) void chain_lds(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
-                                                    LF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
+__device__ __attribute__((noinline)) void chain_lds(ChainProgram G, LF3 m, uint32_t none, LF2 acc, bool fix, float dt)
 {
-    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_lds(acc), nslots,
-                           reps, nj, jbase, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(G, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_lds(acc), uniform(fix) != 0u, dt);
 }
 template <bool MULTI, bool WARM, bool DIRECT>
-__device__ __attribute__((noinline)) void chain_lds_accg(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, LF3 m, uint32_t none,
-                                                         GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
+__device__ __attribute__((noinline)) void chain_lds_accg(ChainProgram G, LF3 m, uint32_t none, GF2 acc, bool fix, float dt)
 {
-    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), nslots,
-                           reps, nj, jbase, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(G, LdsMomenta{uniform_lds(m), uniform(none)}, uniform_ptr(acc), uniform(fix) != 0u, dt);
 }
-
 // momenta and impulses in global memory
 template <bool MULTI, bool WARM, bool DIRECT>
-__device__ __attribute__((noinline)) void chain_glb(GCU2 rows, GCU32 entries, GCU2 slots, GCU4 recs, GF3 m, uint32_t none,
-                                                    GF2 acc, uint32_t nslots, uint32_t reps, uint32_t nj, uint32_t jbase, bool fix, float dt)
+__device__ __attribute__((noinline)) void chain_glb(ChainProgram G, GF3 m, uint32_t none, GF2 acc, bool fix, float dt)
 {
-    chain_run<MULTI, WARM, DIRECT>(rows, entries, slots, recs, GlbMomenta{uniform_ptr(m), uniform(none)}, uniform_ptr(acc), nslots,
-                           reps, nj, jbase, uniform(fix) != 0u, dt);
+    chain_run<MULTI, WARM, DIRECT>(G, GlbMomenta{uniform_ptr(m), uniform(none)}, uniform_ptr(acc), uniform(fix) != 0u, dt);
 }
 
 }  // namespace r2d

@@ -1386,7 +1386,8 @@ __device__ __forceinline__ bool fused_grow(const StepDev& S, uint32_t w, WorldSc
                                            uint32_t& s_slot)
 {
     const uint32_t cap = need + need / 2 + 64;
-    const uint32_t take = k < 2 ? cap + 1 : cap;   // entry and candidate slices end with a scan total
+    const uint32_t take = k != 2 ? cap + 1 : cap;   // entry and candidate slices end with a scan total, item slices with
+                                                    // the chain's idle point
     if (threadIdx.x == 0) {
         // claim [base, base + take) only if it fits: a refused request leaves
         // the free end for smaller ones
@@ -1499,8 +1500,10 @@ __device__ __forceinline__ PointBodies point_bodies(const StepDev& S, const Worl
 // what preStep leaves in the manifold: friction and effective masses.
 // Returns whether updateTGSDepth is live for it: a point whose depth is not
 // within 1e-4 of its original depth, which at the step's start is the same
-// number, so NaN or so deep that 1e-4 vanishes in it (1), and whether one of
-// its bodies is static and an ordering body (2).  place(slot): where the
+// number, so NaN or so deep that 1e-4 vanishes in it (1), and whether the
+// chain needs the reference's sums to the letter (2): one of its bodies is
+// static and an ordering body, or a normal or an arm is not finite.
+// place(slot): where the
 // chain keeps a body's momentum.
 template <bool WARM, class PLACE>
 __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev& D, u4v* recs, uint32_t m, uint32_t base,
@@ -1525,11 +1528,12 @@ __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev
     if (WARM && (valid & MV_WARM)) B.flag_b |= PR_WARM;
     const float fric = sqrt_rn(mua * mub);   // preStep (collision.zig:114)
     S.m_fric[m] = fric;
-    bool live = false;
+    bool live = false, finite = true;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
         const bool on = (valid & (1u << p)) != 0u;
         if (!on && p == 1) continue;
+        if (on) finite = finite && 0.f * n.x + 0.f * n.y + 0.f * r1[p].x + 0.f * r1[p].y + 0.f * r2[p].x + 0.f * r2[p].y == 0.f;
         float mn = 0.f, mt = 0.f;
         if (on) {
             point_masses(B, n, r1[p], r2[p], mn, mt);
@@ -1543,7 +1547,7 @@ __device__ __forceinline__ uint32_t point_build(const StepDev& S, const WorldDev
                     on ? r2[p] : z, mn, mt);
     }
     const uint32_t both = PR_WRITE | PR_STATIC;
-    return (live ? 1u : 0u) | ((B.flag_a & both) == both || (B.flag_b & both) == both ? 2u : 0u);
+    return (live ? 1u : 0u) | ((B.flag_a & both) == both || (B.flag_b & both) == both || !finite ? 2u : 0u);
 }
 
 // updateTGSDepth (collision.zig:73-100) for manifold m where it is live:
@@ -1689,6 +1693,12 @@ __device__ __forceinline__ void body_done(const WorldDev& D, const BodyArrays& A
     }
 }
 
+// a momentum component of -0: the chain then needs the reference's sums to the letter
+__device__ __forceinline__ bool minus_zero(f3v m)
+{
+    return asu(m.x) == 0x80000000u || asu(m.y) == 0x80000000u || asu(m.z) == 0x80000000u;
+}
+
 template <bool WARM>
 __device__ __forceinline__ f3v body_push(const BodyArrays& A, int i, bool last, const BodyState& b, BodyIn in, float sub_dt)
 {
@@ -1758,6 +1768,8 @@ struct ChainLds {
     LU32 rest, dcnt, doff;
     uint32_t n, rest_words, consts;
     LF2 acc;
+    // the impulses of n contact points, and a spare one, beside the constants
+    __device__ __forceinline__ bool holds(uint32_t n) const { return consts + 2u * (n + 1u) <= rest_words; }
     __device__ __forceinline__ ChainLds(LU32 smem, uint32_t free_at, uint32_t free_words, uint32_t n_) : n(n_)
     {
         dcnt = smem;
@@ -1829,6 +1841,9 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     if (plan_in_lds) fill(PL); else fill(PG);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
+    // the point that does nothing, after the others (an item slice has an item to spare)
+    if (t < 4u) recs[(size_t)(nit + uniform(sh.pairs)) * 4u + t] = idle_word((int)t);
+    if (t == 0u) G.entries[2u * kc * nit] = nit + uniform(sh.pairs);
     auto build = [&](uint32_t t0, uint32_t stride) {
         for (uint32_t i = t0; i < n; i += stride) {
             C.m[i] = f3v{D.mx[i], D.my[i], D.L[i]};
@@ -1862,7 +1877,7 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     // accumulated impulses (normal, tangential) of the contact points, by
     // point index less the joints: in LDS after the constants when they fit
     const uint32_t nacc = M + uniform(sh.pairs);
-    if (L.consts + 2u * nacc <= L.rest_words) {
+    if (L.holds(nacc)) {
         for (uint32_t q = t; q < nacc; q += T) L.acc[q] = f2v{0.f, 0.f};
     } else {
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
@@ -1898,8 +1913,13 @@ __device__ __attribute__((noinline)) void chain_bodies(StepArgs KS, LU32 smem, R
             body_move(b, in.mass, in.inertia, sub_dt);
             C.px[i] = b.px; C.py[i] = b.py; C.ang[i] = b.ang;
         }
-        if (s == sub_steps) body_done(D, A, i, stat, b);
-        else C.m[i] = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
+        if (s == sub_steps) {
+            body_done(D, A, i, stat, b);
+        } else {
+            const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
+            C.m[i] = m;
+            if (minus_zero(m)) sh.fix = 1u;
+        }
     }
 }
 
@@ -1917,7 +1937,7 @@ __device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     s = uniform(s);
     for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u, [](uint32_t x) { return x; });
-    const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+    const bool in_lds = L.holds(M + uniform(sh.pairs));
     GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
     if (sh.live)
         for (uint32_t q = t; q < M; q += T) {
@@ -1955,7 +1975,7 @@ __device__ __attribute__((noinline)) void chain_finish(StepArgs KS, LU32 smem, R
     const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M);
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
-    const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
+    const bool in_lds = L.holds(M + uniform(sh.pairs));
     GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
     const size_t cm = S.cap_m;
     for (uint32_t q = threadIdx.x; q < M; q += T) {
@@ -1999,20 +2019,19 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         if (iters == 0u) continue;
         const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters;
         const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
-        const bool in_lds = L.consts + 2u * (M + uniform(sh.pairs)) <= L.rest_words;
-        const GCU2 rows = (GCU2)(S.prog_rows + (size_t)ibase * kc), slots = (GCU2)(S.prog_slots + (size_t)ibase * kc);
-        const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
-        const GCU4 recs = (GCU4)(S.recs + (size_t)ibase * 8);
+        const bool in_lds = L.holds(M + uniform(sh.pairs));
+        const ChainProgram G{(GCU2)(S.prog_rows + (size_t)ibase * kc), (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc),
+                             (GCU2)(S.prog_slots + (size_t)ibase * kc), (GCU4)(S.recs + (size_t)ibase * 8),
+                             uniform(sh.nslots), iters / kc, nj, M + uniform(sh.pairs), 2u * kc * (nj + M), 0u};
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
-        const uint32_t nslots = uniform(sh.nslots), reps = iters / kc;
         const float sub_dt = sh.dt / (float)sub_steps;
-        const bool fix = uniform(sh.fix) != 0u;
+        const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
         if (chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u) {
-            if (in_lds) chain_lds<true, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, 0u, fix, sub_dt);
-            else chain_lds_accg<true, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, 0u, fix, sub_dt);
+            if (in_lds) chain_lds<true, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
+            else chain_lds_accg<true, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
         } else if (threadIdx.x < 64u) {
-            if (in_lds) chain_lds<false, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, L.acc, nslots, reps, nj, 0u, fix, sub_dt);
-            else chain_lds_accg<false, WARM, false>(rows, entries, slots, recs, L.C.m, L.n, accg, nslots, reps, nj, 0u, fix, sub_dt);
+            if (in_lds) chain_lds<false, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
+            else chain_lds_accg<false, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
         }
         __syncthreads();
     }
@@ -2041,11 +2060,18 @@ __device__ __forceinline__ GF3 world_momenta(const StepDev& S, const WorldDev& D
 }
 
 // a world's records in program order: entries, then joints, in blocks of four, each last one
-// perhaps not full (up to 3 + 3 places beyond 2 kc an item)
+// perhaps not full, then the idle point's (up to 8 places beyond 2 kc an item)
 __device__ __forceinline__ GU4 world_records(const StepDev& S, uint32_t w, uint32_t ibase)
 {
     return (GU4)(S.prog_recs + (size_t)ibase * 8u * S.chain_iters + (size_t)w * 32u);
 }
+
+__device__ __forceinline__ GU32 world_entries(const StepDev& S, uint32_t w, uint32_t ibase)
+{
+    return (GU32)(S.prog_entries + (size_t)ibase * 2u * S.chain_iters + (size_t)w * 8u);
+}
+// where the joints' records start
+__device__ __forceinline__ uint32_t joint_entries(uint32_t entries) { return (entries + 3u) & ~3u; }
 
 // the planning state of item j of a world, and where its second point is
 __device__ __forceinline__ void plan_item(const StepDev& S, uint32_t ibase, uint32_t j, uint32_t nit, uint32_t second)
@@ -2115,7 +2141,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     __syncthreads();
     Program G;
     G.rows = (GU2)(S.prog_rows + (size_t)ibase * kc);
-    G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+    G.entries = world_entries(S, w, ibase);
     G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
     const GU4 items = (GU4)(S.plan_items + 2 * (size_t)ibase);
     PlanLds PL((LU32)smem, nit, waves);
@@ -2174,18 +2200,26 @@ __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uin
         }
         if (s == sub_steps) { body_done(D, A, i, stat, b); continue; }
         const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
-        if (touched) *mom = m;
+        if (touched) {
+            *mom = m;
+            if (minus_zero(m)) atomicOr(&S.w_chain[w].flags, 2u);
+        }
         else { D.mx[i] = m.x; D.my[i] = m.y; D.L[i] = m.z; }
     }
     if (s == 0u) {
         // each world's entries over gridDim / worlds workgroups
-        const uint32_t parts = gridDim.x > S.nworlds ? gridDim.x / S.nworlds : 1u, kc = S.chain_iters;
+        const uint32_t parts = gridDim.x > S.nworlds ? gridDim.x / S.nworlds : 1u;
         for (uint32_t b = blockIdx.x; b < parts * S.nworlds; b += gridDim.x) {
             const uint32_t w = b % S.nworlds, ibase = S.w_item_base[w], nj = (uint32_t)S.worlds[w].njoints;
             if (S.w_status[w] != 0 || S.w_item_base[w + 1] == ibase) continue;
-            const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
+            const GU32 entries = world_entries(S, w, ibase);
             const GU4 to = world_records(S, w, ibase);
             const uint32_t n = S.w_chain[w].entries;
+            if (b < S.nworlds && threadIdx.x < 4u) {
+                const uint32_t idle = joint_entries(n) + nj;
+                to[entry_at(idle) + threadIdx.x * ENTRY_WORD] = idle_word((int)threadIdx.x);
+                if (threadIdx.x == 0u) entries[idle] = S.w_item_base[w + 1] - ibase + S.w_chain[w].pairs;
+            }
             for (uint32_t e = (b / S.nworlds) * blockDim.x + threadIdx.x; e < n; e += parts * blockDim.x) {
                 const uint32_t p = entries[e];
                 if (p >= nj) entry_copy(to, e, (GCU4)(S.recs + (size_t)ibase * 8), p);
@@ -2228,7 +2262,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     const uint32_t t = threadIdx.x, nj = (uint32_t)D.njoints, M = nit - nj, mbeg = S.w_man_begin[w], base = D.body_base;
     const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + 1u);
     const bool m_lds = (uint32_t)D.nbodies <= lds_nmax && mwords <= lds_words;
-    const bool a_lds = m_lds && mwords + 2u * nacc <= lds_words;
+    const bool a_lds = m_lds && mwords + 2u * (nacc + 1u) <= lds_words;
     const LF3 m = (LF3)(LU32)smem;
     const LF2 acc = (LF2)((LU32)smem + mwords);
     const GF3 mom = world_momenta(S, D, w);
@@ -2244,8 +2278,8 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         for (uint32_t q = t; q < nacc; q += T) acc[q] = accg[q];
     const uint32_t kc = S.chain_iters;
     const GU4 prog = world_records(S, w, ibase);
-    const GCU32 entries = (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc);
-    const uint32_t jbase = (W.entries + 3u) & ~3u;   // 2 kc nit places hold the entries and a record a joint
+    const GCU32 entries = (GCU32)world_entries(S, w, ibase);
+    const uint32_t jbase = joint_entries(W.entries);
     const GlobalPoses C = global_poses(D);
     for (uint32_t j = t; j < nj && iters > 0u; j += T) {
         u4v q[4];
@@ -2286,18 +2320,17 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     }
     __syncthreads();
     if (iters > 0u) {
-        const uint32_t reps = iters / kc, ns = W.slots;
-        const GCU2 rows = (GCU2)(S.prog_rows + (size_t)ibase * kc), slots = (GCU2)(S.prog_slots + (size_t)ibase * kc);
-        const GCU4 rec = (GCU4)prog;
-        const bool fix = (W.flags & 2u) != 0u;
+        const ChainProgram G{(GCU2)(S.prog_rows + (size_t)ibase * kc), entries, (GCU2)(S.prog_slots + (size_t)ibase * kc),
+                             (GCU4)prog, W.slots, iters / kc, nj, nacc, jbase + nj, jbase};
+        const bool fix = W.flags != 0u;
         if (chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
-            if (a_lds) chain_lds<true, WARM, true>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, jbase, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<true, WARM, true>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
-            else chain_glb<true, WARM, true>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
+            if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
+            else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);
         } else if (t < 64u) {
-            if (a_lds) chain_lds<false, WARM, true>(rows, entries, slots, rec, m, nc, acc, ns, reps, nj, jbase, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<false, WARM, true>(rows, entries, slots, rec, m, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
-            else chain_glb<false, WARM, true>(rows, entries, slots, rec, mom, nc, accg, ns, reps, nj, jbase, fix, sub_dt);
+            if (a_lds) chain_lds<false, WARM, true>(G, m, nc, acc, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
+            else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
         }
         __syncthreads();
     }
