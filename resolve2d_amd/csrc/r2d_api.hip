@@ -216,6 +216,7 @@ struct r2d_world {
     float4* dwsum = nullptr;
     size_t dwcap = 0;
     bool host_valid = true;   // host mirror is current
+    bool host_fixed = true;   // ... at least what no step changes (ids, flags, masses, shapes)
     bool dev_valid = false;   // device body block is current
     bool topo_dirty = true;   // joints / generators / exclusions need upload
     bool in_service = false;  // held by a server until its request completes
@@ -243,6 +244,13 @@ struct r2d_ctx {
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;   // brackets of the last launched batch
     hipEvent_t ev_kend = nullptr;                      // end of the last fused kernel
     r2d_server* server = nullptr;
+    bool lane = false;                                 // a server's
+    // reading results: pinned memory (a table of kReadTable bytes, then hread_bytes), the worlds of the last batch
+    // and the reads since it
+    char* hread = nullptr;
+    size_t hread_bytes = 0;
+    std::vector<r2d_world*> last_batch;
+    uint32_t reads = 0;
     uint64_t live_worlds = 0;   // worlds created on this context and not yet destroyed
     // step scratch
     void* arena = nullptr;
@@ -474,13 +482,108 @@ int upload_bodies(r2d_world* w)
     return R2D_OK;
 }
 
+// Reading results back.  A kernel packs what is asked for into pinned host
+// memory: one launch and one wait, where copies into pageable memory cost
+// about 16 us a world each and move whole blocks, room to grow and fields that
+// no step changes included.
+constexpr size_t kReadMax = (size_t)16 << 20, kReadTable = (size_t)64 << 10;
+struct ReadItem {
+    const uint32_t* block;
+    uint64_t out;          // word offset behind the table
+    uint32_t cap, n, fields, pad;
+};
+constexpr uint32_t kReadAll = (1u << F_NFIELDS) - 1u;
+constexpr uint32_t kReadMoving = (1u << F_PX) | (1u << F_PY) | (1u << F_ANG) | (1u << F_MX) | (1u << F_MY) | (1u << F_L) |
+                                 (1u << F_FX) | (1u << F_FY) | (1u << F_TQ) | (1u << F_AX) | (1u << F_AY) |
+                                 (1u << F_AHW) | (1u << F_AHH);
+
+__global__ __launch_bounds__(256) void k_read_bodies(const ReadItem* items, uint32_t* out)
+{
+    const ReadItem r = items[blockIdx.x];
+    for (uint32_t i = blockIdx.y * 256u + threadIdx.x; i < r.n; i += gridDim.y * 256u) {
+        uint32_t* o = out + r.out + i;
+#pragma unroll
+        for (int f = 0; f < F_NFIELDS; ++f)
+            if (r.fields & (1u << f)) {
+                *o = r.block[(size_t)f * r.cap + i];
+                o += r.n;
+            }
+    }
+}
+
+// pinned memory of at least `bytes` (at most kReadMax) behind the table
+int ensure_read(r2d_ctx* c, size_t bytes)
+{
+    if (c->hread && c->hread_bytes >= bytes) return R2D_OK;
+    size_t b = (size_t)256 << 10;
+    while (b < bytes) b *= 2;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kReadTable + b) != hipSuccess) return R2D_E_OOM;
+    if (c->hread) (void)hipHostFree(c->hread);
+    c->hread = (char*)p;
+    c->hread_bytes = b;
+    return R2D_OK;
+}
+
+uint32_t read_fields(const r2d_world* w) { return w->host_fixed ? kReadMoving : kReadAll; }
+size_t read_bytes(const r2d_world* w) { return (size_t)__builtin_popcount(read_fields(w)) * (size_t)w->n * 4; }
+
+// The bodies of w, and with them those of further worlds of its batch: the
+// k-th read after a batch fetches up to 2^(k-1) worlds, so reading every world
+// of a batch takes few round trips and reading a few fetches at most about
+// twice as many.
 int download_bodies(r2d_world* w)
 {
     if (w->host_valid) return R2D_OK;
-    HIPCHK(hipMemcpyAsync(w->block.data(), w->dblock, (size_t)F_NFIELDS * w->cap * 4, hipMemcpyDeviceToHost,
-                          w->ctx->stream));
-    HIPCHK(hipStreamSynchronize(w->ctx->stream));
-    w->host_valid = true;
+    r2d_ctx* c = w->ctx;
+    if (w->n == 0 || read_bytes(w) > kReadMax) {
+        HIPCHK(hipMemcpyAsync(w->block.data(), w->dblock, (size_t)F_NFIELDS * w->cap * 4, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        w->host_valid = w->host_fixed = true;
+        return R2D_OK;
+    }
+    r2d_world* more[kReadTable / sizeof(ReadItem)];
+    size_t cnt = 0, bytes = read_bytes(w);
+    more[cnt++] = w;
+    const bool of_batch = w->epoch != 0 && w->epoch == c->epoch && w->batch_index < c->last_batch.size() &&
+                          c->last_batch[w->batch_index] == w;
+    if (of_batch) {
+        const size_t want = std::min<size_t>((size_t)1 << std::min<uint32_t>(c->reads, 20u), kReadTable / sizeof(ReadItem));
+        for (size_t i = w->batch_index + 1; i < c->last_batch.size() && cnt < want; ++i) {
+            r2d_world* x = c->last_batch[i];
+            if (!x || x->ctx != c || x->epoch != c->epoch || x->host_valid || !x->dev_valid || x->in_service || x->n == 0)
+                continue;
+            if (bytes + read_bytes(x) > kReadMax) break;
+            bytes += read_bytes(x);
+            more[cnt++] = x;
+        }
+        c->reads += 1;
+    }
+    int rc = ensure_read(c, bytes);
+    if (rc) return rc;
+    ReadItem* items = (ReadItem*)c->hread;
+    uint32_t* data = (uint32_t*)(c->hread + kReadTable);
+    uint64_t at = 0;
+    uint32_t maxn = 0;
+    for (size_t k = 0; k < cnt; ++k) {
+        items[k] = ReadItem{more[k]->dblock, at, (uint32_t)more[k]->cap, (uint32_t)more[k]->n, read_fields(more[k]), 0u};
+        at += read_bytes(more[k]) / 4;
+        maxn = std::max(maxn, (uint32_t)more[k]->n);
+    }
+    hipLaunchKernelGGL(k_read_bodies, dim3((unsigned)cnt, std::min(256u, (maxn + 255u) / 256u)), dim3(256), 0, c->stream, items,
+                       data);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));
+    for (size_t k = 0; k < cnt; ++k) {
+        r2d_world* x = more[k];
+        const uint32_t* p = data + items[k].out;
+        for (int f = 0; f < F_NFIELDS; ++f)
+            if (items[k].fields & (1u << f)) {
+                std::memcpy(x->u(f), p, (size_t)x->n * 4);
+                p += x->n;
+            }
+        x->host_valid = x->host_fixed = true;
+    }
     return R2D_OK;
 }
 
@@ -1381,6 +1484,8 @@ int fused_wait(r2d_ctx* c, Batch& b)
 int batch_finish(r2d_ctx* c, Batch& b)
 {
     c->epoch = g_epoch.fetch_add(1) + 1;   // unique over contexts: a world's epoch names one batch
+    c->last_batch = c->lane ? std::vector<r2d_world*>() : b.worlds;
+    c->reads = 0;
     for (size_t i = 0; i < b.worlds.size(); ++i) {
         b.worlds[i]->host_valid = false;
         b.worlds[i]->epoch = c->epoch;
@@ -1456,23 +1561,32 @@ int step_batch(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, size_t
     return batch_wait(c, b);
 }
 
-void fill_state(r2d_world* w, int32_t s, r2d_body_state* o)
+// states of `m` bodies from slot s0 on (the arrays' addresses are taken once:
+// the stores below could alias the vector that holds them)
+void fill_states(r2d_world* w, size_t s0, size_t m, r2d_body_state* __restrict out)
 {
-    std::memset(o, 0, sizeof *o);
-    o->id = w->u(F_ID)[s];
-    uint32_t fl = w->u(F_FLAGS)[s];
-    o->type = (fl & BF_RECT) ? 1u : 0u;
-    o->is_static = (fl & BF_STATIC) ? 1u : 0u;
-    o->num_normals = o->type ? 4u : 1u;
-    o->pos_x = w->f(F_PX)[s]; o->pos_y = w->f(F_PY)[s];
-    o->mom_x = w->f(F_MX)[s]; o->mom_y = w->f(F_MY)[s];
-    o->force_x = w->f(F_FX)[s]; o->force_y = w->f(F_FY)[s];
-    o->mass = w->f(F_MASS)[s]; o->angle = w->f(F_ANG)[s]; o->ang_momentum = w->f(F_L)[s];
-    o->torque = w->f(F_TQ)[s]; o->inertia = w->f(F_INERTIA)[s]; o->mu = w->f(F_MU)[s];
-    o->aabb_x = w->f(F_AX)[s]; o->aabb_y = w->f(F_AY)[s];
-    o->aabb_half_width = w->f(F_AHW)[s]; o->aabb_half_height = w->f(F_AHH)[s];
-    o->radius = w->f(F_RAD)[s];
-    o->width = w->width[s]; o->height = w->height[s];
+    const float* f[F_NFIELDS];
+    for (int k = 0; k < F_NFIELDS; ++k) f[k] = w->f(k) + s0;
+    const uint32_t *id = w->u(F_ID) + s0, *flags = w->u(F_FLAGS) + s0;
+    const float *width = w->width.data() + s0, *height = w->height.data() + s0;
+    for (size_t i = 0; i < m; ++i) {
+        r2d_body_state* o = out + i;
+        std::memset(o, 0, sizeof *o);
+        const uint32_t fl = flags[i];
+        o->id = id[i];
+        o->type = (fl & BF_RECT) ? 1u : 0u;
+        o->is_static = (fl & BF_STATIC) ? 1u : 0u;
+        o->num_normals = o->type ? 4u : 1u;
+        o->pos_x = f[F_PX][i]; o->pos_y = f[F_PY][i];
+        o->mom_x = f[F_MX][i]; o->mom_y = f[F_MY][i];
+        o->force_x = f[F_FX][i]; o->force_y = f[F_FY][i];
+        o->mass = f[F_MASS][i]; o->angle = f[F_ANG][i]; o->ang_momentum = f[F_L][i];
+        o->torque = f[F_TQ][i]; o->inertia = f[F_INERTIA][i]; o->mu = f[F_MU][i];
+        o->aabb_x = f[F_AX][i]; o->aabb_y = f[F_AY][i];
+        o->aabb_half_width = f[F_AHW][i]; o->aabb_half_height = f[F_AHH][i];
+        o->radius = f[F_RAD][i];
+        o->width = width[i]; o->height = height[i];
+    }
 }
 
 // ---------------------------------------------------------------- serving
@@ -1750,6 +1864,7 @@ R2D_EXPORT int r2d_ctx_destroy(r2d_ctx* c)
     if (c->dworlds) (void)hipFree(c->dworlds);
     if (c->hcounters) (void)hipHostFree(c->hcounters);
     if (c->hstatus) (void)hipHostFree(c->hstatus);
+    if (c->hread) (void)hipHostFree(c->hread);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     (void)hipEventDestroy(c->ev_begin);
     (void)hipEventDestroy(c->ev_end);
@@ -1799,6 +1914,8 @@ R2D_EXPORT int r2d_world_destroy(r2d_world* w)
     // is out of service only once its lane's launches are collected)
     (void)hipStreamSynchronize(w->ctx->stream);
     r2d_ctx* o = w->owner;
+    for (r2d_world*& x : o->last_batch)
+        if (x == w) x = nullptr;
     pool_release(o, w->dblock);
     pool_release(o, w->djoints);
     pool_release(o, w->dgens);
@@ -2156,7 +2273,7 @@ R2D_EXPORT int r2d_get_body(r2d_world* w, uint32_t id, r2d_body_state* out)
     if (s < 0) return R2D_E_INVALID_ID;
     int rc = download_bodies(w);
     if (rc) return rc;
-    fill_state(w, s, out);
+    fill_states(w, (size_t)s, 1, out);
     return R2D_OK;
 }
 
@@ -2181,9 +2298,67 @@ R2D_EXPORT int r2d_get_bodies(r2d_world* w, r2d_body_state* out, size_t cap, siz
     if (rc) return rc;
     if (n) *n = (size_t)w->n;
     if (!out) return R2D_OK;
-    size_t m = std::min(cap, (size_t)w->n);
-    for (size_t i = 0; i < m; ++i) fill_state(w, (int32_t)i, &out[i]);
+    fill_states(w, 0, std::min(cap, (size_t)w->n), out);
     return R2D_OK;
+}
+
+// manifolds [first, first + rows) of the range [*begin, *end): the count and
+// the world's body base to `head`, their fields one after another to `out`
+struct ReadManifolds {
+    StepDev S;
+    const uint32_t *begin, *end, *body_base;
+    uint32_t first, rows;
+};
+constexpr size_t kReadManifoldWords = 6 + 2 * MP_NFIELDS;
+
+__global__ __launch_bounds__(256) void k_read_manifolds(ReadManifolds r, uint32_t* head, uint32_t* out)
+{
+    const uint32_t b = *r.begin, cnt = *r.end - b;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        head[0] = cnt;
+        head[1] = r.body_base ? *r.body_base : 0u;
+    }
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < r.rows && r.first + i < cnt; i += gridDim.x * 256u) {
+        const size_t m = (size_t)b + r.first + i, R = r.rows;
+        const StepDev& S = r.S;
+        uint32_t* o = out + i;
+        o[0] = S.m_ref[m]; o[R] = S.m_inc[m]; o[2 * R] = S.m_valid[m];
+        float* v = reinterpret_cast<float*>(o);
+        v[3 * R] = S.m_nx[m]; v[4 * R] = S.m_ny[m]; v[5 * R] = S.m_fric[m];
+        for (int k = 0; k < 2 * MP_NFIELDS; ++k) v[(6 + k) * R] = S.m_pt[(size_t)k * S.cap_m + m];
+    }
+}
+
+// `m` of the R manifolds read to u / v (the same words)
+void fill_manifolds(r2d_world* w, const uint32_t* u, const float* v, size_t R, size_t m, uint32_t base, r2d_manifold_state* out)
+{
+    const uint32_t* ids = w->u(F_ID);
+    // preStep (collision.zig:102-133) sets the tangent, the friction and the
+    // points' effective masses; after a step without sub-steps they keep their
+    // initial zeros (the kernels precompute them at the record build regardless)
+    const bool pre = w->prestepped;
+    for (size_t i = 0; i < m; ++i) {
+        r2d_manifold_state& o = out[i];
+        std::memset(&o, 0, sizeof o);
+        o.ref_id = ids[u[i] - base];
+        o.inc_id = ids[u[R + i] - base];
+        const uint32_t valid = u[2 * R + i];
+        const float nx = v[3 * R + i], ny = v[4 * R + i];
+        o.normal_x = nx; o.normal_y = ny;
+        o.tangent_x = pre ? ny : 0.0f; o.tangent_y = pre ? -nx : 0.0f;
+        o.friction = pre ? v[5 * R + i] : 0.0f;
+        for (int p = 0; p < 2; ++p) {
+            r2d_manifold_point& q = o.points[p];
+            q.valid = (valid >> p) & 1u;
+            if (!q.valid) continue;
+            auto F = [&](int fld) { return v[(6 + (size_t)fld * 2 + p) * R + i]; };
+            q.acc_pn = F(MP_ACC_PN); q.acc_pt = F(MP_ACC_PT);
+            q.ref_r_x = F(MP_R1X); q.ref_r_y = F(MP_R1Y); q.inc_r_x = F(MP_R2X); q.inc_r_y = F(MP_R2Y);
+            q.pos_x = F(MP_POSX); q.pos_y = F(MP_POSY);
+            q.depth = F(MP_DEPTH); q.original_depth = F(MP_ODEPTH);
+            q.mass_n = pre ? F(MP_MASS_N) : 0.0f; q.mass_t = pre ? F(MP_MASS_T) : 0.0f;
+        }
+    }
 }
 
 R2D_EXPORT int r2d_get_manifolds(r2d_world* w, r2d_manifold_state* out, size_t cap, size_t* n)
@@ -2217,59 +2392,44 @@ R2D_EXPORT int r2d_get_manifolds(r2d_world* w, r2d_manifold_state* out, size_t c
         S = w->fused_src ? fused_view(c) : c->S;
     }
     const uint32_t bidx = from_static ? 0u : w->batch_index;
-    uint32_t b[2];
-    if (from_static || w->fused_src) {
-        HIPCHK(hipMemcpy(b, S.w_man_begin + bidx, 4, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(b + 1, S.w_man_end + bidx, 4, hipMemcpyDeviceToHost));
-    } else {
-        HIPCHK(hipMemcpy(b, S.w_man_begin + bidx, 8, hipMemcpyDeviceToHost));
-    }
-    size_t cnt = b[1] - b[0];
-    if (n) *n = cnt;
-    if (!out) return R2D_OK;
-    size_t m = std::min(cap, cnt);
-    if (m == 0) return R2D_OK;
-    std::vector<uint32_t> ref(m), inc(m), valid(m);
-    std::vector<float> nx(m), ny(m), fr(m), pt((size_t)MP_NFIELDS * 2 * m);
-    HIPCHK(hipMemcpy(ref.data(), S.m_ref + b[0], m * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(inc.data(), S.m_inc + b[0], m * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(valid.data(), S.m_valid + b[0], m * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(nx.data(), S.m_nx + b[0], m * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(ny.data(), S.m_ny + b[0], m * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(fr.data(), S.m_fric + b[0], m * 4, hipMemcpyDeviceToHost));
-    for (int f = 0; f < MP_NFIELDS * 2; ++f)
-        HIPCHK(hipMemcpy(pt.data() + (size_t)f * m, S.m_pt + (size_t)f * S.cap_m + b[0], m * 4, hipMemcpyDeviceToHost));
-    int rc = download_bodies(w);
+    const bool ends = from_static || w->fused_src;   // the range's end is in an array of its own
+    int rc = ensure_read(c, (size_t)1 << 16);
     if (rc) return rc;
-    uint32_t wb[1] = {0u};
-    // batch body base of this world = first body's batch index
-    if (!from_static) HIPCHK(hipMemcpy(wb, &c->dworlds[w->batch_index].body_base, 4, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < m; ++i) {
-        r2d_manifold_state& o = out[i];
-        std::memset(&o, 0, sizeof o);
-        o.ref_id = w->u(F_ID)[ref[i] - wb[0]];
-        o.inc_id = w->u(F_ID)[inc[i] - wb[0]];
-        o.normal_x = nx[i]; o.normal_y = ny[i];
-        // preStep (collision.zig:102-133) sets the tangent, the friction and
-        // the points' effective masses; after a step without sub-steps they
-        // keep their initial zeros (the kernels precompute them at the
-        // record build regardless)
-        const bool pre = w->prestepped;
-        o.tangent_x = pre ? ny[i] : 0.0f; o.tangent_y = pre ? -nx[i] : 0.0f;
-        o.friction = pre ? fr[i] : 0.0f;
-        for (int p = 0; p < 2; ++p) {
-            r2d_manifold_point& q = o.points[p];
-            q.valid = (valid[i] >> p) & 1u;
-            if (!q.valid) continue;
-            auto F = [&](int fld) { return pt[((size_t)fld * 2 + p) * m + i]; };
-            q.acc_pn = F(MP_ACC_PN); q.acc_pt = F(MP_ACC_PT);
-            q.ref_r_x = F(MP_R1X); q.ref_r_y = F(MP_R1Y); q.inc_r_x = F(MP_R2X); q.inc_r_y = F(MP_R2Y);
-            q.pos_x = F(MP_POSX); q.pos_y = F(MP_POSY);
-            q.depth = F(MP_DEPTH); q.original_depth = F(MP_ODEPTH);
-            q.mass_n = pre ? F(MP_MASS_N) : 0.0f; q.mass_t = pre ? F(MP_MASS_T) : 0.0f;
+    ReadManifolds r{};
+    r.S = S;
+    r.begin = S.w_man_begin + bidx;
+    r.end = ends ? S.w_man_end + bidx : S.w_man_begin + bidx + 1;
+    r.body_base = from_static ? nullptr : &c->dworlds[w->batch_index].body_base;
+    // as many as fit the pinned memory at a time; the first read also brings the count
+    for (size_t done = 0;;) {
+        const size_t room = c->hread_bytes / 4 / kReadManifoldWords;
+        r.first = (uint32_t)done;
+        r.rows = out ? (uint32_t)std::min<size_t>(std::min(room, cap - done), 0x7fffffff) : 0u;
+        hipLaunchKernelGGL(k_read_manifolds, dim3(std::max(1u, std::min(256u, (r.rows + 255u) / 256u))), dim3(256), 0, c->stream,
+                           r, (uint32_t*)c->hread, (uint32_t*)(c->hread + kReadTable));
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->stream));
+        const uint32_t* head = (const uint32_t*)c->hread;
+        const size_t cnt = head[0], m = std::min(cap, cnt);
+        const uint32_t base = head[1];
+        if (n) *n = cnt;
+        if (!out || m == 0) return R2D_OK;
+        const size_t got = std::min<size_t>(m - done, r.rows);
+        const uint32_t* u = (const uint32_t*)(c->hread + kReadTable);
+        const float* v = reinterpret_cast<const float*>(u);
+        const size_t R = r.rows;
+        // the bodies' ids: no step changes them
+        if (!w->host_fixed) {
+            std::vector<uint32_t> rows(u, u + kReadManifoldWords * R);
+            if ((rc = download_bodies(w))) return rc;   // uses the same pinned memory
+            fill_manifolds(w, rows.data(), reinterpret_cast<const float*>(rows.data()), R, got, base, out + done);
+        } else {
+            fill_manifolds(w, u, v, R, got, base, out + done);
         }
+        done += got;
+        if (done >= m) return R2D_OK;
+        if ((rc = ensure_read(c, std::min(kReadMax, (m - done) * kReadManifoldWords * 4)))) return rc;
     }
-    return R2D_OK;
 }
 
 R2D_EXPORT int r2d_set_hash_params(r2d_world* w, int mode, float cell, size_t mult)
@@ -2682,6 +2842,7 @@ R2D_EXPORT int r2d_make_bodies(r2d_world* w, size_t n, const r2d_body_options* b
     hipLaunchKernelGGL(k_make_bodies, dim3(blocks), dim3(256), 0, st, w->dblock, w->dcap, (uint32_t)n0,
                        (uint32_t)n, dbo, dkind, da, db, id0);
     HIPCHK(hipGetLastError());
+    w->host_fixed = false;
     // host side: ids, the id -> slot map, the shapes the host keeps
     if ((size_t)id0 + n > w->id2slot.size())
         w->id2slot.resize(std::max<size_t>(64, ((size_t)id0 + n) * 2), -1);
@@ -2731,6 +2892,7 @@ R2D_EXPORT int r2d_serve_create(r2d_ctx* c, const r2d_serve_options* opt, r2d_se
             delete sv;
             return rc;
         }
+        sv->lanes[l].ctx->lane = true;
         sv->lanes[l].ctx->server = sv;
     }
     c->server = sv;
