@@ -771,6 +771,7 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.w_chain, (W + 1) * sizeof(WorldChain));
     add((void**)&S.counters, 64 * 4);
     add((void**)&S.partials, 1024 * 4);
+    add((void**)&S.scan_state, SCANS * SCAN_TILES * 8); add((void**)&S.scan_ticket, SCANS * 4);
     for (auto& p : parts) off += align256(p.second);
     if (c->arena) {
         HIPCHK(hipStreamSynchronize(c->stream));

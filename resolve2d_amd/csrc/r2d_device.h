@@ -102,6 +102,7 @@ enum : int32_t {
 };
 
 // per-step scratch, sized by capacities chosen on the host
+constexpr uint32_t SCANS = 5, SCAN_TILES = 1024;   // scans of a step, tiles of the largest that one kernel does
 constexpr uint32_t UNTOUCHED = 0xffffffffu;
 // a world's chain in the separate launches
 struct WorldChain {
@@ -171,6 +172,8 @@ struct StepDev {
     WorldChain* w_chain;     // [W+1]
     uint32_t* counters;
     uint32_t* partials;                    // scan scratch
+    uint64_t* scan_state;                  // [SCANS * SCAN_TILES] a step's scans: each tile's sum or prefix
+    uint32_t* scan_ticket;                 // [SCANS] next tile
     // whole steps of each world in one workgroup (k_fused)
     WorldScratch* wscr;        // [W] the world's slices of the arrays above (a world may move to a larger one)
     uint32_t* fpool;           // [8] next free index and capacity of the entry, candidate, manifold and item arrays

@@ -88,7 +88,8 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t* sm, uint32_t* total)
 
 // ------------------------------------------------------------- scan (u32)
 // Exclusive scan of n = min(*n_dev, cap) (or n_const) values into out[0..n],
-// out[n] = total; three fixed-grid kernels.
+// out[n] = total.  One kernel for arrays of up to SCAN_TILES tiles (k_scan);
+// three fixed-grid kernels for larger ones.
 constexpr int SCAN_BLOCKS = 256;
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ITEMS = 4;
@@ -159,19 +160,104 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const uint32_t* in, 
     }
 }
 
-void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t n_const, uint32_t cap,
-              uint32_t* total_dev, uint32_t* partials, hipStream_t st)
+// Tiles taken in the order of a ticket.  A tile publishes its sum, adds up its
+// predecessors' (64 at a time, each a sum or, from some tile on, a prefix) and
+// publishes its prefix: value and kind in one 64-bit word.  Every tile it waits
+// for has its ticket and runs, so the wait ends; the limit only bounds it.
+// One launch where the three kernels took 4.7 us each, almost all of it the
+// launch: a step has five scans (4,096-body pile, 20 launches fewer with the
+// kernels that clear and prepare folded together: 813 -> 720 us a frame).
+constexpr uint32_t SCAN_EACH = 16, SCAN_TILE = SCAN_THREADS * SCAN_EACH;
+constexpr uint32_t SCAN_SPIN = 1u << 22;
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan(const uint32_t* in, uint32_t* out, const uint32_t* n_dev,
+                                                        uint32_t n_const, uint32_t cap, uint32_t* total_dev,
+                                                        uint64_t* state, uint32_t* ticket, uint32_t* overflow)
 {
+    __shared__ uint32_t sm[16], s_tile, s_before;
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    if (t == 0) s_tile = atomicAdd(ticket, 1u);
+    __syncthreads();
+    const uint32_t tile = s_tile, n = scan_n(n_dev, n_const, cap);
+    const uint32_t tiles = n ? (n + SCAN_TILE - 1u) / SCAN_TILE : 1u;
+    if (tile >= tiles) return;
+    const uint32_t i0 = tile * SCAN_TILE + t * SCAN_EACH;
+    uint32_t v[SCAN_EACH], sum = 0;
+    if (i0 + SCAN_EACH <= n) {
+        const uint4* q = reinterpret_cast<const uint4*>(in + i0);   // arrays start at 256-byte bounds
+#pragma unroll
+        for (uint32_t k = 0; k < SCAN_EACH / 4; ++k) {
+            const uint4 x = q[k];
+            v[4 * k] = x.x; v[4 * k + 1] = x.y; v[4 * k + 2] = x.z; v[4 * k + 3] = x.w;
+        }
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < SCAN_EACH; ++k) v[k] = i0 + k < n ? in[i0 + k] : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < SCAN_EACH; ++k) sum += v[k];
+    uint32_t tot;
+    const uint32_t ex = block_excl_scan(sum, sm, &tot);
+    if (t < 64u) {
+        auto put = [&](uint32_t kind, uint32_t x) {
+            if (lane == 0)
+                __hip_atomic_store(&state[tile], ((uint64_t)kind << 32) | x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        uint32_t before = 0;
+        if (tile > 0u) {
+            put(1u, tot);
+            uint32_t spins = 0;
+            for (int32_t base = (int32_t)tile - 1; base >= 0;) {
+                const int32_t at = base - (int32_t)lane;
+                const uint64_t x = at >= 0 ? __hip_atomic_load(&state[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                           : (uint64_t)2u << 32;
+                const uint32_t kind = (uint32_t)(x >> 32);
+                if (__ballot(kind == 0u)) {
+                    if (++spins > SCAN_SPIN) {
+                        if (lane == 0) atomicOr(overflow, 16u);
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                    continue;
+                }
+                const uint64_t ends = __ballot(kind == 2u);
+                const uint32_t last = ends ? (uint32_t)__builtin_ctzll(ends) : 63u;   // the nearest prefix ends the sum
+                before += (uint32_t)__shfl((int)wave_incl_scan(lane <= last ? (uint32_t)x : 0u), 63);
+                if (ends) break;
+                base -= 64;
+            }
+        }
+        put(2u, before + tot);
+        if (lane == 0) s_before = before;
+    }
+    __syncthreads();
+    uint32_t run = s_before + ex;
+#pragma unroll
+    for (uint32_t k = 0; k < SCAN_EACH; ++k) {
+        if (i0 + k < n) out[i0 + k] = run;
+        run += v[k];
+    }
+    if (tile == tiles - 1u && t == 0) {
+        out[n] = s_before + tot;
+        if (total_dev) *total_dev = s_before + tot;
+    }
+}
+
+void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t n_const, uint32_t cap,
+              uint32_t* total_dev, const StepDev& S, int which, hipStream_t st)
+{
+    uint32_t* partials = S.partials;
+    const uint64_t tiles = ((uint64_t)cap + SCAN_TILE - 1u) / SCAN_TILE;
+    if (tiles <= SCAN_TILES) {
+        hipLaunchKernelGGL(k_scan, dim3((unsigned)std::max<uint64_t>(tiles, 1u)), dim3(SCAN_THREADS), 0, st, in, out, n_dev, n_const,
+                           cap, total_dev, S.scan_state + (size_t)which * SCAN_TILES, S.scan_ticket + which,
+                           S.counters + C_OVERFLOW);
+        return;
+    }
     hipLaunchKernelGGL(k_scan_reduce, dim3(SCAN_BLOCKS), dim3(SCAN_THREADS), 0, st, in, n_dev, n_const, cap, partials);
     hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(SCAN_THREADS), 0, st, partials, out, n_dev, n_const, cap,
                        total_dev);
     hipLaunchKernelGGL(k_scan_down, dim3(SCAN_BLOCKS), dim3(SCAN_THREADS), 0, st, in, out, n_dev, n_const, cap,
                        partials);
-}
-
-__global__ void k_zero_u32(uint32_t* p, uint32_t n)
-{
-    for (uint32_t i = grid_tid(); i < n; i += grid_stride()) p[i] = 0u;
 }
 
 // ---------------------------------------------------------- body geometry
@@ -343,14 +429,6 @@ __device__ __forceinline__ bool excluded(const WorldDev& D, uint32_t ida, uint32
 }
 
 // ------------------------------------------------------------ broadphase
-__global__ void k_fill_bworld(StepDev S)
-{
-    // the descriptor's fields read once: the stores below could alias them,
-    // so reading them in the loop would reload them every iteration
-    const uint32_t n = (uint32_t)S.worlds[blockIdx.x].nbodies, base = S.worlds[blockIdx.x].body_base;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) S.bworld[base + i] = blockIdx.x;
-}
-
 // One body's broadphase preparation: cos / sin of the angle, the scheduling
 // flag (a static body orders contacts only if a contact's "+= 0" could change
 // it: a -0 component; joint-touched bodies are added later) and the cell
@@ -407,10 +485,39 @@ __device__ __forceinline__ Prep prep_body(const WorldDev& D, uint32_t sl)
     return o;
 }
 
+// A step's counters, statuses and counts at zero.  The overflow flag is sticky
+// (it is cleared by the host), so a replayed sequence of steps stops
+// committing at the first step whose scratch did not fit.
+__global__ __launch_bounds__(256) void k_begin_step(StepDev S)
+{
+    const uint32_t top = umax(umax(S.nb, S.nbuckets), umax(S.nworlds, SCANS * SCAN_TILES));
+    for (uint32_t x = grid_tid(); x <= top; x += grid_stride()) {
+        if (x < C_OVERFLOW) S.counters[x] = 0u;
+        if (x < SCANS) S.scan_ticket[x] = 0u;
+        if (x < SCANS * SCAN_TILES) S.scan_state[x] = 0ull;
+        if (x <= S.nbuckets) { S.bkt_cnt[x] = 0u; S.bkt_fill[x] = 0u; }
+        if (x <= S.nworlds) {
+            S.w_status[x] = 0;
+            S.w_chain[x] = WorldChain{};
+            if (S.nworlds == 1u) S.w_order[0] = 0u;   // k_world_order is for more
+        }
+        if (x <= S.nb) {
+            S.deg[x] = 0u;
+            S.deg_fill[x] = 0u;
+            if (x < S.nb) S.cmap[x] = UNTOUCHED;
+        }
+    }
+}
+
 __global__ void k_prep(StepDev S)
 {
     for (uint32_t i = grid_tid(); i < S.nb; i += grid_stride()) {
-        uint32_t w = S.bworld[i];
+        uint32_t w = 0, hi = S.nworlds;   // the body's world: the last whose bodies start at or before it
+        while (hi - w > 1) {
+            const uint32_t mid = (w + hi) >> 1;
+            if (S.worlds[mid].body_base <= i) w = mid; else hi = mid;
+        }
+        S.bworld[i] = w;
         const WorldDev& D = S.worlds[w];
         const Prep o = prep_body(D, i - D.body_base);
         S.cc[i] = o.c;
@@ -422,9 +529,31 @@ __global__ void k_prep(StepDev S)
     }
 }
 
-// per cell entry: its body, its bucket; bucket occupancy counts
+// the world of batch joint j
+__device__ __forceinline__ uint32_t joint_world(const StepDev& S, uint32_t j)
+{
+    uint32_t lo = 0, hi = S.nworlds;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (S.worlds[mid].joint_base <= j) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// per cell entry: its body, its bucket; bucket occupancy counts.  And the
+// bodies of distance / offset joints, which write both even when static
+// (DistanceJoint.zig:72-74, OffsetDistanceJoint.zig:100-104): such a static
+// body orders every item that touches it.
 __global__ void k_entries(StepDev S)
 {
+    for (uint32_t j = grid_tid(); j < S.njoints; j += grid_stride()) {
+        const WorldDev& D = S.worlds[joint_world(S, j)];
+        const Joint& J = D.joints[j - D.joint_base];
+        if (J.type <= 1) {
+            if (J.s1 >= 0) atomicOr(&S.sflag[D.body_base + J.s1], SF_RESOURCE);
+            if (J.s2 >= 0) atomicOr(&S.sflag[D.body_base + J.s2], SF_RESOURCE);
+        }
+    }
     uint32_t E = dev_count(&S.counters[C_ENTRIES], S.cap_e);
     if (S.counters[C_ENTRIES] > S.cap_e) { if (grid_tid() == 0) atomicOr(&S.counters[C_OVERFLOW], 1u); return; }
     for (uint32_t e = grid_tid(); e < E; e += grid_stride()) {
@@ -729,24 +858,9 @@ __device__ __forceinline__ void man_build_one(const StepDev& S, const WorldDev& 
     S.m_valid[m] = valid;
 }
 
-__global__ void k_man_build(StepDev S)
+// each world's range of manifolds and of items
+__device__ __forceinline__ void world_ranges(const StepDev& S)
 {
-    uint32_t R = dev_count(&S.counters[C_RAW], S.cap_r);
-    if (S.counters[C_OVERFLOW]) return;
-    if (S.counters[C_MANIFOLDS] > S.cap_m) { if (grid_tid() == 0) atomicOr(&S.counters[C_OVERFLOW], 4u); return; }
-    for (uint32_t q = grid_tid(); q < R; q += grid_stride()) {
-        if (!S.cand_flag[q]) continue;
-        const uint4 cq = S.cand[q];
-        const uint32_t a = cq.x, b = cq.y;
-        const WorldDev& D = S.worlds[S.bworld[a]];
-        man_build_one(S, D, D, S.cand_idx[q], D.body_base, a - D.body_base, b - D.body_base, S.sat_info[q],
-                      mk(S.sat_nx[q], S.sat_ny[q]), S.cc[a], S.cs[a], S.cc[b], S.cs[b]);
-    }
-}
-
-__global__ void k_world_ranges(StepDev S)
-{
-    if (S.counters[C_OVERFLOW]) return;
     uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
     uint32_t R = dev_count(&S.counters[C_RAW], S.cap_r);
     uint32_t E = dev_count(&S.counters[C_ENTRIES], S.cap_e);
@@ -768,6 +882,22 @@ __global__ void k_world_ranges(StepDev S)
         uint32_t jb = (w == S.nworlds) ? S.njoints : S.worlds[w].joint_base;
         S.w_item_base[w] = jb + mb;
         if (w == S.nworlds) S.counters[C_ITEMS] = jb + mb;
+    }
+}
+
+__global__ void k_man_build(StepDev S)
+{
+    uint32_t R = dev_count(&S.counters[C_RAW], S.cap_r);
+    if (S.counters[C_OVERFLOW]) return;
+    if (S.counters[C_MANIFOLDS] > S.cap_m) { if (grid_tid() == 0) atomicOr(&S.counters[C_OVERFLOW], 4u); return; }
+    world_ranges(S);
+    for (uint32_t q = grid_tid(); q < R; q += grid_stride()) {
+        if (!S.cand_flag[q]) continue;
+        const uint4 cq = S.cand[q];
+        const uint32_t a = cq.x, b = cq.y;
+        const WorldDev& D = S.worlds[S.bworld[a]];
+        man_build_one(S, D, D, S.cand_idx[q], D.body_base, a - D.body_base, b - D.body_base, S.sat_info[q],
+                      mk(S.sat_nx[q], S.sat_ny[q]), S.cc[a], S.cs[a], S.cc[b], S.cs[b]);
     }
 }
 
@@ -795,28 +925,6 @@ __global__ __launch_bounds__(1024) void k_world_order(StepDev S)
         uint32_t items = S.w_item_base[w + 1] - S.w_item_base[w];
         uint32_t pos = atomicAdd(&hist[(uint32_t)__builtin_clz(items + 1u)], 1u);
         S.w_order[pos] = w;
-    }
-}
-
-// distance / offset joints write both bodies even when static
-// (DistanceJoint.zig:72-74, OffsetDistanceJoint.zig:100-104): such a static
-// body orders every item that touches it.
-__global__ void k_joint_mark(StepDev S)
-{
-    if (S.counters[C_OVERFLOW]) return;
-    for (uint32_t j = grid_tid(); j < S.njoints; j += grid_stride()) {
-        // world of batch joint j
-        uint32_t lo = 0, hi = S.nworlds;
-        while (hi - lo > 1) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (S.worlds[mid].joint_base <= j) lo = mid; else hi = mid;
-        }
-        const WorldDev& D = S.worlds[lo];
-        const Joint& J = D.joints[j - D.joint_base];
-        if (J.type <= 1) {
-            if (J.s1 >= 0) atomicOr(&S.sflag[D.body_base + J.s1], SF_RESOURCE);
-            if (J.s2 >= 0) atomicOr(&S.sflag[D.body_base + J.s2], SF_RESOURCE);
-        }
     }
 }
 
@@ -848,59 +956,36 @@ __device__ __forceinline__ void chain_touch(const StepDev& S, bool on, uint32_t 
     if (mine) S.cmap[x] = c;
 }
 
-__global__ void k_items_joints(StepDev S)
+// the step's solver items: their ordering bodies, and the items of each
+__global__ void k_items(StepDev S)
 {
     if (S.counters[C_OVERFLOW]) return;
     if (S.counters[C_ITEMS] > S.cap_i) { if (grid_tid() == 0) atomicOr(&S.counters[C_OVERFLOW], 8u); return; }
+    auto put = [&](uint32_t w, uint32_t item, int32_t r0, int32_t r1) {
+        S.it_r0[item] = r0;
+        S.it_r1[item] = r1;
+        if (r0 >= 0) atomicAdd(&S.deg[r0], 1u);
+        if (r1 >= 0) atomicAdd(&S.deg[r1], 1u);
+    };
     for (uint32_t j = grid_tid(); j < S.njoints; j += grid_stride()) {
-        uint32_t lo = 0, hi = S.nworlds;
-        while (hi - lo > 1) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (S.worlds[mid].joint_base <= j) lo = mid; else hi = mid;
-        }
-        const WorldDev& D = S.worlds[lo];
-        uint32_t jl = j - D.joint_base;
+        const uint32_t w = joint_world(S, j);
+        const WorldDev& D = S.worlds[w];
+        const uint32_t jl = j - D.joint_base;
         const Joint& J = D.joints[jl];
-        uint32_t item = S.w_item_base[lo] + jl;
-        int32_t r0 = J.s1 >= 0 ? (int32_t)(D.body_base + J.s1) : -1;
+        const int32_t r0 = J.s1 >= 0 ? (int32_t)(D.body_base + J.s1) : -1;
         int32_t r1 = -1;
         if (J.type <= 1 && J.s2 >= 0 && J.s2 != J.s1) r1 = (int32_t)(D.body_base + J.s2);
-        S.it_r0[item] = r0;
-        S.it_r1[item] = r1;
-        if (r0 >= 0) atomicAdd(&S.deg[r0], 1u);
-        if (r1 >= 0) atomicAdd(&S.deg[r1], 1u);
-        chain_touch(S, r0 >= 0, lo, (uint32_t)r0);
-        chain_touch(S, r1 >= 0, lo, (uint32_t)r1);
+        put(w, S.w_item_base[w] + jl, r0, r1);
+        chain_touch(S, r0 >= 0, w, (uint32_t)r0);
+        chain_touch(S, r1 >= 0, w, (uint32_t)r1);
     }
-}
-
-__global__ void k_items_mans(StepDev S)
-{
-    if (S.counters[C_OVERFLOW] || S.counters[C_ITEMS] > S.cap_i) return;
-    uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
+    const uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
     for (uint32_t m = grid_tid(); m < M; m += grid_stride()) {
-        uint32_t ref = S.m_ref[m], inc = S.m_inc[m];
-        uint32_t w = S.bworld[ref];
-        uint32_t item = S.w_item_base[w] + S.worlds[w].njoints + (m - S.w_man_begin[w]);
-        int32_t r0 = (S.sflag[ref] & SF_RESOURCE) ? (int32_t)ref : -1;
-        int32_t r1 = (S.sflag[inc] & SF_RESOURCE) ? (int32_t)inc : -1;
-        S.it_r0[item] = r0;
-        S.it_r1[item] = r1;
-        if (r0 >= 0) atomicAdd(&S.deg[r0], 1u);
-        if (r1 >= 0) atomicAdd(&S.deg[r1], 1u);
+        const uint32_t ref = S.m_ref[m], inc = S.m_inc[m], w = S.bworld[ref];
+        put(w, S.w_item_base[w] + S.worlds[w].njoints + (m - S.w_man_begin[w]),
+            (S.sflag[ref] & SF_RESOURCE) ? (int32_t)ref : -1, (S.sflag[inc] & SF_RESOURCE) ? (int32_t)inc : -1);
         chain_touch(S, true, w, ref);
         chain_touch(S, true, w, inc);
-    }
-}
-
-// what the step's items are counted into, at zero
-__global__ void k_items_clear(StepDev S)
-{
-    for (uint32_t x = grid_tid(); x <= S.nb; x += grid_stride()) {
-        S.deg[x] = 0u;
-        S.deg_fill[x] = 0u;
-        if (x < S.nb) S.cmap[x] = UNTOUCHED;
-        if (x <= S.nworlds) S.w_chain[x] = WorldChain{};
     }
 }
 
@@ -2099,12 +2184,7 @@ __global__ __launch_bounds__(256) void k_chain_build(StepDev S, float sub_dt)
 {
     if (S.counters[C_OVERFLOW]) return;
     for (uint32_t q = grid_tid(); q < S.njoints; q += grid_stride()) {
-        uint32_t lo = 0, hi = S.nworlds;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (S.worlds[mid].joint_base <= q) lo = mid; else hi = mid;
-        }
-        const uint32_t ibase = S.w_item_base[lo];
+        const uint32_t lo = joint_world(S, q), ibase = S.w_item_base[lo];
         plan_item(S, ibase, q - S.worlds[lo].joint_base, S.w_item_base[lo + 1] - ibase, 0u);
     }
     const uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
@@ -2227,6 +2307,7 @@ __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uin
         }
     }
     if (s != sub_steps) return;
+    if (grid_tid() == 0u) S.counters[C_STEPS] += 1u;   // the step is done
     const size_t cm = S.cap_m;
     const uint32_t M = dev_count(&S.counters[C_MANIFOLDS], S.cap_m);
     for (uint32_t m = grid_tid(); m < M; m += grid_stride()) {
@@ -2647,14 +2728,7 @@ void k_fused(StepDev S /* first: chain_world reads it from the argument segment 
     if (t < 4) atomicAdd(&S.counters[t], cnt[t]);
 }
 
-// step bookkeeping: counters of one step start at zero; the overflow flag is
-// sticky (it is cleared by the host), so a replayed sequence of steps stops
-// committing at the first step whose scratch did not fit.
-__global__ void k_begin_step(uint32_t* counters)
-{
-    if (threadIdx.x < C_OVERFLOW) counters[threadIdx.x] = 0u;
-}
-
+// the end of a step without sub-steps
 __global__ void k_commit_step(uint32_t* counters)
 {
     if (threadIdx.x == 0 && counters[C_OVERFLOW] == 0u) counters[C_STEPS] += 1u;
@@ -2813,26 +2887,16 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
     hipStream_t st = ss.main;
     switch (phase) {
     case PH_BROAD:
-        hipLaunchKernelGGL(k_begin_step, dim3(1), dim3(64), 0, st, S.counters);
+        hipLaunchKernelGGL(k_begin_step, dim3(blocks_for(std::max<uint64_t>(std::max(S.nb, S.nbuckets), SCANS * SCAN_TILES), BS, 1024)),
+                           dim3(BS), 0, st, S);
         tmark(ss, "k_begin_step", st);
-        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(S.nworlds + 1, BS)), dim3(BS), 0, st,
-                           reinterpret_cast<uint32_t*>(S.w_status), S.nworlds + 1);
-        tmark(ss, "k_zero_u32", st);
-        hipLaunchKernelGGL(k_fill_bworld, dim3(S.nworlds), dim3(256), 0, st, S);
-        tmark(ss, "k_fill_bworld", st);
         hipLaunchKernelGGL(k_prep, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
         tmark(ss, "k_prep", st);
-        scan_u32(S.ncell, S.cell_off, nullptr, S.nb, S.nb, &S.counters[C_ENTRIES], S.partials, st);
+        scan_u32(S.ncell, S.cell_off, nullptr, S.nb, S.nb, &S.counters[C_ENTRIES], S, 0, st);
         tmark(ss, "scan ncell", st);
-        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(S.nbuckets + 1, BS)), dim3(BS), 0, st, S.bkt_cnt,
-                           S.nbuckets + 1);
-        tmark(ss, "k_zero_u32", st);
-        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(S.nbuckets + 1, BS)), dim3(BS), 0, st, S.bkt_fill,
-                           S.nbuckets + 1);
-        tmark(ss, "k_zero_u32", st);
         hipLaunchKernelGGL(k_entries, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_entries", st);
-        scan_u32(S.bkt_cnt, S.bkt_off, nullptr, S.nbuckets, S.nbuckets, nullptr, S.partials, st);
+        scan_u32(S.bkt_cnt, S.bkt_off, nullptr, S.nbuckets, S.nbuckets, nullptr, S, 1, st);
         tmark(ss, "scan bkt_cnt", st);
         hipLaunchKernelGGL(k_bucket_fill, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_bucket_fill", st);
@@ -2840,7 +2904,7 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
         tmark(ss, "k_bucket_rank", st);
         hipLaunchKernelGGL(k_ent_cnt, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_ent_cnt", st);
-        scan_u32(S.ent_cnt, S.ent_off, &S.counters[C_ENTRIES], 0, S.cap_e, &S.counters[C_RAW], S.partials, st);
+        scan_u32(S.ent_cnt, S.ent_off, &S.counters[C_ENTRIES], 0, S.cap_e, &S.counters[C_RAW], S, 2, st);
         tmark(ss, "scan ent_cnt", st);
         hipLaunchKernelGGL(k_cand_emit, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_cand_emit", st);
@@ -2848,23 +2912,15 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
     case PH_NARROW:
         hipLaunchKernelGGL(k_narrow, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_narrow", st);
-        scan_u32(S.cand_flag, S.cand_idx, &S.counters[C_RAW], 0, S.cap_r, &S.counters[C_MANIFOLDS], S.partials, st);
+        scan_u32(S.cand_flag, S.cand_idx, &S.counters[C_RAW], 0, S.cap_r, &S.counters[C_MANIFOLDS], S, 3, st);
         tmark(ss, "scan cand_flag", st);
         hipLaunchKernelGGL(k_man_build, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_man_build", st);
         break;
     case PH_SCHED:
-        hipLaunchKernelGGL(k_world_ranges, dim3(blocks_for(S.nworlds + 1, BS)), dim3(BS), 0, st, S);
-        tmark(ss, "k_world_ranges", st);
-        hipLaunchKernelGGL(k_joint_mark, dim3(blocks_for(S.njoints, BS)), dim3(BS), 0, st, S);
-        tmark(ss, "k_joint_mark", st);
-        hipLaunchKernelGGL(k_items_clear, dim3(blocks_for(S.nb + 1, BS)), dim3(BS), 0, st, S);
-        tmark(ss, "k_items_clear", st);
-        hipLaunchKernelGGL(k_items_joints, dim3(blocks_for(S.njoints, BS)), dim3(BS), 0, st, S);
-        tmark(ss, "k_items_joints", st);
-        hipLaunchKernelGGL(k_items_mans, dim3(GRID), dim3(BS), 0, st, S);
-        tmark(ss, "k_items_mans", st);
-        scan_u32(S.deg, S.deg_off, nullptr, S.nb, S.nb, nullptr, S.partials, st);
+        hipLaunchKernelGGL(k_items, dim3(GRID), dim3(BS), 0, st, S);
+        tmark(ss, "k_items", st);
+        scan_u32(S.deg, S.deg_off, nullptr, S.nb, S.nb, nullptr, S, 4, st);
         tmark(ss, "scan deg", st);
         hipLaunchKernelGGL(k_list_fill, dim3(GRID), dim3(BS), 0, st, S);
         tmark(ss, "k_list_fill", st);
@@ -2874,8 +2930,10 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             hipLaunchKernelGGL(k_color, dim3(S.nworlds), dim3(256), 0, st, S);
             tmark(ss, "k_color", st);
         }
-        hipLaunchKernelGGL(k_world_order, dim3(1), dim3(1024), 0, st, S);
-        tmark(ss, "k_world_order", st);
+        if (S.nworlds > 1u) {
+            hipLaunchKernelGGL(k_world_order, dim3(1), dim3(1024), 0, st, S);
+            tmark(ss, "k_world_order", st);
+        }
         if (sp.any_colored) {
             hipLaunchKernelGGL(k_list_rank<true>, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
             tmark(ss, "k_list_rank<true>", st);
@@ -2918,8 +2976,10 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             hipLaunchKernelGGL(k_warm_save, dim3(GRID), dim3(BS), 0, st, S);
             tmark(ss, "k_warm_save", st);
         }
-        hipLaunchKernelGGL(k_commit_step, dim3(1), dim3(64), 0, st, S.counters);
-        tmark(ss, "k_commit_step", st);
+        if (sub_steps == 0) {
+            hipLaunchKernelGGL(k_commit_step, dim3(1), dim3(64), 0, st, S.counters);
+            tmark(ss, "k_commit_step", st);
+        }
         break;
     }
     }
