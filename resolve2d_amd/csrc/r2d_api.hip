@@ -811,11 +811,44 @@ void destroy_graphs(r2d_ctx* c)
     c->graph_key.clear();
 }
 
-// The launch shape of a batch the caller has not tuned: a few worlds (each
-// alone on a CU, latency-bound on their chains) take the 512-lane record
-// kernel; more take the register-slot kernel for small worlds and the
-// 256-thread record kernel for the others.
-int default_variant(size_t nworlds) { return nworlds <= WIDE_MAX_WORLDS ? WIDE_VARIANT : 1; }
+constexpr size_t kFusedLdsMax = 160 * 1024 - 1024;
+
+// Workgroups a CU holds of a batch at once: what its worlds need, one each
+size_t worlds_per_cu(const r2d_ctx* c, size_t nworlds)
+{
+    const size_t cus = c->num_cus > 0 ? (size_t)c->num_cus : 256;
+    return std::max<size_t>(1, (nworlds + cus - 1) / cus);
+}
+
+// The launch shape of a batch the caller has not tuned.  Worlds that are each
+// alone on a CU take 768 threads (256 worlds of 379-501 bodies: 375 us a step,
+// 435 with 256 threads).  Two or three a CU take 256 threads and registers for
+// three workgroups (512 worlds of 273-501: 453 us; for four: 461); more take
+// registers for four, with spills, since a fourth world that waits for one of
+// the three costs more (1,024 worlds of 51-501: 484 us, for three 600, 192
+// threads 506).  Warm starting is compiled into kernels of its own, of 768 and
+// 192 threads (256 worlds: 6.1 and 8.2 ms for 16 steps).
+int default_variant(const r2d_ctx* c, size_t nworlds)
+{
+    const size_t k = worlds_per_cu(c, nworlds);
+    return k == 1 ? WIDE_VARIANT : k <= 3 ? 1 : 10;
+}
+int warm_variant(const r2d_ctx* c, size_t nworlds)
+{
+    return worlds_per_cu(c, nworlds) == 1 ? WARM_WIDE_VARIANT : WARM_VARIANT;
+}
+
+// LDS of a fused launch: a CU's divided by the worlds it is to hold, as far as
+// the largest world needs no more.  What a world has beyond its need holds
+// plans and impulses of worlds with many contacts, which are in global memory
+// otherwise (a world of 501 bodies and 983 items: plan 111 us, in LDS 46).
+size_t fused_lds_share(const r2d_ctx* c, size_t nworlds, uint32_t n, uint32_t tb)
+{
+    const size_t need = fused_lds_bytes(n, tb);
+    const size_t fit = std::max<size_t>(1, (kFusedLdsMax + 1024) / (need + 1024));
+    const size_t share = ((kFusedLdsMax + 1024) / std::min(fit, worlds_per_cu(c, nworlds)) - 1024) & ~(size_t)15;
+    return std::max(need, share);
+}
 
 template <class Fn>
 bool capture_graph(r2d_ctx* c, hipGraphExec_t* out, Fn&& enqueue)
@@ -855,7 +888,6 @@ struct Batch {
 };
 
 // ------------------------------------------------ fused steps: scratch slices
-constexpr size_t kFusedLdsMax = 160 * 1024 - 1024;
 
 uint32_t grow_cap(uint32_t have, uint64_t need)
 {
@@ -1196,7 +1228,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
 
     // solve variant: context override (autotuner), environment, then the
     // default (default_variant)
-    int variant = default_variant(nw);
+    int variant = default_variant(c, nw);
     if (c->solve_variant >= 0) variant = c->solve_variant;
     if (const char* e = std::getenv("R2D_SOLVE_VARIANT")) {
         int v = std::atoi(e);
@@ -1207,8 +1239,8 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         colored = colored || worlds[i]->sched != 0;
         warm = warm || worlds[i]->warm > 0.0f;
     }
-    // warm starting is compiled into one variant's kernels only
-    if (warm) variant = WARM_VARIANT;
+    // warm starting is compiled into kernels of its own
+    if (warm) variant = warm_variant(c, nw);
     b.plan = plan_solve(variant, sizes.data(), nw, c->lds_nmax, colored, warm, c->wide_record);
     b.variant = variant;
     // whole steps per workgroup: worlds of at most FUSED_NMAX bodies in the
@@ -1221,7 +1253,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         maxtb = std::max(maxtb, b.descs[i].table);
     }
     if (fused) {
-        b.fused_lds = fused_lds_bytes(maxn, maxtb);
+        b.fused_lds = fused_lds_share(c, nw, maxn, maxtb);
         fused = b.fused_lds <= kFusedLdsMax;
     }
     b.fused = fused;
@@ -2166,9 +2198,9 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     if (sub_steps > 0 && iters > 0)
         for (const HJoint& h : w->joints)
             if (w->slot_of(h.id1) < 0 || (h.type <= 1 && w->slot_of(h.id2) < 0)) return R2D_E_INVALID_ID;
-    int variant = c->solve_variant >= 0 ? c->solve_variant : default_variant(1);
+    int variant = c->solve_variant >= 0 ? c->solve_variant : default_variant(c, 1);
     if (!fused_available(variant)) variant = 11;
-    const size_t lds = fused_lds_bytes(n, tb);
+    const size_t lds = fused_lds_share(c, 1, n, tb);
     if (lds > kFusedLdsMax) return R2D_E_CAPACITY;
     if (n == 0) {   // nothing moves and no manifold exists
         w->epoch = 0;

@@ -19,17 +19,15 @@ enum { KT_BROAD_BEGIN = 0, KT_NARROW_BEGIN, KT_SCHED_BEGIN, KT_SOLVE_BEGIN, KT_E
 // the four phases of one step, enqueued in this order on one stream
 enum { PH_BROAD = 0, PH_NARROW, PH_SCHED, PH_SOLVE, PH_N };
 
-// solve-kernel variants (register-slot kernel shape + record-kernel workgroup
-// size; table in r2d_kernels.hip)
+// solve variants: shapes of the kernels that run worlds' programs (table in
+// r2d_kernels.hip)
 constexpr int SOLVE_VARIANTS = 15;
-// the default for batches of at most WIDE_MAX_WORLDS worlds (each alone on a
-// CU): records only, 768-thread workgroups, so a world of up to 768 solver
-// items holds one item per lane and its chain never picks up a record
+// the default for worlds that are each alone on a CU
 constexpr int WIDE_VARIANT = 14;
-constexpr size_t WIDE_MAX_WORLDS = 64;
-// the variant every batch with a warm-started world takes (not tunable)
-constexpr int WARM_VARIANT = SOLVE_VARIANTS;
-constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 1;
+// batches with a warm-started world take these (not tunable): several worlds
+// a CU, and one
+constexpr int WARM_VARIANT = SOLVE_VARIANTS, WARM_WIDE_VARIANT = SOLVE_VARIANTS + 1;
+constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 2;
 
 // Iterations of a sub-step that one program covers: all of them up to 16,
 // else their largest divisor up to 16 (the program is then run that often).
