@@ -594,6 +594,42 @@ __device__ __forceinline__ uint32_t count_below(const uint32_t* l, uint32_t c, u
     return r;
 }
 
+// Walks of long cell lists: a wall has hundreds of cells, and one thread walks
+// them while the kernel waits for it.  Sixteen loads are in flight at a time
+// (four for the usual body of up to four cells).
+template <uint32_t W, class F>
+__device__ __forceinline__ bool walk(const uint32_t* l, uint32_t i, uint32_t c, F stop)
+{
+    uint32_t x[W];
+    bool hit = false;
+#pragma unroll
+    for (uint32_t q = 0; q < W; ++q) x[q] = l[umin(i + q, c - 1u)];
+#pragma unroll
+    for (uint32_t q = 0; q < W; ++q) hit = stop(x[q], i + q < c) || hit;
+    return hit;
+}
+
+// how many of l[0, c) equal v
+__device__ __forceinline__ uint32_t count_equal(const uint32_t* l, uint32_t c, uint32_t v)
+{
+    uint32_t r = 0;
+    for (uint32_t i = 0; i < c; i += 16)
+        walk<16>(l, i, c, [&](uint32_t x, bool in) { r += in && x == v; return false; });
+    return r;
+}
+
+// whether some of l[0, c) is one of h[0, n), n of 1 to 4
+__device__ __forceinline__ bool any_equal(const uint32_t* l, uint32_t c, const uint32_t* h, uint32_t n)
+{
+    if (c == 0u) return false;
+    const uint32_t h0 = h[0], h1 = h[umin(1u, n - 1u)], h2 = h[umin(2u, n - 1u)], h3 = h[n - 1u];
+    auto same = [&](uint32_t x, bool) { return x == h0 || x == h1 || x == h2 || x == h3; };   // (the last one may repeat)
+    if (walk<4>(l, 0u, c, same)) return true;
+    for (uint32_t i = 4; i < c; i += 16)
+        if (walk<16>(l, i, c, same)) return true;
+    return false;
+}
+
 // A cell entry's rank among its bucket's members it[0, c): how many are
 // greater than its body a and how many equal it.  Four members per
 // iteration, so their loads are in flight together.
@@ -633,8 +669,10 @@ __global__ void k_bucket_rank(StepDev S)
         uint32_t greater, same;
         bucket_rank_of(it, n, a, greater, same);
         uint32_t dup = 0;
-        if (same > 1)
-            for (uint32_t x = S.cell_off[a]; x < e; ++x) dup += S.ent_bkt[x] == gb;
+        if (same > 1) {
+            const uint32_t x = S.cell_off[a];
+            dup = count_equal(S.ent_bkt + x, e - x, gb);
+        }
         S.bkt_sorted[o + greater + dup] = a;
     }
 }
@@ -700,13 +738,7 @@ __device__ __forceinline__ bool narrow_pair(const WorldDev& D, const B& bodies, 
     // b first appears in a's query list at cell k unless an earlier cell of a
     // hashes to a bucket b also occupies (buckets are deduplicated, so
     // within one bucket b appears once)
-    if (ok) {
-        for (uint32_t j = 0; j < nb && ok; ++j) {
-            uint32_t h = bb[j];
-            for (uint32_t kk = 0; kk < k; ++kk)
-                if (ba[kk] == h) { ok = false; break; }
-        }
-    }
+    for (uint32_t j = 0; j < nb && ok; j += 4) ok = !any_equal(ba, k, bb + j, umin(nb - j, 4u));
     if (!ok) return false;
     Geo ga = load_geo(bodies, sa, ca, sa_sin);
     Geo gb = load_geo(bodies, sb, cb, sb_sin);
@@ -1019,59 +1051,78 @@ constexpr uint32_t COLOR_SPIN_LIMIT = 1u << 22;
 // per world.  The colouring runs as a dataflow over per-body counters in item
 // order: an item waits until every earlier item on its bodies has taken its
 // colour.  Worlds in the reference order take no part.
-__global__ __launch_bounds__(256) void k_color(StepDev S)
+// The counters and the colours used (20 bytes a body) are in LDS under the
+// bodies' chain places when they fit, and 1,024 lanes take items in turn: an
+// item waits behind its lane's earlier ones, and a poll of global memory is
+// about a microsecond (4,096-body pile: 128 -> 34 us).
+constexpr uint32_t COLOR_THREADS = 1024;
+constexpr size_t COLOR_LDS = 159 * 1024;
+__global__ __launch_bounds__(COLOR_THREADS) void k_color(StepDev S, uint32_t lds_words)
 {
+    extern __shared__ __align__(16) uint32_t smem[];
     __shared__ uint32_t s_abort;
     if (S.counters[C_OVERFLOW]) return;
     const uint32_t w = blockIdx.x;
     const WorldDev& D = S.worlds[w];
-    const uint32_t i0 = S.w_item_base[w], nit = S.w_item_base[w + 1] - i0;
-    const uint32_t T = blockDim.x, t = threadIdx.x;
     if (D.sched == 0) return;
-    const uint32_t base = D.body_base;
-    for (int b = t; b < D.nbodies; b += T) {
-        S.cmask[2 * (base + b)] = 0ull;
-        S.cmask[2 * (base + b) + 1] = 0ull;
-        S.g_cnt[base + b] = 0u;
-    }
-    if (t == 0) s_abort = 0u;
-    __syncthreads();
-    uint32_t spins = 0;
-    for (uint32_t p = t; p < nit;) {
-        if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
-        const uint32_t it = i0 + p;
-        const int32_t r0 = S.it_r0[it], r1 = S.it_r1[it];
-        bool ready = r0 < 0 || ld_acq(&S.g_cnt[r0]) == S.it_k0[it];
-        if (ready && r1 >= 0) ready = ld_acq(&S.g_cnt[r1]) == S.it_k1[it];
-        if (ready) {
-            uint64_t m0 = 0, m1 = 0;
-            if (r0 >= 0) { m0 |= S.cmask[2 * r0]; m1 |= S.cmask[2 * r0 + 1]; }
-            if (r1 >= 0) { m0 |= S.cmask[2 * r1]; m1 |= S.cmask[2 * r1 + 1]; }
-            uint32_t c;
-            if (~m0) c = (uint32_t)__builtin_ctzll(~m0);
-            else if (~m1) c = 64u + (uint32_t)__builtin_ctzll(~m1);
-            else c = 128u + p;
-            S.it_color[it] = c;
-            if (c < 128) {
-                const uint32_t hi = c >> 6;
-                const uint64_t bit = 1ull << (c & 63u);
-                if (r0 >= 0) S.cmask[2 * r0 + hi] |= bit;
-                if (r1 >= 0) S.cmask[2 * r1 + hi] |= bit;
-            }
-            if (r0 >= 0) st_rel(&S.g_cnt[r0], S.it_k0[it] + 1u);
-            if (r1 >= 0) st_rel(&S.g_cnt[r1], S.it_k1[it] + 1u);
-            p += T;
-            spins = 0;
-        } else {
-            // every item's predecessors come first, so some item is always ready
-            if (++spins > COLOR_SPIN_LIMIT) {
-                __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                S.w_status[w] = 5;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
+    const uint32_t i0 = S.w_item_base[w], nit = S.w_item_base[w + 1] - i0, base = D.body_base, t = threadIdx.x;
+    const uint32_t nc = S.w_chain[w].bodies;
+    auto run = [&](auto mask, auto count, uint32_t n, auto place) {
+        for (uint32_t b = t; b < n; b += COLOR_THREADS) {
+            mask[2 * b] = 0ull;
+            mask[2 * b + 1] = 0ull;
+            count[b] = 0u;
         }
-    }
+        if (t == 0) s_abort = 0u;
+        __syncthreads();
+        uint32_t spins = 0, cur = ~0u, b0 = 0, b1 = 0, k0 = 0, k1 = 0;
+        int32_t r0 = -1, r1 = -1;
+        for (uint32_t p = t; p < nit;) {
+            const uint32_t it = i0 + p;
+            if (p != cur) {
+                cur = p;
+                r0 = S.it_r0[it]; r1 = S.it_r1[it];
+                k0 = S.it_k0[it]; k1 = S.it_k1[it];
+                b0 = r0 >= 0 ? place((uint32_t)r0) : 0u;
+                b1 = r1 >= 0 ? place((uint32_t)r1) : 0u;
+            }
+            bool ready = r0 < 0 || ld_acq(&count[b0]) == k0;
+            if (ready && r1 >= 0) ready = ld_acq(&count[b1]) == k1;
+            if (ready) {
+                uint64_t m0 = 0, m1 = 0;
+                if (r0 >= 0) { m0 |= mask[2 * b0]; m1 |= mask[2 * b0 + 1]; }
+                if (r1 >= 0) { m0 |= mask[2 * b1]; m1 |= mask[2 * b1 + 1]; }
+                uint32_t c;
+                if (~m0) c = (uint32_t)__builtin_ctzll(~m0);
+                else if (~m1) c = 64u + (uint32_t)__builtin_ctzll(~m1);
+                else c = 128u + p;
+                S.it_color[it] = c;
+                if (c < 128) {
+                    const uint32_t hi = c >> 6;
+                    const uint64_t bit = 1ull << (c & 63u);
+                    if (r0 >= 0) mask[2 * b0 + hi] |= bit;
+                    if (r1 >= 0) mask[2 * b1 + hi] |= bit;
+                }
+                if (r0 >= 0) st_rel(&count[b0], k0 + 1u);
+                if (r1 >= 0) st_rel(&count[b1], k1 + 1u);
+                p += COLOR_THREADS;
+                spins = 0;
+            } else {
+                // every item's predecessors come first, so some item is always ready
+                if (__hip_atomic_load(&s_abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
+                if (++spins > COLOR_SPIN_LIMIT) {
+                    __hip_atomic_store(&s_abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    S.w_status[w] = 5;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+    };
+    if (5u * nc <= lds_words)
+        run((uint64_t*)smem, smem + 4u * nc, nc, [&](uint32_t r) { return S.cmap[r]; });
+    else
+        run(S.cmask + 2 * (size_t)base, S.g_cnt + base, (uint32_t)D.nbodies, [&](uint32_t r) { return r - base; });
 }
 
 // rank of each item among the items sharing one of its resources: in item
@@ -2928,7 +2979,8 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
         hipLaunchKernelGGL(k_list_rank<false>, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
         tmark(ss, "k_list_rank<false>", st);
         if (sp.any_colored) {
-            hipLaunchKernelGGL(k_color, dim3(S.nworlds), dim3(256), 0, st, S);
+            const size_t lds = S.nworlds <= CHAIN_WIDE_WORLDS ? COLOR_LDS : COLOR_LDS / 4;
+            hipLaunchKernelGGL(k_color, dim3(S.nworlds), dim3(COLOR_THREADS), lds, st, S, (uint32_t)(lds / 4u));
             tmark(ss, "k_color", st);
         }
         if (S.nworlds > 1u) {
@@ -2989,6 +3041,7 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
 void set_solve_smem_limit()
 {
     auto allow = [](const void* f) { (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); };
+    allow((const void*)k_color);
     allow((const void*)k_chain_plan<CHAIN_THREADS>);
     allow((const void*)k_chain_plan<CHAIN_NARROW>);
     allow((const void*)k_chain_run<CHAIN_THREADS, false>);

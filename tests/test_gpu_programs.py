@@ -74,8 +74,11 @@ CASES = {
     "momenta-global-one-wave": (("links", 12, 30, 6), 2, 4, 6, True, 1, 0.0),
     "momenta-global-several": (("heap", 900, 14.0, 5), 2, 4, 3, True, 1, 0.0),
     "momenta-global-warm": (("heap", 300, 9.0, 7), 2, 4, 5, True, 1, 0.8),
-    # 700 contacts a body row in a heap too large for LDS plans and impulses
+    # a heap too large for plans and impulses in LDS
     "heap-6000": (("heap", 6000, 30.0, 8), 1, 2, 2, True, 0, 0.0),
+    # the coloured order, its counters in LDS and in global memory
+    "coloured": (("heap", 900, 14.0, 5), 2, 4, 3, True, 0, 0.0),
+    "coloured-9000": (("heap", 9000, 45.0, 9), 1, 2, 2, True, 0, 0.0),
 }
 
 
@@ -93,6 +96,8 @@ def test_program_matches_oracle(oracle, name):
         apply_scene(ops, e)
         if warm:
             e.set_warm_start(warm)
+        if name.startswith("coloured"):
+            e.set_schedule(1)
     for step in range(steps):
         print(f"{name}: step {step + 1} of {steps}", flush=True)
         assert g.process(DT, sub, iters) == o.process(DT, sub, iters) == 0
