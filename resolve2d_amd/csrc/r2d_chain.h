@@ -228,11 +228,26 @@ struct ChainShared {
     float dt;
     uint32_t free_at, free_words;   // LDS from this word on is the solve's
     uint32_t ready, pairs, live, fix, nslots, failed, taken, entries, queued[3];
+    // a plan that the first chain runs behind: LDS words it keeps, rows it has written (PLANNED: all), and the
+    // waves that have met (waves_meet)
+    uint32_t beside, progress, met;
 };
+constexpr uint32_t PLANNED = 0x80000000u;
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
 {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+__device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
+// waits until `waves` waves of the workgroup have called it for the round-th
+// time (from 1 on): a barrier of some of the waves, which all reach it
+__device__ __forceinline__ void waves_meet(uint32_t* met, uint32_t waves, uint32_t round)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if (lane_id() == 0u) __hip_atomic_fetch_add(met, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (__hip_atomic_load(met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < waves * round)
+        __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 // The arguments of an out-of-line function arrive in vector registers: what is
@@ -315,10 +330,16 @@ __device__ __forceinline__ void plan_put(PLAN& P, const Round& R, uint32_t at)
 // The program of a world run by one wave, planned by one wave without
 // barriers; `ready` items are in the ring.  Returns the rows (0: the ordering
 // data was corrupt) and the entries.
-template <class PLAN>
+// PUBLISH: `progress` counts the rows that other waves may read (a round's
+// stores, three at most, are waited for in the next round).
+template <bool PUBLISH = false, class PLAN>
 __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint32_t nit, uint32_t nj, uint32_t iters,
-                                                uint32_t ready, uint32_t& entries)
+                                                uint32_t ready, uint32_t& entries, uint32_t* progress = nullptr)
 {
+    auto publish = [&](uint32_t rows) {
+        asm volatile("" ::: "memory");
+        if (lane_id() == 0u) __hip_atomic_store(progress, rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
     const uint32_t total = nit * iters;
@@ -337,7 +358,18 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
         count += added - R.taken;
         done += R.taken;
         entry += R.lanes;
+        if constexpr (PUBLISH) {
+            // at most this round's last two stores are under way: the rows before it are written
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0f72);   // vmcnt(2)
+            publish(row);
+        }
         row += 1u;
+    }
+    if constexpr (PUBLISH) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0)
+        publish((done == total ? row : 0u) | PLANNED);
     }
     entries = entry;
     return done == total ? row : 0u;

@@ -1906,7 +1906,8 @@ struct ChainLds {
     LF2 acc;
     // the impulses of n contact points, and a spare one, beside the constants
     __device__ __forceinline__ bool holds(uint32_t n) const { return consts + 2u * (n + 1u) <= rest_words; }
-    __device__ __forceinline__ ChainLds(LU32 smem, uint32_t free_at, uint32_t free_words, uint32_t n_) : n(n_)
+    // beside: words that the plan keeps in front of the constants
+    __device__ __forceinline__ ChainLds(LU32 smem, uint32_t free_at, uint32_t free_words, uint32_t n_, uint32_t beside) : n(n_)
     {
         dcnt = smem;
         doff = smem + n;
@@ -1914,19 +1915,117 @@ struct ChainLds {
         C.m = (LF3)lds;
         C.px = (LF)(lds + 4u * (n + 1u)); C.py = C.px + n; C.ang = C.py + n;
         const uint32_t fixed = (4u * (n + 1u) + 3u * n + 1u) & ~1u;
-        rest = lds + fixed;
-        rest_words = free_words - fixed;
+        rest = lds + fixed + beside;
+        rest_words = free_words - fixed - beside;
         C.mass = (LF)rest; C.inertia = C.mass + n; C.flags = (LU32)(C.inertia + n);
         consts = (3u * n + 1u) & ~1u;
         acc = (LF2)(rest + consts);
     }
 };
 
+// the gap before sub-step s's chain (s == sub_steps: after the last one), bodies
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void chain_bodies(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s, uint32_t off)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const uint32_t sub_steps = uniform(sh.sub_steps);
+    const float sub_dt = sh.dt / (float)sub_steps;
+    const int n = D.nbodies;
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)n, uniform(sh.beside));
+    const ChainBodies& C = L.C;
+    const BodyArrays A = body_arrays(D);
+    s = uniform(s);
+    off = uniform(off);
+    for (int i = (int)(threadIdx.x - off); i < n; i += (int)(T - off)) {
+        BodyIn in{0u, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (s == 0u) {
+            in = BodyIn{A.flags[i], A.mass[i], A.inertia[i], A.fx[i], A.fy[i], A.tq[i]};
+            C.mass[i] = in.mass; C.inertia[i] = in.inertia; C.flags[i] = in.f;
+        } else {
+            in.f = C.flags[i]; in.mass = C.mass[i]; in.inertia = C.inertia[i];
+        }
+        const bool stat = (in.f & BF_STATIC) != 0;
+        BodyState b{C.m[i], C.px[i], C.py[i], C.ang[i]};
+        if (s > 0u && !stat) {
+            body_move(b, in.mass, in.inertia, sub_dt);
+            C.px[i] = b.px; C.py[i] = b.py; C.ang[i] = b.ang;
+        }
+        if (s == sub_steps) {
+            body_done(D, A, i, stat, b);
+        } else {
+            const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
+            C.m[i] = m;
+            if (minus_zero(m)) sh.fix = 1u;
+        }
+    }
+}
+
+// the gap, items: the joints' records, moved contact points, carried impulses
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s, uint32_t off)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M),
+                   base = uniform(sh.base), t = threadIdx.x - uniform(off), stride = (uint32_t)T - uniform(off);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
+    const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
+    u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
+    s = uniform(s);
+    for (uint32_t j = t; j < nj; j += stride) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u, [](uint32_t x) { return x; });
+    const bool in_lds = L.holds(M + uniform(sh.pairs));
+    GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+    if (sh.live)
+        for (uint32_t q = t; q < M; q += stride) {
+            const uint32_t p1 = S.it_k0[ibase + nj + q];
+            point_tgs(S, D, recs, L.C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
+                const uint32_t at = p ? p1 - nj : q;
+                if (in_lds) L.acc[at] = f2v{0.f, 0.f};
+                else accg[at] = f2v{0.f, 0.f};
+            });
+        }
+    if constexpr (WARM) {
+        if (!(D.warm > 0.0f)) return;
+        const size_t cm = S.cap_m;
+        for (uint32_t q = t; q < M; q += stride) {
+            // warm starting: the carried impulse per sub-step joins the accumulators
+            const uint32_t m = mbeg + q, valid = S.m_valid[m];
+            if (!(valid & MV_WARM)) continue;
+            for (uint32_t p = 0; p < 2u; ++p) {
+                if (!(valid & (1u << p))) continue;
+                const f2v add{S.m_pt[(MP_WARM_N * 2 + p) * cm + m], S.m_pt[(MP_WARM_T * 2 + p) * cm + m]};
+                const uint32_t at = p ? S.it_k0[ibase + nj + q] - nj : q;
+                if (in_lds) L.acc[at] = L.acc[at] + add;
+                else accg[at] = accg[at] + add;
+            }
+        }
+    }
+}
+
+// a world's program in memory
+__device__ __forceinline__ ChainProgram chain_program(const StepDev& S, uint32_t ibase, uint32_t kc, uint32_t nslots,
+                                                      uint32_t reps, uint32_t nj, uint32_t M, uint32_t pairs)
+{
+    return ChainProgram{(GCU2)(S.prog_rows + (size_t)ibase * kc), (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc),
+                        (GCU2)(S.prog_slots + (size_t)ibase * kc), (GCU4)(S.recs + (size_t)ibase * 8),
+                        nslots, reps, nj, M + pairs, 2u * kc * (nj + M), 0u};
+}
+
 // The plan, and meanwhile the bodies into LDS and the point records: wave 0
 // plans a world run by one wave while the other waves build; a wider world is
 // planned by all waves, then built by all.
+//
+// Where the plan, the constants and the impulses fit LDS side by side, the
+// other waves also do the first sub-step's bodies and items, and wave 1 then
+// runs its chain behind the planner, FOLLOW_ROWS rows at a time (a row takes
+// the planner 0.46 us and the chain 0.28, so the first chain costs little more
+// than the rows of its last part): returns whether it did.
+constexpr uint32_t FOLLOW_ROWS = 24;
 template <int T, bool WARM>
-__device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
+__device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
 {
     const StepDev& S = *(const StepDev*)uniform_ptr(KS);
     ChainShared& sh = *(ChainShared*)uniform_lds(shl);
@@ -1935,7 +2034,7 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + w);
     const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, kc = S.chain_iters;
     const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
-    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n, 0u);
     const ChainBodies& C = L.C;
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     const uint32_t waves = chain_waves(nit, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS);
@@ -1977,9 +2076,10 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
     if (plan_in_lds) fill(PL); else fill(PG);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
-    // the point that does nothing, after the others (an item slice has an item to spare)
-    if (t < 4u) recs[(size_t)(nit + uniform(sh.pairs)) * 4u + t] = idle_word((int)t);
-    if (t == 0u) G.entries[2u * kc * nit] = nit + uniform(sh.pairs);
+    // the point that does nothing, after the others (an item slice has an item
+    // to spare); by wave 1, whose chain may start without a barrier
+    if (t - 64u < 4u) recs[(size_t)(nit + uniform(sh.pairs)) * 4u + (t - 64u)] = idle_word((int)(t - 64u));
+    if (t == 64u) G.entries[2u * kc * nit] = nit + uniform(sh.pairs);
     auto build = [&](uint32_t t0, uint32_t stride) {
         for (uint32_t i = t0; i < n; i += stride) {
             C.m[i] = f3v{D.mx[i], D.my[i], D.L[i]};
@@ -1992,8 +2092,48 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
             if (f & 2u) sh.fix = 1u;
         }
     };
+    const uint32_t nacc = M + uniform(sh.pairs);
+    const uint32_t plan_words = (plan_lds_words(nit, 1u) + 1u) & ~1u;
+    const bool follow = chain && waves == 1u && plan_in_lds && sh.iters == kc && plan_words < L.rest_words &&
+                        L.consts + 2u * (nacc + 1u) <= L.rest_words - plan_words;
     uint32_t ns = 1u;
-    if (chain && waves > 1u) {
+    if (follow) {
+        sh.beside = plan_words;   // the same from every thread
+        if (t < 64u) {
+            uint32_t entries;
+            ns = plan_single<true>(PL, G, nit, nj, kc, ready, entries, &sh.progress);
+        } else {
+            constexpr uint32_t OTHERS = (uint32_t)T / 64u - 1u;
+            LF2 acc = L.acc + plan_words / 2u;
+            build(t - 64u, T - 64u);
+            for (uint32_t q = t - 64u; q < nacc; q += T - 64u) acc[q] = f2v{0.f, 0.f};
+            chain_bodies<T, WARM>(KS, smem, shl, 0u, 64u);
+            waves_meet(&sh.met, OTHERS, 1u);
+            if (nj || sh.live || (WARM && D.warm > 0.0f)) {
+                chain_items<T, WARM>(KS, smem, shl, 0u, 64u);
+                waves_meet(&sh.met, OTHERS, 2u);
+            }
+            if (t < 128u) {
+                ChainProgram P = chain_program(S, ibase, kc, 0u, 1u, nj, M, uniform(sh.pairs));
+                const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
+                for (uint32_t run = 0u;;) {
+                    const uint32_t p = uniform(__hip_atomic_load(&sh.progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+                    const uint32_t have = p & ~PLANNED, rows = have > run ? have - run : 0u;   // (none of a failed plan)
+                    asm volatile("" ::: "memory");   // the rows are read after their count
+                    if (rows >= FOLLOW_ROWS || ((p & PLANNED) && rows != 0u)) {
+                        P.nslots = rows;
+                        chain_lds<false, WARM, false>(P, C.m, n, acc, fix, sub_dt);
+                        P.rows += rows;
+                        run += rows;
+                    } else if (p & PLANNED) {
+                        break;
+                    } else {
+                        __builtin_amdgcn_s_sleep(4);
+                    }
+                }
+            }
+        }
+    } else if (chain && waves > 1u) {
         ns = plan_in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh)
                          : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
         build(t, T);
@@ -2010,96 +2150,16 @@ __device__ __attribute__((noinline)) void chain_prepare(StepArgs KS, LU32 smem, 
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
     __syncthreads();
+    if (follow) return true;
     // accumulated impulses (normal, tangential) of the contact points, by
     // point index less the joints: in LDS after the constants when they fit
-    const uint32_t nacc = M + uniform(sh.pairs);
     if (L.holds(nacc)) {
         for (uint32_t q = t; q < nacc; q += T) L.acc[q] = f2v{0.f, 0.f};
     } else {
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         for (uint32_t q = t; q < nacc; q += T) accg[q] = f2v{0.f, 0.f};
     }
-}
-
-// the gap before sub-step s's chain (s == sub_steps: after the last one), bodies
-template <int T, bool WARM>
-__device__ __attribute__((noinline)) void chain_bodies(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s)
-{
-    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
-    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
-    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
-    const uint32_t sub_steps = uniform(sh.sub_steps);
-    const float sub_dt = sh.dt / (float)sub_steps;
-    const int n = D.nbodies;
-    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)n);
-    const ChainBodies& C = L.C;
-    const BodyArrays A = body_arrays(D);
-    s = uniform(s);
-    for (int i = (int)threadIdx.x; i < n; i += T) {
-        BodyIn in{0u, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (s == 0u) {
-            in = BodyIn{A.flags[i], A.mass[i], A.inertia[i], A.fx[i], A.fy[i], A.tq[i]};
-            C.mass[i] = in.mass; C.inertia[i] = in.inertia; C.flags[i] = in.f;
-        } else {
-            in.f = C.flags[i]; in.mass = C.mass[i]; in.inertia = C.inertia[i];
-        }
-        const bool stat = (in.f & BF_STATIC) != 0;
-        BodyState b{C.m[i], C.px[i], C.py[i], C.ang[i]};
-        if (s > 0u && !stat) {
-            body_move(b, in.mass, in.inertia, sub_dt);
-            C.px[i] = b.px; C.py[i] = b.py; C.ang[i] = b.ang;
-        }
-        if (s == sub_steps) {
-            body_done(D, A, i, stat, b);
-        } else {
-            const f3v m = body_push<WARM>(A, i, s + 1u == sub_steps, b, in, sub_dt);
-            C.m[i] = m;
-            if (minus_zero(m)) sh.fix = 1u;
-        }
-    }
-}
-
-// the gap, items: the joints' records, moved contact points, carried impulses
-template <int T, bool WARM>
-__device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl, uint32_t s)
-{
-    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
-    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
-    const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M),
-                   base = uniform(sh.base), t = threadIdx.x;
-    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
-    const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
-    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
-    u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
-    s = uniform(s);
-    for (uint32_t j = t; j < nj; j += T) joint_record(recs + (size_t)j * 4u, D.joints[j], D, L.C, s == 0u, [](uint32_t x) { return x; });
-    const bool in_lds = L.holds(M + uniform(sh.pairs));
-    GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
-    if (sh.live)
-        for (uint32_t q = t; q < M; q += T) {
-            const uint32_t p1 = S.it_k0[ibase + nj + q];
-            point_tgs(S, D, recs, L.C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
-                const uint32_t at = p ? p1 - nj : q;
-                if (in_lds) L.acc[at] = f2v{0.f, 0.f};
-                else accg[at] = f2v{0.f, 0.f};
-            });
-        }
-    if constexpr (WARM) {
-        if (!(D.warm > 0.0f)) return;
-        const size_t cm = S.cap_m;
-        for (uint32_t q = t; q < M; q += T) {
-            // warm starting: the carried impulse per sub-step joins the accumulators
-            const uint32_t m = mbeg + q, valid = S.m_valid[m];
-            if (!(valid & MV_WARM)) continue;
-            for (uint32_t p = 0; p < 2u; ++p) {
-                if (!(valid & (1u << p))) continue;
-                const f2v add{S.m_pt[(MP_WARM_N * 2 + p) * cm + m], S.m_pt[(MP_WARM_T * 2 + p) * cm + m]};
-                const uint32_t at = p ? S.it_k0[ibase + nj + q] - nj : q;
-                if (in_lds) L.acc[at] = L.acc[at] + add;
-                else accg[at] = accg[at] + add;
-            }
-        }
-    }
+    return false;
 }
 
 // the impulses -> the step's manifold arrays (what r2d_get_manifolds reports)
@@ -2110,7 +2170,7 @@ __device__ __attribute__((noinline)) void chain_finish(StepArgs KS, LU32 smem, R
     ChainShared& sh = *(ChainShared*)uniform_lds(shl);
     const uint32_t ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj), M = uniform(sh.M);
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
-    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
     const bool in_lds = L.holds(M + uniform(sh.pairs));
     GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
     const size_t cm = S.cap_m;
@@ -2137,28 +2197,26 @@ template <int T, bool WARM>
 __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
 {
     ChainShared& sh = *(ChainShared*)shl;
-    chain_prepare<T, WARM>(KS, smem, shl);
+    const bool first = uniform(chain_prepare<T, WARM>(KS, smem, shl)) != 0u;
     if (sh.failed) return;
     const StepDev& S = *(const StepDev*)KS;
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
     const uint32_t sub_steps = uniform(sh.sub_steps), iters = uniform(sh.iters), nj = uniform(sh.nj);
     const bool any = nj + sh.M > 0u, items = nj || sh.live || (WARM && D.warm > 0.0f);
-    for (uint32_t s = 0;; ++s) {
-        chain_bodies<T, WARM>(KS, smem, shl, s);
+    for (uint32_t s = first ? 1u : 0u;; ++s) {   // the first chain may have run behind the planner
+        chain_bodies<T, WARM>(KS, smem, shl, s, 0u);
         if (s == sub_steps) break;
         __syncthreads();
         if (!any) continue;
         if (items) {
-            chain_items<T, WARM>(KS, smem, shl, s);
+            chain_items<T, WARM>(KS, smem, shl, s, 0u);
             __syncthreads();
         }
         if (iters == 0u) continue;
         const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters;
-        const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies);
+        const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
         const bool in_lds = L.holds(M + uniform(sh.pairs));
-        const ChainProgram G{(GCU2)(S.prog_rows + (size_t)ibase * kc), (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc),
-                             (GCU2)(S.prog_slots + (size_t)ibase * kc), (GCU4)(S.recs + (size_t)ibase * 8),
-                             uniform(sh.nslots), iters / kc, nj, M + uniform(sh.pairs), 2u * kc * (nj + M), 0u};
+        const ChainProgram G = chain_program(S, ibase, kc, uniform(sh.nslots), iters / kc, nj, M, uniform(sh.pairs));
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
@@ -2744,7 +2802,7 @@ void k_fused(StepDev S /* first: chain_world reads it from the argument segment 
             if (t == 0) {
                 const uint32_t keep = fused_keep_words(n);
                 s_chain = ChainShared{w, X.i0, X.m0, nj, M, base, sub_steps, iters, dt, keep, lds_words - keep,
-                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}};
+                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}, 0u, 0u, 0u};
             }
             __syncthreads();
             chain_world<MAXT, WARM>((StepArgs)__builtin_amdgcn_kernarg_segment_ptr(), (LU32)smem,
