@@ -444,7 +444,9 @@ __host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, ui
 
 // ----------------------------------------------------------------- the chain
 // momenta (x, y, angular) of a world's bodies in LDS, 16 bytes a body; the
-// place after the last body takes the writes that are not to be kept
+// SPARE places after the last body take the writes that are not to be kept,
+// one a lane: to one place they would be served one after another
+constexpr uint32_t SPARE = 64;
 typedef float f3v __attribute__((ext_vector_type(3)));
 typedef R2D_LDS f3v* LF3;
 typedef R2D_GLB f3v* GF3;
@@ -453,7 +455,7 @@ struct LdsMomenta {
     uint32_t none;
     __device__ __forceinline__ f3v get(uint32_t i) const { return m[i]; }
     __device__ __forceinline__ void put(uint32_t i, f3v v) const { m[i] = v; }
-    __device__ __forceinline__ void put_if(bool keep, uint32_t i, f3v v) const { m[keep ? i : none] = v; }
+    __device__ __forceinline__ void put_if(bool keep, uint32_t i, f3v v) const { m[keep ? i : none + lane_id()] = v; }
 };
 
 // the same in global memory
@@ -724,30 +726,7 @@ __device__ __forceinline__ void chain_run(ChainProgram G, const ST& st, ACC acc,
         load_rec(1);
         load_entry(batch, 3u, 0);
         __builtin_amdgcn_sched_barrier(0);
-        auto run_slot = [&](uint32_t i, int u) __attribute__((always_inline)) {
-            // this row's LDS reads first: the fetches below are issued while
-            // they are under way (joints read something harmless)
-            const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
-            const uint32_t rc = cnt[u], left = point[u] - nj;
-            const uint32_t ai = left < nacc ? left : nacc;   // joints, and lanes without a point: the spare one
-            const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
-            const f2v old = acc[ai];
-            __builtin_amdgcn_sched_barrier(0);
-            load_rec((u + 2) % 3);
-            load_entry(batch, i, (u + 4) % 3);
-            __builtin_amdgcn_sched_barrier(0);
-            uint32_t fl_a = q0.x, fl_b = q0.y;
-            float bias = asf(q1.y);
-            if (rc & ROW_JOINTS) {
-                asm volatile("");   // one branch for the row: not folded into the lanes' test
-                const bool joint = (q0.x & PR_JOINT) != 0u;
-                if (joint) chain_joint(q0, q1, q2, q3, st, dt);
-                // as a point it does nothing
-                fl_a = joint ? 0u : fl_a;
-                fl_b = joint ? 0u : fl_b;
-                bias = joint ? -1.0f : bias;
-            }
-            chain_contact<WARM>(q0, q1, q2, q3, fl_a, fl_b, bias, st, s1, s2, old, acc + ai, lane, (rc >> 8) & 0xffu, fix);
+        auto wait = [&]() {
             // the next slot reads what this one wrote
             if constexpr (MULTI) {
                 if constexpr (LDS_ONLY) {
@@ -762,6 +741,42 @@ __device__ __forceinline__ void chain_run(ChainProgram G, const ST& st, ACC acc,
             } else {
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
             }
+        };
+        auto run_slot = [&](uint32_t i, int u) __attribute__((always_inline)) {
+            // this row's LDS reads first: the fetches below are issued while
+            // they are under way (joints read something harmless)
+            const u4v q0 = rec[u][0], q1 = rec[u][1], q2 = rec[u][2], q3 = rec[u][3];
+            const uint32_t rc = cnt[u], left = point[u] - nj;
+            const uint32_t ai = left < nacc ? left : nacc;   // joints, and lanes without a point: the spare one
+            const f3v s1 = st.get(q0.x & PR_INDEX), s2 = st.get(q0.y & PR_INDEX);
+            const f2v old = acc[ai];
+            __builtin_amdgcn_sched_barrier(0);
+            load_rec((u + 2) % 3);
+            load_entry(batch, i, (u + 4) % 3);
+            __builtin_amdgcn_sched_barrier(0);
+            auto work = [&]() __attribute__((always_inline)) {
+                uint32_t fl_a = q0.x, fl_b = q0.y;
+                float bias = asf(q1.y);
+                if (rc & ROW_JOINTS) {
+                    asm volatile("");   // one branch for the row: not folded into the lanes' test
+                    const bool joint = (q0.x & PR_JOINT) != 0u;
+                    if (joint) chain_joint(q0, q1, q2, q3, st, dt);
+                    // as a point it does nothing
+                    fl_a = joint ? 0u : fl_a;
+                    fl_b = joint ? 0u : fl_b;
+                    bias = joint ? -1.0f : bias;
+                }
+                chain_contact<WARM>(q0, q1, q2, q3, fl_a, fl_b, bias, st, s1, s2, old, acc + ai, lane, (rc >> 8) & 0xffu, fix);
+            };
+            if constexpr (MULTI) {
+                if (rc & 0xffu) {   // this wave has a row in the slot
+                    asm volatile("");
+                    work();
+                }
+            } else {
+                work();
+            }
+            wait();
         };
         // whole rounds of the three buffers, a batch of them at a time, then
         // what is left: a way out of the middle of the loop would make its

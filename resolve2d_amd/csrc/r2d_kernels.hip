@@ -1913,8 +1913,8 @@ struct ChainLds {
         doff = smem + n;
         LU32 lds = smem + free_at;
         C.m = (LF3)lds;
-        C.px = (LF)(lds + 4u * (n + 1u)); C.py = C.px + n; C.ang = C.py + n;
-        const uint32_t fixed = (4u * (n + 1u) + 3u * n + 1u) & ~1u;
+        C.px = (LF)(lds + 4u * (n + SPARE)); C.py = C.px + n; C.ang = C.py + n;
+        const uint32_t fixed = (4u * (n + SPARE) + 3u * n + 1u) & ~1u;
         rest = lds + fixed + beside;
         rest_words = free_words - fixed - beside;
         C.mass = (LF)rest; C.inertia = C.mass + n; C.flags = (LU32)(C.inertia + n);
@@ -2450,7 +2450,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     const WorldDev& D = S.worlds[w];
     const WorldChain W = S.w_chain[w];
     const uint32_t t = threadIdx.x, nj = (uint32_t)D.njoints, M = nit - nj, mbeg = S.w_man_begin[w], base = D.body_base;
-    const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + 1u);
+    const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + SPARE);
     const bool m_lds = (uint32_t)D.nbodies <= lds_nmax && mwords <= lds_words;
     const bool a_lds = m_lds && mwords + 2u * (nacc + 1u) <= lds_words;
     const LF3 m = (LF3)(LU32)smem;
