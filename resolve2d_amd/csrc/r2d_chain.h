@@ -86,11 +86,11 @@ __device__ __forceinline__ uint32_t asu(float x) { return __float_as_uint(x); }
 // iteration off.  An item with one ordering body releases the spare item (the
 // last place), which never becomes ready.
 //
-// Planning state in LDS, 4.5 words an item: succ (both successors, 15 bits
-// each; bit 31: one ordering body), state, second (second point of a pair,
-// counted from 1) and a ring of ready items (x: item | second << 16, y: succ).
-// Worlds that do not fit, or with more items than 15 bits, keep the same in
-// global memory (PlanGlb).
+// Planning state in LDS, 5 words an item: the entry (x: item | second << 16,
+// y: both successors, 15 bits each, SINGLE when there is one ordering body; the
+// second point of a pair counts from 1), the state, and a ring of the ready
+// items' entries, which are copied as they are.  Worlds that do not fit, or
+// with more items than 15 bits, keep the same in global memory (PlanGlb).
 constexpr uint32_t PLAN_MAX_ITEMS = 0x7ffe;
 constexpr uint32_t STATE_BODY = 1u << 16;
 
@@ -103,48 +103,40 @@ __host__ __device__ constexpr uint32_t plan_ring(uint32_t nit, uint32_t waves) {
 // LDS words of PlanLds
 __host__ __device__ constexpr uint32_t plan_lds_words(uint32_t nit, uint32_t waves)
 {
-    return 2u * plan_ring(nit, waves) + 2u * (nit + 1u) + (nit + 2u) / 2u;
+    return 2u * plan_ring(nit, waves) + 3u * (nit + 1u);
 }
 // a state that made its item ready when a release found it
 __device__ __forceinline__ bool state_ready(uint32_t old) { return old - (STATE_BODY + 1u) < STATE_BODY - 1u; }
 
 struct PlanLds {
-    LU32 succ, state;
-    LU16 second;
-    LU2 ring;
+    typedef u2v Raw;
+    LU2 ring, items;
+    LU32 state;
     uint32_t ring_n;
 
     __device__ __forceinline__ PlanLds(LU32 p, uint32_t nit, uint32_t waves)
     {
         ring_n = plan_ring(nit, waves);
         ring = (LU2)p;                      // p is 8-byte aligned
-        succ = p + 2u * ring_n;
-        state = succ + nit + 1u;
-        second = (LU16)(state + nit + 1u);
+        items = ring + ring_n;
+        state = (LU32)(items + nit + 1u);
     }
-    static __device__ __forceinline__ uint32_t pack(uint32_t s0, uint32_t s1)
+    static __device__ __forceinline__ PlanEntry unpack(u2v v)
     {
-        return s0 | ((s1 & 0x7fffu) << 16) | (s1 & SINGLE);
+        return PlanEntry{v.x & 0xffffu, v.x >> 16, v.y & 0x7fffu, ((v.y >> 16) & 0x7fffu) | (v.y & SINGLE)};
     }
-    static __device__ __forceinline__ PlanEntry unpack(uint32_t x, uint32_t y)
+    static __device__ __forceinline__ u2v pack(const PlanEntry& e)
     {
-        return PlanEntry{x & 0xffffu, x >> 16, y & 0x7fffu, ((y >> 16) & 0x7fffu) | (y & SINGLE)};
+        return u2v{e.item | (e.second << 16), e.s0 | ((e.s1 & 0x7fffu) << 16) | (e.s1 & SINGLE)};
     }
     __device__ __forceinline__ void init(uint32_t j, uint32_t s0, uint32_t s1, uint32_t st, uint32_t sec)
     {
-        succ[j] = pack(s0, s1);
+        items[j] = pack(PlanEntry{j, sec, s0, s1});
         state[j] = st;
-        second[j] = (uint16_t)sec;
     }
-    __device__ __forceinline__ PlanEntry read(uint32_t at) const
-    {
-        const u2v v = ring[at];
-        return unpack(v.x, v.y);
-    }
-    __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e)
-    {
-        ring[at] = u2v{e.item | (e.second << 16), pack(e.s0, e.s1)};
-    }
+    __device__ __forceinline__ Raw read(uint32_t at) const { return ring[at]; }
+    __device__ __forceinline__ void push(uint32_t at, Raw e) { ring[at] = e; }
+    __device__ __forceinline__ Raw entry(uint32_t s) const { return items[s]; }
     __device__ __forceinline__ void rearm(uint32_t j, uint32_t by)
     {
         __hip_atomic_fetch_add(&state[j], by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -153,12 +145,14 @@ struct PlanLds {
     {
         return __hip_atomic_fetch_sub(&state[s], STATE_BODY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    __device__ __forceinline__ PlanEntry entry(uint32_t s) const { return unpack(s | ((uint32_t)second[s] << 16), succ[s]); }
 };
 
 // the same in global memory: items (succ 0, succ 1, state, second), ring of
 // ready items (item, second, succ 0, succ 1)
 struct PlanGlb {
+    typedef PlanEntry Raw;
+    static __device__ __forceinline__ PlanEntry unpack(const PlanEntry& e) { return e; }
+    static __device__ __forceinline__ PlanEntry pack(const PlanEntry& e) { return e; }
     GU4 items, ring;
     uint32_t ring_n;
 
@@ -269,55 +263,65 @@ __device__ __forceinline__ P uniform_lds(P p)
 // `entry0` with pairs in the lower lanes and releases their successors
 // (plan_run: the released items are in e0 / e1, r0 / r1 whether the lane
 // released one).
+template <class PLAN>
 struct Round {
+    typename PLAN::Raw self, e0, e1;
     uint32_t taken, lanes, word;   // items, points, second word of the row
     bool take, left;               // this lane's item is in the row / did not fit it
     uint32_t below, pairs;         // pairs in lower lanes / in the row
-    PlanEntry self, e0, e1;
     bool r0, r1;
 };
 
 template <class PLAN>
-__device__ __forceinline__ Round plan_take(PLAN& P, uint32_t first, uint32_t avail, uint32_t lane, uint32_t nj)
+__device__ __forceinline__ Round<PLAN> plan_take(PLAN& P, uint32_t first, uint32_t avail, uint32_t lane, uint32_t nj)
 {
-    Round R;
+    Round<PLAN> R;
     const bool act = lane < avail;
     uint32_t at = first + (act ? lane : 0u);
     at = at < at - P.ring_n ? at : at - P.ring_n;   // at - ring_n wraps round to a large number below the ring's end
     R.self = P.read(at);
-    const bool pair = act && R.self.second != 0u;
+    const PlanEntry e = PLAN::unpack(R.self);
+    const bool pair = act && e.second != 0u;
     R.below = lanes_below(__ballot(pair));
     R.take = act && lane + 1u + R.below + (pair ? 1u : 0u) <= 64u;   // lanes used through this item
     const uint64_t tm = __ballot(R.take);
     R.taken = (uint32_t)__popcll(tm);
     R.pairs = (uint32_t)__popcll(tm & __ballot(pair));
     R.lanes = R.taken + R.pairs;
-    R.word = R.lanes | (R.pairs << 9) | (__ballot(R.take && R.self.item < nj) ? ROW_JOINTS : 0u);
+    R.word = R.lanes | (R.pairs << 9) | (__ballot(R.take && e.item < nj) ? ROW_JOINTS : 0u);
     R.left = act && !R.take;
     return R;
 }
 
-template <class PLAN>
-__device__ __forceinline__ void plan_run(PLAN& P, Round& R, GU32 entries, uint32_t entry0, uint32_t nit, uint32_t lane)
+// entry0: a function, called once the releases are under way (the answer of
+// another LDS operation is waited for with theirs)
+template <class PLAN, class ENTRY0>
+__device__ __forceinline__ void plan_run(PLAN& P, Round<PLAN>& R, GU32 entries, ENTRY0 entry0, uint32_t nit, uint32_t lane)
 {
     R.r0 = R.r1 = false;
+    const PlanEntry e = PLAN::unpack(R.self);
+    uint32_t o0 = 0u, o1 = 0u;
     if (R.take) {
-        const uint32_t j = R.self.item, s0 = R.self.s0, s1 = R.self.s1 & ~SINGLE;
-        P.rearm(j, (R.self.s1 & SINGLE ? STATE_BODY : 2u * STATE_BODY) - 1u);
-        const uint32_t o0 = P.release(s0), o1 = P.release(s1);
-        R.e0 = P.entry(s0);
+        const uint32_t s1 = e.s1 & ~SINGLE;
+        P.rearm(e.item, (e.s1 & SINGLE ? STATE_BODY : 2u * STATE_BODY) - 1u);
+        o0 = P.release(e.s0);
+        o1 = P.release(s1);
+        R.e0 = P.entry(e.s0);
         R.e1 = P.entry(s1);
-        const bool pair = R.self.second != 0u;
-        const uint32_t pos = entry0 + (pair ? 2u * R.below : 2u * R.pairs + (lane - R.below));
-        entries[pos] = j;
-        if (pair) entries[pos + 1u] = nit + R.self.second - 1u;
+    }
+    const uint32_t first = entry0();
+    if (R.take) {
+        const bool pair = e.second != 0u;
+        const uint32_t pos = first + (pair ? 2u * R.below : 2u * R.pairs + (lane - R.below));
+        entries[pos] = e.item;
+        if (pair) entries[pos + 1u] = nit + e.second - 1u;
         R.r0 = state_ready(o0);
         R.r1 = state_ready(o1);
     }
 }
 
 template <class PLAN>
-__device__ __forceinline__ void plan_put(PLAN& P, const Round& R, uint32_t at)
+__device__ __forceinline__ void plan_put(PLAN& P, const Round<PLAN>& R, uint32_t at)
 {
     const uint64_t m0 = __ballot(R.r0), m1 = __ballot(R.r1), m2 = __ballot(R.left);
     const uint32_t c0 = (uint32_t)__popcll(m0), c2 = (uint32_t)__popcll(m2);
@@ -344,10 +348,10 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
     uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
     const uint32_t total = nit * iters;
     while (done < total && count) {
-        Round R = plan_take(P, head, count < 64u ? count : 64u, lane, nj);
+        Round<PLAN> R = plan_take(P, head, count < 64u ? count : 64u, lane, nj);
         R.left = false;                  // stays at the head of the ring
         if (lane == 0) G.rows[row] = u2v{entry, R.word};
-        plan_run(P, R, G.entries, entry, nit, lane);
+        plan_run(P, R, G.entries, [&]() { return entry; }, nit, lane);
         uint32_t tail = head + count;
         if (tail >= P.ring_n) tail -= P.ring_n;
         plan_put(P, R, tail);
@@ -400,15 +404,14 @@ __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32
             const uint32_t rest = count - 64u * wv;
             uint32_t first = head + 64u * wv;
             if (first >= P.ring_n) first -= P.ring_n;
-            Round R = plan_take(P, first, rest < 64u ? rest : 64u, lane, nj);
+            Round<PLAN> R = plan_take(P, first, rest < 64u ? rest : 64u, lane, nj);
             uint32_t e0 = 0u;
             if (lane == 0) {
                 e0 = __hip_atomic_fetch_add(&sh.entries, R.lanes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_fetch_add(&sh.taken, R.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                G.rows[row + wv] = u2v{e0, R.word};
             }
-            e0 = uniform(e0);
-            plan_run(P, R, G.entries, e0, nit, lane);
+            plan_run(P, R, G.entries, [&]() { return e0 = uniform(e0); }, nit, lane);
+            if (lane == 0) G.rows[row + wv] = u2v{e0, R.word};
             const uint32_t add = (uint32_t)(__popcll(__ballot(R.r0)) + __popcll(__ballot(R.r1)) + __popcll(__ballot(R.left)));
             uint32_t at = 0u;
             if (lane == 0)

@@ -2069,7 +2069,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
             P.init(j, s0, s1, need * STATE_BODY + kc, sec);
             if (need == 0u)
                 P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
-                       PlanEntry{j, sec, s0, s1});
+                       P.pack(PlanEntry{j, sec, s0, s1}));
         }
         if (t == 0u) P.init(nit, nit, nit | SINGLE, 0u, 0u);   // the spare item: no iterations, never ready
     };
@@ -2341,7 +2341,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
             if (init) P.init(j, v.x, v.y, v.z, v.w);
             if (v.z < STATE_BODY)
                 P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
-                       PlanEntry{j, v.w, v.x, v.y});
+                       P.pack(PlanEntry{j, v.w, v.x, v.y}));
         }
         if (t == 0u) P.init(nit, nit, nit | SINGLE, 0u, 0u);   // the spare item: no iterations, never ready
     };
