@@ -24,6 +24,8 @@ FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-fvisibility=hidden", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result", "-Xarch_device", "-mllvm=-amdgpu-opt-vgpr-liverange=0",
+    # loops of one wave start at a cache line (20-row pyramid step 261 -> 256 us, 1,024 worlds 27.7 -> 27.3 ms)
+    "-Xarch_device", "-mllvm=-align-all-nofallthru-blocks=6",
 ]
 
 

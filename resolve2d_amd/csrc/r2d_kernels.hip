@@ -2530,311 +2530,491 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         for (uint32_t q = t; q < nacc; q += T) accg[q] = acc[q];
 }
 
+// ------------------------------------------- the other parts of a fused step
+// Like the solve, each a function of its own that reads the argument block and
+// the world's descriptor through the constant address space: inlined together
+// they held 269 scalar registers' worth in spills and, at four workgroups a CU,
+// 80 vector registers.
+struct FusedShared {
+    uint32_t w, lds_words, err, slot;
+    uint32_t E, R, M;
+    WorldScratch X;
+    uint32_t sm[16];
+};
+
+template <int T>
+struct FusedView {
+    const StepDev& S;
+    const WorldDev& D;
+    uint32_t &err, *s_sm;
+    uint32_t w, n, tb, base, nj, t, lds_words, E, R, M;
+    WorldScratch X;
+    FusedLds L;
+    PairCache P;
+    // the entries' buckets and the bucket members are read in serial loops: in
+    // LDS after the pair cache when they fit (E is about 1.5 n for bodies up to
+    // a cell wide)
+    uint32_t *ent_body, *ecnt, *ent_bkt, *items, *sorted;   // ecnt: raw candidates per entry -> offsets
+    uint4* cand;
+    uint32_t* cflag;   // collides per candidate -> manifold offsets
+    __device__ __forceinline__ FusedView(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+        : S(*(const StepDev*)uniform_ptr(KS)),
+          D(*(const WorldDev*)(WorldArgs)(((const StepDev*)uniform_ptr(KS))->worlds + uniform(((FusedShared*)fsl)->w))),
+          err(((FusedShared*)uniform_lds(fsl))->err), s_sm(((FusedShared*)uniform_lds(fsl))->sm)
+    {
+        const FusedShared& fs = *(FusedShared*)uniform_lds(fsl);
+        w = uniform(fs.w);
+        lds_words = uniform(fs.lds_words);
+        E = uniform(fs.E); R = uniform(fs.R); M = uniform(fs.M);
+        X.e0 = uniform(fs.X.e0); X.r0 = uniform(fs.X.r0); X.m0 = uniform(fs.X.m0); X.i0 = uniform(fs.X.i0);
+        n = (uint32_t)D.nbodies; tb = D.table; base = D.body_base; nj = (uint32_t)D.njoints;
+        t = threadIdx.x;
+        L = fused_carve((uint32_t*)uniform_lds(smem), n, tb);
+        P = pair_cache(L.pairs, n);
+        ent_body = S.ent_body + X.e0;
+        ecnt = S.ent_cnt + X.e0;
+        const bool e_lds = 3 * (size_t)E <= (size_t)(lds_words - fused_front_words(n, tb) - PAIR_CACHE_WORDS * n);
+        uint32_t* e_free = L.pairs + PAIR_CACHE_WORDS * n;
+        ent_bkt = e_lds ? e_free : S.ent_bkt + X.e0;
+        items = e_lds ? e_free + E : S.bkt_items + X.e0;
+        sorted = e_lds ? e_free + 2 * E : S.bkt_sorted + X.e0;
+        cand = S.cand + X.r0;
+        cflag = S.cand_flag + X.r0;
+    }
+};
+
+// broadphase, per body (k_prep); returns the cell entries
+template <int T>
+__device__ __attribute__((noinline)) uint32_t fused_cells(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const StepDev& S = V.S;
+    const WorldDev& D = V.D;
+    const uint32_t n = V.n, base = V.base, t = V.t;
+    const FusedLds& L = V.L;
+    const PairCache& P = V.P;
+    uint32_t* const s_sm = V.s_sm;
+    // stale AABBs and flags in LDS for the pair filters below
+    for (uint32_t i = t; i < n; i += T) {
+        const Prep o = prep_body(D, i);
+        P.ax[i] = D.ax[i]; P.ay[i] = D.ay[i]; P.ahw[i] = D.ahw[i]; P.ahh[i] = D.ahh[i];
+        P.flags[i] = D.flags[i];
+        L.cc[i] = o.c;
+        L.cs[i] = o.s;
+        S.sflag[base + i] = o.res;
+        if (o.err) atomicOr(&V.err, o.err == WS_NONFINITE ? 2u : 1u);
+        if (!o.err && o.ncell) { S.cx0[base + i] = o.x0; S.cy0[base + i] = o.y0; S.cnx[base + i] = o.nx; }
+        L.coff[i] = o.ncell;
+    }
+    __syncthreads();
+    return group_scan(L.coff, n, s_sm);
+}
+
+// cell entries and buckets (k_entries .. k_bucket_rank)
+template <int T>
+__device__ __attribute__((noinline)) void fused_buckets(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const StepDev& S = V.S;
+    const uint32_t n = V.n, tb = V.tb, base = V.base, t = V.t, E = V.E;
+    const FusedLds& L = V.L;
+    uint32_t *const ent_body = V.ent_body, *const ent_bkt = V.ent_bkt, *const items = V.items, *const sorted = V.sorted, *const s_sm = V.s_sm;
+    for (uint32_t b = t; b <= tb; b += T) {
+        L.boff[b] = 0u;
+        if (b < tb) L.bfill[b] = 0u;
+    }
+    __syncthreads();
+    // cell entries and bucket occupancy (k_entries)
+    for (uint32_t e = t; e < E; e += T) {
+        uint32_t i = upper_idx(L.coff, n, e);
+        uint32_t k = e - L.coff[i];
+        uint32_t nx = S.cnx[base + i];
+        int64_t yi = S.cy0[base + i] + (int64_t)(k / nx);
+        int64_t xi = S.cx0[base + i] + (int64_t)(k % nx);
+        uint32_t b = (uint32_t)cell_hash((uint64_t)tb, xi, yi);
+        ent_body[e] = i;
+        ent_bkt[e] = b;
+        atomicAdd(&L.boff[b], 1u);
+    }
+    __syncthreads();
+    group_scan(L.boff, tb, s_sm);
+    // bucket members (k_bucket_fill), then in descending slot with a
+    // body's repeats adjacent (k_bucket_rank)
+    for (uint32_t e = t; e < E; e += T) {
+        uint32_t b = ent_bkt[e];
+        uint32_t pos = atomicAdd(&L.bfill[b], 1u);
+        items[L.boff[b] + pos] = ent_body[e];
+    }
+    __syncthreads();
+    for (uint32_t e = t; e < E; e += T) {
+        uint32_t a = ent_body[e], b = ent_bkt[e];
+        uint32_t o = L.boff[b], c = L.boff[b + 1] - o;
+        uint32_t greater, same;
+        bucket_rank_of(items + o, c, a, greater, same);
+        uint32_t dup = 0;
+        if (same > 1)
+            for (uint32_t x = L.coff[a]; x < e; ++x) dup += ent_bkt[x] == b;
+        sorted[o + greater + dup] = a;
+    }
+    __syncthreads();
+}
+
+template <int T>
+__device__ __attribute__((noinline)) uint32_t fused_count(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const uint32_t t = V.t, E = V.E;
+    const FusedLds& L = V.L;
+    const PairCache& P = V.P;
+    uint32_t *const ent_body = V.ent_body, *const ecnt = V.ecnt, *const ent_bkt = V.ent_bkt, *const items = V.items, *const sorted = V.sorted, *const s_sm = V.s_sm;
+    // raw candidates per entry: distinct bucket members above the entry's
+    // body (k_ent_cnt) that pass the both-static and AABB filters; the
+    // passing members among the first 32 as a mask (in `items`, whose
+    // bucket lists are no longer read)
+    for (uint32_t e = t; e < E; e += T) {
+        const uint32_t a = ent_body[e], b = ent_bkt[e];
+        const uint32_t o = L.boff[b], c = L.boff[b + 1] - o;
+        uint32_t q, mask;
+        entry_candidates(P, a, sorted + o, c, q, mask);
+        ecnt[e] = q;
+        items[e] = mask;
+    }
+    __syncthreads();
+    return group_scan(ecnt, E, s_sm);
+}
+
+template <int T>
+__device__ __attribute__((noinline)) void fused_emit(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const uint32_t t = V.t, E = V.E;
+    const FusedLds& L = V.L;
+    const PairCache& P = V.P;
+    uint32_t *const ent_body = V.ent_body, *const ecnt = V.ecnt, *const ent_bkt = V.ent_bkt, *const items = V.items, *const sorted = V.sorted;
+    uint4* const cand = V.cand;
+    // raw candidates in query order (k_cand_emit)
+    for (uint32_t e = t; e < E; e += T) {
+        uint32_t a = ent_body[e], b = ent_bkt[e];
+        uint32_t o = L.boff[b];
+        uint32_t ro = ecnt[e], c = ecnt[e + 1] - ro;
+        uint32_t k = e - L.coff[a];
+        uint32_t q = 0;
+        for (uint32_t mask = items[e]; mask; mask &= mask - 1u, ++q)
+            cand[ro + q] = make_uint4(a, sorted[o + (uint32_t)__builtin_ctz(mask)], k, 0u);
+        for (uint32_t j = 32; q < c; ++j) {
+            const uint32_t bj = sorted[o + j];
+            if (bj == sorted[o + j - 1] || !pair_passes(P, a, bj)) continue;
+            cand[ro + q] = make_uint4(a, bj, k, 0u);
+            ++q;
+        }
+    }
+    __syncthreads();
+}
+
+template <int T>
+__device__ __attribute__((noinline)) uint32_t fused_narrow(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const WorldDev& D = V.D;
+    const uint32_t t = V.t, R = V.R;
+    const FusedLds& L = V.L;
+    uint32_t *const ent_bkt = V.ent_bkt, *const cflag = V.cflag, *const s_sm = V.s_sm;
+    uint4* const cand = V.cand;
+    // ---- narrowphase (k_narrow): the collision overwrites its candidate
+    // (partner, face id | ref-is-a, normal)
+    for (uint32_t q = t; q < R; q += T) {
+        const uint4 cq = cand[q];
+        const uint32_t a = cq.x, b = cq.y;
+        uint32_t info = 0;
+        float nx = 0.f, ny = 0.f;
+        bool hit = narrow_pair_call(D, a, b, cq.z, ent_bkt + L.coff[a], ent_bkt + L.coff[b],
+                                     L.coff[b + 1] - L.coff[b], L.cc[a], L.cs[a], L.cc[b], L.cs[b], info, nx, ny);
+        cflag[q] = hit ? 1u : 0u;
+        if (hit) cand[q] = make_uint4(a | (b << 16), info, __float_as_uint(nx), __float_as_uint(ny));
+    }
+    __syncthreads();
+    return group_scan(cflag, R, s_sm);
+}
+
+template <int T>
+__device__ __attribute__((noinline)) void fused_contacts(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const StepDev& S = V.S;
+    const WorldDev& D = V.D;
+    const uint32_t n = V.n, base = V.base, nj = V.nj, t = V.t, R = V.R;
+    const FusedLds& L = V.L;
+    const WorldScratch& X = V.X;
+    uint32_t* const cflag = V.cflag;
+    uint4* const cand = V.cand;
+    // contact points (k_man_build), manifolds in discovery order
+    for (uint32_t q = t; q < R; q += T) {
+        const uint32_t mi = cflag[q];
+        if (cflag[q + 1] == mi) continue;
+        const uint4 x = cand[q];
+        const uint32_t a = x.x & 0xffffu, b = x.x >> 16;
+        man_build_one(S, D, D, X.m0 + mi, base, a, b, x.y, mk(__uint_as_float(x.z), __uint_as_float(x.w)), L.cc[a],
+                      L.cs[a], L.cc[b], L.cs[b]);
+    }
+    // ---- schedule: distance / offset joints make both bodies ordering (k_joint_mark)
+    for (uint32_t j = t; j < nj; j += T) {
+        const Joint& J = D.joints[j];
+        if (J.type <= 1) {
+            if (J.s1 >= 0) atomicOr(&S.sflag[base + J.s1], SF_RESOURCE);
+            if (J.s2 >= 0) atomicOr(&S.sflag[base + J.s2], SF_RESOURCE);
+        }
+    }
+    for (uint32_t i = t; i < n; i += T) { L.dcnt[i] = 0u; L.dfill[i] = 0u; }
+    __syncthreads();
+}
+
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void fused_schedule(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl, uint32_t sub_steps)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const StepDev& S = V.S;
+    const WorldDev& D = V.D;
+    const uint32_t n = V.n, base = V.base, nj = V.nj, t = V.t, M = V.M;
+    const FusedLds& L = V.L;
+    const WorldScratch& X = V.X;
+    uint32_t* const s_sm = V.s_sm;
+    const uint32_t nit = nj + M;
+    // items: joints, then manifolds, with their ordering bodies (k_items_*)
+    for (uint32_t j = t; j < nit; j += T) {
+        int32_t r0 = -1, r1 = -1;
+        if (j < nj) {
+            const Joint& J = D.joints[j];
+            r0 = J.s1 >= 0 ? (int32_t)(base + J.s1) : -1;
+            if (J.type <= 1 && J.s2 >= 0 && J.s2 != J.s1) r1 = (int32_t)(base + J.s2);
+        } else {
+            const uint32_t m = X.m0 + (j - nj);
+            const uint32_t ref = S.m_ref[m], inc = S.m_inc[m];
+            r0 = (S.sflag[ref] & SF_RESOURCE) ? (int32_t)ref : -1;
+            r1 = (S.sflag[inc] & SF_RESOURCE) ? (int32_t)inc : -1;
+        }
+        S.it_r0[X.i0 + j] = r0;
+        S.it_r1[X.i0 + j] = r1;
+        if (r0 >= 0) atomicAdd(&L.dcnt[r0 - (int32_t)base], 1u);
+        if (r1 >= 0) atomicAdd(&L.dcnt[r1 - (int32_t)base], 1u);
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += T) L.doff[i] = L.dcnt[i];
+    __syncthreads();
+    group_scan(L.doff, n, s_sm);
+    // per-body item lists (k_list_fill), ranks in item order (k_list_rank).
+    // When the lists fit LDS behind the items per body (the cell, trig,
+    // bucket and pair arrays are dead after the contacts), they are filled there in any
+    // order and each entry then finds its rank by counting the smaller
+    // entries of its body's list (independent LDS reads) and goes to that
+    // place of the global lists; else they are filled in global memory and
+    // sorted per body.
+    const uint32_t lds_words = V.lds_words;
+    uint32_t* const lists = S.lists + 2 * (size_t)X.i0;
+    uint32_t* const ul = L.coff;
+    const bool lds_lists = L.doff[n] <= lds_words - (3u * n + 1u);
+    uint32_t* const fill = lds_lists ? ul : lists;
+    for (uint32_t j = t; j < nit; j += T) {
+        const int32_t r0 = S.it_r0[X.i0 + j], r1 = S.it_r1[X.i0 + j];
+        if (r0 >= 0) {
+            const uint32_t x = (uint32_t)r0 - base;
+            fill[L.doff[x] + atomicAdd(&L.dfill[x], 1u)] = j * 2u;
+        }
+        if (r1 >= 0) {
+            const uint32_t x = (uint32_t)r1 - base;
+            fill[L.doff[x] + atomicAdd(&L.dfill[x], 1u)] = j * 2u + 1u;
+        }
+    }
+    __syncthreads();
+    if (lds_lists) {
+        for (uint32_t j = t; j < nit; j += T) {
+#pragma unroll
+            for (uint32_t side = 0; side < 2; ++side) {
+                const int32_t r = side ? S.it_r1[X.i0 + j] : S.it_r0[X.i0 + j];
+                if (r < 0) continue;
+                const uint32_t x = (uint32_t)r - base, o = L.doff[x];
+                const uint32_t v = j * 2u + side;
+                const uint32_t rank = count_below(ul + o, L.dcnt[x], v);
+                lists[o + rank] = v;
+                if (side) S.it_k1[X.i0 + j] = rank; else S.it_k0[X.i0 + j] = rank;
+            }
+        }
+    } else {
+        for (uint32_t x = t; x < n; x += T) {
+            uint32_t* l = lists + L.doff[x];
+            const uint32_t c = L.dcnt[x];
+            for (uint32_t i = 1; i < c; ++i) {
+                uint32_t v = l[i];
+                uint32_t j = i;
+                while (j > 0 && l[j - 1] > v) { l[j] = l[j - 1]; --j; }
+                l[j] = v;
+            }
+            for (uint32_t p = 0; p < c; ++p) {
+                uint32_t v = l[p];
+                if (v & 1u) S.it_k1[X.i0 + (v >> 1)] = p; else S.it_k0[X.i0 + (v >> 1)] = p;
+            }
+        }
+    }
+    __syncthreads();
+    if (WARM && D.warm > 0.0f) {
+        // warm starting: match last step's manifolds, then each body's carried impulse
+        for (uint32_t q = t; q < M; q += T) warm_match(S, D, X.m0 + q, base, sub_steps);
+        __syncthreads();
+        for (uint32_t x = t; x < n; x += T) warm_body_sum(S, D, lists + L.doff[x], L.dcnt[x], x, 0u, nj, X.m0);
+        __syncthreads();
+    }
+}
+
+// Room for the step's entries (stage 0), raw candidates (1) and manifolds and
+// items (2; the counts not known yet are 0): a slice that is too small is replaced, or the world stops before its state changes.
+// The counts are then what the parts read.
+template <int T>
+__device__ __attribute__((noinline)) bool fused_room(StepArgs KS, R2D_LDS FusedShared* fsl, uint32_t E, uint32_t R, uint32_t M,
+                                                     uint32_t stage)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    FusedShared& fs = *(FusedShared*)uniform_lds(fsl);
+    E = uniform(E); R = uniform(R); M = uniform(M); stage = uniform(stage);
+    const uint32_t w = uniform(fs.w), nit = (uint32_t)S.worlds[w].njoints + M;
+    WorldScratch X = fs.X;
+    const bool fits = stage == 0u ? E <= X.ecap : stage == 1u ? R <= X.rcap : M <= X.mcap && nit <= X.icap;
+    bool ok = true;
+    if (!uniform(fits)) {
+        if (stage == 0u) ok = fused_grow(S, w, X, 0, E, fs.slot);
+        else if (stage == 1u) ok = fused_grow(S, w, X, 1, R, fs.slot);
+        else ok = (M <= X.mcap || fused_grow(S, w, X, 2, M, fs.slot)) && (nit <= X.icap || fused_grow(S, w, X, 3, nit, fs.slot));
+        if (!ok) fused_overflow(S, w, E, R, M, stage == 2u ? nit : 0u);
+    }
+    __syncthreads();   // every thread has read the slices
+    if (threadIdx.x == 0) {
+        fs.E = E; fs.R = R; fs.M = M;
+        fs.X = X;
+    }
+    __syncthreads();
+    return ok;
+}
+
+// the end of a step: warm-start tables, counts
+template <int T, bool WARM>
+__device__ __attribute__((noinline)) void fused_done(StepArgs KS, LU32 smem, R2D_LDS FusedShared* fsl, uint32_t step)
+{
+    const FusedView<T> V(KS, smem, fsl);
+    const StepDev& S = V.S;
+    const WorldDev& D = V.D;
+    const uint32_t n = V.n, t = V.t, M = V.M, w = V.w, m0 = V.X.m0, nit = V.nj + M;
+    step = uniform(step);
+    if (WARM && D.warm > 0.0f) {
+        // warm starting: this step's manifolds become the next step's tables
+        for (uint32_t x = t; x < n; x += T) D.wcnt[x] = 0u;
+        __syncthreads();
+        for (uint32_t q = t; q < M; q += T) warm_save(S, D, m0 + q, m0, m0 + M, V.base);
+        __syncthreads();
+    }
+    if (t == 0) {
+        uint32_t* cnt = S.w_cnt + 8 * (size_t)w;
+        cnt[0] = V.E; cnt[1] = V.R; cnt[2] = M; cnt[3] = nit;
+        unsigned long long* sums = reinterpret_cast<unsigned long long*>(S.counters + C_SUMS);
+        atomicAdd(&sums[0], (unsigned long long)n);
+        atomicAdd(&sums[1], (unsigned long long)V.E);
+        atomicAdd(&sums[2], (unsigned long long)V.R);
+        atomicAdd(&sums[3], (unsigned long long)M);
+        atomicAdd(&sums[4], (unsigned long long)nit);
+        S.w_man_begin[w] = m0;
+        S.w_man_end[w] = m0 + M;
+        S.w_done[w] = step + 1;
+        if (S.w_tstamp && step < S.tcap) S.w_tstamp[(size_t)w * (S.tcap + 1) + step + 1] = wall_clock64();
+    }
+}
+
 // One workgroup per world (S.w_order), up to nsteps steps per world counted
 // in S.w_done, so a relaunch after an overflow resumes each world where it
 // stopped.  lds_words: the launch's dynamic LDS.
 template <int MAXT, int WAVES, bool WARM = false>
 __global__ __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WAVES)))
-void k_fused(StepDev S /* first: chain_world reads it from the argument segment */, float dt, uint32_t sub_steps, uint32_t iters, uint32_t nsteps, uint32_t lds_words)
+void k_fused(StepDev /* read from the argument segment, which it starts */, float dt, uint32_t sub_steps, uint32_t iters, uint32_t nsteps, uint32_t lds_words)
 {
     extern __shared__ __align__(16) uint32_t smem[];
-    __shared__ uint32_t s_sm[16];
-    __shared__ uint32_t s_err, s_slot;
+    __shared__ FusedShared s_fs;
     __shared__ ChainShared s_chain;
-    const uint32_t w = S.w_order[blockIdx.x];
-    const WorldDev& D = S.worlds[w];
-    WorldScratch X = S.wscr[w];
-    const uint32_t n = (uint32_t)D.nbodies, tb = D.table, base = D.body_base, nj = (uint32_t)D.njoints;
     const uint32_t t = threadIdx.x;
-    constexpr uint32_t T = MAXT;
-    const FusedLds L = fused_carve(smem, n, tb);
-    uint32_t* cnt = S.w_cnt + 8 * (size_t)w;
-    uint64_t* ts = S.w_tstamp ? S.w_tstamp + (size_t)w * (S.tcap + 1) : nullptr;
-    uint32_t step = S.w_done[w];
-    if (ts && t == 0 && step < nsteps && step <= S.tcap) ts[step] = wall_clock64();
+    constexpr int T = MAXT;
+    const StepArgs KS = (StepArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    const LU32 lds = (LU32)smem;
+    R2D_LDS FusedShared* const fs = (R2D_LDS FusedShared*)&s_fs;
+    // the argument block where it is read (nothing of it is held across a part)
+    auto args = [&]() -> const StepDev& {
+        StepArgs p = KS;
+        asm volatile("" : "+s"(p));
+        return *(const StepDev*)p;
+    };
+    const uint32_t w = args().w_order[blockIdx.x];
     // phase times (profiling): thread 0 adds the wall clock between marks
-    uint64_t* prof = (S.w_prof && t == 0) ? S.w_prof + (size_t)w * FP_N : nullptr;
-    uint64_t tmark = prof ? wall_clock64() : 0;
+    uint64_t tmark = 0;
     auto mark = [&](int ph) {
-        if (prof) {
+        const StepDev& S = args();
+        if (S.w_prof && t == 0) {
             const uint64_t now = wall_clock64();
-            prof[ph] += now - tmark;
+            if (ph >= 0) S.w_prof[(size_t)w * FP_N + ph] += now - tmark;
             tmark = now;
         }
     };
+    uint32_t step;
+    {
+        const StepDev& S = args();
+        step = S.w_done[w];
+        if (t == 0) {
+            s_fs.w = w;
+            s_fs.lds_words = lds_words;
+            s_fs.E = s_fs.R = s_fs.M = 0u;
+            s_fs.X = S.wscr[w];
+            if (S.w_tstamp && step < nsteps && step <= S.tcap) S.w_tstamp[(size_t)w * (S.tcap + 1) + step] = wall_clock64();
+        }
+    }
+    __syncthreads();
+    mark(-1);
     for (; step < nsteps; ++step) {
-        if (S.w_status[w] != WS_OK) break;      // uniform: read before the barrier below
-        // ---- broadphase: per body (k_prep)
-        if (t == 0) s_err = 0u;
+        if (args().w_status[w] != WS_OK) break;      // uniform: read before the barrier below
+        if (t == 0) s_fs.err = 0u;
         __syncthreads();
-        // stale AABBs and flags in LDS for the pair filters below
-        const PairCache P = pair_cache(L.pairs, n);
-        for (uint32_t i = t; i < n; i += T) {
-            const Prep o = prep_body(D, i);
-            P.ax[i] = D.ax[i]; P.ay[i] = D.ay[i]; P.ahw[i] = D.ahw[i]; P.ahh[i] = D.ahh[i];
-            P.flags[i] = D.flags[i];
-            L.cc[i] = o.c;
-            L.cs[i] = o.s;
-            S.sflag[base + i] = o.res;
-            if (o.err) atomicOr(&s_err, o.err == WS_NONFINITE ? 2u : 1u);
-            if (!o.err && o.ncell) { S.cx0[base + i] = o.x0; S.cy0[base + i] = o.y0; S.cnx[base + i] = o.nx; }
-            L.coff[i] = o.ncell;
-        }
-        __syncthreads();
-        if (s_err) {
-            if (t == 0) S.w_status[w] = (s_err & 2u) ? WS_NONFINITE : WS_CELLS;
+        const uint32_t E = uniform(fused_cells<T>(KS, lds, fs));
+        if (s_fs.err) {   // (its scan's barriers lie between)
+            if (t == 0) args().w_status[w] = (s_fs.err & 2u) ? WS_NONFINITE : WS_CELLS;
             break;
         }
-        const uint32_t E = group_scan(L.coff, n, s_sm);
         mark(FP_PREP);
-        if (E > X.ecap && !fused_grow(S, w, X, 0, E, s_slot)) { fused_overflow(S, w, E, 0, 0, 0); break; }
-        uint32_t* ent_body = S.ent_body + X.e0;
-        uint32_t* ecnt = S.ent_cnt + X.e0;      // raw candidates per entry -> offsets
-        // the entries' buckets and the bucket members are read in serial
-        // loops: in LDS after the pair cache when they fit (E is about 1.5 n
-        // for bodies up to a cell wide)
-        const bool e_lds = 3 * (size_t)E <= (size_t)(lds_words - fused_front_words(n, tb) - PAIR_CACHE_WORDS * n);
-        uint32_t* e_free = L.pairs + PAIR_CACHE_WORDS * n;
-        uint32_t* ent_bkt = e_lds ? e_free : S.ent_bkt + X.e0;
-        uint32_t* items = e_lds ? e_free + E : S.bkt_items + X.e0;
-        uint32_t* sorted = e_lds ? e_free + 2 * E : S.bkt_sorted + X.e0;
-        for (uint32_t b = t; b <= tb; b += T) {
-            L.boff[b] = 0u;
-            if (b < tb) L.bfill[b] = 0u;
-        }
-        __syncthreads();
-        // cell entries and bucket occupancy (k_entries)
-        for (uint32_t e = t; e < E; e += T) {
-            uint32_t i = upper_idx(L.coff, n, e);
-            uint32_t k = e - L.coff[i];
-            uint32_t nx = S.cnx[base + i];
-            int64_t yi = S.cy0[base + i] + (int64_t)(k / nx);
-            int64_t xi = S.cx0[base + i] + (int64_t)(k % nx);
-            uint32_t b = (uint32_t)cell_hash((uint64_t)tb, xi, yi);
-            ent_body[e] = i;
-            ent_bkt[e] = b;
-            atomicAdd(&L.boff[b], 1u);
-        }
-        __syncthreads();
-        group_scan(L.boff, tb, s_sm);
-        // bucket members (k_bucket_fill), then in descending slot with a
-        // body's repeats adjacent (k_bucket_rank)
-        for (uint32_t e = t; e < E; e += T) {
-            uint32_t b = ent_bkt[e];
-            uint32_t pos = atomicAdd(&L.bfill[b], 1u);
-            items[L.boff[b] + pos] = ent_body[e];
-        }
-        __syncthreads();
-        for (uint32_t e = t; e < E; e += T) {
-            uint32_t a = ent_body[e], b = ent_bkt[e];
-            uint32_t o = L.boff[b], c = L.boff[b + 1] - o;
-            uint32_t greater, same;
-            bucket_rank_of(items + o, c, a, greater, same);
-            uint32_t dup = 0;
-            if (same > 1)
-                for (uint32_t x = L.coff[a]; x < e; ++x) dup += ent_bkt[x] == b;
-            sorted[o + greater + dup] = a;
-        }
-        __syncthreads();
+        if (!uniform(fused_room<T>(KS, fs, E, 0u, 0u, 0u))) break;
+        fused_buckets<T>(KS, lds, fs);
         mark(FP_BUCKETS);
-        // raw candidates per entry: distinct bucket members above the entry's
-        // body (k_ent_cnt) that pass the both-static and AABB filters; the
-        // passing members among the first 32 as a mask (in `items`, whose
-        // bucket lists are no longer read)
-        for (uint32_t e = t; e < E; e += T) {
-            const uint32_t a = ent_body[e], b = ent_bkt[e];
-            const uint32_t o = L.boff[b], c = L.boff[b + 1] - o;
-            uint32_t q, mask;
-            entry_candidates(P, a, sorted + o, c, q, mask);
-            ecnt[e] = q;
-            items[e] = mask;
-        }
-        __syncthreads();
-        const uint32_t R = group_scan(ecnt, E, s_sm);
-        if (R > X.rcap && !fused_grow(S, w, X, 1, R, s_slot)) { fused_overflow(S, w, E, R, 0, 0); break; }
-        uint4* cand = S.cand + X.r0;
-        uint32_t* cflag = S.cand_flag + X.r0;   // collides per candidate -> manifold offsets
-        // raw candidates in query order (k_cand_emit)
-        for (uint32_t e = t; e < E; e += T) {
-            uint32_t a = ent_body[e], b = ent_bkt[e];
-            uint32_t o = L.boff[b];
-            uint32_t ro = ecnt[e], c = ecnt[e + 1] - ro;
-            uint32_t k = e - L.coff[a];
-            uint32_t q = 0;
-            for (uint32_t mask = items[e]; mask; mask &= mask - 1u, ++q)
-                cand[ro + q] = make_uint4(a, sorted[o + (uint32_t)__builtin_ctz(mask)], k, 0u);
-            for (uint32_t j = 32; q < c; ++j) {
-                const uint32_t bj = sorted[o + j];
-                if (bj == sorted[o + j - 1] || !pair_passes(P, a, bj)) continue;
-                cand[ro + q] = make_uint4(a, bj, k, 0u);
-                ++q;
-            }
-        }
-        __syncthreads();
+        const uint32_t R = uniform(fused_count<T>(KS, lds, fs));
+        if (!uniform(fused_room<T>(KS, fs, E, R, 0u, 1u))) break;
+        fused_emit<T>(KS, lds, fs);
         mark(FP_CANDS);
-        // ---- narrowphase (k_narrow): the collision overwrites its candidate
-        // (partner, face id | ref-is-a, normal)
-        for (uint32_t q = t; q < R; q += T) {
-            const uint4 cq = cand[q];
-            const uint32_t a = cq.x, b = cq.y;
-            uint32_t info = 0;
-            float nx = 0.f, ny = 0.f;
-            bool hit = narrow_pair_call(D, a, b, cq.z, ent_bkt + L.coff[a], ent_bkt + L.coff[b],
-                                         L.coff[b + 1] - L.coff[b], L.cc[a], L.cs[a], L.cc[b], L.cs[b], info, nx, ny);
-            cflag[q] = hit ? 1u : 0u;
-            if (hit) cand[q] = make_uint4(a | (b << 16), info, __float_as_uint(nx), __float_as_uint(ny));
-        }
-        __syncthreads();
-        const uint32_t M = group_scan(cflag, R, s_sm);
+        const uint32_t M = uniform(fused_narrow<T>(KS, lds, fs));
         mark(FP_NARROW);
-        if ((M > X.mcap && !fused_grow(S, w, X, 2, M, s_slot)) ||
-            (nj + M > X.icap && !fused_grow(S, w, X, 3, nj + M, s_slot))) {
-            fused_overflow(S, w, E, R, M, nj + M);
-            break;
-        }
-        uint32_t* lists = S.lists + 2 * (size_t)X.i0;
-        // contact points (k_man_build), manifolds in discovery order
-        for (uint32_t q = t; q < R; q += T) {
-            const uint32_t mi = cflag[q];
-            if (cflag[q + 1] == mi) continue;
-            const uint4 x = cand[q];
-            const uint32_t a = x.x & 0xffffu, b = x.x >> 16;
-            man_build_one(S, D, D, X.m0 + mi, base, a, b, x.y, mk(__uint_as_float(x.z), __uint_as_float(x.w)), L.cc[a],
-                          L.cs[a], L.cc[b], L.cs[b]);
-        }
-        // ---- schedule: distance / offset joints make both bodies ordering (k_joint_mark)
-        for (uint32_t j = t; j < nj; j += T) {
-            const Joint& J = D.joints[j];
-            if (J.type <= 1) {
-                if (J.s1 >= 0) atomicOr(&S.sflag[base + J.s1], SF_RESOURCE);
-                if (J.s2 >= 0) atomicOr(&S.sflag[base + J.s2], SF_RESOURCE);
-            }
-        }
-        for (uint32_t i = t; i < n; i += T) { L.dcnt[i] = 0u; L.dfill[i] = 0u; }
-        __syncthreads();
+        if (!uniform(fused_room<T>(KS, fs, E, R, M, 2u))) break;
+        fused_contacts<T>(KS, lds, fs);
         mark(FP_CONTACTS);
-        const uint32_t nit = nj + M;
-        // items: joints, then manifolds, with their ordering bodies (k_items_*)
-        for (uint32_t j = t; j < nit; j += T) {
-            int32_t r0 = -1, r1 = -1;
-            if (j < nj) {
-                const Joint& J = D.joints[j];
-                r0 = J.s1 >= 0 ? (int32_t)(base + J.s1) : -1;
-                if (J.type <= 1 && J.s2 >= 0 && J.s2 != J.s1) r1 = (int32_t)(base + J.s2);
-            } else {
-                const uint32_t m = X.m0 + (j - nj);
-                const uint32_t ref = S.m_ref[m], inc = S.m_inc[m];
-                r0 = (S.sflag[ref] & SF_RESOURCE) ? (int32_t)ref : -1;
-                r1 = (S.sflag[inc] & SF_RESOURCE) ? (int32_t)inc : -1;
-            }
-            S.it_r0[X.i0 + j] = r0;
-            S.it_r1[X.i0 + j] = r1;
-            if (r0 >= 0) atomicAdd(&L.dcnt[r0 - (int32_t)base], 1u);
-            if (r1 >= 0) atomicAdd(&L.dcnt[r1 - (int32_t)base], 1u);
-        }
-        __syncthreads();
-        for (uint32_t i = t; i < n; i += T) L.doff[i] = L.dcnt[i];
-        __syncthreads();
-        group_scan(L.doff, n, s_sm);
-        // per-body item lists (k_list_fill), ranks in item order (k_list_rank).
-        // When the lists fit LDS behind the items per body (the cell, trig,
-        // bucket and pair arrays are dead after the contacts), they are filled there in any
-        // order and each entry then finds its rank by counting the smaller
-        // entries of its body's list (independent LDS reads) and goes to that
-        // place of the global lists; else they are filled in global memory and
-        // sorted per body.
-        uint32_t* const ul = L.coff;
-        const bool lds_lists = L.doff[n] <= lds_words - (3u * n + 1u);
-        uint32_t* const fill = lds_lists ? ul : lists;
-        for (uint32_t j = t; j < nit; j += T) {
-            const int32_t r0 = S.it_r0[X.i0 + j], r1 = S.it_r1[X.i0 + j];
-            if (r0 >= 0) {
-                const uint32_t x = (uint32_t)r0 - base;
-                fill[L.doff[x] + atomicAdd(&L.dfill[x], 1u)] = j * 2u;
-            }
-            if (r1 >= 0) {
-                const uint32_t x = (uint32_t)r1 - base;
-                fill[L.doff[x] + atomicAdd(&L.dfill[x], 1u)] = j * 2u + 1u;
-            }
-        }
-        __syncthreads();
-        if (lds_lists) {
-            for (uint32_t j = t; j < nit; j += T) {
-#pragma unroll
-                for (uint32_t side = 0; side < 2; ++side) {
-                    const int32_t r = side ? S.it_r1[X.i0 + j] : S.it_r0[X.i0 + j];
-                    if (r < 0) continue;
-                    const uint32_t x = (uint32_t)r - base, o = L.doff[x];
-                    const uint32_t v = j * 2u + side;
-                    const uint32_t rank = count_below(ul + o, L.dcnt[x], v);
-                    lists[o + rank] = v;
-                    if (side) S.it_k1[X.i0 + j] = rank; else S.it_k0[X.i0 + j] = rank;
-                }
-            }
-        } else {
-            for (uint32_t x = t; x < n; x += T) {
-                uint32_t* l = lists + L.doff[x];
-                const uint32_t c = L.dcnt[x];
-                for (uint32_t i = 1; i < c; ++i) {
-                    uint32_t v = l[i];
-                    uint32_t j = i;
-                    while (j > 0 && l[j - 1] > v) { l[j] = l[j - 1]; --j; }
-                    l[j] = v;
-                }
-                for (uint32_t p = 0; p < c; ++p) {
-                    uint32_t v = l[p];
-                    if (v & 1u) S.it_k1[X.i0 + (v >> 1)] = p; else S.it_k0[X.i0 + (v >> 1)] = p;
-                }
-            }
-        }
-        __syncthreads();
-        if (WARM && D.warm > 0.0f) {
-            // warm starting: match last step's manifolds, then each body's carried impulse
-            for (uint32_t q = t; q < M; q += T) warm_match(S, D, X.m0 + q, base, sub_steps);
-            __syncthreads();
-            for (uint32_t x = t; x < n; x += T) warm_body_sum(S, D, lists + L.doff[x], L.dcnt[x], x, 0u, nj, X.m0);
-            __syncthreads();
-        }
+        fused_schedule<T, WARM>(KS, lds, fs, sub_steps);
         mark(FP_SCHED);
         // ---- solve
         // (all of LDS but the items per body and their offsets is dead by now)
         if (sub_steps > 0u) {
             if (t == 0) {
-                const uint32_t keep = fused_keep_words(n);
-                s_chain = ChainShared{w, X.i0, X.m0, nj, M, base, sub_steps, iters, dt, keep, lds_words - keep,
-                                      0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}, 0u, 0u, 0u};
+                const WorldDev& D = args().worlds[w];
+                const uint32_t keep = fused_keep_words((uint32_t)D.nbodies);
+                s_chain = ChainShared{w, s_fs.X.i0, s_fs.X.m0, (uint32_t)D.njoints, M, D.body_base, sub_steps, iters, dt, keep,
+                                      lds_words - keep, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, {0u, 0u, 0u}, 0u, 0u, 0u};
             }
             __syncthreads();
-            chain_world<MAXT, WARM>((StepArgs)__builtin_amdgcn_kernarg_segment_ptr(), (LU32)smem,
-                                    (R2D_LDS ChainShared*)&s_chain);
+            chain_world<MAXT, WARM>(KS, lds, (R2D_LDS ChainShared*)&s_chain);
         }
         __syncthreads();
         mark(FP_SOLVE);
         if (sub_steps > 0u && s_chain.failed) break;   // status set
-        if (WARM && D.warm > 0.0f) {
-            // warm starting: this step's manifolds become the next step's tables
-            for (uint32_t x = t; x < n; x += T) D.wcnt[x] = 0u;
-            __syncthreads();
-            for (uint32_t q = t; q < M; q += T) warm_save(S, D, X.m0 + q, X.m0, X.m0 + M, base);
-            __syncthreads();
-        }
-        if (t == 0) {
-            cnt[0] = E; cnt[1] = R; cnt[2] = M; cnt[3] = nit;
-            unsigned long long* sums = reinterpret_cast<unsigned long long*>(S.counters + C_SUMS);
-            atomicAdd(&sums[0], (unsigned long long)n);
-            atomicAdd(&sums[1], (unsigned long long)E);
-            atomicAdd(&sums[2], (unsigned long long)R);
-            atomicAdd(&sums[3], (unsigned long long)M);
-            atomicAdd(&sums[4], (unsigned long long)nit);
-            S.w_man_begin[w] = X.m0;
-            S.w_man_end[w] = X.m0 + M;
-            S.w_done[w] = step + 1;
-            if (ts && step < S.tcap) ts[step + 1] = wall_clock64();
-        }
+        fused_done<T, WARM>(KS, lds, fs, step);
     }
     // the counts of the world's last step into the call's totals
     __syncthreads();
-    if (t < 4) atomicAdd(&S.counters[t], cnt[t]);
+    if (t < 4) atomicAdd(&args().counters[t], args().w_cnt[8 * (size_t)w + t]);
 }
 
 // the end of a step without sub-steps
