@@ -153,7 +153,7 @@ struct StepDev {
     uint32_t *it_k0, *it_k1;
     uint32_t *deg, *deg_off, *deg_fill;    // [N+1]
     uint32_t* lists;                       // [2*cap_i]
-    uint32_t* it_color;                    // [cap_i] colour (0 in reference order)
+    uint32_t* it_color;                    // [cap_i] the candidates that collide, then colours (coloured order)
     uint64_t* cmask;                       // [2*N] colours used per body (coloured schedule)
     uint4* recs;                           // [8*cap_i] contact point and joint records (two of 64 B an item)
     // the solver's program (r2d_chain.h): iterations one program covers, its

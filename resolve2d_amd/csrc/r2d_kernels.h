@@ -88,7 +88,8 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
                   const SolvePlan& sp);
 
 void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t n_const, uint32_t cap,
-              uint32_t* total_dev, const StepDev& S, int which, hipStream_t st);
+              uint32_t* total_dev, const StepDev& S, int which, hipStream_t st, uint32_t* where = nullptr,
+              uint32_t where_cap = 0);
 
 void set_solve_smem_limit();
 

@@ -55,6 +55,19 @@ def _heap(n, side, seed):
     return b.ops
 
 
+def _swarm(n, seed):
+    """n small discs in one cell: n (n - 1) / 2 candidates, of which few collide."""
+    from resolve2d_amd import scenes
+    rng = np.random.default_rng(seed)
+    b = scenes._Builder()
+    b.gravity(9.81)
+    for x, y in rng.uniform(4.1, 7.9, (n, 2)):
+        b.disc(x, y, 0.01, mu=0.5)
+    return b.ops
+
+
+SCENES = {"links": _links, "heap": _heap, "swarm": _swarm}
+
 # scene, sub-steps, iterations, steps, separate launches, LDS limit, warm
 CASES = {
     # what one program covers: 1, 3, 5, all 16 of 16, 10 of 20, 1 of 17; none
@@ -78,6 +91,8 @@ CASES = {
     "heap-6000": (("heap", 6000, 30.0, 8), 1, 2, 2, True, 0, 0.0),
     # the coloured order, its counters in LDS and in global memory
     "coloured": (("heap", 900, 14.0, 5), 2, 4, 3, True, 0, 0.0),
+    # more candidates than one kernel scans (4.2 M): their collisions' list
+    "candidates-4.5-million": (("swarm", 3000, 10), 1, 2, 2, True, 0, 0.0),
     "coloured-9000": (("heap", 9000, 45.0, 9), 1, 2, 2, True, 0, 0.0),
 }
 
@@ -87,7 +102,7 @@ def test_program_matches_oracle(oracle, name):
     from resolve2d_amd.engine import GpuWorld, apply_scene
     from resolve2d_amd.solver import Context
     scene, sub, iters, steps, separate, limit, warm = CASES[name]
-    ops = (_links if scene[0] == "links" else _heap)(*scene[1:])
+    ops = SCENES[scene[0]](*scene[1:])
     ctx = Context(0)
     ctx.set_lds_limit(limit)
     ctx.set_fused(not separate)
