@@ -59,10 +59,9 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 # host processes at most: the host CPU share that comes with one GPU of an MI355X node
 CPU_SHARE = 16
 
-# fused kernel shape of each solve variant: <slots, workgroup size, waves per SIMD>
-FUSED_SHAPES = {1: "4,256,3", 2: "2,512,3", 3: "3,256,3", 4: "4,256,2", 5: "8,128,2", 7: "4,256,3",
-                9: "0,256,3", 10: "0,256,4", 11: "0,192,3", 12: "0,128,2", 13: "0,512,2",
-                14: "0,768,3"}
+# fused kernel shape of each solve variant: <workgroup size, waves per SIMD>
+FUSED_SHAPES = {1: "256,3", 2: "512,3", 3: "256,3", 4: "256,2", 5: "128,2", 7: "256,3", 9: "256,3", 10: "256,4",
+                11: "192,3", 12: "128,2", 13: "512,2", 14: "768,3"}
 
 
 def traffic_for(name, window, args):
@@ -941,8 +940,7 @@ def main():
         plain = {"value": pw_bs / pw_t, "unit": "body-steps/s",
                  "sample": f"{len(pick)} worlds spread over the batch, one world per launch (r2d_process per "
                            f"step); steps {window[0]}-{window[1]} timed",
-                 "launch": "the library's default shape for one world (k_fused<0,768,3>: a lane per solver item "
-                           "up to 768 items)" if args.variant < 0 else f"variant {args.variant}"}
+                 "launch": "the library's default shape for one world (k_fused<768,3>)" if args.variant < 0 else f"variant {args.variant}"}
         if ph_t:
             plain["horizon"] = {"value": ph_bs / ph_t, "unit": "body-steps/s",
                                 "sample": f"the same worlds over steps 1-{window[1]}"}
@@ -959,7 +957,9 @@ def main():
     # Phase kernels: the solve phase, 112 B per body + 120 B per manifold +
     # 16 B per solver item.
     joint_items = max(0, work["items"] - work["manifolds"])
-    used_variant = tuned["variant"] if tuned else (args.variant if args.variant >= 0 else 1)
+    # untuned: the library's choice by worlds per compute unit (256 of them)
+    shared = -(-args.worlds // 256)
+    used_variant = tuned["variant"] if tuned else args.variant if args.variant >= 0 else 14 if shared == 1 else 1 if shared <= 3 else 10
     if fused_launches:
         kernel = f"k_fused<{FUSED_SHAPES.get(used_variant, '?')}>"
         launch_s = fused_ms / fused_launches / 1e3
@@ -969,7 +969,7 @@ def main():
         per_step = {k: v / max(world_steps, 1) for k, v in fused_phases.items()}
         per_step_note = "per world-step, workgroup wall clock"
     else:
-        kernel = "k_solve"
+        kernel = "k_chain_run"
         names = ["broadphase", "narrowphase", "schedule", "solve"]
         per_step = {n: phase_ms[i] / max(phase_steps, 1) for i, n in enumerate(names)}
         launch_s = per_step["solve"] / 1e3

@@ -271,23 +271,21 @@ int r2d_ctx_fused_counts(r2d_ctx* ctx, uint64_t* out);
  * environment variable R2D_NO_FUSED=1 sets the default to off.  No
  * counterpart in the reference (Solver.process is one world, one step). */
 int r2d_ctx_set_fused(r2d_ctx* ctx, int on);
-/* Launch configuration of the solve kernel: -1 (default) is variant 1;
- * 0..12 select the register-slot kernel's slots x workgroup size, the record
- * kernel's workgroup size, and the fused kernel's shape (table in
- * r2d_kernels.hip; 9-12 solve with records only).
+/* Launch configuration of the solve: -1 (default) chooses by how many worlds
+ * share a compute unit; 0..14 select the shape of the one-kernel step (threads
+ * and registers; 0, 6 and 8 have none) and the threads of the separate
+ * launches' chain (table in r2d_kernels.hip).
  * Every variant gives the same bits; the autotuner (resolve2d_amd/autotune.py)
  * picks the fastest for a batch shape. */
 int r2d_ctx_set_solve_variant(r2d_ctx* ctx, int variant);
-/* Largest world (bodies) whose solver body state is kept in LDS; larger
- * worlds use the solve kernel with body state in global memory.  0 (default)
- * = as many as LDS holds.  Results are identical either way; this is a
+/* Separate launches only: the largest world (bodies) whose momenta are kept in
+ * LDS during a chain; larger worlds' stay in global memory.  0 (default) = as
+ * many as LDS holds.  Results are identical either way; this is a
  * launch-shape knob for the autotuner. */
 int r2d_ctx_set_lds_limit(r2d_ctx* ctx, uint32_t max_bodies);
-/* Phase kernels only: a batch of at most 64 worlds whose solver body state
- * fits LDS takes the record kernel with 512 lanes per world instead of the
- * variant's shape (on, the default: such worlds are alone on their CUs and
- * latency-bound).  Off keeps the variant's record kernel.  Same bits either
- * way; a launch-shape knob with no counterpart in the reference. */
+/* Separate launches only: a batch of at most 256 worlds runs their chains
+ * with 512 threads a world (on, the default: each is alone on its CU).  Off
+ * keeps the variant's threads.  Same bits either way; a launch-shape knob with no counterpart in the reference. */
 int r2d_ctx_set_wide_record(r2d_ctx* ctx, int on);
 /* Totals of the last step of the context: entries, raw candidates,
  * manifolds, solver items (out[4]). */

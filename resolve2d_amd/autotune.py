@@ -1,10 +1,10 @@
 """Autotuner of the step's launch shape for a batch of worlds.
 
 Knobs (all give bit-identical results, so tuning may run on live steps):
-  - solve variant: the register-slot kernel's slots x workgroup size, and the
-    record kernels' workgroup sizes (r2d_ctx_set_solve_variant);
-  - LDS limit: the largest world whose body state the solve kernel keeps in
-    LDS (r2d_ctx_set_lds_limit);
+  - solve variant: threads and registers of the one-kernel step, threads of
+    the separate launches' chain (r2d_ctx_set_solve_variant);
+  - LDS limit: the largest world whose momenta the separate launches' chain
+    keeps in LDS (r2d_ctx_set_lds_limit);
   - whole steps per workgroup (r2d_ctx_set_fused) for variants that have a
     fused kernel.  A fused launch ends with its slowest world, so it is timed
     on calls of several steps, as the caller's calls would run.
@@ -25,8 +25,7 @@ import numpy as np
 from . import _native as N
 
 SOLVE_VARIANTS = 15
-# variants that differ on the phase kernels (9 and 10 are variant 6 there, 12
-# is variant 7; 11 is the record kernel with 192 threads, 13 with 512)
+# variants tried on the phase kernels, whose chain has 256 or 512 threads
 PHASE_VARIANTS = tuple(range(9)) + (11, 13)
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "resolve2d_amd", "autotune.json")
 
@@ -79,8 +78,7 @@ def save_cache(cache: Dict[str, dict], path: str = DEFAULT_CACHE):
     os.replace(tmp, path)
 
 
-# variants with a fused kernel (the register-slot shapes, lockstep walk aside,
-# and the records-only shapes)
+# variants with a fused kernel
 FUSED_VARIANTS = (1, 2, 3, 4, 5, 7, 9, 10, 11, 12, 13, 14)
 
 

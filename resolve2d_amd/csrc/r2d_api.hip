@@ -821,13 +821,12 @@ size_t worlds_per_cu(const r2d_ctx* c, size_t nworlds)
 }
 
 // The launch shape of a batch the caller has not tuned.  Worlds that are each
-// alone on a CU take 768 threads (256 worlds of 379-501 bodies: 375 us a step,
-// 435 with 256 threads).  Two or three a CU take 256 threads and registers for
-// three workgroups (512 worlds of 273-501: 453 us; for four: 461); more take
-// registers for four, with spills, since a fourth world that waits for one of
-// the three costs more (1,024 worlds of 51-501: 484 us, for three 600, 192
-// threads 506).  Warm starting is compiled into kernels of its own, of 768 and
-// 192 threads (256 worlds: 6.1 and 8.2 ms for 16 steps).
+// alone on a CU take 768 threads (256 worlds of 379-501 bodies with 256
+// threads: 384 us a step).  Two or three a CU take 256 threads and registers
+// for three workgroups (512 worlds of 273-501: 403 us; for four: 401); more
+// take registers for four (1,024 worlds of 51-501: 462 us, for three 540, 192
+// threads 487).  Warm starting is compiled into kernels of its own, of 768 and
+// 192 threads.
 int default_variant(const r2d_ctx* c, size_t nworlds)
 {
     const size_t k = worlds_per_cu(c, nworlds);

@@ -6,7 +6,7 @@
 // item on its ordering bodies has run.  That partial order is the same in
 // every sub-step of a step, so it is worked out once per step (plan_*: the
 // items ready now make the next rows, which release their successors) and
-// the sub-steps replay the rows (chain_call).  A row's lanes share no
+// the sub-steps replay the rows (chain_lds and its relatives).  A row's lanes share no
 // ordering body and every body meets its items in the reference's order, so
 // the bits are the sequential loop's.  Nothing polls: a world whose rows all
 // fit one wave runs them in program order, LDS serving one wave's operations
@@ -14,7 +14,7 @@
 // between rows.
 //
 // What bounds it is the length of the dependency chain times one row: two LDS
-// reads, about 90 VALU instructions and an LDS write.  Lanes hold contact
+// reads, about 100 VALU instructions and an LDS write.  Lanes hold contact
 // points, not items: the points of a two-point manifold sit in neighbouring
 // lanes (the reference computes both from the same momenta and adds their
 // impulses up afterwards), which halves the instructions of a row, and a
@@ -434,7 +434,8 @@ __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32
 // Waves that run a world's rows: one for each `rows` rows of 64 its items fill
 // (a pile's chain is 90-150 slots deep for 4 iterations).  In the one-kernel
 // step a slot of several waves costs about two rows of one, so they pay from
-// 96 rows on (97 worlds x 8 steps: 3.40 ms, with 48 4.45 ms).  In the separate
+// 96 rows on (97 worlds x 8 steps, when this line was drawn: 3.40 ms, with 48
+// 4.45 ms; 2.26 now).  In the separate
 // launches, records in program order, wider is better down to a wave for 32
 // rows (solve of a 4,096-body pile, 96 / 48 / 24 rows: 529 / 499 / 498 us;
 // coloured 417 / 311 / 308).

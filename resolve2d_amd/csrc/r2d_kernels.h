@@ -94,7 +94,7 @@ void scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t
 void set_solve_smem_limit();
 
 // Whole steps per workgroup (k_fused) for worlds of at most FUSED_NMAX bodies
-// in the reference order; the variant picks the solve's slot shape.
+// in the reference order; the variant picks threads and workgroups a CU.
 constexpr uint32_t FUSED_NMAX = 1024;
 bool fused_available(int variant);
 // dynamic LDS of the fused kernel for a world of n bodies and tb hash buckets

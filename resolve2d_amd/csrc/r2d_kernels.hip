@@ -1,27 +1,33 @@
 // HIP kernels of one resolve2d step (Solver.process, src/core/lib.zig:189-299)
 // for gfx950, over a batch of independent worlds.
 //
-// Pipeline (every kernel reads its element counts from device memory so the
-// whole step is a fixed launch sequence that can be captured in a hipGraph):
+// Small worlds take every step of a call in one kernel (k_fused, a workgroup
+// per world).  The others take separate launches (every kernel reads its
+// element counts from device memory so the whole step is a fixed launch
+// sequence that can be captured in a hipGraph):
 //
+//   k_begin_step    counters, bucket and body counts, the scans' states cleared
 //   k_prep          per body: cos/sin of the angle, cell range of the stale AABB
-//   scan            cell counts -> entry offsets                (E entries)
+//   k_scan          cell counts -> entry offsets                (E entries)
 //   k_entries       per entry: bucket = hash(cell) % table, bucket counts
-//   scan            bucket counts -> bucket offsets
+//   k_scan          bucket counts -> bucket offsets
 //   k_bucket_fill   per entry: scatter body into its bucket
-//   k_bucket_sort   per bucket: descending body order, duplicates dropped
+//   k_bucket_rank   per entry: its place in descending body order, without duplicates
 //   k_ent_cnt       per entry: bodies in the bucket with a higher slot
-//   scan            -> raw candidate offsets                    (R candidates)
+//   k_scan          -> raw candidate offsets                    (R candidates)
 //   k_cand_emit     per entry: (a, b) raw candidates in the reference's query order
 //   k_narrow        per candidate: first occurrence, filters, SAT
-//   scan            collides flags -> manifold index             (M manifolds)
-//   k_man_build     per manifold: contact points (identifyCollisionPoints)
-//   k_world_ranges  per world: manifold / item ranges
-//   k_items_*       solver items and their ordering resources
-//   scan, k_list_*  per-body ordered item lists -> ranks
-//   k_solve         one workgroup per world: sub-steps, forces, integration,
-//                   pre-step and the sequential-impulse iterations, run as a
-//                   dataflow that reproduces the reference's sequential order.
+//   k_scan          collides flags -> manifold index and list   (M manifolds)
+//   k_man_build     per manifold: contact points (identifyCollisionPoints);
+//                   per world: manifold / item ranges
+//   k_items         solver items and their ordering resources
+//   k_scan, k_list_*  per-body ordered item lists -> ranks
+//   k_color, k_world_order  coloured order only
+//   k_chain_build   per item: its points' records
+//   k_chain_plan    per world: the program of rows, records in its order
+//   k_chain_bodies, k_chain_run  per sub-step: forces, integration, pre-step;
+//                   then the world's program, which reproduces the
+//                   reference's sequential order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1493,8 +1499,7 @@ size_t fused_lds_bytes(uint32_t n, uint32_t tb)
 
 // The fused kernel's narrowphase test of one candidate, as a call: out of
 // line, its registers are allocated apart from the step kernel's, which
-// spills less (45 -> 31 VGPRs for k_fused<0, 192, 3>) and ran the 240-step
-// launch 2 % faster.  It takes only pointers and values (no reference to the
+// spills less.  It takes only pointers and values (no reference to the
 // kernel's argument block, which would be copied to scratch).
 __device__ __attribute__((noinline)) bool narrow_pair_call(const WorldDev& D, uint32_t sa, uint32_t sb, uint32_t k,
                                                          const uint32_t* ba, const uint32_t* bb, uint32_t nb,
@@ -2794,7 +2799,7 @@ __device__ __attribute__((noinline)) void fused_schedule(StepArgs KS, LU32 smem,
     const WorldScratch& X = V.X;
     uint32_t* const s_sm = V.s_sm;
     const uint32_t nit = nj + M;
-    // items: joints, then manifolds, with their ordering bodies (k_items_*)
+    // items: joints, then manifolds, with their ordering bodies
     for (uint32_t j = t; j < nit; j += T) {
         int32_t r0 = -1, r1 = -1;
         if (j < nj) {

@@ -80,8 +80,8 @@ class Context:
         N.check(self.lib.r2d_ctx_set_lds_limit(self.handle, max_bodies), "r2d_ctx_set_lds_limit")
 
     def set_wide_record(self, on: bool):
-        """Phase kernels: batches of at most 64 LDS-state worlds take the
-        512-lane record kernel (default on).  Same bits either way."""
+        """Phase kernels: batches of at most 256 worlds run their chains with
+        512 threads a world (default on).  Same bits either way."""
         N.check(self.lib.r2d_ctx_set_wide_record(self.handle, 1 if on else 0), "r2d_ctx_set_wide_record")
 
     def set_fused(self, on: bool):
