@@ -825,8 +825,10 @@ size_t worlds_per_cu(const r2d_ctx* c, size_t nworlds)
 // threads: 384 us a step).  Two or three a CU take 256 threads and registers
 // for three workgroups (512 worlds of 273-501: 403 us; for four: 401); more
 // take registers for four (1,024 worlds of 51-501: 462 us, for three 540, 192
-// threads 487).  Warm starting is compiled into kernels of its own, of 768 and
-// 192 threads.
+// threads 487).  Warm starting is compiled into kernels of its own, of 768
+// threads and of 256 with registers for four workgroups (20 steps of 1,024
+// settled worlds: 10.8 ms, with 192 threads and registers for three 11.7; 16
+// steps of 600 worlds 7.4 and 8.1, of 300 6.6 and 7.4).
 int default_variant(const r2d_ctx* c, size_t nworlds)
 {
     const size_t k = worlds_per_cu(c, nworlds);

@@ -3078,7 +3078,7 @@ static const SolveVariant kSolveVariants[SOLVE_TABLE] = {
     {CHAIN_NARROW, k_fused<128, 2>, 128},
     {CHAIN_THREADS, k_fused<512, 2>, 512},
     {CHAIN_THREADS, k_fused<768, 3>, 768},      // WIDE_VARIANT
-    {CHAIN_NARROW, k_fused<192, 3, true>, 192}, // WARM_VARIANT (the kernels above carry no warm-start passes)
+    {CHAIN_NARROW, k_fused<256, 4, true>, 256}, // WARM_VARIANT (the kernels above carry no warm-start passes)
     {CHAIN_THREADS, k_fused<768, 3, true>, 768}, // WARM_WIDE_VARIANT
 };
 

@@ -123,3 +123,30 @@ def test_program_matches_oracle(oracle, name):
     g.close()
     o.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("worlds", [257, 513])
+def test_warm_batch_of_several_worlds_a_cu(oracle, worlds):
+    """More warm worlds than CUs: the narrow warm kernel, heaps of 1 to 40 bodies."""
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    from resolve2d_amd.solver import Context
+    ctx = Context(0)
+    scenes = [_heap(1 + (7 * k) % 40, 2.0 + k % 3, 20 + k) for k in range(worlds)]
+    gs = [GpuWorld(ctx) for _ in scenes]
+    for ops, g in zip(scenes, gs):
+        apply_scene(ops, g)
+        g.set_warm_start(0.8)
+    for _ in range(2):
+        ctx.process_batch_handles([g.handle for g in gs], DT, 2, 4, 3)
+    for k in range(0, worlds, 16):
+        o = oracle.OracleWorld("f32")
+        apply_scene(scenes[k], o)
+        o.set_warm_start(0.8)
+        for _ in range(6):
+            assert o.process(DT, 2, 4) == 0
+        a, b = gs[k].bodies(), o.bodies()
+        assert bits_equal(a, b), (k, first_diff(a, b))
+        o.close()
+    for g in gs:
+        g.close()
+    ctx.close()
