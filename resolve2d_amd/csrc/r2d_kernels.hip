@@ -3054,11 +3054,16 @@ static inline unsigned blocks_for(uint64_t n, unsigned bs, unsigned cap = 4096)
 
 typedef void (*FusedFn)(StepDev, float, uint32_t, uint32_t, uint32_t, uint32_t);
 struct SolveVariant {
-    unsigned threads;    // workgroup of the separate launches' chain (CHAIN_THREADS or CHAIN_NARROW)
+    unsigned threads;    // workgroup of the separate launches' chain (CHAIN_THREADS: wide, or CHAIN_NARROW)
     FusedFn fused_fn;    // whole steps per workgroup (nullptr: none)
     unsigned fused_t;    // its workgroup size
 };
-constexpr unsigned CHAIN_THREADS = 512, CHAIN_NARROW = 256;
+// Separate launches' workgroups.  The coloured order's slots hold about 700
+// points of a 4,096-body pile, eleven waves' rows, and take twelve waves
+// (solve 262 -> 237 us a step; sixteen, which spill, 250); the reference
+// order's about 200, and twelve waves cost it their barriers (24 piles 535 ->
+// 547, a pile 413 -> 417).
+constexpr unsigned CHAIN_THREADS = 512, CHAIN_COLORED = 768, CHAIN_NARROW = 256;
 // Solve variants: shapes of the kernels that run worlds' programs.  The fused
 // kernels differ in threads and in waves per SIMD (registers); 0, 6 and 8
 // have none and take the separate launches.
@@ -3260,14 +3265,16 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
     default: {
         const float sub_dt = dt / (float)sub_steps;
         auto pick = [&](auto warm, auto cold) { return sp.any_warm ? warm : cold; };
-        const unsigned T = sp.wide ? CHAIN_THREADS : CHAIN_NARROW;
+        const bool colored = sp.any_colored && !sp.any_warm;
+        const unsigned T = !sp.wide ? CHAIN_NARROW : colored ? CHAIN_COLORED : CHAIN_THREADS;
+        auto width = [&](auto narrow, auto wide, auto widest) { return !sp.wide ? narrow : colored ? widest : wide; };
         const uint32_t words = sp.lds / 4u;
         if (sub_steps > 0) {   // without sub-steps nothing of a world changes
             hipLaunchKernelGGL(pick(k_chain_build<true>, k_chain_build<false>), dim3(GRID), dim3(BS), 0, st, S, sub_dt);
             tmark(ss, "k_chain_build", st);
             if (iters > 0) {
-                hipLaunchKernelGGL(sp.wide ? k_chain_plan<CHAIN_THREADS> : k_chain_plan<CHAIN_NARROW>, dim3(S.nworlds), dim3(T),
-                                   sp.lds, st, S, words);
+                hipLaunchKernelGGL(width(k_chain_plan<CHAIN_NARROW>, k_chain_plan<CHAIN_THREADS>, k_chain_plan<CHAIN_COLORED>),
+                                   dim3(S.nworlds), dim3(T), sp.lds, st, S, words);
                 tmark(ss, "k_chain_plan", st);
             }
         }
@@ -3277,8 +3284,9 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
                                dim3(BS), 0, st, S, s, sub_steps, sub_dt);
             tmark(ss, "k_chain_bodies", st);
             if (s == sub_steps) break;
-            auto run = sp.wide ? pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>)
-                               : pick(k_chain_run<CHAIN_NARROW, true>, k_chain_run<CHAIN_NARROW, false>);
+            auto run = width(pick(k_chain_run<CHAIN_NARROW, true>, k_chain_run<CHAIN_NARROW, false>),
+                             pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>),
+                             k_chain_run<CHAIN_COLORED, false>);
             hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax);
             tmark(ss, "k_chain_run", st);
         }
@@ -3303,6 +3311,8 @@ void set_solve_smem_limit()
     allow((const void*)k_color);
     allow((const void*)k_chain_plan<CHAIN_THREADS>);
     allow((const void*)k_chain_plan<CHAIN_NARROW>);
+    allow((const void*)k_chain_plan<CHAIN_COLORED>);
+    allow((const void*)k_chain_run<CHAIN_COLORED, false>);
     allow((const void*)k_chain_run<CHAIN_THREADS, false>);
     allow((const void*)k_chain_run<CHAIN_THREADS, true>);
     allow((const void*)k_chain_run<CHAIN_NARROW, false>);

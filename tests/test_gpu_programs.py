@@ -150,3 +150,31 @@ def test_warm_batch_of_several_worlds_a_cu(oracle, worlds):
     for g in gs:
         g.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("warm", [0.0, 0.8], ids=["cold", "warm"])
+def test_coloured_beside_reference_order(oracle, warm):
+    """A coloured world whose slots hold more than eight waves' rows, in one
+    batch with a world in the reference order (warm started or not)."""
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    from resolve2d_amd.solver import Context
+    ctx = Context(0)
+    ctx.set_fused(False)
+    scenes = [_heap(3000, 25.0, 30), _heap(200, 7.0, 31)]
+    gs, os = [GpuWorld(ctx) for _ in scenes], [oracle.OracleWorld("f32") for _ in scenes]
+    for ops, g, o in zip(scenes, gs, os):
+        apply_scene(ops, g)
+        apply_scene(ops, o)
+    for e in (gs[0], os[0]):
+        e.set_schedule(1)
+    for e in (gs[1], os[1]):
+        e.set_warm_start(warm)
+    for step in range(3):
+        ctx.process_batch_handles([g.handle for g in gs], DT, 2, 4, 1)
+        for k, (g, o) in enumerate(zip(gs, os)):
+            assert o.process(DT, 2, 4) == 0
+            a, b = g.bodies(), o.bodies()
+            assert bits_equal(a, b), (step, k, first_diff(a, b))
+    for e in gs + os:
+        e.close()
+    ctx.close()
