@@ -302,6 +302,12 @@ int r2d_last_error(char* buf, size_t n);
  * pairs (in[2i] / in[2i+1]; `in` holds 2n floats). */
 int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
 
+/* Test hook with no counterpart in the reference: the rules by which the host
+ * lays out and launches steps, for given sizes (no device needed).
+ * rule 0: in {collision iterations}; out {iterations that a solver program
+ * covers, iterations of the program that ends a sub-step}. */
+int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out);
+
 /* Measurement hook with no counterpart in the reference: the device's
  * measured peaks, for rooflines against what the hardware delivers.
  * out[0]: HBM read stream (GB/s, 1 GiB read by 16-byte loads, 4 in flight

@@ -716,6 +716,14 @@ WorldDev make_desc(r2d_world* w)
     return d;
 }
 
+// the iterations of each program of a call's worlds
+void set_split(StepDev& S, size_t iters)
+{
+    const ChainSplit c = chain_split(iters);
+    S.chain_iters = c.each;
+    S.chain_rest = c.rest;
+}
+
 // carve the step scratch for the current capacities
 int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, uint32_t e, uint32_t r, uint32_t m,
                    uint32_t it, uint32_t k)
@@ -1066,7 +1074,7 @@ int fused_layout(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
     }
     // as much again free for worlds that outgrow their slices during the call
-    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, chain_iters(b.iters), false))) return rc;
+    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, chain_split(b.iters).room(), false))) return rc;
     // workgroups take the largest worlds first (the longest steps start first)
     c->forder.resize(nw);
     for (size_t i = 0; i < nw; ++i) c->forder[i] = (uint32_t)i;
@@ -1106,7 +1114,7 @@ int fused_regrow(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
         c->hstatus[i] = WS_OK;
     }
-    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, chain_iters(b.iters), true);
+    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, chain_split(b.iters).room(), true);
     if (rc) return rc;
     if ((rc = fused_upload_tables(c))) return rc;
     HIPCHK(hipMemcpyAsync(c->S.w_status, c->hstatus, nw * 4, hipMemcpyHostToDevice, c->stream));
@@ -1270,7 +1278,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     uint32_t est_r = std::max<uint32_t>(c->cap_r, (uint32_t)(8 * b.N + 1024));
     uint32_t est_m = std::max<uint32_t>(c->cap_m, (uint32_t)(4 * b.N + 1024));
     return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m,
-                          (uint32_t)b.J + est_m, chain_iters(b.iters));
+                          (uint32_t)b.J + est_m, chain_split(b.iters).room());
 }
 
 // sum the phase times of the timed steps recorded so far
@@ -1307,7 +1315,7 @@ int batch_launch(r2d_ctx* c, Batch& b)
     StepDev S = c->S;
     S.nb = (uint32_t)b.N; S.nworlds = (uint32_t)nw; S.nbuckets = (uint32_t)b.B; S.njoints = (uint32_t)b.J;
     S.worlds = c->dworlds;
-    S.chain_iters = chain_iters(b.iters);
+    set_split(S, b.iters);
     const Streams ss = c->streams();
     const uint32_t sub = (uint32_t)b.sub, iters = (uint32_t)b.iters;
     auto eager_phase = [&](int ph) { launch_phase(S, ss, ph, b.dt, sub, iters, b.plan); };
@@ -1381,7 +1389,7 @@ int fused_launch(r2d_ctx* c, Batch& b)
     StepDev F = fused_view(c);
     F.nb = (uint32_t)b.N; F.nworlds = (uint32_t)nw; F.nbuckets = (uint32_t)b.B; F.njoints = (uint32_t)b.J;
     F.worlds = c->dworlds;
-    F.chain_iters = chain_iters(b.iters);
+    set_split(F, b.iters);
     if (c->profiling) {
         // The timing buffers grow rarely and by a lot: a launch that follows a
         // hipMalloc closely can stall all of its waves for several ms at once
@@ -1563,7 +1571,7 @@ int batch_wait(r2d_ctx* c, Batch& b)
             if (c->hcounters[C_OVERFLOW] & 4u) m = c->hcounters[C_MANIFOLDS] * 2;
             if (c->hcounters[C_OVERFLOW] & 8u) it = c->hcounters[C_ITEMS] * 2;
             int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e + 1, r + 1,
-                                    m + 1, it + 1, chain_iters(b.iters));
+                                    m + 1, it + 1, chain_split(b.iters).room());
             if (rc) return rc;
         }
         if (b.done >= b.steps) break;
@@ -2231,7 +2239,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     WorldDev* ddesc = nullptr;
     static_layout(base, &F, &ddesc);
     F.nb = n; F.nbuckets = tb; F.njoints = nj;
-    F.chain_iters = chain_iters(iters);
+    set_split(F, iters);
     // host values the asynchronous uploads read; the call waits for the
     // stream before they go out of scope
     WorldDev d = w->desc;
@@ -2716,6 +2724,20 @@ R2D_EXPORT int r2d_debug_peaks(r2d_ctx* c, double* out)
     out[1] = (double)(2 * n16 * 16) / t_copy / 1e9;
     out[2] = (double)lds_blocks * threads * 16.0 * 8.0 * rounds / t_lds / 1e9;
     return R2D_OK;
+}
+
+R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
+{
+    if (!in || !out) return R2D_E_INVALID_ARG;
+    switch (rule) {
+    case 0: {
+        const ChainSplit s = chain_split(in[0]);
+        out[0] = s.each;
+        out[1] = s.rest;
+        return R2D_OK;
+    }
+    }
+    return R2D_E_INVALID_ARG;
 }
 
 R2D_EXPORT int r2d_last_error(char* buf, size_t n)

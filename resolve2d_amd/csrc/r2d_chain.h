@@ -137,9 +137,9 @@ struct PlanLds {
     __device__ __forceinline__ Raw read(uint32_t at) const { return ring[at]; }
     __device__ __forceinline__ void push(uint32_t at, Raw e) { ring[at] = e; }
     __device__ __forceinline__ Raw entry(uint32_t s) const { return items[s]; }
-    __device__ __forceinline__ void rearm(uint32_t j, uint32_t by)
+    __device__ __forceinline__ uint32_t rearm(uint32_t j, uint32_t by)
     {
-        __hip_atomic_fetch_add(&state[j], by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return __hip_atomic_fetch_add(&state[j], by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __device__ __forceinline__ uint32_t release(uint32_t s)
     {
@@ -171,9 +171,9 @@ struct PlanGlb {
     }
     __device__ __forceinline__ void push(uint32_t at, const PlanEntry& e) { ring[at] = u4v{e.item, e.second, e.s0, e.s1}; }
     __device__ __forceinline__ GU32 state_of(uint32_t j) const { return (GU32)(items + j) + 2; }
-    __device__ __forceinline__ void rearm(uint32_t j, uint32_t by)
+    __device__ __forceinline__ uint32_t rearm(uint32_t j, uint32_t by)
     {
-        __hip_atomic_fetch_add(state_of(j), by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return __hip_atomic_fetch_add(state_of(j), by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __device__ __forceinline__ uint32_t release(uint32_t s)
     {
@@ -225,6 +225,7 @@ struct ChainShared {
     // a plan that the first chain runs behind: LDS words it keeps, rows it has written (PLANNED: all), and the
     // waves that have met (waves_meet)
     uint32_t beside, progress, met;
+    uint32_t rest_slots;   // of the program after the others (StepDev::chain_rest)
 };
 constexpr uint32_t PLANNED = 0x80000000u;
 
@@ -332,8 +333,9 @@ __device__ __forceinline__ void plan_put(PLAN& P, const Round<PLAN>& R, uint32_t
 }
 
 // The program of a world run by one wave, planned by one wave without
-// barriers; `ready` items are in the ring.  Returns the rows (0: the ordering
-// data was corrupt) and the entries.
+// barriers; `ready` items are in the ring from its start on, `entries` are
+// written already.  Returns the rows (0: the ordering data was corrupt) and
+// adds the entries.
 // PUBLISH: `progress` counts the rows that other waves may read (a round's
 // stores, three at most, are waited for in the next round).
 template <bool PUBLISH = false, class PLAN>
@@ -345,7 +347,7 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
         if (lane_id() == 0u) __hip_atomic_store(progress, rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t head = 0, count = ready, entry = 0, row = 0, done = 0;
+    uint32_t head = 0, count = ready, entry = entries, row = 0, done = 0;
     const uint32_t total = nit * iters;
     while (done < total && count) {
         Round<PLAN> R = plan_take(P, head, count < 64u ? count : 64u, lane, nj);
@@ -382,7 +384,8 @@ __device__ __forceinline__ uint32_t plan_single(PLAN& P, const Program& G, uint3
 // The program of a world run by `waves` waves of the workgroup, planned by
 // all of them: wave w takes the w-th 64 ready items.  Items that do not fit
 // a row go back to the end of the ring.  A barrier per slot; called by the
-// whole workgroup.  sh.taken, sh.entries, sh.queued start at 0.
+// whole workgroup.  sh.taken and sh.queued start at 0, sh.entries at the
+// entries written already.
 template <class PLAN>
 __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32_t nit, uint32_t nj, uint32_t iters,
                                                uint32_t ready, uint32_t waves, ChainShared& sh)
@@ -429,6 +432,57 @@ __device__ __forceinline__ uint32_t plan_multi(PLAN& P, const Program& G, uint32
     }
     __syncthreads();
     return sh.taken == limit ? slot : 0u;
+}
+
+// Planned through, every item waits for the bodies it waited for at first and
+// has no iterations left: with `iters` more it can be planned again.  Lanes t,
+// t + stride, ... ; `ready` (0 before) counts the items that wait for nothing,
+// which are in the ring from its start on.
+template <class PLAN>
+__device__ __forceinline__ void plan_again(PLAN& P, uint32_t nit, uint32_t iters, uint32_t t, uint32_t stride, uint32_t* ready)
+{
+    for (uint32_t j = t; j < nit; j += stride)
+        if (P.rearm(j, iters) < STATE_BODY)
+            P.push(__hip_atomic_fetch_add(ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), P.entry(j));
+}
+
+// A world's program, and the one for the rest of its iterations, with rows and
+// slots from kc * nit on and the entries after the first one's.  By one wave,
+// or (SEVERAL) by the whole workgroup.  Returns the slots of the first, with
+// those of the second in `rest_slots` (0: the ordering data was corrupt).
+template <bool SEVERAL, class PLAN>
+__device__ __forceinline__ uint32_t plan_world(PLAN& P, Program G, uint32_t nit, uint32_t nj, uint32_t kc, uint32_t rest,
+                                               uint32_t ready, uint32_t waves, ChainShared& sh, uint32_t& entries,
+                                               uint32_t& rest_slots)
+{
+    uint32_t first = 0u;
+    rest_slots = 0u;
+    for (uint32_t iters = kc;;) {   // (one copy of the planner: its instructions are what it waits for)
+        uint32_t ns;
+        if constexpr (SEVERAL) ns = plan_multi(P, G, nit, nj, iters, ready, waves, sh);
+        else ns = plan_single(P, G, nit, nj, iters, ready, entries);
+        if (first) {
+            rest_slots = ns;
+            return ns ? first : 0u;
+        }
+        if (rest == 0u || ns == 0u) return ns;
+        first = ns;
+        iters = rest;
+        G.rows += (size_t)kc * nit;
+        G.slots += (size_t)kc * nit;
+        if constexpr (SEVERAL) {
+            __syncthreads();   // sh.taken has been read
+            if (threadIdx.x == 0) sh.ready = sh.taken = sh.queued[0] = 0u;
+            __syncthreads();
+            plan_again(P, nit, rest, threadIdx.x, blockDim.x, &sh.ready);
+            __syncthreads();
+            ready = uniform(sh.ready);
+        } else {
+            plan_again(P, nit, rest, lane_id(), 64u, &sh.taken);   // (one wave's: no one else counts in it)
+            asm volatile("" ::: "memory");
+            ready = uniform(__hip_atomic_load(&sh.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        }
+    }
 }
 
 // Waves that run a world's rows: one for each `rows` rows of 64 its items fill
@@ -639,6 +693,15 @@ struct ChainProgram {
     GCU4 recs;
     uint32_t nslots, reps, nj, nacc, idle, jbase;
 };
+// the program after it (plan_world): rows and slots from `rows` on
+__device__ __forceinline__ ChainProgram rest_program(ChainProgram G, uint32_t rows, uint32_t nslots)
+{
+    G.rows += rows;
+    G.slots += rows;
+    G.nslots = nslots;
+    G.reps = 1u;
+    return G;
+}
 
 // Runs a program `reps` times over.  MULTI: the workgroup's waves run the rows
 // of a slot side by side, a workgroup barrier after each slot (every wave of

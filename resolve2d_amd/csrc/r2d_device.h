@@ -110,7 +110,8 @@ struct WorldChain {
     uint32_t pairs;     // manifolds of two points
     uint32_t flags;     // 1: updateTGSDepth is live; 2: some static body is an ordering body
     uint32_t slots;     // of its program
-    uint32_t entries;   // of its program
+    uint32_t rest_slots;   // ... and of the shorter one after it
+    uint32_t entries;   // of both
 };
 
 struct StepDev {
@@ -156,13 +157,15 @@ struct StepDev {
     uint32_t* it_color;                    // [cap_i] the candidates that collide, then colours (coloured order)
     uint64_t* cmask;                       // [2*N] colours used per body (coloured schedule)
     uint4* recs;                           // [8*cap_i] contact point and joint records (two of 64 B an item)
-    // the solver's program (r2d_chain.h): iterations one program covers, its
-    // rows and entries, and planning state when it does not fit LDS
-    uint32_t chain_iters;
-    uint2* prog_rows;                      // [chain_iters * cap_i]
-    uint32_t* prog_entries;                // [2 * chain_iters * cap_i]
-    uint2* prog_slots;                     // [chain_iters * cap_i]
-    uint4* prog_recs;                      // [8 * chain_iters * cap_i + 32 W] separate launches: records in program order
+    // the solver's program (r2d_chain.h): iterations it covers, those of the
+    // shorter one that ends a sub-step (0: none), their rows and entries, and
+    // planning state when it does not fit LDS
+    uint32_t chain_iters, chain_rest;
+    __host__ __device__ uint32_t chain_room() const { return chain_iters + chain_rest; }
+    uint2* prog_rows;                      // [chain_room * cap_i]
+    uint32_t* prog_entries;                // [2 * chain_room * cap_i]
+    uint2* prog_slots;                     // [chain_room * cap_i]
+    uint4* prog_recs;                      // [8 * chain_room * cap_i + 32 W] separate launches: records in program order
     uint4* plan_items;                     // [2 * cap_i]
     uint4* plan_ring;                      // [2 * cap_i]
     // the solve in separate launches

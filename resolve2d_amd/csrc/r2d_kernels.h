@@ -30,15 +30,29 @@ constexpr int WARM_VARIANT = SOLVE_VARIANTS, WARM_WIDE_VARIANT = SOLVE_VARIANTS 
 constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 2;
 
 // Iterations of a sub-step that one program covers: all of them up to 16,
-// else their largest divisor up to 16 (the program is then run that often).
-// A program's size grows with the iterations it covers.
-constexpr uint32_t CHAIN_ITERS_MAX = 16;
-inline uint32_t chain_iters(size_t iters)
+// else their largest divisor from 4 to 16 (the program is then run that
+// often), else 4, with a program of its own for the rest (17 = 4 x 4 + 1).  A
+// program's size grows with the iterations it covers, and what a program
+// covers runs overlapped: an iteration by itself costs the whole depth of the
+// world's contacts.  Four are enough for that (ms a step of 16 iterations by
+// programs of 1 / 4 / 8 / 16: 20-row pyramid 2.18 / 0.79 / 0.62 / 0.95, 60
+// rows 10.0 / 4.7 / 3.4 / 2.7, world of 387 bodies 0.58 / 0.61 / 0.64 / 0.99,
+// 97 worlds 0.78 / 0.80 / 1.09 / 1.34, 4,096-body pile 1.47 / 1.24 / 1.33 /
+// 1.54).  17 iterations, one at a time and by fours: pyramids of 20 and 60
+// rows 2.29 -> 0.96 and 9.5 -> 5.2 ms, 4,096-body pile 1.43 -> 1.31; shallow
+// worlds pay for planning more, 387 bodies 0.61 -> 0.65, 97 worlds 0.79 -> 0.89.
+constexpr uint32_t CHAIN_ITERS_MAX = 16, CHAIN_ITERS_ENOUGH = 4;
+struct ChainSplit {
+    uint32_t each, rest;   // iterations of the program, and of the one that ends a sub-step
+    uint32_t room() const { return each + rest; }
+};
+inline ChainSplit chain_split(size_t iters)
 {
-    if (iters == 0) return 1u;
-    for (uint32_t k = CHAIN_ITERS_MAX; k > 1u; --k)
-        if (iters % k == 0) return k;
-    return 1u;
+    if (iters == 0) return ChainSplit{1u, 0u};
+    if (iters <= CHAIN_ITERS_MAX) return ChainSplit{(uint32_t)iters, 0u};
+    for (uint32_t k = CHAIN_ITERS_MAX; k >= CHAIN_ITERS_ENOUGH; --k)
+        if (iters % k == 0) return ChainSplit{k, 0u};
+    return ChainSplit{CHAIN_ITERS_ENOUGH, (uint32_t)(iters % CHAIN_ITERS_ENOUGH)};
 }
 
 // The separate launches' chain: batches of at most this many worlds (one per

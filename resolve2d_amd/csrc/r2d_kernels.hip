@@ -2026,12 +2026,12 @@ __device__ __attribute__((noinline)) void chain_items(StepArgs KS, LU32 smem, R2
 }
 
 // a world's program in memory
-__device__ __forceinline__ ChainProgram chain_program(const StepDev& S, uint32_t ibase, uint32_t kc, uint32_t nslots,
+__device__ __forceinline__ ChainProgram chain_program(const StepDev& S, uint32_t ibase, uint32_t room, uint32_t nslots,
                                                       uint32_t reps, uint32_t nj, uint32_t M, uint32_t pairs)
 {
-    return ChainProgram{(GCU2)(S.prog_rows + (size_t)ibase * kc), (GCU32)(S.prog_entries + (size_t)ibase * 2u * kc),
-                        (GCU2)(S.prog_slots + (size_t)ibase * kc), (GCU4)(S.recs + (size_t)ibase * 8),
-                        nslots, reps, nj, M + pairs, 2u * kc * (nj + M), 0u};
+    return ChainProgram{(GCU2)(S.prog_rows + (size_t)ibase * room), (GCU32)(S.prog_entries + (size_t)ibase * 2u * room),
+                        (GCU2)(S.prog_slots + (size_t)ibase * room), (GCU4)(S.recs + (size_t)ibase * 8),
+                        nslots, reps, nj, M + pairs, 2u * room * (nj + M), 0u};
 }
 
 // The plan, and meanwhile the bodies into LDS and the point records: wave 0
@@ -2052,7 +2052,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const uint32_t w = uniform(sh.w), ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj),
                    M = uniform(sh.M), base = uniform(sh.base);
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + w);
-    const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, kc = S.chain_iters;
+    const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, kc = S.chain_iters, room = S.chain_room();
     const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n, 0u);
     const ChainBodies& C = L.C;
@@ -2061,9 +2061,9 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const bool chain = nit > 0u && sh.iters > 0u;
     const bool plan_in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words;
     Program G;
-    G.rows = (GU2)(S.prog_rows + (size_t)ibase * kc);
-    G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * kc);
-    G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
+    G.rows = (GU2)(S.prog_rows + (size_t)ibase * room);
+    G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * room);
+    G.slots = (GU2)(S.prog_slots + (size_t)ibase * room);
     PlanLds PL(L.rest, nit, waves);
     PlanGlb PG((GU4)(S.plan_items + 2 * (size_t)ibase), (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
     const uint32_t* lists = S.lists + 2 * (size_t)ibase;
@@ -2099,7 +2099,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     // the point that does nothing, after the others (an item slice has an item
     // to spare); by wave 1, whose chain may start without a barrier
     if (t - 64u < 4u) recs[(size_t)(nit + uniform(sh.pairs)) * 4u + (t - 64u)] = idle_word((int)(t - 64u));
-    if (t == 64u) G.entries[2u * kc * nit] = nit + uniform(sh.pairs);
+    if (t == 64u) G.entries[2u * room * nit] = nit + uniform(sh.pairs);
     auto build = [&](uint32_t t0, uint32_t stride) {
         for (uint32_t i = t0; i < n; i += stride) {
             C.m[i] = f3v{D.mx[i], D.my[i], D.L[i]};
@@ -2116,11 +2116,10 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const uint32_t plan_words = (plan_lds_words(nit, 1u) + 1u) & ~1u;
     const bool follow = chain && waves == 1u && plan_in_lds && sh.iters == kc && plan_words < L.rest_words &&
                         L.consts + 2u * (nacc + 1u) <= L.rest_words - plan_words;
-    uint32_t ns = 1u;
+    uint32_t ns = 1u, rest_slots = 0u, entries = 0u;
     if (follow) {
         sh.beside = plan_words;   // the same from every thread
         if (t < 64u) {
-            uint32_t entries;
             ns = plan_single<true>(PL, G, nit, nj, kc, ready, entries, &sh.progress);
         } else {
             constexpr uint32_t OTHERS = (uint32_t)T / 64u - 1u;
@@ -2134,7 +2133,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
                 waves_meet(&sh.met, OTHERS, 2u);
             }
             if (t < 128u) {
-                ChainProgram P = chain_program(S, ibase, kc, 0u, 1u, nj, M, uniform(sh.pairs));
+                ChainProgram P = chain_program(S, ibase, room, 0u, 1u, nj, M, uniform(sh.pairs));
                 const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
                 for (uint32_t run = 0u;;) {
                     const uint32_t p = uniform(__hip_atomic_load(&sh.progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
@@ -2154,18 +2153,19 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
             }
         }
     } else if (chain && waves > 1u) {
-        ns = plan_in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh)
-                         : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
+        ns = plan_in_lds ? plan_world<true>(PL, G, nit, nj, kc, S.chain_rest, ready, waves, sh, entries, rest_slots)
+                         : plan_world<true>(PG, G, nit, nj, kc, S.chain_rest, ready, waves, sh, entries, rest_slots);
         build(t, T);
     } else if (t < 64u) {
-        uint32_t entries;
         if (chain)
-            ns = plan_in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
+            ns = plan_in_lds ? plan_world<false>(PL, G, nit, nj, kc, S.chain_rest, ready, 1u, sh, entries, rest_slots)
+                             : plan_world<false>(PG, G, nit, nj, kc, S.chain_rest, ready, 1u, sh, entries, rest_slots);
     } else {
         build(t - 64u, T - 64u);
     }
     if (t == 0) {
         sh.nslots = ns;
+        sh.rest_slots = rest_slots;
         sh.failed = ns == 0u;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2233,19 +2233,23 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
             __syncthreads();
         }
         if (iters == 0u) continue;
-        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters;
+        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters, rest_slots = uniform(sh.rest_slots);
         const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
         const bool in_lds = L.holds(M + uniform(sh.pairs));
-        const ChainProgram G = chain_program(S, ibase, kc, uniform(sh.nslots), iters / kc, nj, M, uniform(sh.pairs));
+        ChainProgram G = chain_program(S, ibase, S.chain_room(), uniform(sh.nslots), iters / kc, nj, M, uniform(sh.pairs));
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
-        if (chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u) {
-            if (in_lds) chain_lds<true, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
-            else chain_lds_accg<true, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
-        } else if (threadIdx.x < 64u) {
-            if (in_lds) chain_lds<false, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
-            else chain_lds_accg<false, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
+        const bool several = chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u;
+        for (uint32_t part = 0; part < (rest_slots ? 2u : 1u); ++part) {
+            if (part) G = rest_program(G, kc * (nj + M), rest_slots);
+            if (several) {
+                if (in_lds) chain_lds<true, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
+                else chain_lds_accg<true, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
+            } else if (threadIdx.x < 64u) {
+                if (in_lds) chain_lds<false, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
+                else chain_lds_accg<false, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
+            }
         }
         __syncthreads();
     }
@@ -2274,15 +2278,15 @@ __device__ __forceinline__ GF3 world_momenta(const StepDev& S, const WorldDev& D
 }
 
 // a world's records in program order: entries, then joints, in blocks of four, each last one
-// perhaps not full, then the idle point's (up to 8 places beyond 2 kc an item)
+// perhaps not full, then the idle point's (up to 8 places beyond 2 chain_room an item)
 __device__ __forceinline__ GU4 world_records(const StepDev& S, uint32_t w, uint32_t ibase)
 {
-    return (GU4)(S.prog_recs + (size_t)ibase * 8u * S.chain_iters + (size_t)w * 32u);
+    return (GU4)(S.prog_recs + (size_t)ibase * 8u * S.chain_room() + (size_t)w * 32u);
 }
 
 __device__ __forceinline__ GU32 world_entries(const StepDev& S, uint32_t w, uint32_t ibase)
 {
-    return (GU32)(S.prog_entries + (size_t)ibase * 2u * S.chain_iters + (size_t)w * 8u);
+    return (GU32)(S.prog_entries + (size_t)ibase * 2u * S.chain_room() + (size_t)w * 8u);
 }
 // where the joints' records start
 __device__ __forceinline__ uint32_t joint_entries(uint32_t entries) { return (entries + 3u) & ~3u; }
@@ -2342,6 +2346,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, nj = (uint32_t)S.worlds[w].njoints;
     if (S.w_status[w] != 0 || nit == 0u) return;
     const uint32_t t = threadIdx.x, kc = S.chain_iters, waves = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
+    const size_t rows = (size_t)ibase * S.chain_room();
     const bool in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= lds_words;
     if (t == 0) {
         sh.ready = sh.taken = sh.entries = 0u;
@@ -2349,9 +2354,9 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     }
     __syncthreads();
     Program G;
-    G.rows = (GU2)(S.prog_rows + (size_t)ibase * kc);
+    G.rows = (GU2)(S.prog_rows + rows);
     G.entries = world_entries(S, w, ibase);
-    G.slots = (GU2)(S.prog_slots + (size_t)ibase * kc);
+    G.slots = (GU2)(S.prog_slots + rows);
     const GU4 items = (GU4)(S.plan_items + 2 * (size_t)ibase);
     PlanLds PL((LU32)smem, nit, waves);
     PlanGlb PG(items, (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
@@ -2368,13 +2373,17 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     if (in_lds) start(PL, true); else start(PG, false);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
-    uint32_t ns = 0u, entries = 0u;
+    uint32_t ns = 0u, rest_slots = 0u, entries = 0u;
+    const uint32_t rest = S.chain_rest;
     if (waves > 1u)
-        ns = in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh) : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
+        ns = in_lds ? plan_world<true>(PL, G, nit, nj, kc, rest, ready, waves, sh, entries, rest_slots)
+                    : plan_world<true>(PG, G, nit, nj, kc, rest, ready, waves, sh, entries, rest_slots);
     else if (t < 64u)
-        ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
+        ns = in_lds ? plan_world<false>(PL, G, nit, nj, kc, rest, ready, 1u, sh, entries, rest_slots)
+                    : plan_world<false>(PG, G, nit, nj, kc, rest, ready, 1u, sh, entries, rest_slots);
     if (t == 0) {
         S.w_chain[w].slots = ns;
+        S.w_chain[w].rest_slots = rest_slots;
         S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2530,17 +2539,22 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     }
     __syncthreads();
     if (iters > 0u) {
-        const ChainProgram G{(GCU2)(S.prog_rows + (size_t)ibase * kc), entries, (GCU2)(S.prog_slots + (size_t)ibase * kc),
-                             (GCU4)prog, W.slots, iters / kc, nj, nacc, jbase + nj, jbase};
+        const size_t rows = (size_t)ibase * S.chain_room();
+        ChainProgram G{(GCU2)(S.prog_rows + rows), entries, (GCU2)(S.prog_slots + rows), (GCU4)prog, W.slots, iters / kc,
+                       nj, nacc, jbase + nj, jbase};
         const bool fix = W.flags != 0u;
-        if (chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
-            if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
-            else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);
-        } else if (t < 64u) {
-            if (a_lds) chain_lds<false, WARM, true>(G, m, nc, acc, fix, sub_dt);
-            else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
-            else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
+        const bool several = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u;
+        for (uint32_t part = 0; part < (W.rest_slots ? 2u : 1u); ++part) {
+            if (part) G = rest_program(G, kc * nit, W.rest_slots);
+            if (several) {
+                if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
+                else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
+                else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);
+            } else if (t < 64u) {
+                if (a_lds) chain_lds<false, WARM, true>(G, m, nc, acc, fix, sub_dt);
+                else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
+                else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
+            }
         }
         __syncthreads();
     }
