@@ -29,6 +29,20 @@ FLAGS = [
 ]
 
 
+def verify(out_dir: str) -> list:
+    """Compile every source with the compiler's machine verifier on (a minute
+    and a half, so not part of build) and return what it refused: (source,
+    messages).  A kernel that outgrew its registers has come out of the
+    compiler with an undefined register, and faulted."""
+    runs = []
+    for src in SOURCES:
+        cmd = [HIPCC] + FLAGS + ["-Xarch_device", "-mllvm=-verify-machineinstrs", "-c", os.path.join(CSRC, src), "-o",
+                                 os.path.join(out_dir, src + ".o")]
+        runs.append((src, subprocess.Popen(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True)))
+    done = [(src, p.communicate()[1], p.returncode) for src, p in runs]
+    return [(src, err) for src, err, rc in done if rc != 0]
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     objs = []
