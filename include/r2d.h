@@ -305,7 +305,12 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
 /* Test hook with no counterpart in the reference: the rules by which the host
  * lays out and launches steps, for given sizes (no device needed).
  * rule 0: in {collision iterations}; out {iterations that a solver program
- * covers, iterations of the program that ends a sub-step}. */
+ * covers, iterations of the program that ends a sub-step}.
+ * rule 1: in {bodies, buckets, worlds, joints, cell entries, raw candidates,
+ * manifolds, solver items, iterations of the programs}; out {bytes of the step
+ * scratch that holds them}.
+ * rule 2: in {cell entries, raw candidates, manifolds, solver items,
+ * iterations of the programs}; out {bytes of the one-kernel step's slices}. */
 int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out);
 
 /* Measurement hook with no counterpart in the reference: the device's

@@ -258,6 +258,8 @@ struct r2d_ctx {
     StepDev S{};
     uint32_t cap_n = 0, cap_b = 0, cap_w = 0, cap_j = 0;
     uint32_t cap_e = 0, cap_r = 0, cap_m = 0, cap_i = 0, cap_k = 0;
+    uint32_t chain_most = CHAIN_ITERS_MAX, fchain_most = CHAIN_ITERS_MAX;   // iterations a program of the arenas may cover
+    size_t scratch_limit = 0;
     WorldDev* dworlds = nullptr;
     size_t dworlds_cap = 0;
     uint32_t* hcounters = nullptr;     // pinned
@@ -717,34 +719,35 @@ WorldDev make_desc(r2d_world* w)
 }
 
 // the iterations of each program of a call's worlds
-void set_split(StepDev& S, size_t iters)
+void set_split(StepDev& S, const ChainSplit& c)
 {
-    const ChainSplit c = chain_split(iters);
     S.chain_iters = c.each;
     S.chain_rest = c.rest;
 }
 
-// carve the step scratch for the current capacities
-int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, uint32_t e, uint32_t r, uint32_t m,
-                   uint32_t it, uint32_t k)
+// Device memory of the step scratch.  R2D_SCRATCH_LIMIT (bytes) refuses a
+// larger piece, as a full device does.
+hipError_t scratch_alloc(const r2d_ctx* c, void** p, size_t bytes)
 {
-    if (k <= c->cap_k && n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w && j <= c->cap_j && e <= c->cap_e && r <= c->cap_r &&
-        m <= c->cap_m && it <= c->cap_i && c->arena)
-        return R2D_OK;
-    auto grow = [](uint32_t have, uint32_t need) {
-        if (need <= have) return have;
-        uint64_t v = (uint64_t)need + need / 2 + 256;
-        return (uint32_t)std::min<uint64_t>(v, 0xffffff00ull);
-    };
-    c->cap_k = std::max(c->cap_k, k);
-    c->cap_n = grow(c->cap_n, n); c->cap_b = grow(c->cap_b, b); c->cap_w = grow(c->cap_w, wn);
-    c->cap_j = grow(c->cap_j, j); c->cap_e = grow(c->cap_e, e); c->cap_r = grow(c->cap_r, r);
-    c->cap_m = grow(c->cap_m, m); c->cap_i = grow(c->cap_i, std::max(it, c->cap_m + c->cap_j));
-    size_t N = c->cap_n, B = c->cap_b, W = c->cap_w, E = c->cap_e, R = c->cap_r, M = c->cap_m, I = c->cap_i;
-    size_t off = 0;
-    std::vector<std::pair<void**, size_t>> parts;
-    StepDev& S = c->S;
-    auto add = [&](void** p, size_t bytes) { parts.push_back({p, bytes}); };
+    const hipError_t e = c->scratch_limit && bytes > c->scratch_limit ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();   // answered here: not an error of a later launch
+    }
+    return e;
+}
+
+// Elements the step scratch holds: bodies, buckets, worlds, joints, cell
+// entries, raw candidates, manifolds, solver items, iterations of programs
+struct ScratchCaps {
+    size_t n, b, w, j, e, r, m, i, k;
+};
+
+// every array of the step scratch: add(pointer, bytes)
+template <class Add>
+void scratch_arrays(StepDev& S, const ScratchCaps& c, Add add)
+{
+    const size_t N = c.n, B = c.b, W = c.w, E = c.e, R = c.r, M = c.m, I = c.i, K = c.k;
     add((void**)&S.bworld, N * 4);
     add((void**)&S.cx0, N * 8); add((void**)&S.cy0, N * 8);
     add((void**)&S.cnx, N * 4); add((void**)&S.cny, N * 4);
@@ -761,16 +764,15 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.m_ref, M * 4); add((void**)&S.m_inc, M * 4);
     add((void**)&S.m_nx, M * 4); add((void**)&S.m_ny, M * 4); add((void**)&S.m_fric, M * 4);
     add((void**)&S.m_prev1, M * 4); add((void**)&S.m_prev2, M * 4); add((void**)&S.m_valid, M * 4);
-    add((void**)&S.m_pt, (size_t)MP_NFIELDS * 2 * M * 4);
+    add((void**)&S.m_pt, MP_NFIELDS * 2 * M * 4);
     add((void**)&S.w_man_begin, (W + 1) * 4); add((void**)&S.w_item_base, (W + 1) * 4);
     add((void**)&S.w_status, (W + 1) * 4); add((void**)&S.w_order, (W + 1) * 4);
     add((void**)&S.it_r0, I * 4); add((void**)&S.it_r1, I * 4);
     add((void**)&S.it_k0, I * 4); add((void**)&S.it_k1, I * 4);
     add((void**)&S.deg, (N + 1) * 4); add((void**)&S.deg_off, (N + 1) * 4); add((void**)&S.deg_fill, (N + 1) * 4);
     add((void**)&S.lists, 2 * I * 4);
-    add((void**)&S.it_color, I * 4);
+    add((void**)&S.it_color, std::max(I, M) * 4);   // also lists the candidates that collide
     add((void**)&S.recs, I * 128);
-    const size_t K = c->cap_k;
     add((void**)&S.prog_rows, K * I * 8); add((void**)&S.prog_entries, (2 * K * I + 8 * W) * 4); add((void**)&S.prog_slots, K * I * 8);
     add((void**)&S.prog_recs, 2 * K * I * 64 + W * 512);
     add((void**)&S.plan_items, 2 * I * 16); add((void**)&S.plan_ring, 2 * I * 16);
@@ -780,18 +782,61 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
     add((void**)&S.counters, 64 * 4);
     add((void**)&S.partials, 1024 * 4);
     add((void**)&S.scan_state, SCANS * SCAN_TILES * 8); add((void**)&S.scan_ticket, SCANS * 4);
-    for (auto& p : parts) off += align256(p.second);
+}
+
+// Iterations that programs of the separate launches may cover (most), largest
+// first, and whether the arrays get room to grow.  An item takes 220 bytes and
+// 152 more for each iteration of its programs, 2.7 KB in all with 16: where
+// the device has no room for that, the programs are made shorter (the same
+// bits; 60-row pyramid, 16 iterations by 16 / 4 / 1: 2.7 / 4.7 / 10 ms).
+constexpr struct {
+    uint32_t most;
+    bool room;
+} kScratchTries[] = {{CHAIN_ITERS_MAX, true}, {CHAIN_SHORT, true}, {1u, true}, {1u, false}};
+constexpr size_t kProgramPlaces = (size_t)1 << 30;   // places of a program that its entries can name
+
+// carve the step scratch for the current capacities; iters: the call's iterations
+int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, uint32_t e, uint32_t r, uint32_t m,
+                   uint32_t it, size_t iters)
+{
+    if (chain_split(iters, c->chain_most).room() <= c->cap_k && n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w &&
+        j <= c->cap_j && e <= c->cap_e && r <= c->cap_r && m <= c->cap_m && it <= c->cap_i && c->arena)
+        return R2D_OK;
     if (c->arena) {
         HIPCHK(hipStreamSynchronize(c->stream));
         HIPCHK(hipFree(c->arena));
         c->arena = nullptr;
     }
-    if (hipMalloc(&c->arena, off) != hipSuccess) { c->arena = nullptr; c->arena_bytes = 0; return R2D_E_OOM; }
-    c->arena_bytes = off;
-    char* base = (char*)c->arena;
-    size_t o = 0;
-    for (auto& p : parts) { *p.first = base + o; o += align256(p.second); }
-    HIPCHK(hipMemsetAsync(c->arena, 0, off, c->stream));
+    StepDev& S = c->S;
+    ScratchCaps caps{};
+    size_t bytes = 0;
+    for (const auto& t : kScratchTries) {
+        auto grow = [&](uint32_t have, uint32_t need) -> size_t {
+            if (need <= have) return t.room ? have : need;
+            const uint64_t v = t.room ? (uint64_t)need + need / 2 + 256 : need;
+            return (size_t)std::min<uint64_t>(v, 0xffffff00ull);
+        };
+        caps = ScratchCaps{grow(c->cap_n, n), grow(c->cap_b, b), grow(c->cap_w, wn), grow(c->cap_j, j), grow(c->cap_e, e),
+                           grow(c->cap_r, r), grow(c->cap_m, m), grow(c->cap_i, it), chain_split(iters, t.most).room()};
+        // what longer calls got, unless it is in the way now
+        if (t.most == CHAIN_ITERS_MAX && c->chain_most == CHAIN_ITERS_MAX) caps.k = std::max<size_t>(caps.k, c->cap_k);
+        if (2 * caps.k * caps.i + 8 * caps.w > kProgramPlaces) continue;
+        bytes = 0;
+        scratch_arrays(S, caps, [&](void**, size_t x) { bytes += align256(x); });
+        if (scratch_alloc(c, &c->arena, bytes) == hipSuccess) {
+            c->chain_most = t.most;
+            break;
+        }
+    }
+    if (!c->arena) { c->arena_bytes = 0; return R2D_E_OOM; }
+    c->arena_bytes = bytes;
+    char* at = (char*)c->arena;
+    scratch_arrays(S, caps, [&](void** p, size_t x) { *p = at; at += align256(x); });
+    c->cap_n = (uint32_t)caps.n; c->cap_b = (uint32_t)caps.b; c->cap_w = (uint32_t)caps.w; c->cap_j = (uint32_t)caps.j;
+    c->cap_e = (uint32_t)caps.e; c->cap_r = (uint32_t)caps.r; c->cap_m = (uint32_t)caps.m; c->cap_i = (uint32_t)caps.i;
+    c->cap_k = (uint32_t)caps.k;
+    const size_t W = caps.w;
+    HIPCHK(hipMemsetAsync(c->arena, 0, bytes, c->stream));
     S.cap_e = c->cap_e; S.cap_r = c->cap_r; S.cap_m = c->cap_m; S.cap_i = c->cap_i;
     if (c->hstatus_cap < W + 1) {
         if (c->hstatus) HIPCHK(hipHostFree(c->hstatus));
@@ -905,40 +950,54 @@ uint32_t grow_cap(uint32_t have, uint64_t need)
     return (uint32_t)std::min<uint64_t>(v, 0xffffff00ull);
 }
 
+// its arrays (E cell entries, R raw candidates, M manifolds, I solver items, K
+// iterations of programs): add(pointer, bytes)
+template <class Add>
+void fused_arrays(StepDev& F, size_t E, size_t R, size_t M, size_t I, size_t K, Add add)
+{
+    add((void**)&F.bkt_items, E * 4); add((void**)&F.bkt_sorted, E * 4);
+    add((void**)&F.ent_body, E * 4); add((void**)&F.ent_bkt, E * 4);
+    add((void**)&F.ent_cnt, E * 4);
+    add((void**)&F.cand, R * 16); add((void**)&F.cand_flag, R * 4);
+    add((void**)&F.m_ref, M * 4); add((void**)&F.m_inc, M * 4);
+    add((void**)&F.m_nx, M * 4); add((void**)&F.m_ny, M * 4); add((void**)&F.m_fric, M * 4);
+    add((void**)&F.m_prev1, M * 4); add((void**)&F.m_prev2, M * 4); add((void**)&F.m_valid, M * 4);
+    add((void**)&F.m_pt, MP_NFIELDS * 2 * M * 4);
+    add((void**)&F.it_r0, I * 4); add((void**)&F.it_r1, I * 4);
+    add((void**)&F.it_k0, I * 4); add((void**)&F.it_k1, I * 4);
+    add((void**)&F.lists, 2 * I * 4);
+    add((void**)&F.recs, I * 128);
+    add((void**)&F.prog_rows, K * I * 8); add((void**)&F.prog_entries, 2 * K * I * 4);
+    add((void**)&F.prog_slots, K * I * 8);
+    add((void**)&F.plan_items, 2 * I * 16); add((void**)&F.plan_ring, 2 * I * 16);
+}
+
 // The fused arena: every world's slices of the entry, candidate, manifold and
 // item arrays.  With `preserve` the manifold arrays keep their contents (the
 // slices of worlds that finished before an overflow relaunch stay readable).
-int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64_t ti, uint32_t iters, bool preserve)
+int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64_t ti, size_t iters, bool preserve)
 {
-    if (te <= c->fcap_e && tr <= c->fcap_r && tm <= c->fcap_m && ti <= c->fcap_i && iters <= c->fcap_k && c->farena)
+    if (te <= c->fcap_e && tr <= c->fcap_r && tm <= c->fcap_m && ti <= c->fcap_i &&
+        chain_split(iters, c->fchain_most).room() <= c->fcap_k && c->farena)
         return R2D_OK;
     if (std::max(std::max(te, tr), std::max(tm, ti)) >= 0x7fffff00ull) return R2D_E_CAPACITY;
     const uint32_t E = grow_cap(c->fcap_e, te), R = grow_cap(c->fcap_r, tr), M = grow_cap(c->fcap_m, tm),
-                   I = grow_cap(c->fcap_i, ti), K = std::max(c->fcap_k, iters);
+                   I = grow_cap(c->fcap_i, ti);
     StepDev F{};
-    std::vector<std::pair<void**, size_t>> parts;
-    auto add = [&](void** p, size_t bytes) { parts.push_back({p, bytes}); };
-    add((void**)&F.bkt_items, (size_t)E * 4); add((void**)&F.bkt_sorted, (size_t)E * 4);
-    add((void**)&F.ent_body, (size_t)E * 4); add((void**)&F.ent_bkt, (size_t)E * 4);
-    add((void**)&F.ent_cnt, (size_t)E * 4);
-    add((void**)&F.cand, (size_t)R * 16); add((void**)&F.cand_flag, (size_t)R * 4);
-    add((void**)&F.m_ref, (size_t)M * 4); add((void**)&F.m_inc, (size_t)M * 4);
-    add((void**)&F.m_nx, (size_t)M * 4); add((void**)&F.m_ny, (size_t)M * 4); add((void**)&F.m_fric, (size_t)M * 4);
-    add((void**)&F.m_prev1, (size_t)M * 4); add((void**)&F.m_prev2, (size_t)M * 4); add((void**)&F.m_valid, (size_t)M * 4);
-    add((void**)&F.m_pt, (size_t)MP_NFIELDS * 2 * M * 4);
-    add((void**)&F.it_r0, (size_t)I * 4); add((void**)&F.it_r1, (size_t)I * 4);
-    add((void**)&F.it_k0, (size_t)I * 4); add((void**)&F.it_k1, (size_t)I * 4);
-    add((void**)&F.lists, 2 * (size_t)I * 4);
-    add((void**)&F.recs, (size_t)I * 128);
-    add((void**)&F.prog_rows, (size_t)K * I * 8); add((void**)&F.prog_entries, 2 * (size_t)K * I * 4);
-    add((void**)&F.prog_slots, (size_t)K * I * 8);
-    add((void**)&F.plan_items, 2 * (size_t)I * 16); add((void**)&F.plan_ring, 2 * (size_t)I * 16);
-    size_t bytes = 0;
-    for (auto& p : parts) bytes += align256(p.second);
     void* arena = nullptr;
-    if (hipMalloc(&arena, bytes) != hipSuccess) return R2D_E_OOM;
-    size_t o = 0;
-    for (auto& p : parts) { *p.first = (char*)arena + o; o += align256(p.second); }
+    size_t bytes = 0;
+    uint32_t K = 0, most = 0;
+    for (const auto& t : kScratchTries) {   // shorter programs where memory holds no longer ones
+        most = t.most;
+        K = chain_split(iters, most).room();
+        if (most == CHAIN_ITERS_MAX && c->fchain_most == CHAIN_ITERS_MAX) K = std::max(K, c->fcap_k);
+        bytes = 0;
+        fused_arrays(F, E, R, M, I, K, [&](void**, size_t x) { bytes += align256(x); });
+        if (scratch_alloc(c, &arena, bytes) == hipSuccess) break;
+    }
+    if (!arena) return R2D_E_OOM;
+    char* at = (char*)arena;
+    fused_arrays(F, E, R, M, I, K, [&](void** p, size_t x) { *p = at; at += align256(x); });
     StepDev& O = c->SF;
     if (c->farena && preserve) {
         const size_t om = c->fcap_m;
@@ -957,6 +1016,7 @@ int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64
     c->farena = arena;
     c->farena_bytes = bytes;
     c->fcap_e = E; c->fcap_r = R; c->fcap_m = M; c->fcap_i = I; c->fcap_k = K;
+    c->fchain_most = most;
     O.bkt_items = F.bkt_items; O.bkt_sorted = F.bkt_sorted; O.ent_body = F.ent_body; O.ent_bkt = F.ent_bkt;
     O.ent_cnt = F.ent_cnt; O.cand = F.cand; O.cand_flag = F.cand_flag; O.m_ref = F.m_ref; O.m_inc = F.m_inc; O.m_nx = F.m_nx; O.m_ny = F.m_ny;
     O.m_fric = F.m_fric; O.m_prev1 = F.m_prev1; O.m_prev2 = F.m_prev2; O.m_valid = F.m_valid; O.m_pt = F.m_pt;
@@ -1074,7 +1134,7 @@ int fused_layout(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
     }
     // as much again free for worlds that outgrow their slices during the call
-    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, chain_split(b.iters).room(), false))) return rc;
+    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, b.iters, false))) return rc;
     // workgroups take the largest worlds first (the longest steps start first)
     c->forder.resize(nw);
     for (size_t i = 0; i < nw; ++i) c->forder[i] = (uint32_t)i;
@@ -1114,7 +1174,7 @@ int fused_regrow(r2d_ctx* c, Batch& b)
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
         c->hstatus[i] = WS_OK;
     }
-    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, chain_split(b.iters).room(), true);
+    int rc = ensure_fused_arena(c, te + te / 2, tr + tr / 2, tm + tm / 2, ti + ti / 2, b.iters, true);
     if (rc) return rc;
     if ((rc = fused_upload_tables(c))) return rc;
     HIPCHK(hipMemcpyAsync(c->S.w_status, c->hstatus, nw * 4, hipMemcpyHostToDevice, c->stream));
@@ -1270,15 +1330,16 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     if (fused) {
         // the step scratch holds the per-body and per-world arrays; the
         // worlds' slices live in the fused arena
-        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1, 1)))
+        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1, 0)))
             return rc;
         return fused_layout(c, b);
     }
     uint32_t est_e = std::max<uint32_t>(c->cap_e, (uint32_t)(4 * b.N + 1024));
     uint32_t est_r = std::max<uint32_t>(c->cap_r, (uint32_t)(8 * b.N + 1024));
     uint32_t est_m = std::max<uint32_t>(c->cap_m, (uint32_t)(4 * b.N + 1024));
-    return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m,
-                          (uint32_t)b.J + est_m, chain_split(b.iters).room());
+    // convex bodies touch at most three others each on average; settled piles and stacks have 1.4 to 2.3 manifolds a body
+    uint32_t est_i = std::max<uint32_t>(c->cap_i, (uint32_t)(b.J + 2 * b.N + 1024));
+    return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m, est_i, b.iters);
 }
 
 // sum the phase times of the timed steps recorded so far
@@ -1315,7 +1376,7 @@ int batch_launch(r2d_ctx* c, Batch& b)
     StepDev S = c->S;
     S.nb = (uint32_t)b.N; S.nworlds = (uint32_t)nw; S.nbuckets = (uint32_t)b.B; S.njoints = (uint32_t)b.J;
     S.worlds = c->dworlds;
-    set_split(S, b.iters);
+    set_split(S, chain_split(b.iters, c->chain_most));
     const Streams ss = c->streams();
     const uint32_t sub = (uint32_t)b.sub, iters = (uint32_t)b.iters;
     auto eager_phase = [&](int ph) { launch_phase(S, ss, ph, b.dt, sub, iters, b.plan); };
@@ -1389,7 +1450,7 @@ int fused_launch(r2d_ctx* c, Batch& b)
     StepDev F = fused_view(c);
     F.nb = (uint32_t)b.N; F.nworlds = (uint32_t)nw; F.nbuckets = (uint32_t)b.B; F.njoints = (uint32_t)b.J;
     F.worlds = c->dworlds;
-    set_split(F, b.iters);
+    set_split(F, chain_split(b.iters, c->fchain_most));
     if (c->profiling) {
         // The timing buffers grow rarely and by a lot: a launch that follows a
         // hipMalloc closely can stall all of its waves for several ms at once
@@ -1561,17 +1622,13 @@ int batch_wait(r2d_ctx* c, Batch& b)
         }
         for (int k = 0; k < 4; ++k) c->last_counts[k] = c->hcounters[k];
         if (c->hcounters[C_OVERFLOW]) {
-            uint32_t e = std::max(c->hcounters[C_ENTRIES], c->cap_e);
-            uint32_t r = std::max(c->hcounters[C_RAW], c->cap_r);
-            uint32_t m = std::max(c->hcounters[C_MANIFOLDS], c->cap_m);
-            uint32_t it = std::max(c->hcounters[C_ITEMS], c->cap_i);
+            uint32_t e = c->cap_e, r = c->cap_r, m = c->cap_m, it = c->cap_i;
             // a count is only known once the counts before it fit; grow the first short buffer
-            if (c->hcounters[C_OVERFLOW] & 1u) e = c->hcounters[C_ENTRIES] * 2;
-            if (c->hcounters[C_OVERFLOW] & 2u) r = c->hcounters[C_RAW] * 2;
-            if (c->hcounters[C_OVERFLOW] & 4u) m = c->hcounters[C_MANIFOLDS] * 2;
-            if (c->hcounters[C_OVERFLOW] & 8u) it = c->hcounters[C_ITEMS] * 2;
-            int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e + 1, r + 1,
-                                    m + 1, it + 1, chain_split(b.iters).room());
+            if (c->hcounters[C_OVERFLOW] & 1u) e = c->hcounters[C_ENTRIES] * 2 + 1;
+            if (c->hcounters[C_OVERFLOW] & 2u) r = c->hcounters[C_RAW] * 2 + 1;
+            if (c->hcounters[C_OVERFLOW] & 4u) m = c->hcounters[C_MANIFOLDS] * 2 + 1;
+            if (c->hcounters[C_OVERFLOW] & 8u) it = c->hcounters[C_ITEMS] + c->hcounters[C_ITEMS] / 4;
+            int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e, r, m, it, b.iters);
             if (rc) return rc;
         }
         if (b.done >= b.steps) break;
@@ -1880,6 +1937,7 @@ R2D_EXPORT int r2d_ctx_create(int device, r2d_ctx** out)
     if (const char* e = std::getenv("R2D_NO_FUSED")) c->fused_enabled = !(e[0] == '1');
     set_solve_smem_limit();
     if (const char* e = std::getenv("R2D_NO_GRAPH")) c->use_graph = !(e[0] == '1');
+    if (const char* e = std::getenv("R2D_SCRATCH_LIMIT")) c->scratch_limit = (size_t)std::strtoull(e, nullptr, 10);
     if (const char* e = std::getenv("R2D_TRACE_KERNELS")) {
         if (e[0] == '1') {
             c->trace = new (std::nothrow) KernelTrace();
@@ -2239,7 +2297,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     WorldDev* ddesc = nullptr;
     static_layout(base, &F, &ddesc);
     F.nb = n; F.nbuckets = tb; F.njoints = nj;
-    set_split(F, iters);
+    set_split(F, chain_split(iters));
     // host values the asynchronous uploads read; the call waits for the
     // stream before they go out of scope
     WorldDev d = w->desc;
@@ -2734,6 +2792,16 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
         const ChainSplit s = chain_split(in[0]);
         out[0] = s.each;
         out[1] = s.rest;
+        return R2D_OK;
+    }
+    case 1:
+    case 2: {
+        StepDev S{};
+        size_t bytes = 0;
+        auto add = [&](void**, size_t x) { bytes += align256(x); };
+        if (rule == 1) scratch_arrays(S, ScratchCaps{in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], in[8]}, add);
+        else fused_arrays(S, in[0], in[1], in[2], in[3], in[4], add);
+        out[0] = bytes;
         return R2D_OK;
     }
     }

@@ -55,16 +55,16 @@ typedef const R2D_GLB u4v* GCU4;
 //     14-15 inverse inertias
 //   fixed position (2): 2-3 direction, 4 bias, 5 / 6 limits, 12 inverse mass
 //   motor (3): 2 inertia, 3 target, 4 beta, 5 / 6 limits, 7 torque
-constexpr uint32_t PR_INDEX = (1u << 26) - 1u;
+constexpr uint32_t PR_INDEX = (1u << 29) - 1u;   // more bodies than memory holds the scratch of
 enum : uint32_t {
     PR_WRITE = 1u << 31,      // word 0 / 1, contacts: body a / b is an ordering body (its momentum is written)
                               // and this is the manifold's first point
     PR_STATIC = 1u << 30,     // word 0 / 1, contacts: the body is static (an ordering one gets "+= 0")
-    PR_JOINT = 1u << 26,      // word 0
-    PR_SELF = 1u << 27,       // word 0, joints: both ends on one body
-    PR_SKIP = 1u << 28,       // word 0, joints: changes nothing this sub-step
-    PR_WARM = 1u << 26,       // word 1, contacts: warm started (no minimum impulse)
-    PR_TYPE_SHIFT = 28        // word 1, joints: type
+    PR_JOINT = 1u << 29,      // word 0
+    PR_SELF = 1u << 31,       // word 0, joints: both ends on one body
+    PR_SKIP = 1u << 30,       // word 0, joints: changes nothing this sub-step
+    PR_WARM = 1u << 29,       // word 1, contacts: warm started (no minimum impulse)
+    PR_TYPE_SHIFT = 30        // word 1, joints: type
 };
 
 // the record of a lane without a point: bias -1, no body to write

@@ -46,11 +46,14 @@ struct ChainSplit {
     uint32_t each, rest;   // iterations of the program, and of the one that ends a sub-step
     uint32_t room() const { return each + rest; }
 };
-inline ChainSplit chain_split(size_t iters)
+// most: a smaller bound where memory holds no more (CHAIN_SHORT: fours, and
+// ones; 1: ones)
+constexpr uint32_t CHAIN_SHORT = 2 * CHAIN_ITERS_ENOUGH - 1;
+inline ChainSplit chain_split(size_t iters, uint32_t most = CHAIN_ITERS_MAX)
 {
-    if (iters == 0) return ChainSplit{1u, 0u};
-    if (iters <= CHAIN_ITERS_MAX) return ChainSplit{(uint32_t)iters, 0u};
-    for (uint32_t k = CHAIN_ITERS_MAX; k >= CHAIN_ITERS_ENOUGH; --k)
+    if (iters == 0 || most < CHAIN_SHORT) return ChainSplit{1u, 0u};
+    if (iters <= most) return ChainSplit{(uint32_t)iters, 0u};
+    for (uint32_t k = most; k >= CHAIN_ITERS_ENOUGH; --k)
         if (iters % k == 0) return ChainSplit{k, 0u};
     return ChainSplit{CHAIN_ITERS_ENOUGH, (uint32_t)(iters % CHAIN_ITERS_ENOUGH)};
 }
