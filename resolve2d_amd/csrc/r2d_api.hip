@@ -1294,6 +1294,8 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         sizes[i] = (uint32_t)w->n;
     }
     if (b.N >= 0x7fffffffull || b.B >= 0x7fffffffull) return R2D_E_CAPACITY;
+    for (uint32_t n : sizes)
+        if (n > CHAIN_BODIES) return R2D_E_CAPACITY;
 
     // solve variant: context override (autotuner), environment, then the
     // default (default_variant)

@@ -55,16 +55,16 @@ typedef const R2D_GLB u4v* GCU4;
 //     14-15 inverse inertias
 //   fixed position (2): 2-3 direction, 4 bias, 5 / 6 limits, 12 inverse mass
 //   motor (3): 2 inertia, 3 target, 4 beta, 5 / 6 limits, 7 torque
-constexpr uint32_t PR_INDEX = (1u << 29) - 1u;   // more bodies than memory holds the scratch of
+constexpr uint32_t PR_INDEX = CHAIN_BODIES - 1u;
 enum : uint32_t {
     PR_WRITE = 1u << 31,      // word 0 / 1, contacts: body a / b is an ordering body (its momentum is written)
                               // and this is the manifold's first point
     PR_STATIC = 1u << 30,     // word 0 / 1, contacts: the body is static (an ordering one gets "+= 0")
     PR_JOINT = 1u << 29,      // word 0
-    PR_SELF = 1u << 31,       // word 0, joints: both ends on one body
-    PR_SKIP = 1u << 30,       // word 0, joints: changes nothing this sub-step
-    PR_WARM = 1u << 29,       // word 1, contacts: warm started (no minimum impulse)
-    PR_TYPE_SHIFT = 30        // word 1, joints: type
+    PR_SELF = 1u << 27,       // word 0, joints: both ends on one body
+    PR_SKIP = 1u << 28,       // word 0, joints: changes nothing this sub-step
+    PR_WARM = 1u << 27,       // word 1, contacts: warm started (no minimum impulse)
+    PR_TYPE_SHIFT = 28        // word 1, joints: type
 };
 
 // the record of a lane without a point: bias -1, no body to write
@@ -446,43 +446,48 @@ __device__ __forceinline__ void plan_again(PLAN& P, uint32_t nit, uint32_t iters
             P.push(__hip_atomic_fetch_add(ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP), P.entry(j));
 }
 
-// A world's program, and the one for the rest of its iterations, with rows and
-// slots from kc * nit on and the entries after the first one's.  By one wave,
-// or (SEVERAL) by the whole workgroup.  Returns the slots of the first, with
-// those of the second in `rest_slots` (0: the ordering data was corrupt).
-template <bool SEVERAL, class PLAN>
-__device__ __forceinline__ uint32_t plan_world(PLAN& P, Program G, uint32_t nit, uint32_t nj, uint32_t kc, uint32_t rest,
-                                               uint32_t ready, uint32_t waves, ChainShared& sh, uint32_t& entries,
-                                               uint32_t& rest_slots)
+// The program for the rest of a world's iterations (StepDev::chain_rest), after
+// a plan of kc: its rows and slots from kc * nit on, its entries after the
+// others (sh.entries).  Called by the whole workgroup after a barrier, with
+// sh.taken at 0 in a world of one wave; ends with one.  sh.rest_slots is 0 if
+// the ordering data was corrupt.  A function of its own: few calls need it,
+// and in the planner's place it costs the others (97 worlds 283 -> 287 us a
+// step).
+struct PlanMemory {
+    LU32 lds;          // of PlanLds, when it fits
+    GU4 items, ring;   // of PlanGlb
+    Program program;
+};
+__device__ __attribute__((noinline)) void plan_rest(PlanMemory X, bool in_lds, uint32_t nit, uint32_t nj, uint32_t kc, uint32_t rest,
+                                                    uint32_t waves, R2D_LDS ChainShared* shl)
 {
-    uint32_t first = 0u;
-    rest_slots = 0u;
-    for (uint32_t iters = kc;;) {   // (one copy of the planner: its instructions are what it waits for)
-        uint32_t ns;
-        if constexpr (SEVERAL) ns = plan_multi(P, G, nit, nj, iters, ready, waves, sh);
-        else ns = plan_single(P, G, nit, nj, iters, ready, entries);
-        if (first) {
-            rest_slots = ns;
-            return ns ? first : 0u;
-        }
-        if (rest == 0u || ns == 0u) return ns;
-        first = ns;
-        iters = rest;
-        G.rows += (size_t)kc * nit;
-        G.slots += (size_t)kc * nit;
-        if constexpr (SEVERAL) {
-            __syncthreads();   // sh.taken has been read
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    nit = uniform(nit); nj = uniform(nj); kc = uniform(kc); rest = uniform(rest); waves = uniform(waves);
+    const Program G{uniform_ptr(X.program.rows) + (size_t)kc * nit, uniform_ptr(X.program.entries),
+                    uniform_ptr(X.program.slots) + (size_t)kc * nit};
+    auto plan = [&](auto P) {
+        if (waves > 1u) {
             if (threadIdx.x == 0) sh.ready = sh.taken = sh.queued[0] = 0u;
             __syncthreads();
             plan_again(P, nit, rest, threadIdx.x, blockDim.x, &sh.ready);
             __syncthreads();
-            ready = uniform(sh.ready);
-        } else {
-            plan_again(P, nit, rest, lane_id(), 64u, &sh.taken);   // (one wave's: no one else counts in it)
+            const uint32_t ns = plan_multi(P, G, nit, nj, rest, uniform(sh.ready), waves, sh);
+            if (threadIdx.x == 0) sh.rest_slots = ns;
+        } else if (threadIdx.x < 64u) {
+            plan_again(P, nit, rest, lane_id(), 64u, &sh.taken);
             asm volatile("" ::: "memory");
-            ready = uniform(__hip_atomic_load(&sh.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+            uint32_t entries = uniform(sh.entries);
+            const uint32_t ready = uniform(__hip_atomic_load(&sh.taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)),
+                           ns = plan_single(P, G, nit, nj, rest, ready, entries);
+            if (threadIdx.x == 0) {
+                sh.rest_slots = ns;
+                sh.entries = entries;
+            }
         }
-    }
+    };
+    if (uniform(in_lds)) plan(PlanLds(uniform_lds(X.lds), nit, waves));
+    else plan(PlanGlb(uniform_ptr(X.items), uniform_ptr(X.ring), nit, waves));
+    __syncthreads();
 }
 
 // Waves that run a world's rows: one for each `rows` rows of 64 its items fill

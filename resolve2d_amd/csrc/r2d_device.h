@@ -104,6 +104,8 @@ enum : int32_t {
 // per-step scratch, sized by capacities chosen on the host
 constexpr uint32_t SCANS = 5, SCAN_TILES = 1024;   // scans of a step, tiles of the largest that one kernel does
 constexpr uint32_t UNTOUCHED = 0xffffffffu;
+// bodies of a world that records can name (their scratch is 250 GB)
+constexpr uint32_t CHAIN_BODIES = 1u << 27;
 // a world's chain in the separate launches
 struct WorldChain {
     uint32_t bodies;    // places: bodies its items touch

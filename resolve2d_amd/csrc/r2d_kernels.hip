@@ -2116,7 +2116,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const uint32_t plan_words = (plan_lds_words(nit, 1u) + 1u) & ~1u;
     const bool follow = chain && waves == 1u && plan_in_lds && sh.iters == kc && plan_words < L.rest_words &&
                         L.consts + 2u * (nacc + 1u) <= L.rest_words - plan_words;
-    uint32_t ns = 1u, rest_slots = 0u, entries = 0u;
+    uint32_t ns = 1u, entries = 0u;
     if (follow) {
         sh.beside = plan_words;   // the same from every thread
         if (t < 64u) {
@@ -2153,24 +2153,31 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
             }
         }
     } else if (chain && waves > 1u) {
-        ns = plan_in_lds ? plan_world<true>(PL, G, nit, nj, kc, S.chain_rest, ready, waves, sh, entries, rest_slots)
-                         : plan_world<true>(PG, G, nit, nj, kc, S.chain_rest, ready, waves, sh, entries, rest_slots);
+        ns = plan_in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh)
+                         : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
         build(t, T);
     } else if (t < 64u) {
         if (chain)
-            ns = plan_in_lds ? plan_world<false>(PL, G, nit, nj, kc, S.chain_rest, ready, 1u, sh, entries, rest_slots)
-                             : plan_world<false>(PG, G, nit, nj, kc, S.chain_rest, ready, 1u, sh, entries, rest_slots);
+            ns = plan_in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
     } else {
         build(t - 64u, T - 64u);
     }
     if (t == 0) {
         sh.nslots = ns;
-        sh.rest_slots = rest_slots;
+        if (waves == 1u) sh.entries = entries;
         sh.failed = ns == 0u;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
     __syncthreads();
     if (follow) return true;
+    if (S.chain_rest && chain && !sh.failed) {
+        plan_rest(PlanMemory{L.rest, PG.items, PG.ring, G}, plan_in_lds, nit, nj, kc, S.chain_rest, waves, shl);
+        if (sh.rest_slots == 0u) {   // (read by all before the barrier that ends the step)
+            if (t == 0) { sh.failed = 1u; S.w_status[w] = WS_STALL; }
+            __syncthreads();
+            return false;
+        }
+    }
     // accumulated impulses (normal, tangential) of the contact points, by
     // point index less the joints: in LDS after the constants when they fit
     if (L.holds(nacc)) {
@@ -2241,8 +2248,8 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
         const bool several = chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u;
-        for (uint32_t part = 0; part < (rest_slots ? 2u : 1u); ++part) {
-            if (part) G = rest_program(G, kc * (nj + M), rest_slots);
+#pragma clang loop unroll(disable)
+        for (uint32_t left = rest_slots;;) {
             if (several) {
                 if (in_lds) chain_lds<true, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
                 else chain_lds_accg<true, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
@@ -2250,6 +2257,9 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
                 if (in_lds) chain_lds<false, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
                 else chain_lds_accg<false, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
             }
+            if (left == 0u) break;
+            G = rest_program(G, kc * (nj + M), left);
+            left = 0u;
         }
         __syncthreads();
     }
@@ -2373,17 +2383,26 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     if (in_lds) start(PL, true); else start(PG, false);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
-    uint32_t ns = 0u, rest_slots = 0u, entries = 0u;
-    const uint32_t rest = S.chain_rest;
+    uint32_t ns = 0u, entries = 0u;
     if (waves > 1u)
-        ns = in_lds ? plan_world<true>(PL, G, nit, nj, kc, rest, ready, waves, sh, entries, rest_slots)
-                    : plan_world<true>(PG, G, nit, nj, kc, rest, ready, waves, sh, entries, rest_slots);
+        ns = in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh) : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
     else if (t < 64u)
-        ns = in_lds ? plan_world<false>(PL, G, nit, nj, kc, rest, ready, 1u, sh, entries, rest_slots)
-                    : plan_world<false>(PG, G, nit, nj, kc, rest, ready, 1u, sh, entries, rest_slots);
+        ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
+    if (S.chain_rest) {
+        if (t == 0) {
+            sh.failed = ns == 0u;
+            if (waves == 1u) sh.entries = entries;
+        }
+        __syncthreads();
+        if (!sh.failed) {
+            plan_rest(PlanMemory{(LU32)smem, items, PG.ring, G}, in_lds, nit, nj, kc, S.chain_rest, waves, (R2D_LDS ChainShared*)&sh);
+            if (sh.rest_slots == 0u) ns = 0u;
+            entries = sh.entries;
+            if (t == 0) S.w_chain[w].rest_slots = sh.rest_slots;
+        }
+    }
     if (t == 0) {
         S.w_chain[w].slots = ns;
-        S.w_chain[w].rest_slots = rest_slots;
         S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2544,8 +2563,8 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
                        nj, nacc, jbase + nj, jbase};
         const bool fix = W.flags != 0u;
         const bool several = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u;
-        for (uint32_t part = 0; part < (W.rest_slots ? 2u : 1u); ++part) {
-            if (part) G = rest_program(G, kc * nit, W.rest_slots);
+#pragma clang loop unroll(disable)
+        for (uint32_t left = W.rest_slots;;) {
             if (several) {
                 if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
                 else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
@@ -2555,6 +2574,9 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
                 else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
                 else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
             }
+            if (left == 0u) break;
+            G = rest_program(G, kc * nit, left);
+            left = 0u;
         }
         __syncthreads();
     }
