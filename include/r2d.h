@@ -309,6 +309,8 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
  * rule 1: in {bodies, buckets, worlds, joints, cell entries, raw candidates,
  * manifolds, solver items, iterations of the programs}; out {bytes of the step
  * scratch that holds them}.
+ * rule 3: in {bodies, buckets, joints, collision iterations}; out {bytes of
+ * step scratch that a world is charged for}.
  * rule 2: in {cell entries, raw candidates, manifolds, solver items,
  * iterations of the programs}; out {bytes of the one-kernel step's slices}. */
 int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out);
@@ -405,7 +407,9 @@ typedef struct {
 } r2d_serve_summary;
 
 /* Bytes a world is charged at admission: its device state plus its share of
- * the step scratch at the library's initial per-body estimates. */
+ * the step scratch at the library's initial estimates.  The scratch grows with
+ * collision_iters up to 16 (about 4 KB a body at 4 iterations, 10 KB at 16):
+ * without a server on the world's context it is counted for 4. */
 int r2d_world_footprint(r2d_world* w, size_t* bytes);
 int r2d_serve_create(r2d_ctx* ctx, const r2d_serve_options* opt, r2d_server** out);
 /* Waits for the launched step; worlds of unfinished requests are released. */

@@ -981,8 +981,9 @@ int ensure_fused_arena(r2d_ctx* c, uint64_t te, uint64_t tr, uint64_t tm, uint64
         chain_split(iters, c->fchain_most).room() <= c->fcap_k && c->farena)
         return R2D_OK;
     if (std::max(std::max(te, tr), std::max(tm, ti)) >= 0x7fffff00ull) return R2D_E_CAPACITY;
-    const uint32_t E = grow_cap(c->fcap_e, te), R = grow_cap(c->fcap_r, tr), M = grow_cap(c->fcap_m, tm),
-                   I = grow_cap(c->fcap_i, ti);
+    // (a new batch's slices come with their reserve)
+    auto grow = [&](uint32_t have, uint64_t need) { return preserve ? grow_cap(have, need) : (uint32_t)std::max<uint64_t>(have, need); };
+    const uint32_t E = grow(c->fcap_e, te), R = grow(c->fcap_r, tr), M = grow(c->fcap_m, tm), I = grow(c->fcap_i, ti);
     StepDev F{};
     void* arena = nullptr;
     size_t bytes = 0;
@@ -1075,17 +1076,29 @@ int ensure_fused_world(r2d_ctx* c, size_t W)
     return R2D_OK;
 }
 
-// slice capacities of a world: what it used before, else estimates (per
-// body 4 cell entries, 32 raw candidates -- a settled pile has about 24 --
-// and 3 manifolds)
+// slice capacities of a world: estimates (per body 4 cell entries, 32 raw
+// candidates -- a settled pile has about 24 -- and 3 manifolds), or what it
+// used before
+void first_slices(uint32_t n, uint32_t nj, uint32_t cap[4])
+{
+    cap[0] = 4 * n + 64;
+    cap[1] = 32 * n + 256;
+    cap[2] = 3 * n + 64;
+    cap[3] = nj + cap[2];
+}
+
 void fused_caps(const r2d_world* w, uint32_t cap[4])
 {
-    const uint32_t n = (uint32_t)w->n, nj = (uint32_t)w->joints.size();
-    cap[0] = w->fz[0] ? w->fz[0] : 4 * n + 64;
-    cap[1] = w->fz[1] ? w->fz[1] : 32 * n + 256;
-    cap[2] = w->fz[2] ? w->fz[2] : 3 * n + 64;
+    const uint32_t nj = (uint32_t)w->joints.size();
+    first_slices((uint32_t)w->n, nj, cap);
+    for (int k = 0; k < 4; ++k)
+        if (w->fz[k]) cap[k] = w->fz[k];
     cap[3] = std::max(w->fz[3] ? w->fz[3] : nj + cap[2], nj + 1);
 }
+
+// free space for worlds that outgrow their slices during a call: at most as
+// much again as the slices, at least half as much
+constexpr size_t FUSED_RESERVE = 2;
 
 // end of the used part of each array (entries, candidates, manifolds, items)
 void fused_used(const r2d_ctx* c, uint64_t end[4])
@@ -1133,8 +1146,9 @@ int fused_layout(r2d_ctx* c, Batch& b)
                                   cap[3]};
         te += (uint64_t)cap[0] + 1; tr += (uint64_t)cap[1] + 1; tm += cap[2]; ti += (uint64_t)cap[3] + 1;
     }
-    // as much again free for worlds that outgrow their slices during the call
-    if ((rc = ensure_fused_arena(c, 2 * te, 2 * tr, 2 * tm, 2 * ti, b.iters, false))) return rc;
+    const bool room = te + te / 2 <= c->fcap_e && tr + tr / 2 <= c->fcap_r && tm + tm / 2 <= c->fcap_m && ti + ti / 2 <= c->fcap_i;
+    const uint64_t f = room ? 1 : FUSED_RESERVE;
+    if ((rc = ensure_fused_arena(c, f * te, f * tr, f * tm, f * ti, b.iters, false))) return rc;
     // workgroups take the largest worlds first (the longest steps start first)
     c->forder.resize(nw);
     for (size_t i = 0; i < nw; ++i) c->forder[i] = (uint32_t)i;
@@ -1691,28 +1705,46 @@ void fill_states(r2d_world* w, size_t s0, size_t m, r2d_body_state* __restrict o
 }
 
 // ---------------------------------------------------------------- serving
-// Admission estimate of one resident world: its device block and topology
-// plus its share of the step scratch at the initial capacity estimates: the
-// phase kernels' (per body: cell ranges, 4 cell entries, 8 raw candidates, 4
-// manifolds and 4 solver items) or the fused kernel's slices and their free
-// reserve, whichever is larger (per body 2 x (4 entries x 20 B + 32
-// candidates x 32 B + 3 manifolds x 128 B + 3 items x 156 B)); per hash
-// bucket 12 B; per joint one solver item.
-constexpr size_t kScratchClassic = 96 + 4 * 24 + 8 * 36 + 4 * 128 + 4 * 160;
-constexpr size_t kScratchFused = 96 + 2 * (4 * 20 + 32 * 32 + 3 * 128 + 3 * 156);
-constexpr size_t kScratchPerBody = kScratchClassic > kScratchFused ? kScratchClassic : kScratchFused;
-constexpr size_t kScratchPerBucket = 12;
-constexpr size_t kScratchPerJoint = 160;
-constexpr size_t kScratchPerWorld = 20 + sizeof(WorldDev);
+// What a world of n bodies, `table` buckets and nj joints adds to the step
+// scratch when it is first allocated, with programs for `iters` iterations:
+// the separate launches' arrays with their room to grow, or, if more and the
+// world is small enough, the per-body arrays and the one-kernel step's slices
+// with their reserve.  From the arrays themselves (scratch_arrays,
+// fused_arrays), so that it follows them.
+size_t scratch_share(size_t n, size_t table, size_t nj, size_t iters)
+{
+    const size_t k = chain_split(iters).room();
+    auto step = [&](size_t e, size_t r, size_t m, size_t i) {
+        auto bytes = [&](const ScratchCaps& c) {
+            StepDev S;
+            size_t sum = 0;
+            scratch_arrays(S, c, [&](void**, size_t x) { sum += x; });
+            return sum;
+        };
+        auto room = [](size_t x) { return x + (x + 1) / 2; };
+        return bytes(ScratchCaps{room(n), room(table), room(1), room(nj), room(e), room(r), room(m), room(i), k}) -
+               bytes(ScratchCaps{0, 0, 0, 0, 0, 0, 0, 0, k});
+    };
+    const size_t separate = step(4 * n, 8 * n, 4 * n, nj + 2 * n);
+    if (n > FUSED_NMAX) return separate;
+    uint32_t cap[4];
+    first_slices((uint32_t)n, (uint32_t)nj, cap);
+    StepDev F;
+    size_t slices = 0;
+    fused_arrays(F, FUSED_RESERVE * ((size_t)cap[0] + 1), FUSED_RESERVE * ((size_t)cap[1] + 1), FUSED_RESERVE * (size_t)cap[2],
+                 FUSED_RESERVE * ((size_t)cap[3] + 1), k, [&](void**, size_t x) { slices += x; });
+    return std::max(separate, step(0, 0, 0, 0) + slices);
+}
 
-size_t world_footprint(const r2d_world* w)
+// What admission charges for a world: its device block and topology and its
+// share of the step scratch
+size_t world_footprint(const r2d_world* w, size_t iters)
 {
     size_t n = (size_t)w->n;
     size_t dev = (size_t)F_NFIELDS * std::max<size_t>(std::max(w->cap, w->dcap), 16) * 4 +
                  std::max<size_t>(16, w->joints.size()) * sizeof(Joint) +
                  std::max<size_t>(16, w->gens.size()) * sizeof(Gen) + std::max<size_t>(16, w->excl.size()) * 8;
-    return dev + n * kScratchPerBody + (size_t)table_size(w) * kScratchPerBucket +
-           w->joints.size() * kScratchPerJoint + kScratchPerWorld;
+    return dev + sizeof(WorldDev) + scratch_share(n, table_size(w), w->joints.size(), iters);
 }
 
 double now_ms()
@@ -2796,6 +2828,9 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
         out[1] = s.rest;
         return R2D_OK;
     }
+    case 3:
+        out[0] = scratch_share(in[0], in[1], in[2], in[3]);
+        return R2D_OK;
     case 1:
     case 2: {
         StepDev S{};
@@ -2996,7 +3031,7 @@ R2D_EXPORT int r2d_make_bodies(r2d_world* w, size_t n, const r2d_body_options* b
 R2D_EXPORT int r2d_world_footprint(r2d_world* w, size_t* bytes)
 {
     if (!w || !bytes) return R2D_E_INVALID_ARG;
-    *bytes = world_footprint(w);
+    *bytes = world_footprint(w, w->owner->server ? w->owner->server->opt.collision_iters : CHAIN_ITERS_ENOUGH);
     return R2D_OK;
 }
 
@@ -3053,7 +3088,7 @@ R2D_EXPORT int r2d_serve_submit(r2d_server* sv, r2d_world* w, uint32_t steps, ui
     if (sv->opt.sub_steps > 0 && sv->opt.collision_iters > 0)
         for (const HJoint& h : w->joints)
             if (w->slot_of(h.id1) < 0 || (h.type <= 1 && w->slot_of(h.id2) < 0)) return R2D_E_INVALID_ID;
-    size_t bytes = world_footprint(w);
+    size_t bytes = world_footprint(w, sv->opt.collision_iters);
     if (bytes > sv->opt.hbm_budget_bytes) { sv->rejected += 1; return R2D_E_CAPACITY; }
     r2d_server::Req q;
     q.w = w;

@@ -83,8 +83,7 @@ def test_short_of_memory_one_kernel(oracle, monkeypatch, fit):
     n, iters = 300, 16
     bodies = n + 1
     slices = [4 * bodies + 65, 32 * bodies + 257, 3 * bodies + 64, 3 * bodies + 65]
-    grown = [_room(2 * x) for x in slices]
-    limit = rule(2, *grown, 1 if fit != "16" else 16)[0] - (fit == "none")
+    limit = rule(2, *[2 * x for x in slices], 1 if fit != "16" else 16)[0] - (fit == "none")
     monkeypatch.setenv("R2D_SCRATCH_LIMIT", str(limit))
     ctx = Context(0)
     g, o = GpuWorld(ctx), oracle.OracleWorld("f32")
@@ -99,3 +98,26 @@ def test_short_of_memory_one_kernel(oracle, monkeypatch, fit):
         _same(g, o, step)
     for e in (g, o, ctx):
         e.close()
+
+
+def test_admission_follows_the_iterations(gpu_ctx):
+    """A budget for two worlds at 4 iterations holds only one at 8."""
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    from resolve2d_amd.serve import Server
+    for iters, at_once in ((4, 2), (8, 1)):
+        ws = [GpuWorld(gpu_ctx) for _ in range(2)]
+        for k, w in enumerate(ws):
+            apply_scene(_heap(1500, 25.0, 50 + k), w)
+        budget = sum(w.footprint() for w in ws)
+        sv = Server(gpu_ctx, budget, max_worlds=4, collision_iters=iters)
+        try:
+            assert (sum(w.footprint() for w in ws) > budget) == (iters == 8)
+            for w in ws:
+                sv.submit(w, 2)
+            assert sv.tick()["running"] == at_once
+            sv.drain()
+            assert sv.stats()["peak_resident_bytes"] <= budget
+        finally:
+            sv.close()
+            for w in ws:
+                w.close()

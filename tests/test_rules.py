@@ -43,3 +43,26 @@ def test_step_scratch_falls_back_to_less_than_before_programs(n, joints):
     before = 84 * _room(n) + 12 * _room(table) + 24 * e + 36 * r + 128 * m + 176 * _room(m + _room(joints))
     assert now(1, lambda x: x) < before
     assert now(1, lambda x: x) < now(1, _room) < now(rule(0, 17)[0] + rule(0, 17)[1], _room) < now(16, _room)
+
+
+@pytest.mark.parametrize("iters", [1, 4, 16, 17])
+@pytest.mark.parametrize("sizes", [[8192], [16] * 40, [300, 50, 1024, 700], [1500, 4096, 2000]],
+                         ids=["one", "small", "mixed", "large"])
+def test_admission_charges_what_is_allocated(sizes, iters):
+    """The charges of a batch's worlds cover what the batch's first step
+    allocates beyond an empty one's (256 bytes of alignment an array)."""
+    each, rest = rule(0, iters)[:2]
+    k = each + rest
+    joints = [n // 3 for n in sizes]
+    charge = sum(rule(3, n, 2 * n, j, iters)[0] for n, j in zip(sizes, joints))
+    N, J, W = sum(sizes), sum(joints), len(sizes)
+
+    def step(n, w, j, e, r, m, i):
+        return rule(1, *[_room(x) for x in (n, 2 * n, w, j, e, r, m, i)], k)[0]
+
+    separate = step(N, W, J, 4 * N + 1024, 8 * N + 1024, 4 * N + 1024, J + 2 * N + 1024) - step(0, 0, 0, *[1024] * 4)
+    assert charge + 60 * 256 >= separate
+    if max(sizes) <= 1024:
+        slices = rule(2, 2 * sum(4 * n + 65 for n in sizes), 2 * sum(32 * n + 257 for n in sizes),
+                      2 * sum(3 * n + 64 for n in sizes), 2 * sum(3 * n + 65 + j for n, j in zip(sizes, joints)), k)[0]
+        assert charge + 60 * 256 >= slices + step(N, W, J, 1, 1, 1, 1) - step(0, 0, 0, 1, 1, 1, 1)
