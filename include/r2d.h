@@ -309,6 +309,9 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
  * rule 1: in {bodies, buckets, worlds, joints, cell entries, raw candidates,
  * manifolds, solver items, iterations of the programs}; out {bytes of the step
  * scratch that holds them}.
+ * rule 4: in {worlds a compute unit, workgroups that its registers hold,
+ * bodies and buckets of the largest world}; out {bytes of LDS of a one-kernel
+ * step's workgroup}.
  * rule 3: in {bodies, buckets, joints, collision iterations}; out {bytes of
  * step scratch that a world is charged for}.
  * rule 2: in {cell entries, raw candidates, manifolds, solver items,

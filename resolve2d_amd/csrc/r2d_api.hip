@@ -892,15 +892,24 @@ int warm_variant(const r2d_ctx* c, size_t nworlds)
     return worlds_per_cu(c, nworlds) == 1 ? WARM_WIDE_VARIANT : WARM_VARIANT;
 }
 
-// LDS of a fused launch: a CU's divided by the worlds it is to hold, as far as
-// the largest world needs no more.  What a world has beyond its need holds
-// plans and impulses of worlds with many contacts, which are in global memory
-// otherwise (a world of 501 bodies and 983 items: plan 111 us, in LDS 46).
-size_t fused_lds_share(const r2d_ctx* c, size_t nworlds, uint32_t n, uint32_t tb)
+// LDS of a fused launch: a CU's divided by the worlds it is to hold -- those
+// of the batch, at most as many as its registers hold workgroups (`groups`) --
+// as far as the largest world needs no more.  What a world has beyond its need
+// holds plans and impulses of worlds with many contacts, which are in global
+// memory otherwise (a world of 501 bodies and 983 items: plan 111 us, in LDS
+// 46).  Divided by five worlds where four are there at once, 1,100 worlds of
+// up to 300 bodies took 362 us a step, 2,048 527; by four 343 and 517.
+// In whole pieces of LDS, 1,280 bytes each, 1 KB of them for the kernel's
+// fixed variables: a third of 160 KB is 42.7 pieces, and three workgroups of 43
+// are not there at once (700 worlds of 50-500 bodies: 470 us a step, by 42
+// pieces 407; 600 of 50-300 338 and 325).
+constexpr size_t kLdsPiece = 1280, kLdsPieces = 128, kLdsFixed = 1024;
+static_assert(kLdsPieces * kLdsPiece - kLdsFixed == kFusedLdsMax, "a workgroup alone takes all of LDS");
+size_t fused_lds_share(size_t worlds_a_cu, size_t groups, uint32_t n, uint32_t tb)
 {
     const size_t need = fused_lds_bytes(n, tb);
-    const size_t fit = std::max<size_t>(1, (kFusedLdsMax + 1024) / (need + 1024));
-    const size_t share = ((kFusedLdsMax + 1024) / std::min(fit, worlds_per_cu(c, nworlds)) - 1024) & ~(size_t)15;
+    const size_t fit = std::max<size_t>(1, kLdsPieces / ((need + kLdsFixed + kLdsPiece - 1) / kLdsPiece));
+    const size_t share = kLdsPieces / std::min(std::min(fit, groups), worlds_a_cu) * kLdsPiece - kLdsFixed;
     return std::max(need, share);
 }
 
@@ -1338,7 +1347,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         maxtb = std::max(maxtb, b.descs[i].table);
     }
     if (fused) {
-        b.fused_lds = fused_lds_share(c, nw, maxn, maxtb);
+        b.fused_lds = fused_lds_share(worlds_per_cu(c, nw), fused_groups(variant), maxn, maxtb);
         fused = b.fused_lds <= kFusedLdsMax;
     }
     b.fused = fused;
@@ -2301,7 +2310,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
             if (w->slot_of(h.id1) < 0 || (h.type <= 1 && w->slot_of(h.id2) < 0)) return R2D_E_INVALID_ID;
     int variant = c->solve_variant >= 0 ? c->solve_variant : default_variant(c, 1);
     if (!fused_available(variant)) variant = 11;
-    const size_t lds = fused_lds_share(c, 1, n, tb);
+    const size_t lds = fused_lds_share(1, 1, n, tb);
     if (lds > kFusedLdsMax) return R2D_E_CAPACITY;
     if (n == 0) {   // nothing moves and no manifold exists
         w->epoch = 0;
@@ -2828,6 +2837,9 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
         out[1] = s.rest;
         return R2D_OK;
     }
+    case 4:
+        out[0] = fused_lds_share(in[0], in[1], (uint32_t)in[2], (uint32_t)in[3]);
+        return R2D_OK;
     case 3:
         out[0] = scratch_share(in[0], in[1], in[2], in[3]);
         return R2D_OK;

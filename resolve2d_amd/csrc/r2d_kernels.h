@@ -117,6 +117,8 @@ bool fused_available(int variant);
 // dynamic LDS of the fused kernel for a world of n bodies and tb hash buckets
 size_t fused_lds_bytes(uint32_t n, uint32_t tb);
 uint32_t fused_threads(int variant);
+// workgroups of it that a compute unit's registers hold
+uint32_t fused_groups(int variant);
 // one workgroup per world (S.w_order), up to nsteps steps per world (S.w_done)
 // the fused kernel of a variant as compiled (registers, LDS, scratch): for error reports
 hipError_t fused_attributes(int variant, hipFuncAttributes* out);

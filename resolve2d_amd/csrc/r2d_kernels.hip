@@ -3132,6 +3132,12 @@ uint32_t fused_threads(int v)
 // loops stride by MAXT): set_solve_smem_limit checks each against the width
 // it would be launched with, and a mismatch leaves the variant without one
 static bool g_fused_width_ok[SOLVE_TABLE];
+static uint32_t g_fused_groups[SOLVE_TABLE];
+
+uint32_t fused_groups(int v)
+{
+    return std::max(1u, g_fused_groups[v]);
+}
 
 bool fused_available(int v)
 {
@@ -3359,6 +3365,10 @@ void set_solve_smem_limit()
             hipFuncAttributes fa{};
             g_fused_width_ok[v] = hipFuncGetAttributes(&fa, (const void*)kSolveVariants[v].fused_fn) == hipSuccess &&
                                   fa.maxThreadsPerBlock == (int)fused_threads(v);
+            int groups = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, (const void*)kSolveVariants[v].fused_fn,
+                                                             (int)fused_threads(v), 0) == hipSuccess)
+                g_fused_groups[v] = (uint32_t)std::max(groups, 1);
         }
     }
     (void)hipGetLastError();   // a refused attribute is not an error of a later call

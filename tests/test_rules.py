@@ -66,3 +66,19 @@ def test_admission_charges_what_is_allocated(sizes, iters):
         slices = rule(2, 2 * sum(4 * n + 65 for n in sizes), 2 * sum(32 * n + 257 for n in sizes),
                       2 * sum(3 * n + 64 for n in sizes), 2 * sum(3 * n + 65 + j for n, j in zip(sizes, joints)), k)[0]
         assert charge + 60 * 256 >= slices + step(N, W, J, 1, 1, 1, 1) - step(0, 0, 0, 1, 1, 1, 1)
+
+
+@pytest.mark.parametrize("bodies", [50, 200, 300, 501, 1024])
+def test_lds_is_divided_among_the_workgroups_there_at_once(bodies):
+    """More worlds than a compute unit's registers hold workgroups: LDS is
+    divided by those, not by worlds that wait for them; and so that as many are
+    there at once (pieces of 1,280 bytes, 1 KB for fixed variables)."""
+    pieces = lambda x: -(-(x + 1024) // 1280)
+    share = [[rule(4, worlds, groups, bodies, 2 * bodies)[0] for worlds in range(1, 13)] for groups in range(1, 13)]
+    least = share[11][11]
+    for groups, row in enumerate(share, 1):
+        assert row == sorted(row, reverse=True)
+        assert set(row[groups:]) <= {row[groups - 1]}        # no less for the worlds that wait
+        for worlds, x in enumerate(row, 1):
+            assert pieces(x) * min(worlds, groups, 128 // pieces(least)) <= 128
+    assert share[0][0] == 159 * 1024
