@@ -1652,7 +1652,11 @@ int batch_wait(r2d_ctx* c, Batch& b)
             if (c->hcounters[C_OVERFLOW] & 1u) e = c->hcounters[C_ENTRIES] * 2 + 1;
             if (c->hcounters[C_OVERFLOW] & 2u) r = c->hcounters[C_RAW] * 2 + 1;
             if (c->hcounters[C_OVERFLOW] & 4u) m = c->hcounters[C_MANIFOLDS] * 2 + 1;
-            if (c->hcounters[C_OVERFLOW] & 8u) it = c->hcounters[C_ITEMS] + c->hcounters[C_ITEMS] / 4;
+            // (the steps after the one that stopped clear the count of items, which are joints and manifolds)
+            if (c->hcounters[C_OVERFLOW] & 8u) {
+                const uint64_t items = b.J + c->hcounters[C_MANIFOLDS];
+                it = (uint32_t)std::min<uint64_t>(items + items / 4, 0x7fffffffu);
+            }
             int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e, r, m, it, b.iters);
             if (rc) return rc;
         }

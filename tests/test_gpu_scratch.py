@@ -45,6 +45,24 @@ def test_items_beyond_the_estimate(oracle, side, short, coloured):
         e.close()
 
 
+def test_items_beyond_the_estimate_within_a_call(oracle):
+    """The same where the step that stops is not the call's last one."""
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    from resolve2d_amd.solver import Context
+    ctx = Context(0)
+    ctx.set_fused(False)
+    g, o = GpuWorld(ctx), oracle.OracleWorld("f32")
+    for e in (g, o):
+        apply_scene(_heap(800, 14.0, 40), e)
+    for call in range(2):
+        ctx.process_batch_handles([g.handle], DT, 1, 2, 3)
+        for _ in range(3):
+            assert o.process(DT, 1, 2) == 0
+        _same(g, o, call)
+    for e in (g, o, ctx):
+        e.close()
+
+
 @pytest.mark.parametrize("iters", [4, 16, 17])
 @pytest.mark.parametrize("fit", ["16", "7", "1", "1 without room", "none"])
 def test_short_of_memory(oracle, monkeypatch, fit, iters):
