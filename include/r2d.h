@@ -284,8 +284,9 @@ int r2d_ctx_set_solve_variant(r2d_ctx* ctx, int variant);
  * launch-shape knob for the autotuner. */
 int r2d_ctx_set_lds_limit(r2d_ctx* ctx, uint32_t max_bodies);
 /* Separate launches only: a batch of at most 256 worlds runs their chains
- * with 512 threads a world (on, the default: each is alone on its CU).  Off
- * keeps the variant's threads.  Same bits either way; a launch-shape knob with no counterpart in the reference. */
+ * with 512 threads a world (on, the default: each is alone on its CU), or 768
+ * in the coloured order.  Off: with 256, unless a variant of 512 is chosen.
+ * Same bits either way; a launch-shape knob with no counterpart in the reference. */
 int r2d_ctx_set_wide_record(r2d_ctx* ctx, int on);
 /* Totals of the last step of the context: entries, raw candidates,
  * manifolds, solver items (out[4]). */
@@ -309,6 +310,9 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
  * rule 1: in {bodies, buckets, worlds, joints, cell entries, raw candidates,
  * manifolds, solver items, iterations of the programs}; out {bytes of the step
  * scratch that holds them}.
+ * rule 5: in {chosen variant + 1 (0: none), worlds, bodies of each, whether
+ * one is coloured, whether one is warm started, r2d_ctx_set_wide_record}; out
+ * {threads of the separate launches' chains, bytes of LDS}.
  * rule 4: in {worlds a compute unit, workgroups that its registers hold,
  * bodies and buckets of the largest world}; out {bytes of LDS of a one-kernel
  * step's workgroup}.

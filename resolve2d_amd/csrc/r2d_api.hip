@@ -283,7 +283,7 @@ struct r2d_ctx {
     std::vector<WorldDev> uploaded_descs;
     int solve_variant = -1;                       // -1: choose by world size
     uint32_t lds_nmax = 0;                        // 0: LDS body state up to the LDS capacity
-    bool wide_record = true;                      // batches of <= 64 LDS worlds may take the 512-lane record kernel
+    bool wide_record = true;                      // separate launches: batches of up to 256 worlds take wide chains
 
     KernelTrace* trace = nullptr;                 // per-kernel timing (R2D_TRACE_KERNELS)
 
@@ -1322,11 +1322,10 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
 
     // solve variant: context override (autotuner), environment, then the
     // default (default_variant)
-    int variant = default_variant(c, nw);
-    if (c->solve_variant >= 0) variant = c->solve_variant;
+    int chosen = c->solve_variant;
     if (const char* e = std::getenv("R2D_SOLVE_VARIANT")) {
         int v = std::atoi(e);
-        if (v >= 0 && v < SOLVE_VARIANTS) variant = v;
+        if (v >= 0 && v < SOLVE_VARIANTS) chosen = v;
     }
     bool colored = false, warm = false;
     for (size_t i = 0; i < nw; ++i) {
@@ -1334,8 +1333,9 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
         warm = warm || worlds[i]->warm > 0.0f;
     }
     // warm starting is compiled into kernels of its own
-    if (warm) variant = warm_variant(c, nw);
-    b.plan = plan_solve(variant, sizes.data(), nw, c->lds_nmax, colored, warm, c->wide_record);
+    if (warm) chosen = -1;
+    const int variant = warm ? warm_variant(c, nw) : chosen >= 0 ? chosen : default_variant(c, nw);
+    b.plan = plan_solve(chosen, sizes.data(), nw, c->lds_nmax, colored, warm, c->wide_record);
     b.variant = variant;
     // whole steps per workgroup: worlds of at most FUSED_NMAX bodies in the
     // reference order whose broadphase and solve arrays fit LDS
@@ -2839,6 +2839,14 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
         const ChainSplit s = chain_split(in[0]);
         out[0] = s.each;
         out[1] = s.rest;
+        return R2D_OK;
+    }
+    case 5: {
+        const uint32_t n = (uint32_t)in[2];
+        std::vector<uint32_t> sizes(std::max<size_t>(1, in[1]), n);
+        const SolvePlan p = plan_solve((int)in[0] - 1, sizes.data(), sizes.size(), 0, in[3] != 0, in[4] != 0, in[5] != 0);
+        out[0] = p.threads;
+        out[1] = p.lds;
         return R2D_OK;
     }
     case 4:

@@ -67,13 +67,13 @@ constexpr size_t CHAIN_LDS = 159 * 1024, CHAIN_LDS_MIN = 16 * 1024, CHAIN_LDS_BO
 struct SolvePlan {
     uint32_t lds = 0;          // dynamic LDS of a world's workgroup
     uint32_t lds_nmax = 0;     // bodies a world may have to keep its momenta in LDS
-    uint32_t wide = 0;         // wide workgroups
+    uint32_t threads = 0;      // of the chain's workgroups
     uint32_t any_colored = 0;  // some world uses the coloured schedule
     uint32_t any_warm = 0;     // some world is warm started
 };
-// lds_limit: largest world (bodies) that keeps its momenta in LDS (0: as many
+// chosen: the variant that the caller chose (-1: none); lds_limit: largest world (bodies) that keeps its momenta in LDS (0: as many
 // as LDS holds)
-SolvePlan plan_solve(int variant, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
+SolvePlan plan_solve(int chosen, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
                      bool any_warm, bool allow_wide = true);
 
 // Optional per-kernel timing (a context created with R2D_TRACE_KERNELS set):

@@ -3217,15 +3217,16 @@ static inline void tmark(const Streams& ss, const char* name, hipStream_t st)
     if (ss.trace) ss.trace->mark(name, st);
 }
 
-SolvePlan plan_solve(int variant, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
+SolvePlan plan_solve(int chosen, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
                      bool any_warm, bool allow_wide)
 {
     SolvePlan p;
     p.any_colored = any_colored ? 1u : 0u;
     p.any_warm = any_warm ? 1u : 0u;
     p.lds_nmax = lds_limit ? lds_limit : 0xffffffffu;
-    p.wide = nw <= CHAIN_WIDE_WORLDS && allow_wide ? 1u : 0u;
-    if (variant >= 0 && variant < SOLVE_TABLE && kSolveVariants[variant].threads == CHAIN_THREADS) p.wide = 1u;
+    const bool wide = (nw <= CHAIN_WIDE_WORLDS && allow_wide) ||
+                      (chosen >= 0 && chosen < SOLVE_TABLE && kSolveVariants[chosen].threads == CHAIN_THREADS);
+    p.threads = !wide ? CHAIN_NARROW : any_colored && !any_warm ? CHAIN_COLORED : CHAIN_THREADS;
     // LDS: worlds that are alone on their CU take all of it; of larger batches
     // each world takes what its momenta (16 bytes a touched body), impulses (8
     // a point) and plan (18 an item) commonly need, so that CUs hold several
@@ -3307,9 +3308,10 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
     default: {
         const float sub_dt = dt / (float)sub_steps;
         auto pick = [&](auto warm, auto cold) { return sp.any_warm ? warm : cold; };
-        const bool colored = sp.any_colored && !sp.any_warm;
-        const unsigned T = !sp.wide ? CHAIN_NARROW : colored ? CHAIN_COLORED : CHAIN_THREADS;
-        auto width = [&](auto narrow, auto wide, auto widest) { return !sp.wide ? narrow : colored ? widest : wide; };
+        const unsigned T = sp.threads;
+        auto width = [&](auto narrow, auto wide, auto widest) {
+            return T == CHAIN_NARROW ? narrow : T == CHAIN_COLORED ? widest : wide;
+        };
         const uint32_t words = sp.lds / 4u;
         if (sub_steps > 0) {   // without sub-steps nothing of a world changes
             hipLaunchKernelGGL(pick(k_chain_build<true>, k_chain_build<false>), dim3(GRID), dim3(BS), 0, st, S, sub_dt);

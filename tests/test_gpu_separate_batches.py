@@ -1,0 +1,49 @@
+"""The separate launches where a batch is larger than the compute units (narrow
+chains and a share of LDS each) and with narrow chains asked for.  Bit for bit
+against the oracle."""
+import pytest
+
+from helpers import bits_equal, first_diff
+from test_gpu_programs import _heap
+
+pytestmark = pytest.mark.gpu
+
+DT = 1.0 / 60.0
+
+
+def _check(oracle, ctx, scenes, warm, coloured, pick, steps=2):
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    ctx.set_fused(False)
+
+    def make(k, w):
+        apply_scene(scenes[k], w)
+        if coloured and k % 5 == 0:   # (a world is one or the other)
+            w.set_schedule(1)
+        elif warm and k % 3 != 1:
+            w.set_warm_start(0.8)
+        return w
+
+    gs = [make(k, GpuWorld(ctx)) for k in range(len(scenes))]
+    for _ in range(2):
+        ctx.process_batch_handles([g.handle for g in gs], DT, 2, 4, steps)
+    for k in pick:
+        o = make(k, oracle.OracleWorld("f32"))
+        for _ in range(2 * steps):
+            assert o.process(DT, 2, 4) == 0
+        a, b = gs[k].bodies(), o.bodies()
+        assert bits_equal(a, b), (k, first_diff(a, b))
+        mg, mo = gs[k].manifolds(), o.manifolds()
+        assert mg.shape == mo.shape and bits_equal(mg, mo), (k, first_diff(mg, mo))
+        o.close()
+    for g in gs:
+        g.close()
+
+
+@pytest.mark.parametrize("warm,coloured", [(False, False), (True, False), (False, True)], ids=["cold", "warm", "coloured"])
+def test_narrow_chains(oracle, warm, coloured):
+    from resolve2d_amd.solver import Context
+    ctx = Context(0)
+    ctx.set_wide_record(False)
+    scenes = [_heap(900, 14.0, 90), _heap(200, 7.0, 91), _heap(20, 3.0, 92)]
+    _check(oracle, ctx, scenes, warm, coloured, range(3))
+    ctx.close()

@@ -82,3 +82,16 @@ def test_lds_is_divided_among_the_workgroups_there_at_once(bodies):
         for worlds, x in enumerate(row, 1):
             assert pieces(x) * min(worlds, groups, 128 // pieces(least)) <= 128
     assert share[0][0] == 159 * 1024
+
+
+@pytest.mark.parametrize("coloured,warm", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_wide_chains_can_be_switched_off(coloured, warm):
+    """r2d_ctx_set_wide_record(0) narrows the chains of batches whose caller
+    chose no variant; a variant of 512 threads (0, 13, 14) stays wide."""
+    for worlds in (1, 40, 256):
+        assert rule(5, 0, worlds, 5000, coloured, warm, 1)[0] >= 512
+        assert rule(5, 0, worlds, 5000, coloured, warm, 0)[0] == 256
+    assert rule(5, 0, 257, 5000, coloured, warm, 1)[0] == 256
+    for variant in range(15):
+        wide = rule(5, variant + 1, 40, 5000, coloured, warm, 0)[0]
+        assert (wide >= 512) == (variant in (0, 13, 14)), variant
