@@ -39,6 +39,22 @@ def _check(oracle, ctx, scenes, warm, coloured, pick, steps=2):
         g.close()
 
 
+@pytest.mark.parametrize("limit", [0, 1], ids=["lds", "momenta-global"])
+@pytest.mark.parametrize("warm,coloured", [(False, False), (True, False), (False, True), (True, True)],
+                         ids=["cold", "warm", "coloured", "warm-coloured"])
+def test_more_worlds_than_compute_units(oracle, warm, coloured, limit):
+    """257 worlds of 1 to 40 bodies, and among them heaps whose plan (20 bytes an
+    item), impulses (8 a point) and colours (20 a body) a share of LDS does not
+    hold: 24 KB for 600 bodies."""
+    from resolve2d_amd.solver import Context
+    ctx = Context(0)
+    ctx.set_lds_limit(limit)
+    dense = {0: (600, 11.0), 57: (600, 12.0), 128: (300, 7.0), 255: (450, 10.0), 256: (200, 5.0)}
+    scenes = [_heap(*dense[k], 60 + k) if k in dense else _heap(1 + (7 * k) % 40, 2.0 + k % 3, 60 + k) for k in range(257)]
+    _check(oracle, ctx, scenes, warm, coloured, list(dense) + list(range(3, 257, 16)))
+    ctx.close()
+
+
 @pytest.mark.parametrize("warm,coloured", [(False, False), (True, False), (False, True)], ids=["cold", "warm", "coloured"])
 def test_narrow_chains(oracle, warm, coloured):
     from resolve2d_amd.solver import Context
