@@ -285,7 +285,7 @@ int r2d_ctx_set_solve_variant(r2d_ctx* ctx, int variant);
 int r2d_ctx_set_lds_limit(r2d_ctx* ctx, uint32_t max_bodies);
 /* Separate launches only: a batch of at most 256 worlds runs their chains
  * with 512 threads a world (on, the default: each is alone on its CU), or 768
- * in the coloured order.  Off: with 256, unless a variant of 512 is chosen.
+ * in the coloured order from 3,000 bodies on.  Off: with 256, unless a variant of 512 is chosen.
  * Same bits either way; a launch-shape knob with no counterpart in the reference. */
 int r2d_ctx_set_wide_record(r2d_ctx* ctx, int on);
 /* Totals of the last step of the context: entries, raw candidates,

@@ -3096,10 +3096,14 @@ struct SolveVariant {
 };
 // Separate launches' workgroups.  The coloured order's slots hold about 700
 // points of a 4,096-body pile, eleven waves' rows, and take twelve waves
-// (solve 262 -> 237 us a step; sixteen, which spill, 250); the reference
+// (solve 287 -> 257 us a step; sixteen, which spill, were slower); the reference
 // order's about 200, and twelve waves cost it their barriers (24 piles 535 ->
-// 547, a pile 413 -> 417).
+// 547, a pile 413 -> 417).  So do coloured worlds whose slots eight waves
+// hold, up to 3,000 bodies (solve by eight and twelve waves, 24 piles of 300 /
+// 1,000 / 2,500 / 3,000 / 3,500 / 4,096 bodies: 145 / 193 / 261 / 295 / 324 /
+// 361 and 148 / 196 / 269 / 293 / 306 / 334 us).
 constexpr unsigned CHAIN_THREADS = 512, CHAIN_COLORED = 768, CHAIN_NARROW = 256;
+constexpr uint32_t CHAIN_COLORED_BODIES = 3000;
 // Solve variants: shapes of the kernels that run worlds' programs.  The fused
 // kernels differ in threads and in waves per SIMD (registers); 0, 6 and 8
 // have none and take the separate launches.
@@ -3226,12 +3230,12 @@ SolvePlan plan_solve(int chosen, const uint32_t* nbodies, size_t nw, uint32_t ld
     p.lds_nmax = lds_limit ? lds_limit : 0xffffffffu;
     const bool wide = (nw <= CHAIN_WIDE_WORLDS && allow_wide) ||
                       (chosen >= 0 && chosen < SOLVE_TABLE && kSolveVariants[chosen].threads == CHAIN_THREADS);
-    p.threads = !wide ? CHAIN_NARROW : any_colored && !any_warm ? CHAIN_COLORED : CHAIN_THREADS;
     // LDS: worlds that are alone on their CU take all of it; of larger batches
     // each world takes what its momenta (16 bytes a touched body), impulses (8
-    // a point) and plan (18 an item) commonly need, so that CUs hold several
+    // a point) and plan (20 an item) commonly need, so that CUs hold several
     uint32_t maxn = 0;
     for (size_t i = 0; i < nw; ++i) maxn = std::max(maxn, nbodies[i]);
+    p.threads = !wide ? CHAIN_NARROW : any_colored && !any_warm && maxn >= CHAIN_COLORED_BODIES ? CHAIN_COLORED : CHAIN_THREADS;
     const size_t want = std::max<size_t>(CHAIN_LDS_MIN, (size_t)maxn * CHAIN_LDS_BODY);
     p.lds = (uint32_t)(nw <= CHAIN_WIDE_WORLDS ? CHAIN_LDS : std::min<size_t>(CHAIN_LDS, want));
     return p;

@@ -95,3 +95,9 @@ def test_wide_chains_can_be_switched_off(coloured, warm):
     for variant in range(15):
         wide = rule(5, variant + 1, 40, 5000, coloured, warm, 0)[0]
         assert (wide >= 512) == (variant in (0, 13, 14)), variant
+
+
+def test_twelve_waves_for_coloured_worlds_that_fill_them():
+    for worlds in (1, 24, 256):
+        assert [rule(5, 0, worlds, n, 1, 0, 1)[0] for n in (10, 2999, 3000, 9000)] == [512, 512, 768, 768]
+        assert [rule(5, 0, worlds, n, c, w, 1)[0] for n in (10, 9000) for c, w in ((0, 0), (0, 1), (1, 1))] == [512] * 6
