@@ -843,7 +843,8 @@ def main():
             return copy
 
         cands = [c for c in autotune.candidates(lds_limits=(0,))
-                 if c[2] or (c[0] in (1, 11) and not args.tune_fused_only)]
+                 if c[2] or (c[0] in (1, 13) and not args.tune_fused_only)]
+        cands = autotune.distinct(cands, args.worlds)
         tuned = autotune.tune(ctx, None, dt, S, K_IT, rounds=1, cands=cands, cache_path=None,
                               steps_per_sample=K, make_batch=fresh_copy, refine=3, refine_steps=K, log=log)
         log(f"autotune: variant {tuned['variant']} fused {tuned['fused']} ({tuned['step_ms']:.3f} ms per step)")

@@ -14,8 +14,10 @@ takes whole steps per workgroup, else the sum of the four phases' HIP
 events -- candidates interleaved round by round so the slowly changing state
 does not favour any of them; the median decides.  The winner is kept per
 batch shape -- worlds, largest world and total bodies, each rounded up to a
-power of two -- in a JSON file, so later runs of the same shape reuse it.
+power of two -- sub-steps, iterations and build of the library in a JSON file,
+so later runs of the same shape reuse it.
 """
+import hashlib
 import json
 import os
 from typing import Callable, Dict, Iterable, Optional, Sequence, Tuple
@@ -61,6 +63,14 @@ def shape_key(shape: Tuple[int, int, int]) -> str:
     return "w{}_n{}_b{}".format(*shape)
 
 
+def cache_key(shape: Tuple[int, int, int], sub_steps: int, iters: int) -> str:
+    """The choice depends on the batch's shape, the call and the kernels: the
+    library's own bytes name its build."""
+    with open(N.LIB_PATH, "rb") as f:
+        build = hashlib.sha1(f.read()).hexdigest()[:12]
+    return f"{shape_key(shape)}_s{sub_steps}_k{iters}_{build}"
+
+
 def load_cache(path: str = DEFAULT_CACHE) -> Dict[str, dict]:
     try:
         with open(path) as f:
@@ -78,8 +88,13 @@ def save_cache(cache: Dict[str, dict], path: str = DEFAULT_CACHE):
     os.replace(tmp, path)
 
 
-# variants with a fused kernel
-FUSED_VARIANTS = (1, 2, 3, 4, 5, 7, 9, 10, 11, 12, 13, 14)
+# variants with a fused kernel: its threads and waves per SIMD
+FUSED_SHAPES = {1: (256, 3), 2: (512, 3), 3: (256, 3), 4: (256, 2), 5: (128, 2), 7: (256, 3), 9: (256, 3), 10: (256, 4),
+                11: (192, 3), 12: (128, 2), 13: (512, 2), 14: (768, 3)}
+FUSED_VARIANTS = tuple(FUSED_SHAPES)
+# variants whose phase kernels' chains are wide whatever the batch, and the
+# largest batch whose chains are wide whatever the variant
+WIDE_VARIANTS, WIDE_WORLDS = (0, 13, 14), 256
 
 
 def candidates(variants: Optional[Iterable[int]] = None, lds_limits: Iterable[int] = (0, 1024),
@@ -94,6 +109,19 @@ def candidates(variants: Optional[Iterable[int]] = None, lds_limits: Iterable[in
                 continue
             for lim in ((0,) if f else lds_limits):
                 out.append((v, lim, bool(f)))
+    return out
+
+
+def distinct(cands, worlds: int) -> list:
+    """The candidates without those that launch the same kernels as an earlier
+    one does on a batch of that many worlds: several variants share a shape."""
+    seen, out = set(), []
+    for c in cands:
+        v, lim, fused = c[0], c[1], c[2] if len(c) > 2 else True
+        shape = (True, FUSED_SHAPES[v]) if fused else (False, lim, v in WIDE_VARIANTS or worlds <= WIDE_WORLDS)
+        if shape not in seen:
+            seen.add(shape)
+            out.append(c)
     return out
 
 
@@ -133,7 +161,7 @@ def tune(ctx, handles: Sequence, dt: float, sub_steps: int, iters: int, rounds: 
     if handles is None:
         probe = make_batch()
         handles = [w.handle for w in probe]
-    key = shape_key(batch_shape(ctx, handles))
+    key = cache_key(batch_shape(ctx, handles), sub_steps, iters)
     if probe is not None:
         for w in probe:
             w.close()
@@ -141,7 +169,7 @@ def tune(ctx, handles: Sequence, dt: float, sub_steps: int, iters: int, rounds: 
     if key in cache:
         apply(ctx, cache[key])
         return dict(cache[key], key=key, cached=True)
-    cands = cands or candidates()
+    cands = cands or distinct(candidates(), len(handles))
     times = {c: [] for c in cands}
     was = ctx.profiling
 

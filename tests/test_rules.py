@@ -101,3 +101,31 @@ def test_twelve_waves_for_coloured_worlds_that_fill_them():
     for worlds in (1, 24, 256):
         assert [rule(5, 0, worlds, n, 1, 0, 1)[0] for n in (10, 2999, 3000, 9000)] == [512, 512, 768, 768]
         assert [rule(5, 0, worlds, n, c, w, 1)[0] for n in (10, 9000) for c, w in ((0, 0), (0, 1), (1, 1))] == [512] * 6
+
+
+def test_autotuner_times_each_shape_once():
+    from resolve2d_amd import autotune
+    fused = [(v, 0, True) for v in autotune.FUSED_VARIANTS]
+    phases = [(v, lim, False) for v in autotune.PHASE_VARIANTS for lim in (0, 1024)]
+    for worlds in (1, 256, 257, 1024):
+        kept = autotune.distinct(fused + phases, worlds)
+        assert [c[0] for c in kept if c[2]] == [1, 2, 4, 5, 10, 11, 13, 14]
+        # the library's own rule for the chains' threads
+        threads = lambda v: min(512, rule(5, v + 1, worlds, 5000, 0, 0, 1)[0])
+        want = []
+        for v, lim, _ in phases:
+            if (threads(v), lim) not in want:
+                want.append((threads(v), lim))
+        assert [(threads(v), lim) for v, lim, f in kept if not f] == want
+        assert autotune.distinct(kept, worlds) == kept
+
+
+def test_autotuner_keeps_choices_by_call_and_build(monkeypatch, tmp_path):
+    from resolve2d_amd import _native, autotune
+    shape = (1024, 512, 262144)
+    keys = [autotune.cache_key(shape, 4, 4), autotune.cache_key(shape, 4, 16), autotune.cache_key(shape, 2, 4)]
+    lib = tmp_path / "lib.so"
+    lib.write_bytes(b"another build")
+    monkeypatch.setattr(_native, "LIB_PATH", str(lib))
+    keys.append(autotune.cache_key(shape, 4, 4))
+    assert len(set(keys)) == 4 and all(k.startswith(autotune.shape_key(shape)) for k in keys)
