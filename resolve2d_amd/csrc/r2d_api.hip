@@ -1988,7 +1988,6 @@ R2D_EXPORT int r2d_ctx_create(int device, r2d_ctx** out)
     if (const char* e = std::getenv("R2D_TRACE_KERNELS")) {
         if (e[0] == '1') {
             c->trace = new (std::nothrow) KernelTrace();
-            if (c->trace) c->trace->main = c->stream;
             c->use_graph = false;   // an event after every launch: eager launches
         }
     }

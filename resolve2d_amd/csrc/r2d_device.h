@@ -110,7 +110,8 @@ constexpr uint32_t CHAIN_BODIES = 1u << 27;
 struct WorldChain {
     uint32_t bodies;    // places: bodies its items touch
     uint32_t pairs;     // manifolds of two points
-    uint32_t flags;     // 1: updateTGSDepth is live; 2: some static body is an ordering body
+    uint32_t flags;     // 1: updateTGSDepth is live; 2: the reference's sums to the letter (a static ordering body,
+                        // a normal or an arm that is not finite, a momentum component of -0)
     uint32_t slots;     // of its program
     uint32_t rest_slots;   // ... and of the shorter one after it
     uint32_t entries;   // of both

@@ -82,12 +82,10 @@ struct KernelTrace {
     struct Mark {
         const char* name;
         hipEvent_t ev;
-        hipStream_t st;
     };
     std::vector<Mark> marks;
     std::vector<hipEvent_t> pool;
     std::map<std::string, std::pair<double, uint64_t>> totals;
-    hipStream_t main = nullptr;
     void mark(const char* name, hipStream_t st);
     void flush();                 // synchronise and add the recorded intervals
     void report(FILE* f);

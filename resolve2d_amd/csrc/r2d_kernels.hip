@@ -1485,7 +1485,7 @@ __device__ __forceinline__ FusedLds fused_carve(uint32_t* lds, uint32_t n, uint3
 // Words per body after the front part: the pair cache and room for the
 // bucket arrays.  The solve then has the whole of LDS but dcnt and doff: 16
 // words a body with 2 n buckets, 7 of them momenta and poses, and in the rest
-// the plan (4 words an item), then 3 words a body and the impulses (2 a
+// the plan (5 words an item), then 3 words a body and the impulses (2 a
 // point).  A world of 500 bodies takes 36 KB: four to a CU.
 constexpr uint32_t FUSED_TAIL_WORDS = 8;
 // Least dynamic LDS of a launch: room for the plan of a small world with many
@@ -3106,7 +3106,8 @@ constexpr unsigned CHAIN_THREADS = 512, CHAIN_COLORED = 768, CHAIN_NARROW = 256;
 constexpr uint32_t CHAIN_COLORED_BODIES = 3000;
 // Solve variants: shapes of the kernels that run worlds' programs.  The fused
 // kernels differ in threads and in waves per SIMD (registers); 0, 6 and 8
-// have none and take the separate launches.
+// have none and take the separate launches.  1, 3, 7 and 9 are alike, and 5
+// and 12: the numbers are the interface's and stay.
 static const SolveVariant kSolveVariants[SOLVE_TABLE] = {
     {CHAIN_THREADS, nullptr, 0},
     {CHAIN_NARROW, k_fused<256, 3>, 256},
@@ -3171,26 +3172,25 @@ void KernelTrace::mark(const char* name, hipStream_t st)
     }
     hipEvent_t e = pool[marks.size()];
     if (hipEventRecord(e, st) != hipSuccess) return;
-    marks.push_back({name, e, st});
+    marks.push_back({name, e});
 }
 
 void KernelTrace::flush()
 {
     if (marks.empty()) return;
     (void)hipDeviceSynchronize();
-    // a main-stream kernel's interval starts at the previous main-stream mark;
-    // a side-stream kernel's at the last main-stream mark before it (the fork)
-    const Mark* prev_main = nullptr;
+    // a kernel's interval starts at the mark before it
+    const Mark* before = nullptr;
     for (const Mark& m : marks) {
-        if (prev_main && m.name[0]) {
+        if (before && m.name[0]) {
             float ms = 0.f;
-            if (hipEventElapsedTime(&ms, prev_main->ev, m.ev) == hipSuccess) {
+            if (hipEventElapsedTime(&ms, before->ev, m.ev) == hipSuccess) {
                 auto& t = totals[m.name];
                 t.first += ms;
                 t.second += 1;
             }
         }
-        if (m.st == main) prev_main = &m;
+        before = &m;
     }
     marks.clear();
 }
