@@ -698,7 +698,7 @@ struct ChainProgram {
     GCU4 recs;
     uint32_t nslots, reps, nj, nacc, idle, jbase;
 };
-// the program after it (plan_world): rows and slots from `rows` on
+// the program after it (plan_rest): rows and slots from `rows` on
 __device__ __forceinline__ ChainProgram rest_program(ChainProgram G, uint32_t rows, uint32_t nslots)
 {
     G.rows += rows;

@@ -2345,9 +2345,12 @@ __global__ __launch_bounds__(256) void k_chain_build(StepDev S, float sub_dt)
     }
 }
 
-// the program of each world, one workgroup each
+// The program of each world, one workgroup each; with `rest`, in a launch after
+// it, the one for the rest of the iterations: its rows and slots from
+// chain_iters * nit on, its entries after the others.  (Planned through, every
+// item waits for what it waited for at first.)
 template <int T>
-__global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
+__global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words, uint32_t rest)
 {
     extern __shared__ __align__(16) uint32_t smem[];
     __shared__ ChainShared sh;
@@ -2355,11 +2358,14 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     const uint32_t w = S.w_order[blockIdx.x];
     const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, nj = (uint32_t)S.worlds[w].njoints;
     if (S.w_status[w] != 0 || nit == 0u) return;
-    const uint32_t t = threadIdx.x, kc = S.chain_iters, waves = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
-    const size_t rows = (size_t)ibase * S.chain_room();
+    const uint32_t t = threadIdx.x, kc = rest ? rest : S.chain_iters,
+                   waves = chain_waves(nit, S.chain_iters, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
+    const size_t rows = (size_t)ibase * S.chain_room() + (rest ? (size_t)S.chain_iters * nit : 0u);
+    const uint32_t before = rest ? S.w_chain[w].entries : 0u;
     const bool in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= lds_words;
     if (t == 0) {
-        sh.ready = sh.taken = sh.entries = 0u;
+        sh.ready = sh.taken = 0u;
+        sh.entries = before;
         sh.queued[0] = sh.queued[1] = sh.queued[2] = 0u;
     }
     __syncthreads();
@@ -2372,8 +2378,9 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     PlanGlb PG(items, (GU4)(S.plan_ring + 2 * (size_t)ibase), nit, waves);
     auto start = [&](auto& P, bool init) {
         for (uint32_t j = t; j < nit; j += T) {
-            const u4v v = items[j];
-            if (init) P.init(j, v.x, v.y, v.z, v.w);
+            u4v v = items[j];
+            if (rest) v.z = (v.z & ~(STATE_BODY - 1u)) + rest;
+            if (init || rest) P.init(j, v.x, v.y, v.z, v.w);
             if (v.z < STATE_BODY)
                 P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
                        P.pack(PlanEntry{j, v.w, v.x, v.y}));
@@ -2383,26 +2390,13 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words)
     if (in_lds) start(PL, true); else start(PG, false);
     __syncthreads();
     const uint32_t ready = uniform(sh.ready);
-    uint32_t ns = 0u, entries = 0u;
+    uint32_t ns = 0u, entries = before;
     if (waves > 1u)
         ns = in_lds ? plan_multi(PL, G, nit, nj, kc, ready, waves, sh) : plan_multi(PG, G, nit, nj, kc, ready, waves, sh);
     else if (t < 64u)
         ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
-    if (S.chain_rest) {
-        if (t == 0) {
-            sh.failed = ns == 0u;
-            if (waves == 1u) sh.entries = entries;
-        }
-        __syncthreads();
-        if (!sh.failed) {
-            plan_rest(PlanMemory{(LU32)smem, items, PG.ring, G}, in_lds, nit, nj, kc, S.chain_rest, waves, (R2D_LDS ChainShared*)&sh);
-            if (sh.rest_slots == 0u) ns = 0u;
-            entries = sh.entries;
-            if (t == 0) S.w_chain[w].rest_slots = sh.rest_slots;
-        }
-    }
     if (t == 0) {
-        S.w_chain[w].slots = ns;
+        if (rest) S.w_chain[w].rest_slots = ns; else S.w_chain[w].slots = ns;
         S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2483,12 +2477,14 @@ __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uin
 }
 
 // Sub-step s's joint records, moved contact points and carried impulses, and
-// its K iterations, one workgroup per world.  Momenta in LDS for worlds of at
+// its iterations, one workgroup per world; with `rest`, in a launch after it,
+// only the iterations that end the sub-step (a loop over both programs in one
+// launch cost those without a rest 3 us a step of a 4,096-body pile).  Momenta in LDS for worlds of at
 // most lds_nmax bodies whose places fit it, and beside them the impulses when
 // they fit too; otherwise they stay in global memory.
 template <int T, bool WARM>
 __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t iters, float sub_dt, uint32_t lds_words,
-                                                 uint32_t lds_nmax)
+                                                 uint32_t lds_nmax, uint32_t rest)
 {
     extern __shared__ __align__(16) uint32_t smem[];
     if (S.counters[C_OVERFLOW]) return;
@@ -2508,7 +2504,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     if (m_lds)
         for (uint32_t c = t; c < nc; c += T) m[c] = mom[c];
-    if (s == 0u)
+    if (s == 0u && !rest)
         for (uint32_t q = t; q < nacc; q += T) {
             if (a_lds) acc[q] = f2v{0.f, 0.f}; else accg[q] = f2v{0.f, 0.f};
         }
@@ -2519,14 +2515,14 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     const GCU32 entries = (GCU32)world_entries(S, w, ibase);
     const uint32_t jbase = joint_entries(W.entries);
     const GlobalPoses C = global_poses(D);
-    for (uint32_t j = t; j < nj && iters > 0u; j += T) {
+    for (uint32_t j = t; j < nj && iters > 0u && !rest; j += T) {
         u4v q[4];
         joint_record(q, D.joints[j], D, C, s == 0u, [&](uint32_t x) { return S.cmap[base + x]; });
         const GU4 to = prog + entry_at(jbase + j);
         for (int p = 0; p < 4; ++p) to[p * ENTRY_WORD] = q[p];
     }
     __syncthreads();
-    if (W.flags & 1u) {
+    if ((W.flags & 1u) && !rest) {
         for (uint32_t q = t; q < M; q += T) {
             const uint32_t p1 = S.it_k0[ibase + nj + q];
             point_tgs(S, D, recs, C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
@@ -2541,7 +2537,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         }
     }
     if constexpr (WARM) {
-        if (D.warm > 0.0f) {
+        if (D.warm > 0.0f && !rest) {
             const size_t cm = S.cap_m;
             for (uint32_t q = t; q < M; q += T) {
                 // warm starting: the carried impulse per sub-step joins the accumulators
@@ -2558,25 +2554,18 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     }
     __syncthreads();
     if (iters > 0u) {
-        const size_t rows = (size_t)ibase * S.chain_room();
-        ChainProgram G{(GCU2)(S.prog_rows + rows), entries, (GCU2)(S.prog_slots + rows), (GCU4)prog, W.slots, iters / kc,
-                       nj, nacc, jbase + nj, jbase};
+        const size_t rows = (size_t)ibase * S.chain_room() + (rest ? (size_t)kc * nit : 0u);
+        const ChainProgram G{(GCU2)(S.prog_rows + rows), entries, (GCU2)(S.prog_slots + rows), (GCU4)prog,
+                             rest ? W.rest_slots : W.slots, rest ? 1u : iters / kc, nj, nacc, jbase + nj, jbase};
         const bool fix = W.flags != 0u;
-        const bool several = chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u;
-#pragma clang loop unroll(disable)
-        for (uint32_t left = W.rest_slots;;) {
-            if (several) {
-                if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
-                else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
-                else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);
-            } else if (t < 64u) {
-                if (a_lds) chain_lds<false, WARM, true>(G, m, nc, acc, fix, sub_dt);
-                else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
-                else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
-            }
-            if (left == 0u) break;
-            G = rest_program(G, kc * nit, left);
-            left = 0u;
+        if (chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
+            if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
+            else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);
+        } else if (t < 64u) {
+            if (a_lds) chain_lds<false, WARM, true>(G, m, nc, acc, fix, sub_dt);
+            else if (m_lds) chain_lds_accg<false, WARM, true>(G, m, nc, accg, fix, sub_dt);
+            else chain_glb<false, WARM, true>(G, mom, nc, accg, fix, sub_dt);
         }
         __syncthreads();
     }
@@ -3322,8 +3311,13 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             tmark(ss, "k_chain_build", st);
             if (iters > 0) {
                 hipLaunchKernelGGL(width(k_chain_plan<CHAIN_NARROW>, k_chain_plan<CHAIN_THREADS>, k_chain_plan<CHAIN_COLORED>),
-                                   dim3(S.nworlds), dim3(T), sp.lds, st, S, words);
+                                   dim3(S.nworlds), dim3(T), sp.lds, st, S, words, 0u);
                 tmark(ss, "k_chain_plan", st);
+                if (S.chain_rest) {
+                    hipLaunchKernelGGL(width(k_chain_plan<CHAIN_NARROW>, k_chain_plan<CHAIN_THREADS>, k_chain_plan<CHAIN_COLORED>),
+                                       dim3(S.nworlds), dim3(T), sp.lds, st, S, words, S.chain_rest);
+                    tmark(ss, "k_chain_plan (rest)", st);
+                }
             }
         }
         for (uint32_t s = 0; sub_steps > 0; ++s) {
@@ -3335,8 +3329,12 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             auto run = width(pick(k_chain_run<CHAIN_NARROW, true>, k_chain_run<CHAIN_NARROW, false>),
                              pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>),
                              k_chain_run<CHAIN_COLORED, false>);
-            hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax);
+            hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax, 0u);
             tmark(ss, "k_chain_run", st);
+            if (S.chain_rest && iters > 0u) {
+                hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax, S.chain_rest);
+                tmark(ss, "k_chain_run (rest)", st);
+            }
         }
         if (sp.any_warm) {
             hipLaunchKernelGGL(k_warm_clear, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
