@@ -39,8 +39,8 @@ constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 2;
 // rows 10.0 / 4.7 / 3.4 / 2.7, world of 387 bodies 0.58 / 0.61 / 0.64 / 0.99,
 // 97 worlds 0.78 / 0.80 / 1.09 / 1.34, 4,096-body pile 1.47 / 1.24 / 1.33 /
 // 1.54).  17 iterations, one at a time and by fours: pyramids of 20 and 60
-// rows 2.29 -> 0.96 and 9.5 -> 5.2 ms, 4,096-body pile 1.43 -> 1.31; shallow
-// worlds pay for planning more, 387 bodies 0.61 -> 0.65, 97 worlds 0.79 -> 0.89.
+// rows 2.29 -> 0.96 and 9.5 -> 5.2 ms, 4,096-body pile 1.43 -> 1.34; shallow
+// worlds pay for planning more, 387 bodies 0.61 -> 0.65, 97 worlds 0.79 -> 0.88.
 constexpr uint32_t CHAIN_ITERS_MAX = 16, CHAIN_ITERS_ENOUGH = 4;
 struct ChainSplit {
     uint32_t each, rest;   // iterations of the program, and of the one that ends a sub-step
@@ -71,8 +71,9 @@ struct SolvePlan {
     uint32_t any_colored = 0;  // some world uses the coloured schedule
     uint32_t any_warm = 0;     // some world is warm started
 };
-// chosen: the variant that the caller chose (-1: none); lds_limit: largest world (bodies) that keeps its momenta in LDS (0: as many
-// as LDS holds)
+// chosen: the variant that the caller chose (-1: none); lds_limit: largest
+// world (bodies) that keeps its momenta in LDS (0: as many as LDS holds);
+// allow_wide: small batches may take wide chains whose caller chose none
 SolvePlan plan_solve(int chosen, const uint32_t* nbodies, size_t nw, uint32_t lds_limit, bool any_colored,
                      bool any_warm, bool allow_wide = true);
 

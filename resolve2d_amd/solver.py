@@ -81,7 +81,8 @@ class Context:
 
     def set_wide_record(self, on: bool):
         """Phase kernels: batches of at most 256 worlds run their chains with
-        512 threads a world (default on).  Same bits either way."""
+        512 or 768 threads a world (default on); off, with 256 unless a solve
+        variant of 512 is chosen.  Same bits either way."""
         N.check(self.lib.r2d_ctx_set_wide_record(self.handle, 1 if on else 0), "r2d_ctx_set_wide_record")
 
     def set_fused(self, on: bool):
