@@ -310,6 +310,8 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
  * rule 1: in {bodies, buckets, worlds, joints, cell entries, raw candidates,
  * manifolds, solver items, iterations of the programs}; out {bytes of the step
  * scratch that holds them}.
+ * rule 6: in {solver items, collision iterations, waves of the workgroup}; out
+ * {waves that run a world's program in the one-kernel step}.
  * rule 5: in {chosen variant + 1 (0: none), worlds, bodies of each, whether
  * one is coloured, whether one is warm started, r2d_ctx_set_wide_record}; out
  * {threads of the separate launches' chains, bytes of LDS}.

@@ -2840,6 +2840,9 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
         out[1] = s.rest;
         return R2D_OK;
     }
+    case 6:
+        out[0] = fused_waves((uint32_t)in[0], chain_split(in[1]).each, (uint32_t)in[2]);
+        return R2D_OK;
     case 5: {
         const uint32_t n = (uint32_t)in[2];
         std::vector<uint32_t> sizes(std::max<size_t>(1, in[1]), n);

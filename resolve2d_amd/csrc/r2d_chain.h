@@ -490,21 +490,6 @@ __device__ __attribute__((noinline)) void plan_rest(PlanMemory X, bool in_lds, u
     __syncthreads();
 }
 
-// Waves that run a world's rows: one for each `rows` rows of 64 its items fill
-// (a pile's chain is 90-150 slots deep for 4 iterations).  In the one-kernel
-// step a slot of several waves costs about two rows of one, so they pay from
-// 96 rows on (97 worlds x 8 steps, when this line was drawn: 3.40 ms, with 48
-// 4.45 ms; 2.26 now).  In the separate
-// launches, records in program order, wider is better down to a wave for 32
-// rows (solve of a 4,096-body pile, 96 / 48 / 24 rows: 529 / 499 / 498 us;
-// coloured 417 / 311 / 308).
-constexpr uint32_t FUSED_WAVE_ROWS = 96, CHAIN_WAVE_ROWS = 32;
-__host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, uint32_t most, uint32_t rows)
-{
-    const uint32_t w = (uint32_t)(((uint64_t)nit * iters / 64u + rows - 1u) / rows);
-    return w < 1u ? 1u : (w < most ? w : most);
-}
-
 // ----------------------------------------------------------------- the chain
 // momenta (x, y, angular) of a world's bodies in LDS, 16 bytes a body; the
 // SPARE places after the last body take the writes that are not to be kept,

@@ -58,6 +58,30 @@ inline ChainSplit chain_split(size_t iters, uint32_t most = CHAIN_ITERS_MAX)
     return ChainSplit{CHAIN_ITERS_ENOUGH, (uint32_t)(iters % CHAIN_ITERS_ENOUGH)};
 }
 
+// Waves that run a world's rows: one for each `rows` rows of 64 its items fill
+// (a pile's chain is 90-150 slots deep for 4 iterations).  In the one-kernel
+// step a slot of several waves costs about two rows of one, so they pay from
+// 96 rows on (97 worlds x 8 steps, when this line was drawn: 3.40 ms, with 48
+// 4.45 ms; 2.26 now).  In the separate
+// launches, records in program order, wider is better down to a wave for 32
+// rows (solve of a 4,096-body pile, 96 / 48 / 24 rows: 529 / 499 / 498 us;
+// coloured 417 / 311 / 308).
+// Whether several pay in the one-kernel step is asked of four iterations at
+// most: more of them make a program longer, not wider.  Asked of all, sixteen
+// iterations took several waves from 384 items on (20-row pyramid 954 us a
+// step, now 512; 387 bodies 988 and 602; 97 worlds 1,340 and 802).
+constexpr uint32_t FUSED_WAVE_ROWS = 96, CHAIN_WAVE_ROWS = 32, FUSED_WAVE_ITERS = 4;
+__host__ __device__ inline uint32_t chain_waves(uint32_t nit, uint32_t iters, uint32_t most, uint32_t rows)
+{
+    const uint32_t w = (uint32_t)(((uint64_t)nit * iters / 64u + rows - 1u) / rows);
+    return w < 1u ? 1u : (w < most ? w : most);
+}
+__host__ __device__ inline uint32_t fused_waves(uint32_t nit, uint32_t iters, uint32_t most)
+{
+    const bool several = chain_waves(nit, iters < FUSED_WAVE_ITERS ? iters : FUSED_WAVE_ITERS, most, FUSED_WAVE_ROWS) > 1u;
+    return several ? chain_waves(nit, iters, most, FUSED_WAVE_ROWS) : 1u;
+}
+
 // The separate launches' chain: batches of at most this many worlds (one per
 // CU) take wide workgroups and all of LDS.
 constexpr size_t CHAIN_WIDE_WORLDS = 256;

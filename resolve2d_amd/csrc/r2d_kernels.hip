@@ -2057,7 +2057,7 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n, 0u);
     const ChainBodies& C = L.C;
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
-    const uint32_t waves = chain_waves(nit, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS);
+    const uint32_t waves = fused_waves(nit, kc, (uint32_t)T / 64u);
     const bool chain = nit > 0u && sh.iters > 0u;
     const bool plan_in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words;
     Program G;
@@ -2247,7 +2247,7 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
-        const bool several = chain_waves(nj + M, kc, (uint32_t)T / 64u, FUSED_WAVE_ROWS) > 1u;
+        const bool several = fused_waves(nj + M, kc, (uint32_t)T / 64u) > 1u;
 #pragma clang loop unroll(disable)
         for (uint32_t left = rest_slots;;) {
             if (several) {

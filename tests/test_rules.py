@@ -129,3 +129,13 @@ def test_autotuner_keeps_choices_by_call_and_build(monkeypatch, tmp_path):
     monkeypatch.setattr(_native, "LIB_PATH", str(lib))
     keys.append(autotune.cache_key(shape, 4, 4))
     assert len(set(keys)) == 4 and all(k.startswith(autotune.shape_key(shape)) for k in keys)
+
+
+@pytest.mark.parametrize("waves", [4, 12])
+def test_more_iterations_do_not_spread_a_small_world(waves):
+    """One wave runs a world in the one-kernel step up to 1,536 items, however
+    many iterations (fewer iterations: up to more)."""
+    for iters in (4, 8, 16, 17, 100):
+        assert [rule(6, n, iters, waves)[0] for n in (0, 1, 400, 1536)] == [1] * 4
+        assert rule(6, 1600, iters, waves)[0] > 1
+    assert rule(6, 3000, 1, waves)[0] == rule(6, 3000, 2, waves)[0] == 1
