@@ -171,7 +171,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const uint32_t* in, 
     }
 }
 
-// Tiles taken in the order of a ticket.  A tile publishes its sum, adds up its
+// The single-pass scan with decoupled look-back (Merrill and Garland).  Tiles
+// taken in the order of a ticket.  A tile publishes its sum, adds up its
 // predecessors' (64 at a time, each a sum or, from some tile on, a prefix) and
 // publishes its prefix: value and kind in one 64-bit word.  Every tile it waits
 // for has its ticket and runs, so the wait ends; the limit only bounds it.
