@@ -815,17 +815,11 @@ constexpr struct {
 } kScratchTries[] = {{CHAIN_ITERS_MAX, true}, {CHAIN_SHORT, true}, {1u, true}, {1u, false}};
 constexpr size_t kProgramPlaces = (size_t)1 << 30;   // places of a program that its entries can name
 
-// programs of the separate launches for a call, where they may cover `most`
-ChainSplit separate_split(size_t sub_steps, size_t iters, uint32_t most)
-{
-    return chain_split(iters, std::min(most, chain_most(sub_steps, iters)));
-}
-
-// carve the step scratch for the current capacities, and a call's sub-steps and iterations
+// carve the step scratch for the current capacities; iters: the call's iterations
 int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, uint32_t e, uint32_t r, uint32_t m,
-                   uint32_t it, size_t sub_steps, size_t iters)
+                   uint32_t it, size_t iters)
 {
-    if (separate_split(sub_steps, iters, c->chain_most).room() <= c->cap_k && n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w &&
+    if (chain_split(iters, c->chain_most).room() <= c->cap_k && n <= c->cap_n && b <= c->cap_b && wn <= c->cap_w &&
         j <= c->cap_j && e <= c->cap_e && r <= c->cap_r && m <= c->cap_m && it <= c->cap_i && c->arena)
         return R2D_OK;
     if (c->arena) {
@@ -843,7 +837,7 @@ int ensure_scratch(r2d_ctx* c, uint32_t n, uint32_t b, uint32_t wn, uint32_t j, 
             return (size_t)std::min<uint64_t>(v, 0xffffff00ull);
         };
         caps = ScratchCaps{grow(c->cap_n, n), grow(c->cap_b, b), grow(c->cap_w, wn), grow(c->cap_j, j), grow(c->cap_e, e),
-                           grow(c->cap_r, r), grow(c->cap_m, m), grow(c->cap_i, it), separate_split(sub_steps, iters, t.most).room()};
+                           grow(c->cap_r, r), grow(c->cap_m, m), grow(c->cap_i, it), chain_split(iters, t.most).room()};
         // what longer calls got, unless it is in the way now
         if (t.most == CHAIN_ITERS_MAX && c->chain_most == CHAIN_ITERS_MAX) caps.k = std::max<size_t>(caps.k, c->cap_k);
         if (2 * caps.k * caps.i + 8 * caps.w > kProgramPlaces) continue;
@@ -973,7 +967,6 @@ struct Batch {
     std::vector<int32_t> world_status;   // device status per world of the last wait
     bool fused = false;                  // whole steps per workgroup (k_fused)
     size_t fused_lds = 0;
-    uint32_t fused_most = CHAIN_ITERS_MAX;   // iterations its programs may cover
     int variant = 0;
 };
 
@@ -1376,14 +1369,13 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     if (fused) {
         b.fused_lds = fused_lds_share(worlds_per_cu(c, nw), fused_groups(variant), maxn, maxtb);
         fused = b.fused_lds <= kFusedLdsMax;
-        b.fused_most = fused_most(sub_steps, iters, maxn);
     }
     b.fused = fused;
     int rc;
     if (fused) {
         // the step scratch holds the per-body and per-world arrays; the
         // worlds' slices live in the fused arena
-        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1, 0, 0)))
+        if ((rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, 1, 1, 1, 1, 0)))
             return rc;
         return fused_layout(c, b);
     }
@@ -1392,8 +1384,7 @@ int batch_prepare(r2d_ctx* c, r2d_world* const* worlds, size_t nw, float dt, siz
     uint32_t est_m = std::max<uint32_t>(c->cap_m, (uint32_t)(4 * b.N + 1024));
     // convex bodies touch at most three others each on average; settled piles and stacks have 1.4 to 2.3 manifolds a body
     uint32_t est_i = std::max<uint32_t>(c->cap_i, (uint32_t)(b.J + 2 * b.N + 1024));
-    return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m, est_i,
-                          b.sub, b.iters);
+    return ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, est_e, est_r, est_m, est_i, b.iters);
 }
 
 // sum the phase times of the timed steps recorded so far
@@ -1430,7 +1421,7 @@ int batch_launch(r2d_ctx* c, Batch& b)
     StepDev S = c->S;
     S.nb = (uint32_t)b.N; S.nworlds = (uint32_t)nw; S.nbuckets = (uint32_t)b.B; S.njoints = (uint32_t)b.J;
     S.worlds = c->dworlds;
-    set_split(S, separate_split(b.sub, b.iters, c->chain_most));
+    set_split(S, chain_split(b.iters, c->chain_most));
     const Streams ss = c->streams();
     const uint32_t sub = (uint32_t)b.sub, iters = (uint32_t)b.iters;
     auto eager_phase = [&](int ph) { launch_phase(S, ss, ph, b.dt, sub, iters, b.plan); };
@@ -1504,7 +1495,7 @@ int fused_launch(r2d_ctx* c, Batch& b)
     StepDev F = fused_view(c);
     F.nb = (uint32_t)b.N; F.nworlds = (uint32_t)nw; F.nbuckets = (uint32_t)b.B; F.njoints = (uint32_t)b.J;
     F.worlds = c->dworlds;
-    set_split(F, chain_split(b.iters, std::min(c->fchain_most, b.fused_most)));
+    set_split(F, chain_split(b.iters, c->fchain_most));
     if (c->profiling) {
         // The timing buffers grow rarely and by a lot: a launch that follows a
         // hipMalloc closely can stall all of its waves for several ms at once
@@ -1689,7 +1680,7 @@ int batch_wait(r2d_ctx* c, Batch& b)
                 const uint64_t items = b.J + c->hcounters[C_MANIFOLDS];
                 it = (uint32_t)std::min<uint64_t>(items + items / 4, 0x7fffffffu);
             }
-            int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e, r, m, it, b.sub, b.iters);
+            int rc = ensure_scratch(c, (uint32_t)b.N, (uint32_t)b.B, (uint32_t)nw, (uint32_t)b.J, e, r, m, it, b.iters);
             if (rc) return rc;
         }
         if (b.done >= b.steps) break;
@@ -2375,7 +2366,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     WorldDev* ddesc = nullptr;
     static_layout(base, &F, &ddesc);
     F.nb = n; F.nbuckets = tb; F.njoints = nj;
-    set_split(F, chain_split(iters, fused_most(sub_steps, iters, n)));
+    set_split(F, chain_split(iters));
     // host values the asynchronous uploads read; the call waits for the
     // stream before they go out of scope
     WorldDev d = w->desc;
@@ -2875,12 +2866,6 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
     case 6:
         out[0] = fused_waves((uint32_t)in[0], chain_split(in[1]).each, (uint32_t)in[2]);
         return R2D_OK;
-    case 7: {
-        const ChainSplit s = separate_split(in[0], in[1], CHAIN_ITERS_MAX);
-        out[0] = s.each;
-        out[1] = s.rest;
-        return R2D_OK;
-    }
     case 5: {
         const uint32_t n = (uint32_t)in[2];
         std::vector<uint32_t> sizes(std::max<size_t>(1, in[1]), n);

@@ -51,32 +51,11 @@ struct ChainSplit {
 constexpr uint32_t CHAIN_SHORT = 2 * CHAIN_ITERS_ENOUGH - 1;
 inline ChainSplit chain_split(size_t iters, uint32_t most = CHAIN_ITERS_MAX)
 {
-    if (iters == 0) return ChainSplit{1u, 0u};
+    if (iters == 0 || most < CHAIN_SHORT) return ChainSplit{1u, 0u};
     if (iters <= most) return ChainSplit{(uint32_t)iters, 0u};
-    if (most <= 1) return ChainSplit{1u, 0u};
-    for (uint32_t k = most; k >= (most < CHAIN_ITERS_ENOUGH ? 2u : CHAIN_ITERS_ENOUGH); --k)
+    for (uint32_t k = most; k >= CHAIN_ITERS_ENOUGH; --k)
         if (iters % k == 0) return ChainSplit{k, 0u};
-    const uint32_t each = most < CHAIN_ITERS_ENOUGH ? most : CHAIN_ITERS_ENOUGH;
-    return ChainSplit{each, (uint32_t)(iters % each)};
-}
-// The separate launches plan before the first chain, and a step of one
-// sub-step runs what they plan that one time: programs for a quarter of the
-// iterations, but two (one sub-step of 8 iterations by programs of 8 and of 2:
-// 4,096-body pile 737 and 479 us a step, 24 piles 750 and 531, 60-row pyramid
-// 1,153 and 1,180; piles with more items than LDS plans, which programs of all
-// iterations made slower than no programs at all: 2.7, 1.2 and 2.0 ms).
-inline uint32_t chain_most(size_t sub_steps, size_t iters)
-{
-    if (sub_steps > 1) return CHAIN_ITERS_MAX;
-    return (uint32_t)(iters / 4 < 2 ? 2 : iters / 4 < CHAIN_ITERS_MAX ? iters / 4 : CHAIN_ITERS_MAX);
-}
-// So does the one-kernel step with the worlds that several waves plan (from
-// about 800 bodies on; 1,000 bodies, 8 iterations: 531 and 293 us); one wave's
-// first chain runs behind its planner.
-constexpr uint32_t FUSED_SEVERAL_BODIES = 800;
-inline uint32_t fused_most(size_t sub_steps, size_t iters, uint32_t bodies)
-{
-    return bodies >= FUSED_SEVERAL_BODIES ? chain_most(sub_steps, iters) : CHAIN_ITERS_MAX;
+    return ChainSplit{CHAIN_ITERS_ENOUGH, (uint32_t)(iters % CHAIN_ITERS_ENOUGH)};
 }
 
 // Waves that run a world's rows: one for each `rows` rows of 64 its items fill

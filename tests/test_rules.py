@@ -131,16 +131,6 @@ def test_autotuner_keeps_choices_by_call_and_build(monkeypatch, tmp_path):
     assert len(set(keys)) == 4 and all(k.startswith(autotune.shape_key(shape)) for k in keys)
 
 
-@pytest.mark.parametrize("iters", list(range(1, 70)) + [127, 1009])
-def test_one_sub_step_plans_short_programs(iters):
-    """What one sub-step plans it runs once: programs of a quarter of the
-    iterations, but two; more sub-steps as before.  Never more room."""
-    assert rule(7, 2, iters)[:2] == rule(7, 4, iters)[:2] == rule(0, iters)[:2]
-    each, rest = rule(7, 1, iters)[:2]
-    assert 1 <= each <= max(2, iters // 4) and (iters - rest) % each == 0 and rest < each
-    assert each >= min(iters, 2) and each + rest <= sum(rule(0, iters)[:2])
-
-
 @pytest.mark.parametrize("waves", [4, 12])
 def test_more_iterations_do_not_spread_a_small_world(waves):
     """One wave runs a world in the one-kernel step up to 1,536 items, however
