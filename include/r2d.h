@@ -312,6 +312,8 @@ int r2d_debug_eval(r2d_ctx* ctx, int op, const float* in, float* out, size_t n);
  * scratch that holds them}.
  * rule 6: in {solver items, collision iterations, waves of the workgroup}; out
  * {waves that run a world's program in the one-kernel step}.
+ * rule 7: in {sub-steps, collision iterations}; out {iterations of the programs
+ * of worlds that are slow to plan (0: as the other worlds)}.
  * rule 5: in {chosen variant + 1 (0: none), worlds, bodies of each, whether
  * one is coloured, whether one is warm started, r2d_ctx_set_wide_record}; out
  * {threads of the separate launches' chains, bytes of LDS}.

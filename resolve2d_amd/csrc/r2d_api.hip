@@ -739,8 +739,9 @@ WorldDev make_desc(r2d_world* w)
 }
 
 // the iterations of each program of a call's worlds
-void set_split(StepDev& S, const ChainSplit& c)
+void set_split(StepDev& S, const ChainSplit& c, size_t sub_steps, size_t iters)
 {
+    S.chain_less = chain_less(sub_steps, iters, c.each);
     S.chain_iters = c.each;
     S.chain_rest = c.rest;
 }
@@ -1421,7 +1422,7 @@ int batch_launch(r2d_ctx* c, Batch& b)
     StepDev S = c->S;
     S.nb = (uint32_t)b.N; S.nworlds = (uint32_t)nw; S.nbuckets = (uint32_t)b.B; S.njoints = (uint32_t)b.J;
     S.worlds = c->dworlds;
-    set_split(S, chain_split(b.iters, c->chain_most));
+    set_split(S, chain_split(b.iters, c->chain_most), b.sub, b.iters);
     const Streams ss = c->streams();
     const uint32_t sub = (uint32_t)b.sub, iters = (uint32_t)b.iters;
     auto eager_phase = [&](int ph) { launch_phase(S, ss, ph, b.dt, sub, iters, b.plan); };
@@ -1495,7 +1496,7 @@ int fused_launch(r2d_ctx* c, Batch& b)
     StepDev F = fused_view(c);
     F.nb = (uint32_t)b.N; F.nworlds = (uint32_t)nw; F.nbuckets = (uint32_t)b.B; F.njoints = (uint32_t)b.J;
     F.worlds = c->dworlds;
-    set_split(F, chain_split(b.iters, c->fchain_most));
+    set_split(F, chain_split(b.iters, c->fchain_most), b.sub, b.iters);
     if (c->profiling) {
         // The timing buffers grow rarely and by a lot: a launch that follows a
         // hipMalloc closely can stall all of its waves for several ms at once
@@ -2366,7 +2367,7 @@ R2D_EXPORT int r2d_process_static(r2d_world* w, float dt, size_t sub_steps, size
     WorldDev* ddesc = nullptr;
     static_layout(base, &F, &ddesc);
     F.nb = n; F.nbuckets = tb; F.njoints = nj;
-    set_split(F, chain_split(iters));
+    set_split(F, chain_split(iters), sub_steps, iters);
     // host values the asynchronous uploads read; the call waits for the
     // stream before they go out of scope
     WorldDev d = w->desc;
@@ -2865,6 +2866,9 @@ R2D_EXPORT int r2d_debug_rule(int rule, const uint64_t* in, uint64_t* out)
     }
     case 6:
         out[0] = fused_waves((uint32_t)in[0], chain_split(in[1]).each, (uint32_t)in[2]);
+        return R2D_OK;
+    case 7:
+        out[0] = chain_less(in[0], in[1], chain_split(in[1]).each);
         return R2D_OK;
     case 5: {
         const uint32_t n = (uint32_t)in[2];

@@ -112,6 +112,7 @@ struct WorldChain {
     uint32_t pairs;     // manifolds of two points
     uint32_t flags;     // 1: updateTGSDepth is live; 2: the reference's sums to the letter (a static ordering body,
                         // a normal or an arm that is not finite, a momentum component of -0)
+    uint32_t iters;     // of its program
     uint32_t slots;     // of its program
     uint32_t rest_slots;   // ... and of the shorter one after it
     uint32_t entries;   // of both
@@ -164,6 +165,7 @@ struct StepDev {
     // shorter one that ends a sub-step (0: none), their rows and entries, and
     // planning state when it does not fit LDS
     uint32_t chain_iters, chain_rest;
+    uint32_t chain_less;                   // iterations of the programs of worlds that are slow to plan (0: as the others)
     __host__ __device__ uint32_t chain_room() const { return chain_iters + chain_rest; }
     uint2* prog_rows;                      // [chain_room * cap_i]
     uint32_t* prog_entries;                // [2 * chain_room * cap_i]

@@ -58,6 +58,23 @@ inline ChainSplit chain_split(size_t iters, uint32_t most = CHAIN_ITERS_MAX)
     return ChainSplit{CHAIN_ITERS_ENOUGH, (uint32_t)(iters % CHAIN_ITERS_ENOUGH)};
 }
 
+// Iterations of the programs of worlds that are slow to plan, in a step of one
+// sub-step, which runs what it plans that one time: their largest divisor up
+// to a quarter of them, but two, or one of two (0: as the other worlds).  Slow are plans in
+// global memory and, in the one-kernel step, plans by several waves; one
+// wave's first chain runs behind its planner.  One sub-step of 8 iterations by
+// programs of 8 and of 2, and before there were programs: a disturbed
+// 4,096-body pile of more items than LDS plans 2.75, 1.17 and 2.00 ms a step,
+// 1,000 bodies 521, 355 and 509 us.  (All worlds by such programs: deep ones lose more than their plan
+// costs, a rope of 900 links 1,160 us a step of 4 iterations, then 2,840.)
+inline uint32_t chain_less(size_t sub_steps, size_t iters, uint32_t each)
+{
+    if (sub_steps != 1) return 0u;
+    for (size_t k = iters == 2 ? 1 : iters / 4 < 2 ? 2 : iters / 4; k > 0; --k)
+        if (iters % k == 0) return k < each ? (uint32_t)k : 0u;
+    return 0u;
+}
+
 // Waves that run a world's rows: one for each `rows` rows of 64 its items fill
 // (a pile's chain is 90-150 slots deep for 4 iterations).  In the one-kernel
 // step a slot of several waves costs about two rows of one, so they pay from

@@ -2053,14 +2053,16 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     const uint32_t w = uniform(sh.w), ibase = uniform(sh.ibase), mbeg = uniform(sh.mbeg), nj = uniform(sh.nj),
                    M = uniform(sh.M), base = uniform(sh.base);
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + w);
-    const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, kc = S.chain_iters, room = S.chain_room();
+    const uint32_t t = threadIdx.x, n = (uint32_t)D.nbodies, nit = nj + M, room = S.chain_room();
     const float sub_dt = sh.dt / (float)uniform(sh.sub_steps);
     const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), n, 0u);
     const ChainBodies& C = L.C;
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
-    const uint32_t waves = fused_waves(nit, kc, (uint32_t)T / 64u);
+    const uint32_t waves = fused_waves(nit, S.chain_iters, (uint32_t)T / 64u);
     const bool chain = nit > 0u && sh.iters > 0u;
     const bool plan_in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words;
+    const bool slow = S.chain_less != 0u && (waves > 1u || !plan_in_lds);
+    const uint32_t kc = slow ? S.chain_less : S.chain_iters;
     Program G;
     G.rows = (GU2)(S.prog_rows + (size_t)ibase * room);
     G.entries = (GU32)(S.prog_entries + (size_t)ibase * 2u * room);
@@ -2165,13 +2167,14 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     }
     if (t == 0) {
         sh.nslots = ns;
+        sh.kc = kc;
         if (waves == 1u) sh.entries = entries;
         sh.failed = ns == 0u;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
     __syncthreads();
     if (follow) return true;
-    if (S.chain_rest && chain && !sh.failed) {
+    if (S.chain_rest && chain && !slow && !sh.failed) {
         plan_rest(PlanMemory{L.rest, PG.items, PG.ring, G}, plan_in_lds, nit, nj, kc, S.chain_rest, waves, shl);
         if (sh.rest_slots == 0u) {   // (read by all before the barrier that ends the step)
             if (t == 0) { sh.failed = 1u; S.w_status[w] = WS_STALL; }
@@ -2241,14 +2244,14 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
             __syncthreads();
         }
         if (iters == 0u) continue;
-        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = S.chain_iters, rest_slots = uniform(sh.rest_slots);
+        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = uniform(sh.kc), rest_slots = uniform(sh.rest_slots);
         const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
         const bool in_lds = L.holds(M + uniform(sh.pairs));
         ChainProgram G = chain_program(S, ibase, S.chain_room(), uniform(sh.nslots), iters / kc, nj, M, uniform(sh.pairs));
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
-        const bool several = fused_waves(nj + M, kc, (uint32_t)T / 64u) > 1u;
+        const bool several = fused_waves(nj + M, S.chain_iters, (uint32_t)T / 64u) > 1u;
 #pragma clang loop unroll(disable)
         for (uint32_t left = rest_slots;;) {
             if (several) {
@@ -2359,11 +2362,13 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words,
     const uint32_t w = S.w_order[blockIdx.x];
     const uint32_t ibase = S.w_item_base[w], nit = S.w_item_base[w + 1] - ibase, nj = (uint32_t)S.worlds[w].njoints;
     if (S.w_status[w] != 0 || nit == 0u) return;
-    const uint32_t t = threadIdx.x, kc = rest ? rest : S.chain_iters,
-                   waves = chain_waves(nit, S.chain_iters, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
+    const uint32_t t = threadIdx.x, waves = chain_waves(nit, S.chain_iters, (uint32_t)T / 64u, CHAIN_WAVE_ROWS);
     const size_t rows = (size_t)ibase * S.chain_room() + (rest ? (size_t)S.chain_iters * nit : 0u);
     const uint32_t before = rest ? S.w_chain[w].entries : 0u;
     const bool in_lds = nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= lds_words;
+    const bool slow = S.chain_less != 0u && !in_lds;
+    if (rest && slow) return;   // its programs have no rest
+    const uint32_t kc = rest ? rest : slow ? S.chain_less : S.chain_iters;
     if (t == 0) {
         sh.ready = sh.taken = 0u;
         sh.entries = before;
@@ -2380,8 +2385,8 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words,
     auto start = [&](auto& P, bool init) {
         for (uint32_t j = t; j < nit; j += T) {
             u4v v = items[j];
-            if (rest) v.z = (v.z & ~(STATE_BODY - 1u)) + rest;
-            if (init || rest) P.init(j, v.x, v.y, v.z, v.w);
+            v.z = (v.z & ~(STATE_BODY - 1u)) + kc;
+            if (init || rest || slow) P.init(j, v.x, v.y, v.z, v.w);
             if (v.z < STATE_BODY)
                 P.push(__hip_atomic_fetch_add(&sh.ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
                        P.pack(PlanEntry{j, v.w, v.x, v.y}));
@@ -2398,6 +2403,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words,
         ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
     if (t == 0) {
         if (rest) S.w_chain[w].rest_slots = ns; else S.w_chain[w].slots = ns;
+        if (!rest) S.w_chain[w].iters = kc;
         S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2494,6 +2500,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     if (S.w_status[w] != 0 || nit == 0u) return;
     const WorldDev& D = S.worlds[w];
     const WorldChain W = S.w_chain[w];
+    if (rest && W.rest_slots == 0u) return;
     const uint32_t t = threadIdx.x, nj = (uint32_t)D.njoints, M = nit - nj, mbeg = S.w_man_begin[w], base = D.body_base;
     const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + SPARE);
     const bool m_lds = (uint32_t)D.nbodies <= lds_nmax && mwords <= lds_words;
@@ -2511,7 +2518,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         }
     else if (a_lds)
         for (uint32_t q = t; q < nacc; q += T) acc[q] = accg[q];
-    const uint32_t kc = S.chain_iters;
+    const uint32_t kc = W.iters;
     const GU4 prog = world_records(S, w, ibase);
     const GCU32 entries = (GCU32)world_entries(S, w, ibase);
     const uint32_t jbase = joint_entries(W.entries);
@@ -2559,7 +2566,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         const ChainProgram G{(GCU2)(S.prog_rows + rows), entries, (GCU2)(S.prog_slots + rows), (GCU4)prog,
                              rest ? W.rest_slots : W.slots, rest ? 1u : iters / kc, nj, nacc, jbase + nj, jbase};
         const bool fix = W.flags != 0u;
-        if (chain_waves(nit, kc, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
+        if (chain_waves(nit, S.chain_iters, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
             if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
             else if (m_lds) chain_lds_accg<true, WARM, true>(G, m, nc, accg, fix, sub_dt);
             else chain_glb<true, WARM, true>(G, mom, nc, accg, fix, sub_dt);

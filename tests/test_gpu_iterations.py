@@ -78,3 +78,32 @@ def test_prime_counts_keep_the_overlap():
         assert best(iters) < 5 * four, (iters, best(iters), four)
     w.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("iters", [2, 3, 5, 8, 10, 16, 31])
+@pytest.mark.parametrize("form", ["one-wave", "one-wave-separate", "several-waves-separate", "plan-global-separate",
+                                  "momenta-global-warm", "coloured", "large-fused"])
+def test_one_sub_step(oracle, form, iters):
+    """One sub-step: worlds that are slow to plan run short programs."""
+    from resolve2d_amd.engine import GpuWorld, apply_scene
+    from resolve2d_amd.solver import Context
+    scene, separate, limit, warm, coloured = FORMS.get(form, (("heap", 900, 14.0, 5), False, 0, 0.0, False))
+    ctx = Context(0)
+    ctx.set_lds_limit(limit)
+    ctx.set_fused(not separate)
+    g, o = GpuWorld(ctx), oracle.OracleWorld("f32")
+    for e in (g, o):
+        apply_scene(SCENES[scene[0]](*scene[1:]), e)
+        if warm:
+            e.set_warm_start(warm)
+        if coloured:
+            e.set_schedule(1)
+    for step in range(3):
+        print(f"{form}, {iters} iterations: step {step + 1} of 3", flush=True)
+        assert g.process(DT, 1, iters) == o.process(DT, 1, iters) == 0
+        a, b = g.bodies(), o.bodies()
+        assert bits_equal(a, b), (step, first_diff(a, b))
+        mg, mo = g.manifolds(), o.manifolds()
+        assert mg.shape == mo.shape and bits_equal(mg, mo), (step, first_diff(mg, mo))
+    for e in (g, o, ctx):
+        e.close()

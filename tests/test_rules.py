@@ -139,3 +139,15 @@ def test_more_iterations_do_not_spread_a_small_world(waves):
         assert [rule(6, n, iters, waves)[0] for n in (0, 1, 400, 1536)] == [1] * 4
         assert rule(6, 1600, iters, waves)[0] > 1
     assert rule(6, 3000, 1, waves)[0] == rule(6, 3000, 2, waves)[0] == 1
+
+
+@pytest.mark.parametrize("iters", list(range(1, 70)) + [127, 1009])
+def test_one_sub_step_has_short_programs_for_slow_plans(iters):
+    """A divisor of the iterations, at most a quarter of them or two, shorter
+    than the other worlds' programs; only in steps of one sub-step."""
+    assert rule(7, 0, iters)[0] == rule(7, 2, iters)[0] == rule(7, 4, iters)[0] == 0
+    less = rule(7, 1, iters)[0]
+    if less == 0:   # theirs are that short
+        assert iters != 2 and rule(0, iters)[0] <= max(2, iters // 4)
+    else:
+        assert iters % less == 0 and less <= max(2, iters // 4) and less < rule(0, iters)[0]
