@@ -226,7 +226,7 @@ struct ChainShared {
     // waves that have met (waves_meet)
     uint32_t beside, progress, met;
     uint32_t rest_slots;   // of the program after the others (StepDev::chain_rest)
-    uint32_t kc;           // iterations of the program
+    uint32_t reps, slow;   // runs of the program a sub-step; its world is slow to plan (StepDev::chain_less)
 };
 constexpr uint32_t PLANNED = 0x80000000u;
 

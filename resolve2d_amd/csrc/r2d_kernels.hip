@@ -2167,19 +2167,39 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     }
     if (t == 0) {
         sh.nslots = ns;
-        sh.kc = kc;
+        sh.reps = sh.iters / kc;
+        sh.slow = slow;
         if (waves == 1u) sh.entries = entries;
         sh.failed = ns == 0u;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
     __syncthreads();
-    if (follow) return true;
-    if (S.chain_rest && chain && !slow && !sh.failed) {
-        plan_rest(PlanMemory{L.rest, PG.items, PG.ring, G}, plan_in_lds, nit, nj, kc, S.chain_rest, waves, shl);
-        if (sh.rest_slots == 0u) {   // (read by all before the barrier that ends the step)
-            if (t == 0) { sh.failed = 1u; S.w_status[w] = WS_STALL; }
-            __syncthreads();
-            return false;
+    return follow;
+}
+
+// Between plan and first chain, where that has not run behind the planner: the
+// program for the rest of the iterations, and the impulses at zero.
+// A function of its own: in the planner's it costs every step 1.5 %.
+template <int T>
+__device__ __attribute__((noinline)) void chain_ready(StepArgs KS, LU32 smem, R2D_LDS ChainShared* shl)
+{
+    const StepDev& S = *(const StepDev*)uniform_ptr(KS);
+    ChainShared& sh = *(ChainShared*)uniform_lds(shl);
+    const uint32_t w = uniform(sh.w), ibase = uniform(sh.ibase), nj = uniform(sh.nj), M = uniform(sh.M), nit = nj + M,
+                   t = threadIdx.x, nacc = M + uniform(sh.pairs);
+    const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + w);
+    const ChainLds L(uniform_lds(smem), uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, 0u);
+    const GU4 ring = (GU4)(S.plan_ring + 2 * (size_t)ibase);
+    if (S.chain_rest && !uniform(sh.slow) && nit > 0u && sh.iters > 0u) {
+        const uint32_t room = S.chain_room(), waves = fused_waves(nit, S.chain_iters, (uint32_t)T / 64u);
+        const Program G{(GU2)(S.prog_rows + (size_t)ibase * room), (GU32)(S.prog_entries + (size_t)ibase * 2u * room),
+                        (GU2)(S.prog_slots + (size_t)ibase * room)};
+        plan_rest(PlanMemory{L.rest, (GU4)(S.plan_items + 2 * (size_t)ibase), ring, G},
+                  nit <= PLAN_MAX_ITEMS && plan_lds_words(nit, waves) <= L.rest_words, nit, nj, S.chain_iters, S.chain_rest,
+                  waves, shl);
+        if (t == 0 && sh.rest_slots == 0u) {
+            sh.failed = 1u;
+            S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
         }
     }
     // accumulated impulses (normal, tangential) of the contact points, by
@@ -2187,10 +2207,10 @@ __device__ __attribute__((noinline)) bool chain_prepare(StepArgs KS, LU32 smem, 
     if (L.holds(nacc)) {
         for (uint32_t q = t; q < nacc; q += T) L.acc[q] = f2v{0.f, 0.f};
     } else {
-        GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
+        GF2 accg = (GF2)ring;
         for (uint32_t q = t; q < nacc; q += T) accg[q] = f2v{0.f, 0.f};
     }
-    return false;
+    __syncthreads();
 }
 
 // the impulses -> the step's manifold arrays (what r2d_get_manifolds reports)
@@ -2230,11 +2250,15 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
     ChainShared& sh = *(ChainShared*)shl;
     const bool first = uniform(chain_prepare<T, WARM>(KS, smem, shl)) != 0u;
     if (sh.failed) return;
+    if (!first) {   // else the first chain has run behind the planner
+        chain_ready<T>(KS, smem, shl);
+        if (sh.failed) return;
+    }
     const StepDev& S = *(const StepDev*)KS;
     const WorldDev& D = *(const WorldDev*)(WorldArgs)(S.worlds + uniform(sh.w));
     const uint32_t sub_steps = uniform(sh.sub_steps), iters = uniform(sh.iters), nj = uniform(sh.nj);
     const bool any = nj + sh.M > 0u, items = nj || sh.live || (WARM && D.warm > 0.0f);
-    for (uint32_t s = first ? 1u : 0u;; ++s) {   // the first chain may have run behind the planner
+    for (uint32_t s = first ? 1u : 0u;; ++s) {
         chain_bodies<T, WARM>(KS, smem, shl, s, 0u);
         if (s == sub_steps) break;
         __syncthreads();
@@ -2244,16 +2268,16 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
             __syncthreads();
         }
         if (iters == 0u) continue;
-        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase), kc = uniform(sh.kc), rest_slots = uniform(sh.rest_slots);
+        const uint32_t M = uniform(sh.M), ibase = uniform(sh.ibase);
         const ChainLds L(smem, uniform(sh.free_at), uniform(sh.free_words), (uint32_t)D.nbodies, uniform(sh.beside));
         const bool in_lds = L.holds(M + uniform(sh.pairs));
-        ChainProgram G = chain_program(S, ibase, S.chain_room(), uniform(sh.nslots), iters / kc, nj, M, uniform(sh.pairs));
+        ChainProgram G = chain_program(S, ibase, S.chain_room(), uniform(sh.nslots), uniform(sh.reps), nj, M, uniform(sh.pairs));
         GF2 accg = (GF2)(S.plan_ring + 2 * (size_t)ibase);
         const float sub_dt = sh.dt / (float)sub_steps;
         const bool fix = (uniform(sh.fix) | uniform(sh.live)) != 0u;
         const bool several = fused_waves(nj + M, S.chain_iters, (uint32_t)T / 64u) > 1u;
 #pragma clang loop unroll(disable)
-        for (uint32_t left = rest_slots;;) {
+        for (uint32_t left = S.chain_rest ? uniform(sh.rest_slots) : 0u;;) {
             if (several) {
                 if (in_lds) chain_lds<true, WARM, false>(G, L.C.m, L.n, L.acc, fix, sub_dt);
                 else chain_lds_accg<true, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
@@ -2262,7 +2286,7 @@ __device__ __forceinline__ void chain_world(StepArgs KS, LU32 smem, R2D_LDS Chai
                 else chain_lds_accg<false, WARM, false>(G, L.C.m, L.n, accg, fix, sub_dt);
             }
             if (left == 0u) break;
-            G = rest_program(G, kc * (nj + M), left);
+            G = rest_program(G, S.chain_iters * (nj + M), left);
             left = 0u;
         }
         __syncthreads();
