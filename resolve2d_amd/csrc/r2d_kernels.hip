@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 
 #include "r2d_device.h"
 #include "r2d_chain.h"
@@ -3158,11 +3159,11 @@ uint32_t fused_threads(int v)
 // loops stride by MAXT): set_solve_smem_limit checks each against the width
 // it would be launched with, and a mismatch leaves the variant without one
 static bool g_fused_width_ok[SOLVE_TABLE];
-static uint32_t g_fused_groups[SOLVE_TABLE];
+static std::atomic<uint32_t> g_fused_groups[SOLVE_TABLE];   // asked once: the same for every context
 
 uint32_t fused_groups(int v)
 {
-    return std::max(1u, g_fused_groups[v]);
+    return std::max(1u, g_fused_groups[v].load(std::memory_order_relaxed));
 }
 
 bool fused_available(int v)
@@ -3402,9 +3403,10 @@ void set_solve_smem_limit()
             g_fused_width_ok[v] = hipFuncGetAttributes(&fa, (const void*)kSolveVariants[v].fused_fn) == hipSuccess &&
                                   fa.maxThreadsPerBlock == (int)fused_threads(v);
             int groups = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, (const void*)kSolveVariants[v].fused_fn,
+            if (g_fused_groups[v].load(std::memory_order_relaxed) == 0u &&
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, (const void*)kSolveVariants[v].fused_fn,
                                                              (int)fused_threads(v), 0) == hipSuccess)
-                g_fused_groups[v] = (uint32_t)std::max(groups, 1);
+                g_fused_groups[v].store((uint32_t)std::max(groups, 1), std::memory_order_relaxed);
         }
     }
     (void)hipGetLastError();   // a refused attribute is not an error of a later call
