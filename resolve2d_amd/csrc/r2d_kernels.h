@@ -34,11 +34,10 @@ constexpr int SOLVE_TABLE = SOLVE_VARIANTS + 2;
 // often), else 4, with a program of its own for the rest (17 = 4 x 4 + 1).  A
 // program's size grows with the iterations it covers, and what a program
 // covers runs overlapped: an iteration by itself costs the whole depth of the
-// world's contacts.  Four are enough for that (ms a step of 16 iterations by
-// programs of 1 / 4 / 8 / 16: 20-row pyramid 2.18 / 0.79 / 0.62 / 0.95, 60
-// rows 10.0 / 4.7 / 3.4 / 2.7, world of 387 bodies 0.58 / 0.61 / 0.64 / 0.99,
-// 97 worlds 0.78 / 0.80 / 1.09 / 1.34, 4,096-body pile 1.47 / 1.24 / 1.33 /
-// 1.54).  17 iterations, one at a time and by fours: pyramids of 20 and 60
+// world's contacts.  Four take most of that away (ms a step of 16 iterations by
+// programs of 1 / 4 / 16: 20-row pyramid 2.18 / 0.79 / 0.51, 60 rows 10.0 /
+// 4.7 / 2.7, world of 387 bodies 0.58 / 0.61 / 0.60, 97 worlds 0.78 / 0.80 /
+// 0.80, 4,096-body pile 1.47 / 1.24 / 1.54).  17 iterations, one at a time and by fours: pyramids of 20 and 60
 // rows 2.29 -> 0.96 and 9.5 -> 5.2 ms, 4,096-body pile 1.43 -> 1.34; shallow
 // worlds pay for planning more, 387 bodies 0.61 -> 0.65, 97 worlds 0.79 -> 0.88.
 constexpr uint32_t CHAIN_ITERS_MAX = 16, CHAIN_ITERS_ENOUGH = 4;
@@ -60,13 +59,14 @@ inline ChainSplit chain_split(size_t iters, uint32_t most = CHAIN_ITERS_MAX)
 
 // Iterations of the programs of worlds that are slow to plan, in a step of one
 // sub-step, which runs what it plans that one time: their largest divisor up
-// to a quarter of them, but two, or one of two (0: as the other worlds).  Slow are plans in
-// global memory and, in the one-kernel step, plans by several waves; one
-// wave's first chain runs behind its planner.  One sub-step of 8 iterations by
-// programs of 8 and of 2, and before there were programs: a disturbed
-// 4,096-body pile of more items than LDS plans 2.75, 1.17 and 2.00 ms a step,
-// 1,000 bodies 521, 355 and 509 us.  (All worlds by such programs: deep ones lose more than their plan
-// costs, a rope of 900 links 1,160 us a step of 4 iterations, then 2,840.)
+// to a quarter of them (up to two, of three to eleven; one, of two), or 0: as
+// the other worlds.  Slow are plans in global memory and, in the one-kernel
+// step, plans by several waves; one wave's first chain runs behind its planner.
+// One sub-step of 8 iterations by programs of 8 and of 2, and before there were
+// programs: a disturbed 4,096-body pile of more items than LDS plans 2.75, 1.18
+// and 2.00 ms a step, 1,000 bodies 521, 355 and 509 us.  (All worlds by such
+// programs: deep ones lose more than their plan costs, a rope of 900 links
+// 1,160 us a step of 4 iterations, then 2,840.)
 inline uint32_t chain_less(size_t sub_steps, size_t iters, uint32_t each)
 {
     if (sub_steps != 1) return 0u;
