@@ -112,7 +112,7 @@ struct WorldChain {
     uint32_t pairs;     // manifolds of two points
     uint32_t flags;     // 1: updateTGSDepth is live; 2: the reference's sums to the letter (a static ordering body,
                         // a normal or an arm that is not finite, a momentum component of -0)
-    uint32_t iters;     // of its program
+    uint32_t reps;      // runs of its program a sub-step
     uint32_t slots;     // of its program
     uint32_t rest_slots;   // ... and of the shorter one after it
     uint32_t entries;   // of both

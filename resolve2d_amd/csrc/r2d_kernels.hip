@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "r2d_device.h"
 #include "r2d_chain.h"
@@ -2379,7 +2380,7 @@ __global__ __launch_bounds__(256) void k_chain_build(StepDev S, float sub_dt)
 // chain_iters * nit on, its entries after the others.  (Planned through, every
 // item waits for what it waited for at first.)
 template <int T>
-__global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words, uint32_t rest)
+__global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t iters, uint32_t lds_words, uint32_t rest)
 {
     extern __shared__ __align__(16) uint32_t smem[];
     __shared__ ChainShared sh;
@@ -2428,7 +2429,7 @@ __global__ __launch_bounds__(T) void k_chain_plan(StepDev S, uint32_t lds_words,
         ns = in_lds ? plan_single(PL, G, nit, nj, kc, ready, entries) : plan_single(PG, G, nit, nj, kc, ready, entries);
     if (t == 0) {
         if (rest) S.w_chain[w].rest_slots = ns; else S.w_chain[w].slots = ns;
-        if (!rest) S.w_chain[w].iters = kc;
+        if (!rest) S.w_chain[w].reps = iters / kc;
         S.w_chain[w].entries = waves > 1u ? sh.entries : entries;
         if (ns == 0u) S.w_status[w] = WS_STALL;   // corrupt ordering data: the world stops
     }
@@ -2509,14 +2510,14 @@ __global__ __launch_bounds__(256) void k_chain_bodies(StepDev S, uint32_t s, uin
 }
 
 // Sub-step s's joint records, moved contact points and carried impulses, and
-// its iterations, one workgroup per world; with `rest`, in a launch after it,
-// only the iterations that end the sub-step (a loop over both programs in one
-// launch cost those without a rest 3 us a step of a 4,096-body pile).  Momenta in LDS for worlds of at
-// most lds_nmax bodies whose places fit it, and beside them the impulses when
-// they fit too; otherwise they stay in global memory.
-template <int T, bool WARM>
+// its iterations, one workgroup per world; REST, in a launch after it, only
+// the iterations that end the sub-step (told apart at run time they cost those
+// without a rest 0.5 us of 30.6 a launch, coloured pile of 4,096 bodies).  Momenta in LDS for worlds of
+// at most lds_nmax bodies whose places fit it, and beside them the impulses
+// when they fit too; otherwise they stay in global memory.
+template <int T, bool WARM, bool REST>
 __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t iters, float sub_dt, uint32_t lds_words,
-                                                 uint32_t lds_nmax, uint32_t rest)
+                                                 uint32_t lds_nmax)
 {
     extern __shared__ __align__(16) uint32_t smem[];
     if (S.counters[C_OVERFLOW]) return;
@@ -2525,7 +2526,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     if (S.w_status[w] != 0 || nit == 0u) return;
     const WorldDev& D = S.worlds[w];
     const WorldChain W = S.w_chain[w];
-    if (rest && W.rest_slots == 0u) return;
+    if (REST && W.rest_slots == 0u) return;
     const uint32_t t = threadIdx.x, nj = (uint32_t)D.njoints, M = nit - nj, mbeg = S.w_man_begin[w], base = D.body_base;
     const uint32_t nc = W.bodies, nacc = M + W.pairs, mwords = 4u * (nc + SPARE);
     const bool m_lds = (uint32_t)D.nbodies <= lds_nmax && mwords <= lds_words;
@@ -2537,25 +2538,24 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     u4v* recs = reinterpret_cast<u4v*>(S.recs + (size_t)ibase * 8);
     if (m_lds)
         for (uint32_t c = t; c < nc; c += T) m[c] = mom[c];
-    if (s == 0u && !rest)
+    if (s == 0u && !REST)
         for (uint32_t q = t; q < nacc; q += T) {
             if (a_lds) acc[q] = f2v{0.f, 0.f}; else accg[q] = f2v{0.f, 0.f};
         }
     else if (a_lds)
         for (uint32_t q = t; q < nacc; q += T) acc[q] = accg[q];
-    const uint32_t kc = W.iters;
     const GU4 prog = world_records(S, w, ibase);
     const GCU32 entries = (GCU32)world_entries(S, w, ibase);
     const uint32_t jbase = joint_entries(W.entries);
     const GlobalPoses C = global_poses(D);
-    for (uint32_t j = t; j < nj && iters > 0u && !rest; j += T) {
+    for (uint32_t j = t; j < nj && iters > 0u && !REST; j += T) {
         u4v q[4];
         joint_record(q, D.joints[j], D, C, s == 0u, [&](uint32_t x) { return S.cmap[base + x]; });
         const GU4 to = prog + entry_at(jbase + j);
         for (int p = 0; p < 4; ++p) to[p * ENTRY_WORD] = q[p];
     }
     __syncthreads();
-    if ((W.flags & 1u) && !rest) {
+    if ((W.flags & 1u) && !REST) {
         for (uint32_t q = t; q < M; q += T) {
             const uint32_t p1 = S.it_k0[ibase + nj + q];
             point_tgs(S, D, recs, C, mbeg + q, base, nj + q, p1, sub_dt, [&](int p) {
@@ -2570,7 +2570,7 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
         }
     }
     if constexpr (WARM) {
-        if (D.warm > 0.0f && !rest) {
+        if (D.warm > 0.0f && !REST) {
             const size_t cm = S.cap_m;
             for (uint32_t q = t; q < M; q += T) {
                 // warm starting: the carried impulse per sub-step joins the accumulators
@@ -2587,9 +2587,9 @@ __global__ __launch_bounds__(T) void k_chain_run(StepDev S, uint32_t s, uint32_t
     }
     __syncthreads();
     if (iters > 0u) {
-        const size_t rows = (size_t)ibase * S.chain_room() + (rest ? (size_t)kc * nit : 0u);
+        const size_t rows = (size_t)ibase * S.chain_room() + (REST ? (size_t)S.chain_iters * nit : 0u);
         const ChainProgram G{(GCU2)(S.prog_rows + rows), entries, (GCU2)(S.prog_slots + rows), (GCU4)prog,
-                             rest ? W.rest_slots : W.slots, rest ? 1u : iters / kc, nj, nacc, jbase + nj, jbase};
+                             REST ? W.rest_slots : W.slots, REST ? 1u : W.reps, nj, nacc, jbase + nj, jbase};
         const bool fix = W.flags != 0u;
         if (chain_waves(nit, S.chain_iters, (uint32_t)T / 64u, CHAIN_WAVE_ROWS) > 1u) {
             if (a_lds) chain_lds<true, WARM, true>(G, m, nc, acc, fix, sub_dt);
@@ -3344,11 +3344,11 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
             tmark(ss, "k_chain_build", st);
             if (iters > 0) {
                 hipLaunchKernelGGL(width(k_chain_plan<CHAIN_NARROW>, k_chain_plan<CHAIN_THREADS>, k_chain_plan<CHAIN_COLORED>),
-                                   dim3(S.nworlds), dim3(T), sp.lds, st, S, words, 0u);
+                                   dim3(S.nworlds), dim3(T), sp.lds, st, S, iters, words, 0u);
                 tmark(ss, "k_chain_plan", st);
                 if (S.chain_rest) {
                     hipLaunchKernelGGL(width(k_chain_plan<CHAIN_NARROW>, k_chain_plan<CHAIN_THREADS>, k_chain_plan<CHAIN_COLORED>),
-                                       dim3(S.nworlds), dim3(T), sp.lds, st, S, words, S.chain_rest);
+                                       dim3(S.nworlds), dim3(T), sp.lds, st, S, iters, words, S.chain_rest);
                     tmark(ss, "k_chain_plan (rest)", st);
                 }
             }
@@ -3359,15 +3359,16 @@ void launch_phase(const StepDev& S, const Streams& ss, int phase, float dt, uint
                                dim3(BS), 0, st, S, s, sub_steps, sub_dt);
             tmark(ss, "k_chain_bodies", st);
             if (s == sub_steps) break;
-            auto run = width(pick(k_chain_run<CHAIN_NARROW, true>, k_chain_run<CHAIN_NARROW, false>),
-                             pick(k_chain_run<CHAIN_THREADS, true>, k_chain_run<CHAIN_THREADS, false>),
-                             k_chain_run<CHAIN_COLORED, false>);
-            hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax, 0u);
-            tmark(ss, "k_chain_run", st);
-            if (S.chain_rest && iters > 0u) {
-                hipLaunchKernelGGL(run, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax, S.chain_rest);
-                tmark(ss, "k_chain_run (rest)", st);
-            }
+            auto run = [&](auto rest, const char* name) {
+                constexpr bool REST = decltype(rest)::value;
+                auto f = width(pick(k_chain_run<CHAIN_NARROW, true, REST>, k_chain_run<CHAIN_NARROW, false, REST>),
+                               pick(k_chain_run<CHAIN_THREADS, true, REST>, k_chain_run<CHAIN_THREADS, false, REST>),
+                               k_chain_run<CHAIN_COLORED, false, REST>);
+                hipLaunchKernelGGL(f, dim3(S.nworlds), dim3(T), sp.lds, st, S, s, iters, sub_dt, words, sp.lds_nmax);
+                tmark(ss, name, st);
+            };
+            run(std::false_type{}, "k_chain_run");
+            if (S.chain_rest && iters > 0u) run(std::true_type{}, "k_chain_run (rest)");
         }
         if (sp.any_warm) {
             hipLaunchKernelGGL(k_warm_clear, dim3(blocks_for(S.nb, BS)), dim3(BS), 0, st, S);
@@ -3391,11 +3392,16 @@ void set_solve_smem_limit()
     allow((const void*)k_chain_plan<CHAIN_THREADS>);
     allow((const void*)k_chain_plan<CHAIN_NARROW>);
     allow((const void*)k_chain_plan<CHAIN_COLORED>);
-    allow((const void*)k_chain_run<CHAIN_COLORED, false>);
-    allow((const void*)k_chain_run<CHAIN_THREADS, false>);
-    allow((const void*)k_chain_run<CHAIN_THREADS, true>);
-    allow((const void*)k_chain_run<CHAIN_NARROW, false>);
-    allow((const void*)k_chain_run<CHAIN_NARROW, true>);
+    auto chains = [&](auto rest) {
+        constexpr bool REST = decltype(rest)::value;
+        allow((const void*)k_chain_run<CHAIN_COLORED, false, REST>);
+        allow((const void*)k_chain_run<CHAIN_THREADS, false, REST>);
+        allow((const void*)k_chain_run<CHAIN_THREADS, true, REST>);
+        allow((const void*)k_chain_run<CHAIN_NARROW, false, REST>);
+        allow((const void*)k_chain_run<CHAIN_NARROW, true, REST>);
+    };
+    chains(std::false_type{});
+    chains(std::true_type{});
     for (int v = 0; v < SOLVE_TABLE; ++v) {
         if (kSolveVariants[v].fused_fn) {
             allow((const void*)kSolveVariants[v].fused_fn);
