@@ -533,10 +533,12 @@ size_t read_bytes(const r2d_world* w) { return (size_t)__builtin_popcount(read_f
 
 // The bodies of w, and with them those of further worlds of its batch: worlds
 // read in even steps (every one, every tenth, backwards) are fetched ahead,
-// twice as many each time, so that reading a whole batch takes few round trips
-// and no read fetches more than the reads before it did.  A world out of step
-// is copied by itself (14 us; by the kernel 18) until READ_ODD of them show
-// that many are wanted.  (Fetching the worlds that follow whatever the steps
+// twice as many each time (neighbours from the second read on, others from the
+// third: one more round trip, 15 us of 230 for 21 piles), so that reading a
+// whole batch takes few round trips and no read fetches more than one world
+// beyond what the reads before it did.  A world out of step is copied by itself
+// (14 us; by the kernel 18) until READ_ODD of them show that many are wanted.
+// (Fetching the worlds that follow whatever the steps
 // were: 16 of 600 worlds evenly spaced 514 us and at random 682, by copies 250
 // and 255, like this 131 and 245; all 600 2.2 ms, backwards 12.0, by copies
 // 9.2, like this 2.2 either way.)
@@ -565,8 +567,9 @@ int download_bodies(r2d_world* w)
         } else {
             c->read_odd += 1;
             const bool many = c->read_odd > READ_ODD;
-            c->read_run = many ? std::min<uint32_t>(1u << std::min(c->read_odd - READ_ODD, 16u), (uint32_t)(kReadTable / sizeof(ReadItem))) : 1;
             c->read_stride = many ? 1 : c->read_last < 0 ? 0 : at - c->read_last;
+            c->read_run = many ? std::min<uint32_t>(1u << std::min(c->read_odd - READ_ODD, 16u), (uint32_t)(kReadTable / sizeof(ReadItem)))
+                               : c->read_stride == 1 || c->read_stride == -1 ? 2 : 1;
         }
         int64_t i = at + c->read_stride;
         for (; c->read_stride && i >= 0 && i < worlds && cnt < c->read_run; i += c->read_stride) {
